@@ -171,9 +171,12 @@ int launch_table_reorder(int precision, long count, const void* src, void* dst, 
                          hipStream_t s);
 
 // power series: one Horner stage  u_out = psi + (-i dt / n) H u_in
-int launch_horner_pair(int precision, int batch, int nx, int ny, int nz, const void* u_in, void* u_out,
-                       const void* psi, const float2* V, double c1, double c2, double inv_2m, double inv_dx2,
-                       int variant, hipStream_t s);
+// stages (2 .. horner_chain_stages) consecutive Horner stages in one launch, time-step factors
+// c[0] .. c[stages - 1]; u_out must alias neither u_in nor psi
+int horner_chain_stages(int precision);
+int launch_horner_chain(int precision, int stages, int batch, int nx, int ny, int nz, const void* u_in, void* u_out,
+                        const void* psi, const float2* V, const double* c, double inv_2m, double inv_dx2,
+                        hipStream_t s);
 int launch_horner_stage(int precision, int batch, int nx, int ny, int nz, const void* u_in, void* u_out,
                         const void* psi, const float2* V, double dt_over_n, double inv_2m, double inv_dx2,
                         int tile_x, hipStream_t s);

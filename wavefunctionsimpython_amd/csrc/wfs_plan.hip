@@ -21,6 +21,7 @@ struct wfs_plan {
   void* kfull[3];         // exp(-i k_d^2 dt / 2m) / N_d, state precision, ntab copies
   void* khalf[3];         // exp(-i k_d^2 dt / 4m) / N_d, state precision, ntab copies
   void* scratch[2];       // power-series ping-pong buffers (lazy)
+  void* state2;           // power series: a second state (lazy, calls of several steps)
   double* obs_work;       // observable partial records
   long obs_work_len;
   double* plane_work;     // plane-current partial records (grown on demand)
@@ -202,6 +203,17 @@ int ensure_scratch(wfs_plan* p, hipStream_t s) {
     if (e != hipSuccess) { set_last_error("hipMalloc(%zu) for power-series scratch failed", bytes); return WFS_ERR_ALLOC; }
   }
   return 0;
+}
+
+// The power series' third buffer (a second state for calls of several steps), or null where it
+// cannot be had: under capture before a call has made it, or without the memory for it.
+void* ensure_state_buffer(wfs_plan* p, hipStream_t s) {
+  if (!p->state2 && !capturing(s) &&
+      hipMalloc(&p->state2, size_t(p->batch) * p->n[0] * p->n[1] * p->n[2] * p->elem) != hipSuccess) {
+    (void)hipGetLastError();
+    p->state2 = nullptr;
+  }
+  return p->state2;
 }
 
 // Timing of the launches of one kernel class when profiling is on: the launches made through
@@ -613,40 +625,57 @@ int fourier_steps(wfs_plan* p, void* psi, const void* V, int nsteps, hipStream_t
 int steps_observed(wfs_plan* p, void* psi, const void* V, int nsteps, int every, const wfs_box* boxes, int nb,
                    double* out, hipStream_t s, wfs_between_steps between = nullptr, void* ctx = nullptr);
 
+// one power-series step, psi -> out (out may be psi).  Horner stages n = order .. 1 run fused, up
+// to horner_chain_stages at a time (WFS_K_HORNER variant 2: pairs, 0: one launch per stage), all
+// with the same bits.  A fused launch reads psi around its tile and so never writes psi: where out
+// is psi, a last single stage writes it (16 B per point less than a copy of the result would add
+// to one more fused stage), else the last result is copied.
+int power_series_step(wfs_plan* p, const void* psi, void* out, const float2* V, hipStream_t s) {
+  const double inv_2m = 1.0 / (2.0 * p->mass);
+  const double inv_dx2 = 1.0 / (p->dx[0] * p->dx[0]);   // x spacing on every axis (power_series_operator.cu:58)
+  const int most = p->variant[WFS_K_HORNER] == 0 ? 1
+                   : p->variant[WFS_K_HORNER] == 2 ? 2 : horner_chain_stages(p->precision);
+  const bool in_place = out == psi;
+  const void* u_in = psi;
+  int which = 0;
+  int nn = p->order;
+  while (nn >= 1) {
+    // of the nn stages left: as many as fit; 3 + 1 as 2 + 2 where the last may not be alone anyway
+    int m = std::min(most, nn);
+    if (m == 3 && nn == 4 && !in_place) m = 2;
+    const bool last = m == nn;
+    void* dst = p->scratch[which];
+    if (last && (!in_place || (m == 1 && u_in != psi))) dst = out;
+    ProfileScope scope(p, WFS_K_HORNER, s);
+    if (m == 1) {
+      WFS_TRY(launch_horner_stage(p->precision, p->batch, p->n[0], p->n[1], p->n[2], u_in, dst, psi, V,
+                                  p->dt / double(nn), inv_2m, inv_dx2, 0, s));
+    } else {
+      const double c[3] = {p->dt / double(nn), p->dt / double(nn - 1), nn > 2 ? p->dt / double(nn - 2) : 0.0};
+      WFS_TRY(launch_horner_chain(p->precision, m, p->batch, p->n[0], p->n[1], p->n[2], u_in, dst, psi, V, c, inv_2m,
+                                  inv_dx2, s));
+    }
+    u_in = dst;
+    nn -= m;
+    which ^= 1;
+  }
+  if (u_in != out) WFS_HIP_CHECK(hipMemcpyAsync(out, u_in, grid_points(p) * p->elem, hipMemcpyDeviceToDevice, s));
+  return 0;
+}
+
 int power_series_steps(wfs_plan* p, void* psi, const void* V, int nsteps, hipStream_t s) {
   if (!V) { set_last_error("wfs_step: the power series needs V"); return WFS_ERR_INVALID; }
   WFS_TRY(ensure_scratch(p, s));
-  const double inv_2m = 1.0 / (2.0 * p->mass);
-  const double inv_dx2 = 1.0 / (p->dx[0] * p->dx[0]);   // x spacing on every axis (power_series_operator.cu:58)
-  const size_t bytes = grid_points(p) * p->elem;
-  // variant 1 (default): stages in fused pairs; variant 0: one launch per stage.  Both give
-  // the same bits.  A pair reads psi around its tile, so it never writes psi in place; the
-  // result of the last pair is copied back, a last single stage writes psi directly.
-  const bool pairs = p->variant[WFS_K_HORNER] != 0;
-  for (int step = 0; step < nsteps; ++step) {
-    const void* u_in = psi;
-    int which = 0;
-    int nn = p->order;
-    while (nn >= 1) {
-      ProfileScope scope(p, WFS_K_HORNER, s);
-      if (pairs && nn >= 2) {
-        void* out = p->scratch[which];
-        WFS_TRY(launch_horner_pair(p->precision, p->batch, p->n[0], p->n[1], p->n[2], u_in, out, psi,
-                                   static_cast<const float2*>(V), p->dt / double(nn), p->dt / double(nn - 1),
-                                   inv_2m, inv_dx2, p->variant[WFS_K_HORNER], s));
-        u_in = out;
-        nn -= 2;
-      } else {
-        void* out = (nn == 1 && u_in != psi) ? psi : p->scratch[which];
-        WFS_TRY(launch_horner_stage(p->precision, p->batch, p->n[0], p->n[1], p->n[2], u_in, out, psi,
-                                    static_cast<const float2*>(V), p->dt / double(nn), inv_2m, inv_dx2, 0, s));
-        u_in = out;
-        nn -= 1;
-      }
-      which ^= 1;
-    }
-    if (u_in != psi) WFS_HIP_CHECK(hipMemcpyAsync(psi, u_in, bytes, hipMemcpyDeviceToDevice, s));
+  const float2* v = static_cast<const float2*>(V);
+  // steps two at a time go psi -> a third buffer -> psi, so that neither ends in a copy (256^3,
+  // order 10: 47 of 610 us per step); an odd last step, or a call without that buffer, in place
+  void* other = nsteps > 1 ? ensure_state_buffer(p, s) : nullptr;
+  int step = 0;
+  for (; other && step + 1 < nsteps; step += 2) {
+    WFS_TRY(power_series_step(p, psi, other, v, s));
+    WFS_TRY(power_series_step(p, other, psi, v, s));
   }
+  for (; step < nsteps; ++step) WFS_TRY(power_series_step(p, psi, psi, v, s));
   return 0;
 }
 
@@ -669,6 +698,7 @@ extern "C" int wfs_plan_destroy(wfs_plan* p) {
   }
   for (int i = 0; i < 2; ++i)
     if (p->scratch[i]) (void)hipFree(p->scratch[i]);
+  if (p->state2) (void)hipFree(p->state2);
   if (p->obs_work) (void)hipFree(p->obs_work);
   if (p->plane_work) (void)hipFree(p->plane_work);
   if (p->plane_out) (void)hipFree(p->plane_out);
@@ -721,9 +751,6 @@ extern "C" int wfs_plan_create_batched(const int n[3], const double dx[3], doubl
   p->elem = precision == WFS_C128 ? 16 : 8;
   p->ntab = precision == WFS_C128 ? 1 : kDither;
   for (int k = 0; k < WFS_K_COUNT; ++k) p->variant[k] = 1;
-  // fused stage pairs: 8 x 128 tiles where the z axis fills them (measured fastest at 256^3),
-  // else 16 x 64
-  p->variant[WFS_K_HORNER] = p->n[2] >= 256 ? 5 : p->n[2] >= 128 ? 4 : 1;
   // fused plane pass where the plane fits in LDS; at 128^2 two rounds (two blocks per CU) once
   // there are enough planes to fill the CUs twice over (measured: 1024 planes 13% faster, 128
   // planes 11% slower)

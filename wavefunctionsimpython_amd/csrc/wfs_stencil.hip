@@ -82,255 +82,325 @@ __global__ __launch_bounds__(TZ* TY) void horner_stage_kernel(const cx<R>* __res
   }
 }
 
-// Two Horner stages in one pass (temporal blocking): w = psi + (-i c1) H u, then
-// u_out = psi + (-i c2) H w.  A block owns a TY x TZ (y, z) tile and marches along x
-// through a slab; the LDS holds three x planes of u with a two-point (y, z) halo and
-// three planes of w with a one-point halo.  Per output point it moves about 37 B per two
-// stages (u with halo, psi and V, u_out) instead of 2 x 32.  Faces replicate the edge
-// voxel as in the single stage: w outside the grid is a copy of w at the clamped voxel,
-// and out-of-grid u cells hold u at the clamped voxel.  w is rounded to the state
-// precision exactly as the single stage stores it, so the result equals two single stages
-// bit for bit.  u_out must not alias psi or u_in (other blocks read their halos).
-template <typename R, int TZ, int TY, int NT>
-__global__ __launch_bounds__(NT) void horner2_kernel(const cx<R>* __restrict__ u_in, cx<R>* __restrict__ u_out,
-                                                     const cx<R>* __restrict__ psi, const float2* __restrict__ V,
-                                                     int nx, int ny, int nz, R c1, R c2, R inv_2m, R inv_dx2,
-                                                     int tile_x, int ntiles) {
-  using C = cx<R>;
-  constexpr int UY = TY + 4, UZ = TZ + 4;   // u window (halo 2)
-  constexpr int WY = TY + 2, WZ = TZ + 2;   // w window (halo 1)
-  constexpr int RU = (UY * UZ + NT - 1) / NT;   // u cells per thread
-  constexpr int RW = (WY * WZ + NT - 1) / NT;   // w cells per thread
-  __shared__ C su[3][UY][UZ];
-  __shared__ C sw[3][WY][WZ];
+// S Horner stages in one pass (temporal blocking): w_1 = psi + (-i c_1) H u, w_2 = psi +
+// (-i c_2) H w_1, ..., u_out = w_S.  A block owns a window of uy x w (y, z) cells -- its output
+// tile and a halo of S cells on every side that is not a grid face -- and marches along x.  A
+// thread owns a strip of RC rows at one column.  While plane t of u arrives, stage s works on
+// plane t - s, so the stages of an iteration read only what earlier iterations left behind:
+//   - level s - 1 (u is level 0) holds its plane t - s in one LDS buffer and plane t - s - 1 in the
+//     other, which this iteration overwrites: one barrier a plane;
+//   - a cell's z neighbours, its centre and its previous plane come from LDS, the y neighbours
+//     inside the strip from the thread's own centres, only the rows above and below it from LDS;
+//   - the next plane of level s - 1 is the thread's own, computed by stage s - 1 just before (or
+//     loaded an iteration ahead for u);
+//   - psi and V of a cell are read once, one iteration ahead, and stay in registers for S planes
+//     (three slots, the loop unrolled by three so that nothing is moved).
+// Faces: a neighbour outside the grid is the voxel itself (the reference's clamped index): an LDS
+// position chosen once for z and for the strip's ends, a copy of the edge row for a face inside a
+// strip, the centre for x.  Cells outside the window's valid part compute values that nothing
+// reads.  Each stage rounds as the single-stage kernel does, so the result equals S single stages
+// bit for bit.  u_out must alias neither psi nor u_in (other blocks read their halos).
+//
+// Every fused launch moves 32 B per point (complex64), 16 at S = 2 and 10.7 at S = 3 per stage:
+// at 256^3 two stages take 112 us (4.9 TB/s, the rate of a large copy) and three 136 us, where the
+// arithmetic and the LDS reads of the halo cells bound the launch.  Keeping the centre and the
+// previous plane of every level in registers spilled 30 of them (290 us at S = 3).  The pair
+// kernel before this one held three planes of every level in LDS, took 111 us at 256^3 and, with
+// too few blocks on smaller grids, 49 us at 128^3 (now 20), 46 at 64^3 (7.8), and in complex128
+// 63 us at 64 x 96 x 128 (14.6) and 322 at 256^3 (185).
+struct ChainArgs {
+  int nx, ny, nz;
+  int w;                    // window columns
+  int ty, tz, tx;           // output tile (rows, columns) and x planes per block
+  int nty, ntz, ntx;        // tiles per grid
+  int batch;
+};
+template <typename R, int S> struct ChainCoef { R c[S], inv_2m, inv_dx2; };
 
+// W: the window's columns where they are known at compile time (LDS row offsets become immediates)
+template <typename R, int S, int NT, int RC, int W>
+__global__ __launch_bounds__(NT) void horner_chain_kernel(const cx<R>* __restrict__ u_in, cx<R>* __restrict__ u_out,
+                                                          const cx<R>* __restrict__ psi,
+                                                          const float2* __restrict__ V, const ChainArgs g,
+                                                          const ChainCoef<R, S> k) {
+  using C = cx<R>;
+  static_assert(S == 2 || S == 3, "psi and V are kept in three slots");
+  constexpr int CELLS = NT * RC;
+  constexpr unsigned EB = unsigned(sizeof(C));
+  __shared__ C lev[2][S][CELLS];            // [buffer][level][row][column]
   const int tid = threadIdx.x;
-  // Blocks are dispatched round-robin over the 8 XCDs in linear order.  Give each XCD a
-  // contiguous run of tiles (z fastest, then y, then x slab): the tiles of one XCD march the
-  // same x planes together, so the y/z halo lines one tile fetches are L2 hits for its
-  // neighbours instead of second HBM reads (the order changes nothing in the arithmetic).
-  int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
-  {
-    const long total = long(gridDim.x) * gridDim.y * gridDim.z;
-    if (total % 8 == 0) {
-      const long lin = blockIdx.x + long(gridDim.x) * (blockIdx.y + long(gridDim.y) * blockIdx.z);
-      const long logical = (lin % 8) * (total / 8) + lin / 8;
-      bx = int(logical % gridDim.x);
-      by = int((logical / gridDim.x) % gridDim.y);
-      bz = int(logical / (long(gridDim.x) * gridDim.y));
-    }
-  }
-  const int z0 = bx * TZ, y0 = by * TY;
-  const int packet = bz / ntiles;
-  const int x0 = (bz % ntiles) * tile_x;
-  int x1 = x0 + tile_x;
-  if (x1 > nx) x1 = nx;
-  const long poff = long(packet) * nx * ny * nz;
+  // Blocks are dispatched round-robin over the 8 XCDs.  Each XCD gets a contiguous run of tiles
+  // (z fastest, then y, then x slab), so the tiles of one XCD march the same x planes together and
+  // the halo cells one tile fetches are L2 hits for its neighbours.
+  const long total = long(g.ntz) * g.nty * g.ntx * g.batch;
+  const long q8 = total / 8, r8 = total % 8, xcd = blockIdx.x % 8;
+  long tile = xcd * q8 + (xcd < r8 ? xcd : r8) + blockIdx.x / 8;
+  const int bz = int(tile % g.ntz);
+  tile /= g.ntz;
+  const int by = int(tile % g.nty);
+  tile /= g.nty;
+  const int bx = int(tile % g.ntx);
+  const long poff = (tile / g.ntx) * long(g.nx) * g.ny * g.nz;
   u_in += poff;
   u_out += poff;
   psi += poff;
   V += poff;
+  const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const int w = W ? W : g.w;
+  const int strips = NT / w;
+  const int x0 = bx * g.tx, x1 = min(x0 + g.tx, nx);
+  const int yb = by * g.ty - S;                       // first window row
+  const int zb = g.ntz > 1 ? bz * g.tz - S : 0;       // first window column (whole rows: no halo)
   const long sx = long(ny) * nz;
-  auto clampi = [](int v, int n) { return v < 0 ? 0 : (v >= n ? n - 1 : v); };
-  auto slot = [](int x) { return ((x % 3) + 3) % 3; };
 
-  // Each thread owns the u cells e = tid + NT r and the w cells e = tid + NT r of the two
-  // windows; what depends only on the cell (its voxel's offset within an x plane, its LDS
-  // positions, whether it is a core cell) is computed once.  An out-of-grid w cell is
-  // computed at its clamped voxel from the same u cells, psi and V as that voxel's own w
-  // cell, so it equals the copy the clamped Laplacian implies, with no extra pass.  Plane
-  // bases are block-uniform and in-plane offsets 32-bit (ny nz <= 2^18).
-  unsigned uoff[RU];                        // clamped voxel of u cell r, offset in its plane
+  // the strip: rows j0 .. j0 + RC - 1 of column c
+  const int strip = tid / w, c = tid % w;
+  const int j0 = strip * RC;
+  const int gy0 = yb + j0, gz = zb + c;
+  const bool live = strip < strips && gz >= 0 && gz < nz && gy0 < ny && gy0 + RC > 0;
+  // depth: the stages the strip takes part in, its largest distance from a window edge that is not
+  // a grid face; outmask: its output cells; off: their voxels in an x plane (clamped)
+  int depth = 0;
+  unsigned outmask = 0;
+  unsigned off[RC];
 #pragma unroll
-  for (int r = 0; r < RU; ++r) {
-    const int e = tid + NT * r;
-    const int gy = clampi(y0 - 2 + e / UZ, ny), gz = clampi(z0 - 2 + e % UZ, nz);
-    uoff[r] = unsigned(gy) * unsigned(nz) + unsigned(gz);
-  }
-  unsigned woff[RW];                        // clamped voxel of w cell r, offset in its plane
-  int wsu[RW];                              // that voxel's position in an su plane
-  bool core[RW];                            // w cell r is an output cell of this block
-#pragma unroll
-  for (int r = 0; r < RW; ++r) {
-    const int e = tid + NT * r;
-    const int j = e / WZ, k = e % WZ;
-    const int gy = y0 - 1 + j, gz = z0 - 1 + k;
-    const int cy = clampi(gy, ny), cz = clampi(gz, nz);
-    woff[r] = unsigned(cy) * unsigned(nz) + unsigned(cz);
-    wsu[r] = (cy - (y0 - 2)) * UZ + (cz - (z0 - 2));
-    core[r] = e < WY * WZ && j >= 1 && j <= TY && k >= 1 && k <= TZ && gy < ny && gz < nz;
-  }
-
-  // The next planes' operands are fetched into registers ahead so their latency overlaps the
-  // current plane's arithmetic (u one plane ahead; psi and V of plane x + 2 while plane x is
-  // computed, before w(x + 1) needs those of x + 1); psi and V of a w cell are kept for the
-  // output at the same point one plane later.
-  C ureg[RU];
-  C pahead[RW], pnext[RW], pcur[RW];
-  float2 vahead[RW], vnext[RW], vcur[RW];
-  constexpr unsigned EB = unsigned(sizeof(C));
-
-  auto fetch_u = [&](int x) {
-    const C* __restrict__ base = u_in + long(clampi(x, nx)) * sx;
-#pragma unroll
-    for (int r = 0; r < RU; ++r)
-      if (tid + NT * r < UY * UZ) ureg[r] = byte_at(base, uoff[r] * EB);
-  };
-  auto store_u = [&](int x) {
-    C* dst = &su[slot(x)][0][0];
-#pragma unroll
-    for (int r = 0; r < RU; ++r) {
-      const int e = tid + NT * r;
-      if (e < UY * UZ) dst[e] = ureg[r];
+  for (int i = 0; i < RC; ++i) {
+    const int j = j0 + i, gy = gy0 + i;
+    off[i] = unsigned(min(max(gy, 0), ny - 1)) * unsigned(nz) + unsigned(min(max(gz, 0), nz - 1));
+    int d = S;
+    if (yb > 0) d = min(d, j);
+    if (yb + strips * RC < ny) d = min(d, strips * RC - 1 - j);
+    if (live && gy >= 0 && gy < ny) {
+      depth = max(depth, d);
+      if (gy >= by * g.ty && gy < (by + 1) * g.ty && gz >= bz * g.tz && gz < (bz + 1) * g.tz) outmask |= 1u << i;
     }
-  };
-  // psi and V at the (clamped) voxels of the owned w cells of plane x (x in the grid)
-  auto fetch_pv_to = [&](int x, C (&pd)[RW], float2 (&vd)[RW]) {
-    const C* __restrict__ pb = psi + long(x) * sx;
-    const float2* __restrict__ vb = V + long(x) * sx;
+  }
+  // LDS elements of a level plane: the strip's first cell, its z neighbours, the rows above and
+  // below the strip; a neighbour outside the grid (or the window) is the cell itself
+  const int own = strip < strips ? j0 * w + c : 0;
+  const int ezm = (c > 0 && gz > 0) ? own - 1 : own;
+  const int ezp = (c < w - 1 && gz < nz - 1) ? own + 1 : own;
+  const int etop = (j0 > 0 && gy0 > 0) ? own - w : own;
+  const int ebot = (strip < strips - 1 && gy0 + RC < ny) ? own + RC * w : own + (RC - 1) * w;
+  // a y face inside the strip: row lo - 1 repeats the grid's first row, row hi + 1 its last
+  const int lo = live && gy0 < 0 ? -gy0 : 0;
+  const int hi = live && gy0 + RC > ny ? ny - 1 - gy0 : RC - 1;
+  const bool face = lo > 0 || hi < RC - 1;
+
+  C un[RC];                                           // u(t)
+  C ps[3][RC];                                        // psi, V of plane q in slot (q - t0) mod 3
+  float2 vs[3][RC];
+  const int t0 = max(x0 - S, 0), t1 = x1 - 1 + S;
 #pragma unroll
-    for (int r = 0; r < RW; ++r) {
-      if (tid + NT * r < WY * WZ) {
-        pd[r] = byte_at(pb, woff[r] * EB);
-        vd[r] = byte_at(vb, woff[r] * unsigned(sizeof(float2)));
+  for (int i = 0; i < RC; ++i) {
+    un[i] = mk<R>(R(0), R(0));
+#pragma unroll
+    for (int f = 0; f < 3; ++f) {
+      ps[f][i] = mk<R>(R(0), R(0));
+      vs[f][i] = make_float2(0.0f, 0.0f);
+    }
+  }
+  if (live) {
+#pragma unroll
+    for (int i = 0; i < RC; ++i) un[i] = byte_at(u_in + long(t0) * sx, off[i] * EB);
+  }
+
+  // iteration t, f = (t - t0) mod 3
+  auto iteration = [&](int t, auto fc) {
+    constexpr int f = decltype(fc)::value;
+    const int b = t & 1;
+    // loads of the next iteration: u(t + 1); psi and V of plane t, whose first stage is next
+    C ua[RC], pa[RC];
+    float2 va[RC];
+    if (live) {
+      const C* __restrict__ ub = u_in + long(min(t + 1, nx - 1)) * sx;
+      const C* __restrict__ pb = psi + long(min(t, nx - 1)) * sx;
+      const float2* __restrict__ vb = V + long(min(t, nx - 1)) * sx;
+#pragma unroll
+      for (int i = 0; i < RC; ++i) ua[i] = byte_at(ub, off[i] * EB);
+#pragma unroll
+      for (int i = 0; i < RC; ++i) {
+        pa[i] = byte_at(pb, off[i] * EB);
+        va[i] = byte_at(vb, off[i] * unsigned(sizeof(float2)));
       }
     }
-  };
-  auto fetch_pv = [&](int x) { fetch_pv_to(x, pnext, vnext); };
-  // w plane x from u(x-1), u(x), u(x+1) and pnext/vnext; a plane outside the grid is a copy
-  // of the nearest grid plane
-  auto make_w = [&](int x) {
-    if (x >= 0 && x < nx) {
-      C* dst = &sw[slot(x)][0][0];
-      const C* um = &su[slot(x - 1)][0][0];
-      const C* uc = &su[slot(x)][0][0];
-      const C* up = &su[slot(x + 1)][0][0];
+    C* wr = &lev[b ^ 1][0][0];
+    const C* rd = &lev[b][0][0];
+    C nxt[RC], prv[RC];                               // level s - 1: planes t - s + 1 and t - s - 1
+    if (strip < strips) {
 #pragma unroll
-      for (int r = 0; r < RW; ++r) {
-        const int e = tid + NT * r;
-        if (e < WY * WZ) {
-          const int c = wsu[r];
-          dst[e] = horner_point<R>(uc[c], um[c], up[c], uc[c - UZ], uc[c + UZ], uc[c - 1], uc[c + 1], pnext[r],
-                                   vnext[r], c1, inv_2m, inv_dx2);
+      for (int i = 0; i < RC; ++i) {
+        nxt[i] = un[i];
+        prv[i] = wr[own + i * w];
+        wr[own + i * w] = un[i];
+      }
+    }
+    static_for<S>([&](auto lc) {
+      constexpr int l = decltype(lc)::value, s = l + 1;
+      const int q = t - s;                            // this stage's plane; the first one needed: x0 - (S - s)
+      if (q >= x0 - (S - s) && q >= 0 && q < nx && depth >= s) {
+        const C* cl = rd + l * CELLS;
+        C cur[RC];
+#pragma unroll
+        for (int i = 0; i < RC; ++i) cur[i] = cl[own + i * w];
+        if (q == 0) {
+#pragma unroll
+          for (int i = 0; i < RC; ++i) prv[i] = cur[i];
         }
+        if (q == nx - 1) {
+#pragma unroll
+          for (int i = 0; i < RC; ++i) nxt[i] = cur[i];
+        }
+        C o[RC];
+#pragma unroll
+        for (int i = 0; i < RC; ++i) {
+          const C ym = i > 0 ? cur[i > 0 ? i - 1 : 0] : cl[etop];
+          const C yp = i < RC - 1 ? cur[i < RC - 1 ? i + 1 : 0] : cl[ebot];
+          o[i] = horner_point<R>(cur[i], prv[i], nxt[i], ym, yp, cl[ezm + i * w], cl[ezp + i * w],
+                                 ps[(f + 3 - s) % 3][i], vs[(f + 3 - s) % 3][i], k.c[l], k.inv_2m, k.inv_dx2);
+        }
+        if constexpr (s < S) {
+          if (face) {
+#pragma unroll
+            for (int i = RC - 1; i > 0; --i)
+              if (i == lo) o[i - 1] = o[i];
+#pragma unroll
+            for (int i = 0; i < RC - 1; ++i)
+              if (i == hi) o[i + 1] = o[i];
+          }
+          C* wl = wr + s * CELLS;
+#pragma unroll
+          for (int i = 0; i < RC; ++i) {
+            nxt[i] = o[i];
+            prv[i] = wl[own + i * w];
+            wl[own + i * w] = o[i];
+          }
+        } else {
+          C* __restrict__ ob = u_out + long(q) * sx;
+#pragma unroll
+          for (int i = 0; i < RC; ++i)
+            if (outmask & (1u << i)) byte_at(ob, off[i] * EB) = o[i];
+        }
+      } else if constexpr (s < S) {
+        // no plane for this stage (before its first, past the grid): the next one still needs the
+        // plane before its own
+#pragma unroll
+        for (int i = 0; i < RC; ++i) prv[i] = wr[s * CELLS + own + i * w];
       }
-    } else {
-      const int ws = slot(x), fs = slot(clampi(x, nx));
-      for (int e = tid; e < WY * WZ; e += NT) {
-        const int j = e / WZ, k = e % WZ;
-        sw[ws][j][k] = sw[fs][j][k];
-      }
+    });
+#pragma unroll
+    for (int i = 0; i < RC; ++i) {
+      un[i] = ua[i];
+      ps[f][i] = pa[i];
+      vs[f][i] = va[i];
     }
+    __syncthreads();
   };
-
-  // prologue: u(x0-2..x0+2) and w(x0-1), w(x0); pcur = psi, V of plane x0
-  fetch_u(x0 - 2);
-  store_u(x0 - 2);
-  fetch_u(x0 - 1);
-  store_u(x0 - 1);
-  fetch_u(x0);
-  store_u(x0);
-  if (x0 - 1 >= 0) fetch_pv(x0 - 1);
-  __syncthreads();
-  if (x0 - 1 >= 0) {
-    make_w(x0 - 1);
-    __syncthreads();
-  }
-  fetch_u(x0 + 1);
-  store_u(x0 + 1);           // replaces u(x0-2)
-  fetch_pv(x0);
-  __syncthreads();
-  make_w(x0);
-  __syncthreads();
-  if (x0 - 1 < 0) {
-    make_w(x0 - 1);          // copy of w(x0)
-    __syncthreads();
-  }
-#pragma unroll
-  for (int r = 0; r < RW; ++r) { pcur[r] = pnext[r]; vcur[r] = vnext[r]; }
-  fetch_u(x0 + 2);
-  store_u(x0 + 2);           // replaces u(x0-1)
-  if (x0 + 1 < nx) fetch_pv(x0 + 1);
-  __syncthreads();
-
-#pragma unroll
-  for (int r = 0; r < RW; ++r) {   // defined values where no plane x + 2 is fetched
-    pahead[r] = pnext[r];
-    vahead[r] = vnext[r];
-  }
-  // state at the top of iteration x: su = u(x..x+2), sw = w(x-1), w(x), pnext = psi/V(x+1),
-  // pcur = psi/V(x)
-  for (int x = x0; x < x1; ++x) {
-    fetch_u(x + 3);                           // into registers, stored after this plane
-    if (x + 2 < nx) fetch_pv_to(x + 2, pahead, vahead);   // used by w(x + 2), next iteration
-    make_w(x + 1);                            // replaces w(x-2)
-    __syncthreads();
-    // output plane x at the owned core cells
-    {
-      const C* wm = &sw[slot(x - 1)][0][0];
-      const C* wc = &sw[slot(x)][0][0];
-      const C* wp = &sw[slot(x + 1)][0][0];
-      C* __restrict__ ob = u_out + long(x) * sx;
-#pragma unroll
-      for (int r = 0; r < RW; ++r) {
-        const int e = tid + NT * r;
-        if (core[r])
-          byte_at(ob, woff[r] * EB) = horner_point<R>(wc[e], wm[e], wp[e], wc[e - WZ], wc[e + WZ], wc[e - 1],
-                                                      wc[e + 1], pcur[r], vcur[r], c2, inv_2m, inv_dx2);
-      }
-    }
-    store_u(x + 3);                           // replaces u(x), last read by w(x + 1)
-#pragma unroll
-    for (int r = 0; r < RW; ++r) {
-      pcur[r] = pnext[r];
-      vcur[r] = vnext[r];
-      pnext[r] = pahead[r];
-      vnext[r] = vahead[r];
-    }
-    __syncthreads();
+  for (int t = t0; t <= t1; t += 3) {
+    iteration(t, std::integral_constant<int, 0>{});
+    if (t + 1 > t1) break;
+    iteration(t + 1, std::integral_constant<int, 1>{});
+    if (t + 2 > t1) break;
+    iteration(t + 2, std::integral_constant<int, 2>{});
   }
 }
 
-template <int TZ, int TY, int NT = 256>
-static void launch_pair_f32(int batch, int nx, int ny, int nz, const void* u_in, void* u_out, const void* psi,
-                            const float2* V, double c1, double c2, double inv_2m, double inv_dx2, int tile_x,
-                            int ntiles, hipStream_t s) {
-  dim3 grid((nz + TZ - 1) / TZ, (ny + TY - 1) / TY, unsigned(ntiles * batch));
-  WFS_LAUNCH((horner2_kernel<float, TZ, TY, NT>), grid, dim3(NT), 0, s, static_cast<const float2*>(u_in),
-                     static_cast<float2*>(u_out), static_cast<const float2*>(psi), V, nx, ny, nz, float(c1),
-                     float(c2), float(inv_2m), float(inv_dx2), tile_x, ntiles);
-}
-
-// variant (complex64): 1 = 16 x 64 (y, z) tile, 2 = 8 x 64, 3 = 8 x 128 with 256 threads, 4 = 8 x 128
-// with 512 threads, 5 = 8 x 256 with 1024 threads.  A wider z tile wastes less of the partly used
-// memory lines at its z halo, a deeper y tile less y halo; both cost LDS and so blocks per CU.
-// More threads per tile give each fewer cells (fewer registers) and the CU more wavefronts to
-// hide the plane loads with: 4 and 5 run 16 wavefronts per CU where the LDS of 3 holds 8.
-// Measured at 256^3 (one box, alternating): 120, 120, 120-125, 113 and 111 us per launch; the
-// plan takes 5 where nz >= 256, 4 where nz >= 128, else 1.
-int launch_horner_pair(int precision, int batch, int nx, int ny, int nz, const void* u_in, void* u_out,
-                       const void* psi, const float2* V, double c1, double c2, double inv_2m, double inv_dx2,
-                       int variant, hipStream_t s) {
-  const int tile_x = nx < 32 ? nx : 32;
-  const int ntiles = (nx + tile_x - 1) / tile_x;
-  if (precision == WFS_C128) {
-    constexpr int TZ = 32, TY = 8, NT = 256;
-    dim3 grid((nz + TZ - 1) / TZ, (ny + TY - 1) / TY, unsigned(ntiles * batch));
-    WFS_LAUNCH((horner2_kernel<double, TZ, TY, NT>), grid, dim3(NT), 0, s,
-                       static_cast<const double2*>(u_in), static_cast<double2*>(u_out),
-                       static_cast<const double2*>(psi), V, nx, ny, nz, c1, c2, inv_2m, inv_dx2, tile_x, ntiles);
-  } else if (variant == 1) {
-    launch_pair_f32<64, 16>(batch, nx, ny, nz, u_in, u_out, psi, V, c1, c2, inv_2m, inv_dx2, tile_x, ntiles, s);
-  } else if (variant == 3) {
-    launch_pair_f32<128, 8>(batch, nx, ny, nz, u_in, u_out, psi, V, c1, c2, inv_2m, inv_dx2, tile_x, ntiles, s);
-  } else if (variant == 4) {
-    launch_pair_f32<128, 8, 512>(batch, nx, ny, nz, u_in, u_out, psi, V, c1, c2, inv_2m, inv_dx2, tile_x, ntiles, s);
-  } else if (variant == 5) {
-    launch_pair_f32<256, 8, 1024>(batch, nx, ny, nz, u_in, u_out, psi, V, c1, c2, inv_2m, inv_dx2, tile_x, ntiles, s);
-  } else {
-    launch_pair_f32<64, 8>(batch, nx, ny, nz, u_in, u_out, psi, V, c1, c2, inv_2m, inv_dx2, tile_x, ntiles, s);
+// g: grid and batch, tz = output columns of a tile (at least nz: whole rows)
+template <typename R, int S, int NT, int RC, int W>
+static int launch_chain_form(ChainArgs g, const void* u_in, void* u_out, const void* psi, const float2* V,
+                             const double* c, double inv_2m, double inv_dx2, hipStream_t s) {
+  constexpr long lds = long(2) * S * NT * RC * long(sizeof(cx<R>));
+  static_assert(lds <= 160 * 1024, "levels do not fit in LDS");
+  if (g.tz > g.nz) g.tz = g.nz;
+  g.ntz = (g.nz + g.tz - 1) / g.tz;
+  g.w = g.ntz > 1 ? g.tz + 2 * S : g.nz;
+  const int uy = (NT / g.w) * RC;
+  if ((W && g.w != W) || uy <= 2 * S) {
+    set_last_error("power series: %d stages on %d columns do not fit the window", S, g.w);
+    return WFS_ERR_INVALID;
   }
+  g.ty = uy - 2 * S < g.ny ? uy - 2 * S : g.ny;
+  g.nty = (g.ny + g.ty - 1) / g.ty;
+  g.ty = (g.ny + g.nty - 1) / g.nty;                  // even tiles
+  // x planes per block: a block takes tx + 2 S iterations; of the slab counts up to four rounds of
+  // blocks, the one with the fewest iterations over all rounds
+  constexpr long fit = 160 * 1024 / lds;
+  constexpr long slots = 256 * (fit < 1024 / NT ? fit : 1024 / NT);
+  const long tiles = long(g.ntz) * g.nty * g.batch;
+  const int most = int(g.nx < 4 * slots / tiles + 1 ? g.nx : 4 * slots / tiles + 1);
+  long best = -1;
+  for (int m = 1; m <= most; ++m) {
+    const int tx = (g.nx + m - 1) / m;
+    const int ntx = (g.nx + tx - 1) / tx;
+    const long cost = (tiles * ntx + slots - 1) / slots * (tx + 2 * S);
+    if (best < 0 || cost < best) {
+      best = cost;
+      g.tx = tx;
+      g.ntx = ntx;
+    }
+  }
+  const long blocks = tiles * g.ntx;
+  if (blocks > 0x7fffffffL) { set_last_error("power series: grid too large"); return WFS_ERR_INVALID; }
+  ChainCoef<R, S> k;
+  for (int i = 0; i < S; ++i) k.c[i] = R(c[i]);
+  k.inv_2m = R(inv_2m);
+  k.inv_dx2 = R(inv_dx2);
+  WFS_LAUNCH((horner_chain_kernel<R, S, NT, RC, W>), dim3(unsigned(blocks)), dim3(NT), 0, s,
+             static_cast<const cx<R>*>(u_in), static_cast<cx<R>*>(u_out), static_cast<const cx<R>*>(psi), V, g, k);
   return int(hipGetLastError());
+}
+
+int horner_chain_stages(int precision) { return precision == WFS_C128 ? 2 : 3; }
+
+// The window by grid, measured per launch in us (the other forms beside it):
+// complex64, S = 3: columns past 64 in tiles of 64 (a wide tile has few rows, most of them halo):
+//   256^3 136 (whole rows 157, tiles of 128 143), 192^3 54 (59), 128^3 28 (26); nz <= 64 whole
+//   rows, 512 threads (64^3 11.5 against 15 with 1024) or 256 on small grids (32^3 9.0 against 10.2)
+// complex64, S = 2: whole rows at nz = 256 (256^3 112; tiles of 64 123), else tiles of 64, 512
+//   threads (192^3 43, whole rows 45; 128^3 20, 21; 64 x 64 x 512 20, 27); 96 columns whole (13);
+//   nz <= 64 whole rows, 256 threads (64^3 7.8, with 1024 10.7; 512 x 512 x 64 116, 120)
+// complex128 (S = 2): whole rows, 1024 threads (256^3 185, 256 threads 231; 64 x 96 x 128 14.6,
+//   17.5), 256 threads on small grids (32^3 5.5, 8.2); 512 columns in tiles of 128
+int launch_horner_chain(int precision, int stages, int batch, int nx, int ny, int nz, const void* u_in, void* u_out,
+                        const void* psi, const float2* V, const double* c, double inv_2m, double inv_dx2,
+                        hipStream_t s) {
+  ChainArgs g{};
+  g.nx = nx;
+  g.ny = ny;
+  g.nz = nz;
+  g.batch = batch;
+  g.tz = nz;
+  const bool small = long(batch) * nx * ny * nz <= 1L << 16;
+#define WFS_CHAIN(R, S, NT, RC, W) \
+  return launch_chain_form<R, S, NT, RC, W>(g, u_in, u_out, psi, V, c, inv_2m, inv_dx2, s)
+  if (precision == WFS_C128) {
+    if (stages == 2) {
+      if (small && nz <= 64) WFS_CHAIN(double, 2, 256, 2, 0);
+      if (nz > 256) g.tz = 128;
+      WFS_CHAIN(double, 2, 1024, 2, 0);
+    }
+  } else if (stages == 3) {
+    if (nz <= 64) {
+      if (small) WFS_CHAIN(float, 3, 256, 3, 0);
+      WFS_CHAIN(float, 3, 512, 3, 0);
+    }
+    if (nz % 64 == 0) {
+      g.tz = 64;
+      WFS_CHAIN(float, 3, 1024, 3, 70);
+    }
+    WFS_CHAIN(float, 3, 1024, 3, 0);
+  } else if (stages == 2) {
+    if (nz <= 64) WFS_CHAIN(float, 2, 256, 3, 0);
+    if (nz == 256) WFS_CHAIN(float, 2, 1024, 3, 256);
+    if (nz % 64 == 0) {
+      g.tz = 64;
+      WFS_CHAIN(float, 2, 512, 3, 68);
+    }
+    WFS_CHAIN(float, 2, 512, 3, 0);
+  }
+#undef WFS_CHAIN
+  set_last_error("power series: no fused launch of %d stages", stages);
+  return WFS_ERR_INVALID;
 }
 
 int launch_horner_stage(int precision, int batch, int nx, int ny, int nz, const void* u_in, void* u_out,
