@@ -422,6 +422,25 @@ int wfs_fno_modes(const float* Rr, const float* Ri, const float* X, float* O, in
 int wfs_fno_layer(const float* W, const float* v, const float* Z, const float* bias, const float* Gz,
                   const float* Fz, float* u, float* vn, float* T, int cin, int C, int n, int tm, int act,
                   void* stream);
+/*
+ * Backward of the layers (no reference counterpart).
+ *  wfs_fno_layer_backward  gn = (W^T g + Tg Fz^T) GELU'(u) and Tn = gn Gz^T in one pass over the
+ *                          grid lines (the transposed wfs_fno_layer): g [cin][n^3], W [cin][C],
+ *                          Tg [C][n^2][tm] or NULL (no spectral term), u [C][n^3]
+ *                          or NULL (no GELU factor), gn [C][n^3], Tn [C][n^2][tm] or NULL.  Operand
+ *                          rounding and limits as wfs_fno_layer; u, gn, Tg 16-byte aligned.
+ *  wfs_fno_weight_grad     gW[o][i] += sum_p g[o][p] v[i][p], gb[o] += sum_p g[o][p]; C, cin <= 32,
+ *                          P a multiple of 32, g and v 16-byte aligned; g and v enter the matrix
+ *                          cores as bf16 hi + lo; work of 512 * 1056 floats holds any size.
+ *  wfs_fno_modes_backward  gradients of wfs_fno_modes: gRr, gRi [m3][C][C] accumulated from X and dO
+ *                          [C][2][m3], dX [C][2][m3] written; C <= 256.
+ */
+int wfs_fno_layer_backward(const float* W, const float* g, const float* Tg, const float* u, const float* Gz,
+                           const float* Fz, float* gn, float* Tn, int cin, int C, int n, int tm, void* stream);
+int wfs_fno_weight_grad(const float* g, const float* v, float* gW, float* gb, int C, int cin, long P, float* work,
+                        long work_elems, void* stream);
+int wfs_fno_modes_backward(const float* Rr, const float* Ri, const float* X, const float* dO, float* dX, float* gRr,
+                           float* gRi, int m3, int C, void* stream);
 int wfs_fno_gelu_backward(const float* u, const float* dv, float* du, long n, void* stream);
 /*
  * wfs_spectral_resample (no reference counterpart): the spectrum of an ndst grid from that of

@@ -54,6 +54,9 @@ SIGNATURES = {
     "wfs_fno_axpby": (ctypes.c_int, [_vp, _vp, ctypes.c_float, ctypes.c_float, ctypes.c_long, _vp]),
     "wfs_fno_layer": (ctypes.c_int, [_vp] * 9 + [ctypes.c_int] * 5 + [_vp]),
     "wfs_fno_modes": (ctypes.c_int, [_vp] * 4 + [ctypes.c_int] * 2 + [_vp]),
+    "wfs_fno_layer_backward": (ctypes.c_int, [_vp] * 8 + [ctypes.c_int] * 4 + [_vp]),
+    "wfs_fno_weight_grad": (ctypes.c_int, [_vp] * 4 + [ctypes.c_int] * 2 + [ctypes.c_long, _vp, ctypes.c_long, _vp]),
+    "wfs_fno_modes_backward": (ctypes.c_int, [_vp] * 7 + [ctypes.c_int] * 2 + [_vp]),
     "wfs_fno_pack": (ctypes.c_int, [_vp, ctypes.c_int, _vp, ctypes.c_float, ctypes.c_float, _vp, ctypes.c_long,
                                     _vp]),
     "wfs_fno_unpack": (ctypes.c_int, [_vp, ctypes.c_float, _vp, ctypes.c_long, _vp]),
@@ -521,6 +524,51 @@ def fno_modes(Rr: torch.Tensor, Ri: torch.Tensor, X: torch.Tensor, O: torch.Tens
             raise ValueError(f"{name} must be a contiguous float32 tensor of at least {size} elements")
     check(lib().wfs_fno_modes(ptr(Rr), ptr(Ri), ptr(X), ptr(O), int(m3), int(C), stream_handle(stream)),
           "wfs_fno_modes")
+
+
+def _check_f32(tensors) -> None:
+    """(tensor or None, least element count, name): contiguous float32 device tensors."""
+    for t, size, name in tensors:
+        if t is None:
+            continue
+        _require_device_any(t, name)
+        if t.dtype != torch.float32 or not t.is_contiguous() or t.numel() < size:
+            raise ValueError(f"{name} must be a contiguous float32 tensor of at least {size} elements")
+
+
+def fno_layer_backward(W: torch.Tensor, g: torch.Tensor, Tg: torch.Tensor | None, u: torch.Tensor | None,
+                       Gz: torch.Tensor, Fz: torch.Tensor, gn: torch.Tensor, Tn: torch.Tensor | None, cin: int, C: int,
+                       n: int, tm: int, stream=None) -> None:
+    """gn = (W^T g + Tg Fz^T) GELU'(u), Tn = gn Gz^T per grid line (``wfs_fno_layer_backward``):
+    W [cin][C], g [cin][n^3], Tg and Tn [C][n^2][tm] or None, u [C][n^3] or None, gn [C][n^3]."""
+    P = n ** 3
+    _check_f32([(W, cin * C, "W"), (g, cin * P, "g"), (Tg, C * n * n * tm, "Tg"), (u, C * P, "u"), (Gz, tm * n, "Gz"),
+                (Fz, n * tm, "Fz"), (gn, C * P, "gn"), (Tn, C * n * n * tm, "Tn")])
+    check(lib().wfs_fno_layer_backward(ptr(W), ptr(g), ptr(Tg) if Tg is not None else None,
+                                       ptr(u) if u is not None else None, ptr(Gz), ptr(Fz), ptr(gn),
+                                       ptr(Tn) if Tn is not None else None, int(cin), int(C), int(n), int(tm),
+                                       stream_handle(stream)), "wfs_fno_layer_backward")
+
+
+# floats wfs_fno_weight_grad may need in its workspace (512 records of a 32 x 32 tile and 32 sums)
+WEIGHT_GRAD_WORK = 512 * 33 * 32
+
+
+def fno_weight_grad(g: torch.Tensor, v: torch.Tensor, gW: torch.Tensor, gb: torch.Tensor, C: int, cin: int, P: int,
+                    work: torch.Tensor, stream=None) -> None:
+    """gW[o][i] += sum_p g[o][p] v[i][p], gb[o] += sum_p g[o][p] (``wfs_fno_weight_grad``)."""
+    _check_f32([(g, C * P, "g"), (v, cin * P, "v"), (gW, C * cin, "gW"), (gb, C, "gb"), (work, 1, "work")])
+    check(lib().wfs_fno_weight_grad(ptr(g), ptr(v), ptr(gW), ptr(gb), int(C), int(cin), int(P), ptr(work),
+                                    int(work.numel()), stream_handle(stream)), "wfs_fno_weight_grad")
+
+
+def fno_modes_backward(Rr: torch.Tensor, Ri: torch.Tensor, X: torch.Tensor, dO: torch.Tensor, dX: torch.Tensor,
+                       gRr: torch.Tensor, gRi: torch.Tensor, m3: int, C: int, stream=None) -> None:
+    """Gradients of fno_modes (``wfs_fno_modes_backward``): gRr, gRi accumulated, dX written."""
+    _check_f32([(Rr, m3 * C * C, "Rr"), (Ri, m3 * C * C, "Ri"), (X, 2 * C * m3, "X"), (dO, 2 * C * m3, "dO"),
+                (dX, 2 * C * m3, "dX"), (gRr, m3 * C * C, "gRr"), (gRi, m3 * C * C, "gRi")])
+    check(lib().wfs_fno_modes_backward(ptr(Rr), ptr(Ri), ptr(X), ptr(dO), ptr(dX), ptr(gRr), ptr(gRi), int(m3), int(C),
+                                       stream_handle(stream)), "wfs_fno_modes_backward")
 
 
 def spectral_resample(src: torch.Tensor, dst: torch.Tensor, scale: float | None = None, shift=None,

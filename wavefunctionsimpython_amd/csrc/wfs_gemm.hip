@@ -269,6 +269,14 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(GemmArgs g) {
 // 32-point z chunk of u^T, items 4q..4q+3, is already the A run of v' for the z run q of
 // T = v' Fz.  A chunk takes 12 matrix instructions (W v, Z Gz and v' Fz, two each per
 // 16 k for the hi and lo parts).  C, cin, tm <= 32.
+//
+// BWD: the layer's transposed product in the same form, for the backward pass
+//   vn = (W^T g + T' Fz^T) GELU'(u),  T = vn Gz^T
+// with g in v, T' (the gradient of the layer's z stage) in Z, W stored [cin][C], the two tables
+// exchanged, u in up (null: no factor) and no bias: what the composition writes and reads in
+// between (W^T g, its sum with the spectral term, the product with GELU') stays in registers.
+// At 64^3, C = 32: 59 us, against 150 us for the four launches it replaces (27 + 27 us for the two
+// GEMMs that write W^T g and add the spectral term, 23 for GELU', 73 for the z stage).
 // ---------------------------------------------------------------------------
 struct LayerArgs {
   const float* W;
@@ -282,6 +290,7 @@ struct LayerArgs {
   float* T;            // may be null
   int cin, C, tm, act;
   long rows;           // lines (n * n)
+  const float* up;     // backward form: pre-activations [C][n^3] whose GELU' multiplies vn (may be null)
 };
 
 __device__ __forceinline__ void split4(const float (&x)[4], bf16x4& hi, bf16x4& lo) {
@@ -293,7 +302,7 @@ __device__ __forceinline__ void split4(const float (&x)[4], bf16x4& hi, bf16x4& 
   }
 }
 
-template <int NZC>
+template <int NZC, bool BWD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void fno_layer_kernel(LayerArgs g) {
   constexpr int n = 32 * NZC;
   constexpr int GP = kBK + 4;                        // padded rows of the transform tables
@@ -310,8 +319,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
 
   for (int e = threadIdx.x; e < n * 32; e += blockDim.x) {
     const int z = e / 32, j = e % 32;
-    GzT[z][j] = (g.Z && j < tm) ? f32_to_bf16(g.Gz[j * n + z]) : (unsigned short)0;
-    FzT[j][z] = (g.T && j < tm) ? f32_to_bf16(g.Fz[z * tm + j]) : (unsigned short)0;
+    const float gz = j < tm && (BWD ? g.T : g.Z) ? g.Gz[j * n + z] : 0.0f;
+    const float fz = j < tm && (BWD ? g.Z : g.T) ? g.Fz[z * tm + j] : 0.0f;
+    GzT[z][j] = f32_to_bf16(BWD ? fz : gz);
+    FzT[j][z] = f32_to_bf16(BWD ? gz : fz);
   }
   bf16x4 Wf[4];                                      // B = W^T: (k = c_in, n = c_out = lc)
 #pragma unroll
@@ -319,9 +330,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int k = 8 * s + kq + j;
-      Wf[s][j] = (short)((lc < C && k < cin) ? f32_to_bf16(g.W[lc * cin + k]) : 0);
+      Wf[s][j] = (short)((lc < C && k < cin) ? f32_to_bf16(g.W[BWD ? k * C + lc : lc * cin + k]) : 0);
     }
-  const float bias_c = lc < C ? g.bias[lc] : 0.0f;
+  const float bias_c = !BWD && lc < C ? g.bias[lc] : 0.0f;
   __syncthreads();
 
   // 32-bit byte offsets from the buffers' base addresses (C * n^3 * 4 < 2^32); loads past
@@ -332,6 +343,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
   char* __restrict__ ub = reinterpret_cast<char*>(g.u);
   char* __restrict__ nb = reinterpret_cast<char*>(g.vn);
   char* __restrict__ tb = reinterpret_cast<char*>(g.T);
+  const char* __restrict__ pb = reinterpret_cast<const char*>(g.up);
   const unsigned lcC = unsigned(lc < C ? lc : C - 1);
   const long stride = long(gridDim.x) * (blockDim.x / 64);
   // the A fragments of v^T for one 32-point chunk; the next chunk's (or the next line's
@@ -417,13 +429,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
         for (int h = 0; h < 2; ++h) {
           const int q = 2 * Q + h;
           float val[4], gv[4];
+          const unsigned off = (lcC * P + line + 32 * ch + 8 * q + kq) * 4u;
+          if constexpr (BWD) {
+            float4 up = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (pb) up = *reinterpret_cast<const float4*>(pb + off);
+            const float uv[4] = {up.x, up.y, up.z, up.w};
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            val[j] = acc[4 * q + j] + bias_c;
-            gv[j] = lc < C ? (g.act ? gelu_f(val[j]) : val[j]) : 0.0f;
+            for (int j = 0; j < 4; ++j) {
+              val[j] = acc[4 * q + j];
+              gv[j] = lc < C ? (pb ? val[j] * gelu_grad(uv[j]) : val[j]) : 0.0f;
+            }
+          } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              val[j] = acc[4 * q + j] + bias_c;
+              gv[j] = lc < C ? (g.act ? gelu_f(val[j]) : val[j]) : 0.0f;
+            }
           }
           if (lc < C) {
-            const unsigned off = (unsigned(lc) * P + line + 32 * ch + 8 * q + kq) * 4u;
             if (ub) *reinterpret_cast<float4*>(ub + off) = make_float4(val[0], val[1], val[2], val[3]);
             if (nb) *reinterpret_cast<float4*>(nb + off) = make_float4(gv[0], gv[1], gv[2], gv[3]);
           }
@@ -520,6 +543,166 @@ __global__ __launch_bounds__(256) void fno_modes_kernel(const float* __restrict_
   }
 }
 
+// ---------------------------------------------------------------------------
+// Weight and bias gradients of a pointwise layer, gW[o][i] += sum_p g[o][p] v[i][p] and
+// gb[o] += sum_p g[o][p], for up to 32 channels on both sides: one 32 x 32 tile whose k is the
+// grid.  Both operands are contiguous along k, so a lane's fragments -- 16 points of row lane % 32
+// of g and of v, the two lane halves side by side -- come straight from memory, with no LDS and no
+// barriers.  Both operands are split into bf16 hi + lo (hi hi + lo hi + hi lo, FP32 accumulation,
+// as the GEMM's split operands); the bias sum adds the FP32 values themselves.  Each wavefront
+// takes every (4 gridDim.x)-th run of 32 points, the block's four tiles are added in LDS, and a
+// second kernel adds the blocks' records in a fixed order.
+// Reads 4 (C + cin) P bytes.  The strided GEMM it replaces computed this tile in blocks of 128 x 32
+// with one wavefront in four at work, and the bias in a second pass over g: 114 + 13 us at 64^3,
+// C = cin = 32 (67 MB); this pair of launches takes 15 + 5 us (4.5 TB/s in the first).
+// ---------------------------------------------------------------------------
+constexpr int kGradRecord = 33 * 32;   // floats per block: the tile [o][i], then the bias sums
+
+__device__ __forceinline__ void split8(const float4& a, const float4& b, s16x8& hi, s16x8& lo) {
+  const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const unsigned short h = f32_to_bf16(x[j]);
+    hi[j] = (short)h;
+    lo[j] = (short)f32_to_bf16(x[j] - __uint_as_float(unsigned(h) << 16));
+  }
+}
+
+__global__ __launch_bounds__(256) void fno_weight_grad_kernel(const float* __restrict__ g, const float* __restrict__ v,
+                                                              float* __restrict__ work, int C, int cin, long P) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row = lane & 31;
+  // rows past the channels read a valid row and count as zero
+  const bool ga = row < C, va = row < cin;
+  const float* __restrict__ gr = g + long(ga ? row : 0) * P + 16 * (lane >> 5);
+  const float* __restrict__ vr = v + long(va ? row : 0) * P + 16 * (lane >> 5);
+  f32x16 acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+  float bsum = 0.0f;
+  const long stride = long(gridDim.x) * 4 * 32;
+  long p = (long(blockIdx.x) * 4 + wave) * 32;
+  float4 a[4], b[4];
+  const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  auto load = [&](long at) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      a[j] = *reinterpret_cast<const float4*>(gr + at + 4 * j);
+      b[j] = *reinterpret_cast<const float4*>(vr + at + 4 * j);
+    }
+  };
+  if (p < P) load(p);
+  for (; p < P; p += stride) {
+    float4 ca[4], cb[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      ca[j] = ga ? a[j] : zero;
+      cb[j] = va ? b[j] : zero;
+    }
+    if (p + stride < P) load(p + stride);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) bsum += (ca[j].x + ca[j].y) + (ca[j].z + ca[j].w);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      s16x8 ah, al, bh, bl;
+      split8(ca[2 * h], ca[2 * h + 1], ah, al);
+      split8(cb[2 * h], cb[2 * h + 1], bh, bl);
+      acc = mfma16(al, bh, acc);
+      acc = mfma16(ah, bl, acc);
+      acc = mfma16(ah, bh, acc);
+    }
+  }
+  bsum += __shfl_xor(bsum, 32, 64);
+  // lane: column i = row; items: o = 8(v/4) + 4(lane/32) + v%4
+  __shared__ float red[4][kGradRecord];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) red[wave][(8 * (i / 4) + 4 * (lane >> 5) + i % 4) * 32 + row] = acc[i];
+  if (lane < 32) red[wave][32 * 32 + row] = bsum;
+  __syncthreads();
+  for (int e = threadIdx.x; e < kGradRecord; e += 256)
+    work[long(blockIdx.x) * kGradRecord + e] = (red[0][e] + red[1][e]) + (red[2][e] + red[3][e]);
+}
+
+// block b: row b of the records (32: the bias), 32 columns by 16 strided parts of the blocks
+__global__ __launch_bounds__(512) void fno_weight_grad_sum_kernel(const float* __restrict__ work, int nblk,
+                                                                  float* __restrict__ gW, float* __restrict__ gb,
+                                                                  int C, int cin) {
+  const int col = threadIdx.x & 31, part = threadIdx.x >> 5;
+  const int row = blockIdx.x;
+  float s = 0.0f;
+#pragma unroll 8
+  for (int b = part; b < nblk; b += 16) s += work[long(b) * kGradRecord + row * 32 + col];
+  __shared__ float red[16][32];
+  red[part][col] = s;
+  __syncthreads();
+  if (part == 0) {
+    float t = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) t += red[k][col];
+    if (row < 32) {
+      if (row < C && col < cin) gW[row * cin + col] += t;
+    } else if (col < C) {
+      gb[col] += t;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Backward of the per-mode channel mixing O = R (.) X (fno_modes_kernel), one block per mode q:
+//   gRr[q][i][o] += Xr[i] dOr[o] + Xi[i] dOi[o],  gRi[q][i][o] += Xr[i] dOi[o] - Xi[i] dOr[o]
+//   dXr[i] = sum_o Rr dOr + Ri dOi,               dXi[i] = sum_o Rr dOi - Ri dOr
+// R plain bf16 and dO as bf16 hi + lo in the sums, as the mixing itself takes them; the outer
+// products are FP32.  32 lanes own a row i (o along the lanes, contiguous in memory), the row sums
+// go over the lanes.  R is read and gR read and written once: 24 C^2 bytes per mode, 42 MB at 12
+// modes and C = 32.  The eight strided GEMMs it replaces (K or N of 1 in a 32 x 32 tile) read and
+// wrote gR twice and took 16 and 12 us each; this launch takes 12 us.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void fno_modes_backward_kernel(const float* __restrict__ Rr,
+                                                                 const float* __restrict__ Ri,
+                                                                 const float* __restrict__ X,
+                                                                 const float* __restrict__ dO, float* __restrict__ dX,
+                                                                 float* __restrict__ gRr, float* __restrict__ gRi,
+                                                                 int m3, int C) {
+  __shared__ float x[2][256], d[2][256];
+  const int q = blockIdx.x;
+  for (int e = threadIdx.x; e < 2 * C; e += 256) {
+    const int c = e % C, part = e / C;
+    x[part][c] = X[(long(c) * 2 + part) * m3 + q];
+    d[part][c] = dO[(long(c) * 2 + part) * m3 + q];
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 31;
+  for (int i = threadIdx.x >> 5; i < C; i += 8) {
+    const float xr = x[0][i], xi = x[1][i];
+    float sr = 0.0f, si = 0.0f;
+    for (int o = lane; o < C; o += 32) {
+      const long e = (long(q) * C + i) * C + o;
+      const float dr = d[0][o], di = d[1][o];
+      gRr[e] += __builtin_fmaf(xr, dr, xi * di);
+      gRi[e] += __builtin_fmaf(xr, di, -(xi * dr));
+      const float a = __uint_as_float(unsigned(f32_to_bf16(Rr[e])) << 16);
+      const float b = __uint_as_float(unsigned(f32_to_bf16(Ri[e])) << 16);
+      const float drh = __uint_as_float(unsigned(f32_to_bf16(dr)) << 16);
+      const float dih = __uint_as_float(unsigned(f32_to_bf16(di)) << 16);
+      const float drl = __uint_as_float(unsigned(f32_to_bf16(dr - drh)) << 16);
+      const float dil = __uint_as_float(unsigned(f32_to_bf16(di - dih)) << 16);
+      sr = __builtin_fmaf(a, drh, __builtin_fmaf(a, drl, sr));
+      sr = __builtin_fmaf(b, dih, __builtin_fmaf(b, dil, sr));
+      si = __builtin_fmaf(a, dih, __builtin_fmaf(a, dil, si));
+      si = __builtin_fmaf(-b, drh, __builtin_fmaf(-b, drl, si));
+    }
+#pragma unroll
+    for (int off = 16; off > 0; off >>= 1) {
+      sr += __shfl_xor(sr, off, 64);
+      si += __shfl_xor(si, off, 64);
+    }
+    if (lane == 0) {
+      dX[long(i) * 2 * m3 + q] = sr;
+      dX[(long(i) * 2 + 1) * m3 + q] = si;
+    }
+  }
+}
+
 }  // namespace wfs
 
 using namespace wfs;
@@ -532,6 +715,19 @@ extern "C" int wfs_fno_modes(const float* Rr, const float* Ri, const float* X, f
                      static_cast<hipStream_t>(stream), Rr, Ri, X, O, m3, C);
   WFS_HIP_CHECK(hipGetLastError());
   return 0;
+}
+
+// one wavefront per line, four per block
+template <bool BWD>
+static void launch_layer(const LayerArgs& g, int n, hipStream_t s) {
+  const long want = (g.rows + 3) / 4;
+  const unsigned blocks = unsigned(want < 2048 ? want : 2048);
+  switch (n / 32) {
+    case 1: hipLaunchKernelGGL((fno_layer_kernel<1, BWD>), dim3(blocks), dim3(256), 0, s, g); break;
+    case 2: hipLaunchKernelGGL((fno_layer_kernel<2, BWD>), dim3(blocks), dim3(256), 0, s, g); break;
+    case 3: hipLaunchKernelGGL((fno_layer_kernel<3, BWD>), dim3(blocks), dim3(256), 0, s, g); break;
+    default: hipLaunchKernelGGL((fno_layer_kernel<4, BWD>), dim3(blocks), dim3(256), 0, s, g); break;
+  }
 }
 
 // layer of the Fourier neural operator fused over grid lines (see fno_layer_kernel)
@@ -553,17 +749,68 @@ extern "C" int wfs_fno_layer(const float* W, const float* v, const float* Z, con
     set_last_error("wfs_fno_layer: u, vn and Z must be 16-byte aligned");
     return WFS_ERR_INVALID;
   }
-  LayerArgs g{W, v, Z, bias, Gz, Fz, u, vn, T, cin, C, tm, act, long(n) * n};
-  // one wavefront per line, four per block
-  const long want = (g.rows + 3) / 4;
-  const unsigned blocks = unsigned(want < 2048 ? want : 2048);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (n / 32) {
-    case 1: hipLaunchKernelGGL(fno_layer_kernel<1>, dim3(blocks), dim3(256), 0, s, g); break;
-    case 2: hipLaunchKernelGGL(fno_layer_kernel<2>, dim3(blocks), dim3(256), 0, s, g); break;
-    case 3: hipLaunchKernelGGL(fno_layer_kernel<3>, dim3(blocks), dim3(256), 0, s, g); break;
-    default: hipLaunchKernelGGL(fno_layer_kernel<4>, dim3(blocks), dim3(256), 0, s, g); break;
+  const LayerArgs g{W, v, Z, bias, Gz, Fz, u, vn, T, cin, C, tm, act, long(n) * n, nullptr};
+  launch_layer<false>(g, n, static_cast<hipStream_t>(stream));
+  WFS_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
+extern "C" int wfs_fno_layer_backward(const float* W, const float* g, const float* Tg, const float* u, const float* Gz,
+                                      const float* Fz, float* gn, float* Tn, int cin, int C, int n, int tm,
+                                      void* stream) {
+  if (!W || !g || !gn || (Tg && !Fz) || (Tn && !Gz)) { set_last_error("wfs_fno_layer_backward: null argument"); return WFS_ERR_INVALID; }
+  if (n % 32 != 0 || n < 32 || n > 128 || C < 1 || C > 32 || cin < 1 || cin > 32 || tm < 4 || tm > 32 || tm % 4) {
+    set_last_error("wfs_fno_layer_backward: needs n in {32, 64, 96, 128}, C, cin <= 32 and tm a multiple of 4 up to 32 "
+                   "(n=%d C=%d cin=%d tm=%d)", n, C, cin, tm);
+    return WFS_ERR_UNSUPPORTED;
   }
+  if ((reinterpret_cast<unsigned long>(u) % 16) != 0 || (reinterpret_cast<unsigned long>(gn) % 16) != 0 ||
+      (reinterpret_cast<unsigned long>(Tg) % 16) != 0) {
+    set_last_error("wfs_fno_layer_backward: u, gn and Tg must be 16-byte aligned");
+    return WFS_ERR_INVALID;
+  }
+  const LayerArgs a{W, g, Tg, nullptr, Gz, Fz, nullptr, gn, Tn, cin, C, tm, 0, long(n) * n, u};
+  launch_layer<true>(a, n, static_cast<hipStream_t>(stream));
+  WFS_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
+// gW += g v^T and gb += sum_p g (see fno_weight_grad_kernel)
+extern "C" int wfs_fno_weight_grad(const float* g, const float* v, float* gW, float* gb, int C, int cin, long P,
+                                   float* work, long work_elems, void* stream) {
+  if (!g || !v || !gW || !gb || !work) { set_last_error("wfs_fno_weight_grad: null argument"); return WFS_ERR_INVALID; }
+  if (C < 1 || C > 32 || cin < 1 || cin > 32 || P < 32 || P % 32) {
+    set_last_error("wfs_fno_weight_grad: needs C, cin <= 32 and P a multiple of 32 (C=%d cin=%d P=%ld)", C, cin, P);
+    return WFS_ERR_UNSUPPORTED;
+  }
+  if ((reinterpret_cast<unsigned long>(g) % 16) != 0 || (reinterpret_cast<unsigned long>(v) % 16) != 0) {
+    set_last_error("wfs_fno_weight_grad: g and v must be 16-byte aligned");
+    return WFS_ERR_INVALID;
+  }
+  // about 256 points per wavefront, at most two blocks per CU
+  const long steps = P / 32;
+  long blocks = (steps + 31) / 32;
+  if (blocks > 512) blocks = 512;
+  if (work_elems < blocks * kGradRecord) {
+    set_last_error("wfs_fno_weight_grad: workspace needs %ld floats", blocks * kGradRecord);
+    return WFS_ERR_INVALID;
+  }
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  hipLaunchKernelGGL(fno_weight_grad_kernel, dim3(unsigned(blocks)), dim3(256), 0, s, g, v, work, C, cin, P);
+  WFS_HIP_CHECK(hipGetLastError());
+  hipLaunchKernelGGL(fno_weight_grad_sum_kernel, dim3(33), dim3(512), 0, s, work, int(blocks), gW, gb, C, cin);
+  WFS_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
+extern "C" int wfs_fno_modes_backward(const float* Rr, const float* Ri, const float* X, const float* dO, float* dX,
+                                      float* gRr, float* gRi, int m3, int C, void* stream) {
+  if (!Rr || !Ri || !X || !dO || !dX || !gRr || !gRi || m3 < 1 || C < 1 || C > 256) {
+    set_last_error("wfs_fno_modes_backward: bad argument");
+    return WFS_ERR_INVALID;
+  }
+  hipLaunchKernelGGL(fno_modes_backward_kernel, dim3(unsigned(m3)), dim3(256), 0, static_cast<hipStream_t>(stream), Rr,
+                     Ri, X, dO, dX, gRr, gRi, m3, C);
   WFS_HIP_CHECK(hipGetLastError());
   return 0;
 }

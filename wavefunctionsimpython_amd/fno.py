@@ -93,6 +93,9 @@ class FNO3d:
         # layers as one fused kernel per grid line (wfs_fno_layer) where the sizes allow
         self.fused = (bool(fused) and self.split_activations and self.n % 32 == 0 and 32 <= self.n <= 128
                       and self.C <= 32 and self.cin <= 32 and 2 * self.m <= 32 and self.m % 2 == 0)
+        # the backward pass's own kernels (the GEMM composition serves what they do not take, and
+        # float64 restatements of the device kernels on the CPU)
+        self._native = self.split_activations and torch.device(self.device).type == "cuda"
         rng = np.random.default_rng(seed)
         C, m3 = self.C, self.m ** 3
 
@@ -135,6 +138,8 @@ class FNO3d:
                 "mse": torch.empty(8192, dtype=torch.float64, device=self.device),
                 "mse_out": torch.empty(2, dtype=torch.float64, device=self.device),
             }
+            if self._native:
+                self._ws["wgrad"] = torch.empty(_abi.WEIGHT_GRAD_WORK, **f)
         return self._ws
 
     def _gemm(self, A, B, C, batch, M, N, K, sA, sB, sC, alpha=1.0, beta=0.0, splits=1, flags=0, bias=None,
@@ -148,29 +153,29 @@ class FNO3d:
                        ws["work"] if splits > 1 else None, flags=flags, bias=bias, act=act)
 
     # ------------------------------------------------------------------ spectral convolution
-    def _spectral(self, v: torch.Tensor, l: int, S: torch.Tensor) -> None:
-        """S[c][p] = Re IDFT_m(R_l (.) DFT_m(v)) (written, not accumulated)."""
+    def _spectral(self, v: torch.Tensor, l: int, S: torch.Tensor, X: torch.Tensor | None = None) -> None:
+        """S[c][p] = Re IDFT_m(R_l (.) DFT_m(v)) (written, not accumulated); X as in _spectral_mid."""
         ws = self._workspace()
         C, n, m = self.C, self.n, self.m
         tm = 2 * m
         tb = self.tab
         self._gemm(v, tb["Fz"], ws["T"], 1, C * n * n, tm, n, (0, n, 1), (0, tm, 1), (0, tm, 1), flags=SA)
-        self._spectral_mid(l)
+        self._spectral_mid(l, X)
         self._gemm(ws["Z"], tb["Gz"], S, 1, C * n * n, n, tm, (0, tm, 1), (0, n, 1), (0, n, 1), flags=SA)
 
-    def _spectral_mid(self, l: int) -> None:
+    def _spectral_mid(self, l: int, X: torch.Tensor | None = None) -> None:
         """Z = the spectral path of layer l between its z stages: T (the z-stage DFT of v, in the
-        workspace) -> y and x DFTs -> R_l -> inverse x and y DFTs -> Z (workspace)."""
+        workspace) -> y and x DFTs -> R_l -> inverse x and y DFTs -> Z (workspace).  X: where the
+        layer's modes go (default the workspace); training keeps them for the backward pass."""
         ws = self._workspace()
         C, n, m = self.C, self.n, self.m
         m2, m3, tm = m * m, m ** 3, 2 * m
         tb = self.tab
-        T, U, X, O, Y, Z = ws["T"], ws["U"], ws["X"], ws["O"], ws["Y"], ws["Z"]
+        T, U, O, Y, Z = ws["T"], ws["U"], ws["O"], ws["Y"], ws["Z"]
+        X = ws["X"] if X is None else X
         self._gemm(tb["F2"], T, U, C * n, tm, m, 2 * n, (0, 2 * n, 1), (2 * n * m, m, 1), (tm * m, m, 1), flags=SB)
         self._gemm(tb["F2"], U, X, C, tm, m2, 2 * n, (0, 2 * n, 1), (2 * n * m2, m2, 1), (tm * m2, m2, 1), flags=SB)
-        Rr, Ri = self.params[f"Rr{l}"], self.params[f"Ri{l}"]
-        Xr, Xi, Or, Oi = X, X[m3:], O, O[m3:]
-        self._modes(Rr, Ri, X, O)
+        self._modes(self.params[f"Rr{l}"], self.params[f"Ri{l}"], X, O)
         self._gemm(tb["G2"], O, Y, C, 2 * n, m2, tm, (0, tm, 1), (tm * m2, m2, 1), (2 * n * m2, m2, 1), flags=SB)
         self._gemm(tb["G2"], Y, Z, C * n, 2 * n, m, tm, (0, tm, 1), (tm * m, m, 1), (2 * n * m, m, 1), flags=SB)
 
@@ -192,41 +197,68 @@ class FNO3d:
         _abi.fno_layer(W, v, Z, bias, self.tab["Gz"], self.tab["Fz"], u, vn, T, cin, self.C, self.n, 2 * self.m,
                        act)
 
-    def _spectral_backward(self, dS: torch.Tensor, l: int, v: torch.Tensor, dv: torch.Tensor) -> None:
-        """dv += d/dv of the spectral path given dS; accumulates dR_l (needs X of this layer)."""
-        ws = self._workspace()
-        C, n, m = self.C, self.n, self.m
-        m2, m3, tm = m * m, m ** 3, 2 * m
-        tb = self.tab
-        T, U, X, O, Y, Z = ws["T"], ws["U"], ws["X"], ws["O"], ws["Y"], ws["Z"]
-        # recompute the forward modes X of this layer (cheaper than storing them per layer)
-        self._gemm(v, tb["Fz"], T, 1, C * n * n, tm, n, (0, n, 1), (0, tm, 1), (0, tm, 1), flags=SA)
-        self._gemm(tb["F2"], T, U, C * n, tm, m, 2 * n, (0, 2 * n, 1), (2 * n * m, m, 1), (tm * m, m, 1), flags=SB)
-        self._gemm(tb["F2"], U, X, C, tm, m2, 2 * n, (0, 2 * n, 1), (2 * n * m2, m2, 1), (tm * m2, m2, 1), flags=SB)
-        # inverse stages, transposed: dZ, dY, dO (reuse Z, Y, O)
-        self._gemm(dS, tb["Gz"], Z, 1, C * n * n, tm, n, (0, n, 1), (0, 1, n), (0, tm, 1), flags=SA)
-        self._gemm(tb["G2"], Z, Y, C * n, tm, m, 2 * n, (0, 1, tm), (2 * n * m, m, 1), (tm * m, m, 1), flags=SB)
-        self._gemm(tb["G2"], Y, O, C, tm, m2, 2 * n, (0, 1, tm), (2 * n * m2, m2, 1), (tm * m2, m2, 1), flags=SB)
+    def _layer_backward(self, W, g, Tg, u, gn, Tn, cin: int) -> None:
+        """gn = (W^T g + Tg Fz^T) GELU'(u), Tn = gn Gz^T in one pass over the grid lines."""
+        _abi.fno_layer_backward(W, g, Tg, u, self.tab["Gz"], self.tab["Fz"], gn, Tn, cin, self.C, self.n, 2 * self.m)
+
+    def _weight_grad(self, g: torch.Tensor, v: torch.Tensor, gW: torch.Tensor, gb: torch.Tensor, rows: int,
+                     cols: int) -> None:
+        """gW[o][i] += sum_p g[o][p] v[i][p], gb[o] += sum_p g[o][p] (rows o, cols i)."""
+        P = self.P
+        if (self._native and rows <= 32 and cols <= 32 and P % 32 == 0 and g.data_ptr() % 16 == 0
+                and v.data_ptr() % 16 == 0):
+            _abi.fno_weight_grad(g, v, gW, gb, rows, cols, P, self._workspace()["wgrad"])
+            return
+        # reductions over the grid (K = P): about 1024 points per split
+        sp = max(1, min(self.splits, P // 1024))
+        self._gemm(g, v, gW, 1, rows, cols, P, (0, P, 1), (0, 1, P), (0, cols, 1), beta=1.0, splits=sp, flags=SAB)
+        self._gemm(g, self.ones, gb, 1, rows, 1, P, (0, P, 1), (0, 0, 0), (0, 1, 0), beta=1.0, splits=sp, flags=SA)
+
+    def _modes_backward(self, l: int, X: torch.Tensor, dO: torch.Tensor, dX: torch.Tensor) -> None:
+        """Gradients of _modes: dR_l accumulated from the modes X and dO, dX written."""
+        C, m3 = self.C, self.m ** 3
         Rr, Ri = self.params[f"Rr{l}"], self.params[f"Ri{l}"]
         gRr, gRi = self.grads[f"Rr{l}"], self.grads[f"Ri{l}"]
-        Xr, Xi, dOr, dOi = X, X[m3:], O, O[m3:]
+        if self._native and C <= 256:
+            _abi.fno_modes_backward(Rr, Ri, X, dO, dX, gRr, gRi, m3, C)
+            return
+        Xr, Xi, dOr, dOi = X, X[m3:], dO, dO[m3:]
         sRt, sX = (C * C, C, 1), (1, 2 * m3, 0)
-        # weight gradients (accumulated): dRr = Xr dOr^T + Xi dOi^T, dRi = Xr dOi^T - Xi dOr^T
+        # dRr = Xr dOr^T + Xi dOi^T, dRi = Xr dOi^T - Xi dOr^T
         sA, sB, sC = (1, 2 * m3, 0), (1, 0, 2 * m3), (C * C, C, 1)
         self._gemm(Xr, dOr, gRr, m3, C, C, 1, sA, sB, sC, beta=1.0, flags=SAB)
         self._gemm(Xi, dOi, gRr, m3, C, C, 1, sA, sB, sC, beta=1.0, flags=SAB)
         self._gemm(Xr, dOi, gRi, m3, C, C, 1, sA, sB, sC, beta=1.0, flags=SAB)
         self._gemm(Xi, dOr, gRi, m3, C, C, 1, sA, sB, sC, alpha=-1.0, beta=1.0, flags=SAB)
-        # mode gradients into X (overwrites the forward modes, no longer needed)
-        dX = torch.empty_like(X)
         dXr, dXi = dX, dX[m3:]
         self._gemm(Rr, dOr, dXr, m3, C, 1, C, sRt, sX, sX, flags=SB)
         self._gemm(Ri, dOi, dXr, m3, C, 1, C, sRt, sX, sX, beta=1.0, flags=SB)
         self._gemm(Ri, dOr, dXi, m3, C, 1, C, sRt, sX, sX, alpha=-1.0, flags=SB)
         self._gemm(Rr, dOi, dXi, m3, C, 1, C, sRt, sX, sX, beta=1.0, flags=SB)
-        # forward stages, transposed: dU, dT, then dv += dT Fz^T
+
+    def _spectral_mid_backward(self, l: int, X: torch.Tensor, Tg: torch.Tensor, Zg: torch.Tensor) -> None:
+        """The transposed middle of layer l's spectral path: Tg (the gradient through the last z
+        stage) -> transposed inverse y and x stages -> modes (dR_l accumulated, X the layer's
+        modes) -> transposed forward x and y stages -> Zg (Tg and Zg may be one buffer)."""
+        ws = self._workspace()
+        C, n, m = self.C, self.n, self.m
+        m2, tm = m * m, 2 * m
+        tb = self.tab
+        U, dX, O, Y = ws["U"], ws["X"], ws["O"], ws["Y"]
+        self._gemm(tb["G2"], Tg, Y, C * n, tm, m, 2 * n, (0, 1, tm), (2 * n * m, m, 1), (tm * m, m, 1), flags=SB)
+        self._gemm(tb["G2"], Y, O, C, tm, m2, 2 * n, (0, 1, tm), (2 * n * m2, m2, 1), (tm * m2, m2, 1), flags=SB)
+        self._modes_backward(l, X, O, dX)
         self._gemm(tb["F2"], dX, U, C, 2 * n, m2, tm, (0, 1, 2 * n), (tm * m2, m2, 1), (2 * n * m2, m2, 1), flags=SB)
-        self._gemm(tb["F2"], U, T, C * n, 2 * n, m, tm, (0, 1, 2 * n), (tm * m, m, 1), (2 * n * m, m, 1), flags=SB)
+        self._gemm(tb["F2"], U, Zg, C * n, 2 * n, m, tm, (0, 1, 2 * n), (tm * m, m, 1), (2 * n * m, m, 1), flags=SB)
+
+    def _spectral_backward(self, dS: torch.Tensor, l: int, X: torch.Tensor, dv: torch.Tensor) -> None:
+        """dv += d/dv of the spectral path given dS; accumulates dR_l (X: this layer's modes)."""
+        ws = self._workspace()
+        C, n, tm = self.C, self.n, 2 * self.m
+        tb = self.tab
+        T, Z = ws["T"], ws["Z"]
+        self._gemm(dS, tb["Gz"], Z, 1, C * n * n, tm, n, (0, n, 1), (0, 1, n), (0, tm, 1), flags=SA)
+        self._spectral_mid_backward(l, X, Z, T)
         self._gemm(T, tb["Fz"], dv, 1, C * n * n, n, tm, (0, tm, 1), (0, 1, tm), (0, n, 1), beta=1.0, flags=SA)
 
     # ------------------------------------------------------------------ forward / backward
@@ -250,6 +282,14 @@ class FNO3d:
         pr = self.params
         saved_v: List[torch.Tensor] = []
         saved_u: List[torch.Tensor] = []
+        saved_X: List[torch.Tensor] = []
+
+        def modes_buffer():
+            # the layer's modes, small beside its activations, kept for the backward pass
+            if not keep:
+                return None
+            saved_X.append(torch.empty(C * 2 * self.m ** 3, dtype=self.dtype, device=self.device))
+            return saved_X[-1]
 
         def act_buffer(avoid=None):
             # training keeps every activation for the backward pass; inference ping-pongs between
@@ -264,7 +304,7 @@ class FNO3d:
             # fused pass: u = W v + (last spectral stage) + b, v' = GELU(u), next z-stage DFT
             self._layer(pr["P"], a, None, pr["pb"], None, v, ws["T"], self.cin, act=False)
             for l in range(self.L):
-                self._spectral_mid(l)
+                self._spectral_mid(l, modes_buffer())
                 last = l == self.L - 1
                 u = (torch.empty(C * P, dtype=self.dtype, device=self.device) if keep
                      else ws["d3"] if last else None)
@@ -279,7 +319,7 @@ class FNO3d:
                        bias=pr["pb"])
             for l in range(self.L):
                 u = torch.empty(C * P, dtype=self.dtype, device=self.device) if keep else ws["d3"]
-                self._spectral(v, l, u)
+                self._spectral(v, l, u, modes_buffer())
                 last = l == self.L - 1
                 vn = None if last else act_buffer(v)
                 # u = W v + S + b and v' = GELU(u) in the GEMM's epilogue; u is stored only when
@@ -299,26 +339,35 @@ class FNO3d:
         elif self.rscale != 1.0:
             self._axpby(out, out, self.rscale, 0.0)
         if keep:
-            self._saved = (a, saved_v, saved_u, v)
+            self._saved = (a, saved_v, saved_u, v, saved_X)
         return out
 
     def backward(self, dout: torch.Tensor) -> None:
         """Accumulate parameter gradients for the last forward(keep=True)."""
         if self._saved is None:
             raise RuntimeError("forward(keep=True) must precede backward()")
-        a, saved_v, saved_u, vL = self._saved
+        a, saved_v, saved_u, vL, saved_X = self._saved
         ws = self._workspace()
         C, P = self.C, self.P
         pr, gr = self.params, self.grads
-        # reductions over the grid (K = P): about 1024 points per split
-        sp = max(1, min(self.splits, P // 1024))
         if self.rscale != 1.0:
             dq = ws["dq"]
             self._axpby(dq, dout, self.rscale, 0.0)
             dout = dq
-        self._gemm(dout, vL, gr["Q"], 1, self.cout, C, P, (0, P, 1), (0, 1, P), (0, C, 1), beta=1.0, splits=sp, flags=SAB)
-        self._gemm(dout, self.ones, gr["qb"], 1, self.cout, 1, P, (0, P, 1), (0, 0, 0), (0, 1, 0), beta=1.0,
-                   splits=sp, flags=SA)
+        self._weight_grad(dout, vL, gr["Q"], gr["qb"], self.cout, C)
+        if self.fused and self._native and self.cout <= 32:
+            # g, the gradient of a layer's pre-activation, and T, its (transposed) last z stage,
+            # come out of one pass per layer, as v and the next first z stage do forward
+            g, gn, T, Z = ws["d1"], ws["d2"], ws["T"], ws["Z"]
+            self._layer_backward(pr["Q"], dout, None, None, g, T, self.cout)
+            for l in reversed(range(self.L)):
+                self._weight_grad(g, saved_v[l], gr[f"W{l}"], gr[f"b{l}"], C, C)
+                self._spectral_mid_backward(l, saved_X[l], T, Z)
+                self._layer_backward(pr[f"W{l}"], g, Z, saved_u[l - 1] if l else None, gn, T if l else None, C)
+                g, gn = gn, g
+            self._weight_grad(g, a, gr["P"], gr["pb"], C, self.cin)
+            self._saved = None
+            return
         dv = ws["d1"]
         self._gemm(pr["Q"], dout, dv, 1, C, P, self.cout, (0, 1, C), (0, P, 1), (0, P, 1), flags=SB)
         du, dvp = ws["d2"], ws["d3"]
@@ -328,13 +377,11 @@ class FNO3d:
                 g = du
             else:
                 g = dv
-            self._gemm(g, self.ones, gr[f"b{l}"], 1, C, 1, P, (0, P, 1), (0, 0, 0), (0, 1, 0), beta=1.0, splits=sp, flags=SA)
-            self._gemm(g, saved_v[l], gr[f"W{l}"], 1, C, C, P, (0, P, 1), (0, 1, P), (0, C, 1), beta=1.0, splits=sp, flags=SAB)
+            self._weight_grad(g, saved_v[l], gr[f"W{l}"], gr[f"b{l}"], C, C)
             self._gemm(pr[f"W{l}"], g, dvp, 1, C, P, C, (0, 1, C), (0, P, 1), (0, P, 1), flags=SB)
-            self._spectral_backward(g, l, saved_v[l], dvp)
+            self._spectral_backward(g, l, saved_X[l], dvp)
             dv, dvp = dvp, dv
-        self._gemm(dv, a, gr["P"], 1, C, self.cin, P, (0, P, 1), (0, 1, P), (0, self.cin, 1), beta=1.0, splits=sp, flags=SAB)
-        self._gemm(dv, self.ones, gr["pb"], 1, C, 1, P, (0, P, 1), (0, 0, 0), (0, 1, 0), beta=1.0, splits=sp, flags=SA)
+        self._weight_grad(dv, a, gr["P"], gr["pb"], C, self.cin)
         self._saved = None
 
     def forward_cost(self) -> Dict[str, float]:
