@@ -435,6 +435,14 @@ int wfs_fno_layer(const float* W, const float* v, const float* Z, const float* b
  *  wfs_fno_modes_backward  gradients of wfs_fno_modes: gRr, gRi [m3][C][C] accumulated from X and dO
  *                          [C][2][m3], dX [C][2][m3] written; C <= 256.
  */
+/*
+ * wfs_fno_stage (no reference counterpart): one truncated-DFT stage along an axis,
+ * out[s][i][c] = sum_k A[i][k] in[s][k][c] for every slab s < slabs, i < M, c < ncol: A bf16,
+ * 16-byte aligned, [M rounded up to 32][K rounded up to 16] zero padded; in FP32 taken as bf16 hi +
+ * lo parts, FP32 accumulation (the rounding of wfs_gemm_bf16 with WFS_GEMM_SPLIT_B).  M <= 32 or
+ * K <= 32.  in and out must not overlap.
+ */
+int wfs_fno_stage(const void* A, const float* in, float* out, int M, int K, int ncol, long slabs, void* stream);
 int wfs_fno_layer_backward(const float* W, const float* g, const float* Tg, const float* u, const float* Gz,
                            const float* Fz, float* gn, float* Tn, int cin, int C, int n, int tm, void* stream);
 int wfs_fno_weight_grad(const float* g, const float* v, float* gW, float* gb, int C, int cin, long P, float* work,

@@ -1,4 +1,4 @@
-"""The network's backward kernels against float64 of the same products.
+"""The network's DFT stages and backward kernels against float64 of the same products.
 
 Bounds, per element, in units of the sum of absolute products: an operand carried as bf16 hi + lo
 keeps about 17 bits (2^-17, two operands and the dropped lo lo product: 2^-15.4), FP32 sums of a few
@@ -65,6 +65,23 @@ def test_modes_backward(dev, C, m3):
     dX = np.stack([(Rr * dr[:, None] + Ri * di[:, None]).sum(2), (Rr * di[:, None] - Ri * dr[:, None]).sum(2)])
     scale = (np.abs(Rr) * np.abs(dr[:, None]) + np.abs(Ri) * np.abs(di[:, None])).sum(2).max()
     assert np.abs(t[4].cpu().numpy().transpose(1, 2, 0) - dX).max() < BOUND * scale
+
+
+# reducing (M <= 32) and expanding (K <= 32) stages, few and many columns, partial tiles of both
+@pytest.mark.parametrize("M,K,ncol,slabs", [(24, 256, 12, 96), (24, 128, 144, 5), (256, 24, 144, 5), (128, 32, 16, 2000),
+                                           (12, 96, 6, 7), (96, 12, 6, 7), (32, 16, 1, 1), (16, 8, 3, 50),
+                                           (64, 4, 4, 1)])
+def test_dft_stage(dev, M, K, ncol, slabs):
+    rng = np.random.default_rng(M + K)
+    A = rng.uniform(-1, 1, (M, K))
+    src = rng.standard_normal((slabs, K, ncol))
+    dst = torch.full((slabs * M * ncol + 64,), 7.0, dtype=torch.float32, device=dev)
+    _abi.fno_stage(_abi.fno_stage_table(A, dev), _dev(src, dev), dst, M, K, ncol, slabs)
+    x = np.float64(np.float32(src))
+    got = dst.double().cpu().numpy()
+    ref, scale = np.matmul(_bf16(A), x), np.matmul(np.abs(_bf16(A)), np.abs(x))
+    assert (np.abs(got[:-64].reshape(slabs, M, ncol) - ref) <= BOUND * scale).all()
+    assert (got[-64:] == 7.0).all()
 
 
 @pytest.mark.parametrize("n,C,cin,m,spectral,factor", [(32, 32, 32, 12, True, True), (64, 20, 20, 6, True, True),

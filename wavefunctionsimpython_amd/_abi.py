@@ -55,6 +55,7 @@ SIGNATURES = {
     "wfs_fno_layer": (ctypes.c_int, [_vp] * 9 + [ctypes.c_int] * 5 + [_vp]),
     "wfs_fno_modes": (ctypes.c_int, [_vp] * 4 + [ctypes.c_int] * 2 + [_vp]),
     "wfs_fno_layer_backward": (ctypes.c_int, [_vp] * 8 + [ctypes.c_int] * 4 + [_vp]),
+    "wfs_fno_stage": (ctypes.c_int, [_vp] * 3 + [ctypes.c_int] * 3 + [ctypes.c_long, _vp]),
     "wfs_fno_weight_grad": (ctypes.c_int, [_vp] * 4 + [ctypes.c_int] * 2 + [ctypes.c_long, _vp, ctypes.c_long, _vp]),
     "wfs_fno_modes_backward": (ctypes.c_int, [_vp] * 7 + [ctypes.c_int] * 2 + [_vp]),
     "wfs_fno_pack": (ctypes.c_int, [_vp, ctypes.c_int, _vp, ctypes.c_float, ctypes.c_float, _vp, ctypes.c_long,
@@ -534,6 +535,25 @@ def _check_f32(tensors) -> None:
         _require_device_any(t, name)
         if t.dtype != torch.float32 or not t.is_contiguous() or t.numel() < size:
             raise ValueError(f"{name} must be a contiguous float32 tensor of at least {size} elements")
+
+
+def fno_stage_table(A: np.ndarray, device) -> torch.Tensor:
+    """A transform table [M][K] as wfs_fno_stage reads it: bf16, rows padded to 32, columns to 16."""
+    M, K = A.shape
+    t = torch.zeros((-(-M // 32) * 32, -(-K // 16) * 16), dtype=torch.float32)
+    t[:M, :K] = torch.from_numpy(np.ascontiguousarray(A, dtype=np.float32))
+    return t.to(torch.bfloat16).to(device).contiguous()
+
+
+def fno_stage(A: torch.Tensor, src: torch.Tensor, dst: torch.Tensor, M: int, K: int, ncol: int, slabs: int,
+              stream=None) -> None:
+    """dst[s][i][c] = sum_k A[i][k] src[s][k][c] (``wfs_fno_stage``); A from fno_stage_table."""
+    _require_device_any(A, "A")
+    if A.dtype != torch.bfloat16 or not A.is_contiguous() or tuple(A.shape) != (-(-M // 32) * 32, -(-K // 16) * 16):
+        raise ValueError(f"A must be the padded bf16 table of a {M} x {K} stage")
+    _check_f32([(src, slabs * K * ncol, "src"), (dst, slabs * M * ncol, "dst")])
+    check(lib().wfs_fno_stage(ptr(A), ptr(src), ptr(dst), int(M), int(K), int(ncol), int(slabs), stream_handle(stream)),
+          "wfs_fno_stage")
 
 
 def fno_layer_backward(W: torch.Tensor, g: torch.Tensor, Tg: torch.Tensor | None, u: torch.Tensor | None,

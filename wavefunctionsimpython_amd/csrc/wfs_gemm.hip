@@ -495,6 +495,142 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
 }
 
 // ---------------------------------------------------------------------------
+// One stage of the truncated DFT along an axis between the z stages: for every slab s
+//   out[s][i][c] = sum_k A[i][k] in[s][k][c],   c < ncol,
+// A a transform table in bf16 ([ceil32(M)][ceil16(K)], zero padded), in as bf16 hi + lo, FP32
+// accumulation (the operand rounding of wfs_gemm_bf16).  The columns of all slabs are numbered
+// through, so a tile of 32 columns is full for any ncol; a tile's A fragments (8 consecutive k of a
+// row) are one 16-byte load each, its B fragments eight loads of 32 columns each, both straight
+// from memory: no LDS on the way to the matrix cores and no barriers.
+//
+// Reducing stages (M = 2 m <= 32 rows, K = 2 n): the block's four wavefronts take a quarter of k
+// each and add their tiles in LDS, so that the x stage (m^2 columns per channel, 144 tiles at 12
+// modes and 32 channels) still has four wavefronts a tile.  Expanding stages (K = 2 m <= 32,
+// M = 2 n): a wavefront holds its tile's B fragments and the four wavefronts share the rows.
+// The strided GEMM staged both operands element by element through LDS with 64-bit index
+// arithmetic, a 32 x 32 tile per 12 useful columns: per launch at 128^3, C = 32, m = 12 (y, x,
+// inverse x, inverse y) 44, 23, 7, 33 us; here 16, 5, 5, 15 (the y stages move 63 MB: 4 TB/s).
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ s16x8 load_a8(const unsigned short* __restrict__ A, long at) {
+  return *reinterpret_cast<const s16x8*>(A + at);
+}
+
+// eight rows k0 .. k0 + 7 of a column, rows from K on zero (their addresses clamped)
+__device__ __forceinline__ void load_b8(const float* __restrict__ col, int ncol, int k0, int K, float (&x)[8]) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) x[j] = col[long(k0 + j < K ? k0 + j : K - 1) * ncol];
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    if (k0 + j >= K) x[j] = 0.0f;
+}
+
+__device__ __forceinline__ void split8v(const float (&x)[8], s16x8& hi, s16x8& lo) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const unsigned short h = f32_to_bf16(x[j]);
+    hi[j] = (short)h;
+    lo[j] = (short)f32_to_bf16(x[j] - __uint_as_float(unsigned(h) << 16));
+  }
+}
+
+// M <= 32
+__global__ __launch_bounds__(256) void fno_reduce_stage_kernel(const unsigned short* __restrict__ A,
+                                                               const float* __restrict__ in, float* __restrict__ out,
+                                                               int M, int K, int ncol, long cols) {
+  __shared__ float red[3][64][17];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int half = lane >> 5;
+  const long j = long(blockIdx.x) * 32 + (lane & 31);
+  const long jj = j < cols ? j : cols - 1;
+  const long slab = jj / ncol;
+  const int c = int(jj - slab * ncol);
+  const float* __restrict__ col = in + slab * K * ncol + c;
+  const int kp = (K + 15) / 16 * 16;
+  const long arow = long(lane & 31) * kp;
+  f32x16 acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+  // k steps of 16: wavefront w takes steps w, w + 4, ...; a lane half takes 8 consecutive k
+  const int steps = kp / 16;
+  for (int s = wave; s < steps; s += 8) {
+    // two steps' loads in flight together (past the last step: zero fragments)
+    float x[2][8];
+    s16x8 a[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int k0 = 16 * (s + 4 * u) + 8 * half;
+      load_b8(col, ncol, k0, K, x[u]);
+      a[u] = load_a8(A, arow + (k0 < kp ? k0 : 8 * half));
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      s16x8 bh, bl;
+      split8v(x[u], bh, bl);
+      acc = mfma16(a[u], bl, acc);
+      acc = mfma16(a[u], bh, acc);
+    }
+  }
+  if (wave) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) red[wave - 1][lane][i] = acc[i];
+  }
+  __syncthreads();
+  if (wave == 0 && j < cols) {
+    float* __restrict__ o = out + slab * M * ncol + c;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int row = 8 * (i / 4) + 4 * half + i % 4;
+      const float v = (acc[i] + red[0][lane][i]) + (red[1][lane][i] + red[2][lane][i]);
+      if (row < M) o[long(row) * ncol] = v;
+    }
+  }
+}
+
+// K <= 32; blockIdx.y: this block's share of the 32-row tiles
+__global__ __launch_bounds__(256) void fno_expand_stage_kernel(const unsigned short* __restrict__ A,
+                                                               const float* __restrict__ in, float* __restrict__ out,
+                                                               int M, int K, int ncol, long cols) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int half = lane >> 5;
+  const long j = long(blockIdx.x) * 32 + (lane & 31);
+  const long jj = j < cols ? j : cols - 1;
+  const long slab = jj / ncol;
+  const int c = int(jj - slab * ncol);
+  const float* __restrict__ col = in + slab * K * ncol + c;
+  const int kp = (K + 15) / 16 * 16;
+  s16x8 bh[2], bl[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    float x[8];
+    load_b8(col, ncol, 16 * s + 8 * half, K, x);
+    split8v(x, bh[s], bl[s]);
+  }
+  float* __restrict__ o = out + slab * M * ncol + c;
+  const int tiles = (M + 31) / 32;
+  for (int t = int(blockIdx.y) * 4 + wave; t < tiles; t += 4 * int(gridDim.y)) {
+    const long arow = long(32 * t + (lane & 31)) * kp + 8 * half;
+    f32x16 acc;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+    const s16x8 a0 = load_a8(A, arow);
+    acc = mfma16(a0, bl[0], acc);
+    acc = mfma16(a0, bh[0], acc);
+    if (kp > 16) {
+      const s16x8 a1 = load_a8(A, arow + 16);
+      acc = mfma16(a1, bl[1], acc);
+      acc = mfma16(a1, bh[1], acc);
+    }
+    if (j < cols) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int row = 32 * t + 8 * (i / 4) + 4 * half + i % 4;
+        if (row < M) o[long(row) * ncol] = acc[i];
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Complex per-mode channel mixing of the Fourier neural operator:
 //   O[o][q] = sum_i R[q][i][o] X[i][q]     (complex: Or = Rr Xr - Ri Xi, Oi = Ri Xr + Rr Xi)
 // for m3 modes q and C channels, with the GEMM path's operand rounding (R plain bf16,
@@ -799,6 +935,33 @@ extern "C" int wfs_fno_weight_grad(const float* g, const float* v, float* gW, fl
   hipLaunchKernelGGL(fno_weight_grad_kernel, dim3(unsigned(blocks)), dim3(256), 0, s, g, v, work, C, cin, P);
   WFS_HIP_CHECK(hipGetLastError());
   hipLaunchKernelGGL(fno_weight_grad_sum_kernel, dim3(33), dim3(512), 0, s, work, int(blocks), gW, gb, C, cin);
+  WFS_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
+extern "C" int wfs_fno_stage(const void* A, const float* in, float* out, int M, int K, int ncol, long slabs,
+                             void* stream) {
+  if (!A || !in || !out) { set_last_error("wfs_fno_stage: null argument"); return WFS_ERR_INVALID; }
+  if (M < 1 || K < 1 || ncol < 1 || slabs < 1 || (M > 32 && K > 32) || M > 1 << 20 || K > 1 << 20) {
+    set_last_error("wfs_fno_stage: needs M <= 32 or K <= 32 (M=%d K=%d ncol=%d slabs=%ld)", M, K, ncol, slabs);
+    return WFS_ERR_UNSUPPORTED;
+  }
+  if (reinterpret_cast<unsigned long>(A) % 16) { set_last_error("wfs_fno_stage: A must be 16-byte aligned"); return WFS_ERR_INVALID; }
+  const long cols = slabs * ncol;
+  const long blocks = (cols + 31) / 32;
+  if (blocks > 0x7fffffffL) { set_last_error("wfs_fno_stage: too many columns"); return WFS_ERR_INVALID; }
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const unsigned short* a = static_cast<const unsigned short*>(A);
+  if (M <= 32) {
+    hipLaunchKernelGGL(fno_reduce_stage_kernel, dim3(unsigned(blocks)), dim3(256), 0, s, a, in, out, M, K, ncol, cols);
+  } else {
+    // few columns (the inverse x stage): the row tiles over several blocks as well
+    const long tiles = (M + 31) / 32;
+    const long share = (tiles + 3) / 4;
+    const unsigned gy = unsigned(blocks < 512 ? share : 1);
+    hipLaunchKernelGGL(fno_expand_stage_kernel, dim3(unsigned(blocks), gy), dim3(256), 0, s, a, in, out, M, K, ncol,
+                       cols);
+  }
   WFS_HIP_CHECK(hipGetLastError());
   return 0;
 }

@@ -119,6 +119,10 @@ class FNO3d:
         self.adam_step = 0
         t = dft_tables(self.n, self.m)
         self.tab = {k: torch.from_numpy(v).to(self.device, self.dtype).contiguous() for k, v in t.items()}
+        # the y and x stages' tables (and their transposes) for their own kernel
+        self._stage_tab = ({k: _abi.fno_stage_table(a, self.device) for k, a in
+                            (("F2", t["F2"]), ("F2t", t["F2"].T), ("G2", t["G2"]), ("G2t", t["G2"].T))}
+                           if self._native and 2 * self.m <= 32 else None)
         self.ones = torch.ones(1, dtype=self.dtype, device=self.device)
         self._ws = None
         self._saved = None
@@ -169,15 +173,14 @@ class FNO3d:
         layer's modes go (default the workspace); training keeps them for the backward pass."""
         ws = self._workspace()
         C, n, m = self.C, self.n, self.m
-        m2, m3, tm = m * m, m ** 3, 2 * m
-        tb = self.tab
+        m2 = m * m
         T, U, O, Y, Z = ws["T"], ws["U"], ws["O"], ws["Y"], ws["Z"]
         X = ws["X"] if X is None else X
-        self._gemm(tb["F2"], T, U, C * n, tm, m, 2 * n, (0, 2 * n, 1), (2 * n * m, m, 1), (tm * m, m, 1), flags=SB)
-        self._gemm(tb["F2"], U, X, C, tm, m2, 2 * n, (0, 2 * n, 1), (2 * n * m2, m2, 1), (tm * m2, m2, 1), flags=SB)
+        self._stage("F2", T, U, C * n, m)
+        self._stage("F2", U, X, C, m2)
         self._modes(self.params[f"Rr{l}"], self.params[f"Ri{l}"], X, O)
-        self._gemm(tb["G2"], O, Y, C, 2 * n, m2, tm, (0, tm, 1), (tm * m2, m2, 1), (2 * n * m2, m2, 1), flags=SB)
-        self._gemm(tb["G2"], Y, Z, C * n, 2 * n, m, tm, (0, tm, 1), (tm * m, m, 1), (2 * n * m, m, 1), flags=SB)
+        self._stage("G2", O, Y, C, m2)
+        self._stage("G2", Y, Z, C * n, m)
 
     def _modes(self, Rr, Ri, X, O) -> None:
         """O = R (.) X per mode, complex (Or = Rr Xr - Ri Xi, Oi = Ri Xr + Rr Xi); X, O [C][2][m^3]."""
@@ -191,6 +194,18 @@ class FNO3d:
         self._gemm(Ri, Xi, Or, m3, C, 1, C, sR, sX, sX, alpha=-1.0, beta=1.0, flags=SB)
         self._gemm(Ri, Xr, Oi, m3, C, 1, C, sR, sX, sX, flags=SB)
         self._gemm(Rr, Xi, Oi, m3, C, 1, C, sR, sX, sX, beta=1.0, flags=SB)
+
+    def _stage(self, table: str, src: torch.Tensor, dst: torch.Tensor, slabs: int, ncol: int) -> None:
+        """dst[s] = A src[s] for the slabs s of ncol columns: A the y/x-stage table F2 [2m][2n],
+        G2 [2n][2m], or a transpose (F2t, G2t)."""
+        n, tm = self.n, 2 * self.m
+        M, K = (tm, 2 * n) if table in ("F2", "G2t") else (2 * n, tm)
+        if self._stage_tab is not None:
+            _abi.fno_stage(self._stage_tab[table], src, dst, M, K, ncol, slabs)
+            return
+        sA = (0, 1, M) if table.endswith("t") else (0, K, 1)
+        self._gemm(self.tab[table[:2]], src, dst, slabs, M, ncol, K, sA, (K * ncol, ncol, 1), (M * ncol, ncol, 1),
+                   flags=SB)
 
     def _layer(self, W, v, Z, bias, u, vn, T, cin: int, act: bool) -> None:
         """u = W v + Z Gz + bias, vn = GELU(u) or u, T = vn Fz in one pass over the grid lines."""
@@ -242,14 +257,13 @@ class FNO3d:
         modes) -> transposed forward x and y stages -> Zg (Tg and Zg may be one buffer)."""
         ws = self._workspace()
         C, n, m = self.C, self.n, self.m
-        m2, tm = m * m, 2 * m
-        tb = self.tab
+        m2 = m * m
         U, dX, O, Y = ws["U"], ws["X"], ws["O"], ws["Y"]
-        self._gemm(tb["G2"], Tg, Y, C * n, tm, m, 2 * n, (0, 1, tm), (2 * n * m, m, 1), (tm * m, m, 1), flags=SB)
-        self._gemm(tb["G2"], Y, O, C, tm, m2, 2 * n, (0, 1, tm), (2 * n * m2, m2, 1), (tm * m2, m2, 1), flags=SB)
+        self._stage("G2t", Tg, Y, C * n, m)
+        self._stage("G2t", Y, O, C, m2)
         self._modes_backward(l, X, O, dX)
-        self._gemm(tb["F2"], dX, U, C, 2 * n, m2, tm, (0, 1, 2 * n), (tm * m2, m2, 1), (2 * n * m2, m2, 1), flags=SB)
-        self._gemm(tb["F2"], U, Zg, C * n, 2 * n, m, tm, (0, 1, 2 * n), (tm * m, m, 1), (2 * n * m, m, 1), flags=SB)
+        self._stage("F2t", dX, U, C, m2)
+        self._stage("F2t", U, Zg, C * n, m)
 
     def _spectral_backward(self, dS: torch.Tensor, l: int, X: torch.Tensor, dv: torch.Tensor) -> None:
         """dv += d/dv of the spectral path given dS; accumulates dR_l (X: this layer's modes)."""
