@@ -275,7 +275,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(GemmArgs g) {
 // with g in v, T' (the gradient of the layer's z stage) in Z, W stored [cin][C], the two tables
 // exchanged, u in up (null: no factor) and no bias: what the composition writes and reads in
 // between (W^T g, its sum with the spectral term, the product with GELU') stays in registers.
-// At 64^3, C = 32: 59 us, against 150 us for the four launches it replaces (27 + 27 us for the two
+// At 64^3, C = 32: 47 us, against 150 us for the four launches it replaces (27 + 27 us for the two
 // GEMMs that write W^T g and add the spectral term, 23 for GELU', 73 for the z stage).
 // ---------------------------------------------------------------------------
 struct LayerArgs {
@@ -302,12 +302,13 @@ __device__ __forceinline__ void split4(const float (&x)[4], bf16x4& hi, bf16x4& 
   }
 }
 
-template <int NZC, bool BWD>
+template <int NZC, bool BWD, bool QUADS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void fno_layer_kernel(LayerArgs g) {
   constexpr int n = 32 * NZC;
   constexpr int GP = kBK + 4;                        // padded rows of the transform tables
   __shared__ unsigned short GzT[n][GP];              // A = Gz^T: [z][j]
   __shared__ unsigned short FzT[32][n + 4];          // B = Fz:   [j][z]
+  __shared__ float tiles[4][32][36];                 // per wavefront: a 32 x 32 (channel, z) chunk
   const int lane = threadIdx.x & 63;
   const int lc = lane & 31;
   const int kq = 4 * (lane >> 5);
@@ -336,8 +337,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
   __syncthreads();
 
   // 32-bit byte offsets from the buffers' base addresses (C * n^3 * 4 < 2^32); loads past
-  // the operand's extent read a clamped valid element and are zeroed, so no load is
-  // conditional
+  // the operand's extent read a valid element instead, whose weight (W, table) is zero, so no
+  // load is conditional; rows past C come out of no store
   const char* __restrict__ vb = reinterpret_cast<const char*>(g.v);
   const char* __restrict__ zb = reinterpret_cast<const char*>(g.Z);
   char* __restrict__ ub = reinterpret_cast<char*>(g.u);
@@ -348,15 +349,58 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
   const long stride = long(gridDim.x) * (blockDim.x / 64);
   // the A fragments of v^T for one 32-point chunk; the next chunk's (or the next line's
   // first chunk's) are loaded while the current one is computed
-  auto load_v = [&](unsigned ru, int ch, float (&x)[16]) {
-    const unsigned zoff = ru * n + 32 * ch + lc;
+  // QUADS (cin a multiple of 4): the channels 8 s + kq .. + 3 exist together or not at all, so four
+  // lane offsets and four scalar bases address all rows
+  unsigned vrow[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+  for (int s = 0; s < 4; ++s) vrow[s] = unsigned(8 * s + kq < cin ? 8 * s + kq : 0) * P + unsigned(lc);
+  auto load_v = [&](unsigned ru, int ch, float (&x)[16]) {
+    const unsigned at = ru * n + 32 * ch;
+    if constexpr (QUADS) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int c = 8 * s + kq + j;
-        x[4 * s + j] = *reinterpret_cast<const float*>(vb + ((c < cin ? unsigned(c) : unsigned(cin - 1)) * P + zoff) * 4u);
+        const char* __restrict__ base = vb + (long(j) * P + at) * 4;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) x[4 * s + j] = *reinterpret_cast<const float*>(base + vrow[s] * 4u);
       }
+    } else {
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int c = 8 * s + kq + j;
+          x[4 * s + j] =
+              *reinterpret_cast<const float*>(vb + ((c < cin ? unsigned(c) : unsigned(cin - 1)) * P + at + lc) * 4u);
+        }
+    }
+  };
+  // A chunk goes to and comes from memory as whole 128-byte lines: lane l holds z = 4 (l % 8) ..
+  // + 3 of channel 8 i + l / 8 in part i.  The wavefront's own LDS tile turns that into the
+  // matrix layout (four consecutive z of channel l % 32) and back.  Stored from the matrix layout,
+  // an instruction wrote 32-byte pieces of 32 channels, whose lines lie n^3 floats apart (a power
+  // of two at 64 and 128: one memory channel): a bare copy in that pattern takes 202 us at 128^3,
+  // in whole lines 114.  A 128^3 layer went from 250 to 188 us (422 to 246 where u is stored too,
+  // backward 401 to 285), a 64^3 one from 43 to 35 (46 to 38, 56 to 47).  What is left is those
+  // power-of-two strides: with 4 KiB more between channels a layer takes 170 us.  Loading up or Z
+  // a chunk or a line ahead was slower (backward 320 us, spilled registers).
+  float (*tile)[36] = tiles[threadIdx.x >> 6];
+  const int mc = lane >> 3, mz = 4 * (lane & 7);
+  auto to_memory = [&](char* base, unsigned at) {
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int c = 8 * i + mc;
+      const float4 y = *reinterpret_cast<const float4*>(&tile[c][mz]);
+      if (c < C) *reinterpret_cast<float4*>(base + (unsigned(c) * P + at + unsigned(mz)) * 4u) = y;
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+  auto load_up = [&](unsigned ru, int ch, float4 (&y)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const unsigned c = unsigned(8 * i + mc < C ? 8 * i + mc : C - 1);
+      y[i] = *reinterpret_cast<const float4*>(pb + (c * P + ru * n + 32 * ch + unsigned(mz)) * 4u);
+    }
   };
   float xv[16];
   long r = long(blockIdx.x) * (blockDim.x / 64) + (threadIdx.x >> 6);
@@ -368,14 +412,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
     for (int s = 0; s < 4; ++s) { Zh[s] = bf16x4{0, 0, 0, 0}; Zl[s] = bf16x4{0, 0, 0, 0}; }
     if (zb) {
       // four consecutive j per lane: one 16-byte load (tm is a multiple of 4, so a quad lies
-      // wholly inside or wholly past the row; past it, the row's last quad is read and dropped)
+      // wholly inside or wholly past the row; past it, the row's last quad meets zero table rows)
       const unsigned row = (lcC * unsigned(rows) + ru) * unsigned(tm);
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const int k0 = 8 * s + kq;
         const float4 y = *reinterpret_cast<const float4*>(zb + (row + unsigned(k0 < tm ? k0 : tm - 4)) * 4u);
-        const bool ok = k0 < tm && lc < C;
-        float x[4] = {ok ? y.x : 0.0f, ok ? y.y : 0.0f, ok ? y.z : 0.0f, ok ? y.w : 0.0f};
+        const float x[4] = {y.x, y.y, y.z, y.w};
         split4(x, Zh[s], Zl[s]);
       }
     }
@@ -386,9 +429,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
     const long rnext = r + stride;
     // chunk ch of this line from x (its loads were issued one chunk earlier)
     auto process = [&](int ch, float (&x)[16]) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        if (8 * (i / 4) + kq + (i % 4) >= cin) x[i] = 0.0f;   // channels past cin
+      float4 up[4];
+      if constexpr (BWD) {
+        if (pb) load_up(ru, ch, up);
+      }
       f32x16 acc;
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
@@ -422,41 +466,58 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
       }
       // lane: column c = lc; items 4q..4q+3: z = 32 ch + 8 q + kq + 0..3; the items of q = 2Q
       // and 2Q + 1 are the A operand of one 16-k step of T = v' Fz
+      const unsigned at = line + 32 * ch;
+      float gv[16];
+      if constexpr (BWD) {
+        if (pb) {
 #pragma unroll
-      for (int Q = 0; Q < 2; ++Q) {
-        bf16x4 ahq[2], alq[2], bq[2];
+          for (int i = 0; i < 4; ++i) *reinterpret_cast<float4*>(&tile[8 * i + mc][mz]) = up[i];
+          __builtin_amdgcn_wave_barrier();
+        }
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int q = 2 * Q + h;
-          float val[4], gv[4];
-          const unsigned off = (lcC * P + line + 32 * ch + 8 * q + kq) * 4u;
-          if constexpr (BWD) {
-            float4 up = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (pb) up = *reinterpret_cast<const float4*>(pb + off);
-            const float uv[4] = {up.x, up.y, up.z, up.w};
+        for (int q = 0; q < 4; ++q) {
+          float4 y = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+          if (pb) y = *reinterpret_cast<const float4*>(&tile[lc][8 * q + kq]);
+          const float uv[4] = {y.x, y.y, y.z, y.w};
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              val[j] = acc[4 * q + j];
-              gv[j] = lc < C ? (pb ? val[j] * gelu_grad(uv[j]) : val[j]) : 0.0f;
-            }
-          } else {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              val[j] = acc[4 * q + j] + bias_c;
-              gv[j] = lc < C ? (g.act ? gelu_f(val[j]) : val[j]) : 0.0f;
-            }
+          for (int j = 0; j < 4; ++j) {
+            const float val = acc[4 * q + j];
+            gv[4 * q + j] = pb ? val * gelu_grad(uv[j]) : val;
           }
-          if (lc < C) {
-            if (ub) *reinterpret_cast<float4*>(ub + off) = make_float4(val[0], val[1], val[2], val[3]);
-            if (nb) *reinterpret_cast<float4*>(nb + off) = make_float4(gv[0], gv[1], gv[2], gv[3]);
-          }
-          if (tb) {
-            split4(gv, ahq[h], alq[h]);
+        }
+        __builtin_amdgcn_wave_barrier();
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[i] = acc[i] + bias_c;
+        if (ub) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<float4*>(&tile[lc][8 * q + kq]) =
+                make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
+          to_memory(ub, at);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) gv[i] = g.act ? gelu_f(acc[i]) : acc[i];
+      }
+      if (nb) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<float4*>(&tile[lc][8 * q + kq]) =
+              make_float4(gv[4 * q], gv[4 * q + 1], gv[4 * q + 2], gv[4 * q + 3]);
+        to_memory(nb, at);
+      }
+      if (tb) {
+#pragma unroll
+        for (int Q = 0; Q < 2; ++Q) {
+          bf16x4 ahq[2], alq[2], bq[2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int q = 2 * Q + h;
+            const float gq[4] = {gv[4 * q], gv[4 * q + 1], gv[4 * q + 2], gv[4 * q + 3]};
+            split4(gq, ahq[h], alq[h]);
 #pragma unroll
             for (int j = 0; j < 4; ++j) bq[h][j] = (short)FzT[lc][32 * ch + 8 * q + kq + j];
           }
-        }
-        if (tb) {
           const s16x8 b = cat8(bq[0], bq[1]);
           accT = mfma16(cat8(alq[0], alq[1]), b, accT);
           accT = mfma16(cat8(ahq[0], ahq[1]), b, accT);
@@ -858,12 +919,16 @@ template <bool BWD>
 static void launch_layer(const LayerArgs& g, int n, hipStream_t s) {
   const long want = (g.rows + 3) / 4;
   const unsigned blocks = unsigned(want < 2048 ? want : 2048);
+#define WFS_LAYER(NZC)                                                                                    \
+  if (g.cin % 4 == 0) hipLaunchKernelGGL((fno_layer_kernel<NZC, BWD, true>), dim3(blocks), dim3(256), 0, s, g); \
+  else hipLaunchKernelGGL((fno_layer_kernel<NZC, BWD, false>), dim3(blocks), dim3(256), 0, s, g);
   switch (n / 32) {
-    case 1: hipLaunchKernelGGL((fno_layer_kernel<1, BWD>), dim3(blocks), dim3(256), 0, s, g); break;
-    case 2: hipLaunchKernelGGL((fno_layer_kernel<2, BWD>), dim3(blocks), dim3(256), 0, s, g); break;
-    case 3: hipLaunchKernelGGL((fno_layer_kernel<3, BWD>), dim3(blocks), dim3(256), 0, s, g); break;
-    default: hipLaunchKernelGGL((fno_layer_kernel<4, BWD>), dim3(blocks), dim3(256), 0, s, g); break;
+    case 1: WFS_LAYER(1) break;
+    case 2: WFS_LAYER(2) break;
+    case 3: WFS_LAYER(3) break;
+    default: WFS_LAYER(4) break;
   }
+#undef WFS_LAYER
 }
 
 // layer of the Fourier neural operator fused over grid lines (see fno_layer_kernel)
