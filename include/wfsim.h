@@ -423,6 +423,14 @@ int wfs_fno_layer(const float* W, const float* v, const float* Z, const float* b
                   const float* Fz, float* u, float* vn, float* T, int cin, int C, int n, int tm, int act,
                   void* stream);
 /*
+ * wfs_fno_last_layer (no reference counterpart): u = W v + Z Gz + b as wfs_fno_layer, and in the
+ * same pass out = base + rscale (Q u + qb), Q [cout][C] taken as bf16, base (may be NULL: zero) and
+ * out [cout][n^3], cout <= 2.  u [C][n^3] is stored where it is not NULL.  out may be base.
+ */
+int wfs_fno_last_layer(const float* W, const float* v, const float* Z, const float* bias, const float* Gz,
+                       const float* Q, const float* qb, const float* base, float rscale, float* u, float* out, int cin,
+                       int C, int cout, int n, int tm, void* stream);
+/*
  * Backward of the layers (no reference counterpart).
  *  wfs_fno_layer_backward  gn = (W^T g + Tg Fz^T) GELU'(u) and Tn = gn Gz^T in one pass over the
  *                          grid lines (the transposed wfs_fno_layer): g [cin][n^3], W [cin][C],

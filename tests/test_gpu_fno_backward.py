@@ -56,7 +56,7 @@ def test_modes_backward(dev, C, m3):
     t = [_dev(x, dev) for x in (Rr, Ri, X, dO, np.zeros_like(X), gr, gi)]
     _abi.fno_modes_backward(*t, m3, C)
     Rr, Ri = _bf16(Rr), _bf16(Ri)
-    X, dO, gr, gi = (np.float64(np.float32(x)) for x in (X, dO, gr, gi))
+    X, dO, gr, gi = (x.astype(np.float32).astype(np.float64) for x in (X, dO, gr, gi))
     (xr, xi), (dr, di) = X.transpose(1, 2, 0), dO.transpose(1, 2, 0)          # [q][c]
     want = {5: gr + xr[:, :, None] * dr[:, None] + xi[:, :, None] * di[:, None],
             6: gi + xr[:, :, None] * di[:, None] - xi[:, :, None] * dr[:, None]}
@@ -113,3 +113,31 @@ def test_layer_backward(dev, n, C, cin, m, spectral, factor):
     tscale = got.abs().reshape(-1, n) @ Gd.abs().t()
     # (the sine of frequency 0 is zero on both sides)
     assert bool(((Tn.double().reshape(-1, tm) - want).abs() <= BOUND * tscale).all())
+
+
+@pytest.mark.parametrize("n,C,cin,cout,m,spectral,residual,keep", [(32, 32, 32, 2, 12, True, True, False),
+                                                                   (64, 20, 20, 1, 6, True, False, True),
+                                                                   (96, 7, 5, 2, 16, False, True, True)])
+def test_last_layer(dev, n, C, cin, cout, m, spectral, residual, keep):
+    rng = np.random.default_rng(n + cout)
+    tm, P = 2 * m, n ** 3
+    Gz = dft_tables(n, m)["Gz"]
+    W, v, b = rng.standard_normal((C, cin)), rng.standard_normal((cin, P)), rng.standard_normal(C)
+    Z, Q, qb = rng.standard_normal((C, n * n, tm)), rng.standard_normal((cout, C)), rng.standard_normal(cout)
+    base = rng.standard_normal((cout, P))
+    W_, v_, b_, Z_, Gz_, Q_, qb_, base_ = (_dev(x, dev) for x in (W, v, b, Z, Gz, Q, qb, base))
+    u = torch.empty(C * P, dtype=torch.float32, device=dev) if keep else None
+    out = torch.empty(cout * P, dtype=torch.float32, device=dev)
+    _abi.fno_last_layer(W_, v_, Z_ if spectral else None, b_, Gz_, Q_, qb_, base_ if residual else None, 0.5, u, out,
+                        cin, C, cout, n, tm)
+    Wd, Gd, Qd = (torch.from_numpy(_bf16(x)).to(dev) for x in (W, Gz, Q))
+    ref = Wd @ v_.double() + b_.double()[:, None]
+    scale = Wd.abs() @ v_.double().abs() + b_.double().abs()[:, None]
+    if spectral:
+        ref = ref + (Z_.double().reshape(-1, tm) @ Gd).reshape(C, P)
+        scale = scale + (Z_.double().abs().reshape(-1, tm) @ Gd.abs()).reshape(C, P)
+    if keep:
+        assert bool(((u.double().reshape(C, P) - ref).abs() <= BOUND * scale).all())
+    want = 0.5 * (Qd @ ref + qb_.double()[:, None]) + (base_.double() if residual else 0.0)
+    oscale = Qd.abs() @ scale + qb_.double().abs()[:, None] + base_.double().abs()
+    assert bool(((out.double().reshape(cout, P) - want).abs() <= BOUND * oscale).all())

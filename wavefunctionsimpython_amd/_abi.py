@@ -54,6 +54,7 @@ SIGNATURES = {
     "wfs_fno_axpby": (ctypes.c_int, [_vp, _vp, ctypes.c_float, ctypes.c_float, ctypes.c_long, _vp]),
     "wfs_fno_layer": (ctypes.c_int, [_vp] * 9 + [ctypes.c_int] * 5 + [_vp]),
     "wfs_fno_modes": (ctypes.c_int, [_vp] * 4 + [ctypes.c_int] * 2 + [_vp]),
+    "wfs_fno_last_layer": (ctypes.c_int, [_vp] * 8 + [ctypes.c_float] + [_vp] * 2 + [ctypes.c_int] * 5 + [_vp]),
     "wfs_fno_layer_backward": (ctypes.c_int, [_vp] * 8 + [ctypes.c_int] * 4 + [_vp]),
     "wfs_fno_stage": (ctypes.c_int, [_vp] * 3 + [ctypes.c_int] * 3 + [ctypes.c_long, _vp]),
     "wfs_fno_weight_grad": (ctypes.c_int, [_vp] * 4 + [ctypes.c_int] * 2 + [ctypes.c_long, _vp, ctypes.c_long, _vp]),
@@ -554,6 +555,20 @@ def fno_stage(A: torch.Tensor, src: torch.Tensor, dst: torch.Tensor, M: int, K: 
     _check_f32([(src, slabs * K * ncol, "src"), (dst, slabs * M * ncol, "dst")])
     check(lib().wfs_fno_stage(ptr(A), ptr(src), ptr(dst), int(M), int(K), int(ncol), int(slabs), stream_handle(stream)),
           "wfs_fno_stage")
+
+
+def fno_last_layer(W: torch.Tensor, v: torch.Tensor, Z: torch.Tensor | None, bias: torch.Tensor, Gz: torch.Tensor,
+                   Q: torch.Tensor, qb: torch.Tensor, base: torch.Tensor | None, rscale: float,
+                   u: torch.Tensor | None, out: torch.Tensor, cin: int, C: int, cout: int, n: int, tm: int,
+                   stream=None) -> None:
+    """u = W v + Z Gz + b and out = base + rscale (Q u + qb) in one pass (``wfs_fno_last_layer``)."""
+    P = n ** 3
+    _check_f32([(W, C * cin, "W"), (v, cin * P, "v"), (Z, C * n * n * tm, "Z"), (bias, C, "bias"), (Gz, tm * n, "Gz"),
+                (Q, cout * C, "Q"), (qb, cout, "qb"), (base, cout * P, "base"), (u, C * P, "u"), (out, cout * P, "out")])
+    opt = [ptr(t) if t is not None else None for t in (Z, base, u)]
+    check(lib().wfs_fno_last_layer(ptr(W), ptr(v), opt[0], ptr(bias), ptr(Gz), ptr(Q), ptr(qb), opt[1], float(rscale),
+                                   opt[2], ptr(out), int(cin), int(C), int(cout), int(n), int(tm),
+                                   stream_handle(stream)), "wfs_fno_last_layer")
 
 
 def fno_layer_backward(W: torch.Tensor, g: torch.Tensor, Tg: torch.Tensor | None, u: torch.Tensor | None,

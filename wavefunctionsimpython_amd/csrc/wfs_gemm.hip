@@ -277,6 +277,11 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(GemmArgs g) {
 // between (W^T g, its sum with the spectral term, the product with GELU') stays in registers.
 // At 64^3, C = 32: 47 us, against 150 us for the four launches it replaces (27 + 27 us for the two
 // GEMMs that write W^T g and add the spectral term, 23 for GELU', 73 for the z stage).
+//
+// LAYER_LAST: the last layer with the projection, out = base + rscale (Q u + qb) for one or two
+// rows (Q bf16 as in the GEMM, u FP32): the lanes sum their half of the channels of one z from the
+// chunk's LDS tile.  Without it the layer wrote u and a GEMM with 2 useful rows of 32 and an
+// elementwise pass read it back: 161 + 79 + 14 us at 128^3, C = 32; here 111 (165 where u is stored).
 // ---------------------------------------------------------------------------
 struct LayerArgs {
   const float* W;
@@ -290,8 +295,16 @@ struct LayerArgs {
   float* T;            // may be null
   int cin, C, tm, act;
   long rows;           // lines (n * n)
-  const float* up;     // backward form: pre-activations [C][n^3] whose GELU' multiplies vn (may be null)
+  const float* up = nullptr;   // backward form: pre-activations [C][n^3] whose GELU' multiplies vn (may be null)
+  // last form: out = base + rscale (Q u + qb), cout <= 2 rows
+  const float* Q = nullptr;    // [cout][C]
+  const float* qb = nullptr;
+  const float* base = nullptr; // [cout][n^3] (may be null: zero)
+  float* out = nullptr;        // [cout][n^3]
+  float rscale = 1.0f;
+  int cout = 0;
 };
+enum { LAYER_FORWARD = 0, LAYER_BACKWARD = 1, LAYER_LAST = 2 };
 
 __device__ __forceinline__ void split4(const float (&x)[4], bf16x4& hi, bf16x4& lo) {
 #pragma unroll
@@ -302,8 +315,9 @@ __device__ __forceinline__ void split4(const float (&x)[4], bf16x4& hi, bf16x4& 
   }
 }
 
-template <int NZC, bool BWD, bool QUADS>
+template <int NZC, int MODE, bool QUADS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void fno_layer_kernel(LayerArgs g) {
+  constexpr bool BWD = MODE == LAYER_BACKWARD;
   constexpr int n = 32 * NZC;
   constexpr int GP = kBK + 4;                        // padded rows of the transform tables
   __shared__ unsigned short GzT[n][GP];              // A = Gz^T: [z][j]
@@ -324,6 +338,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
     const float fz = j < tm && (BWD ? g.Z : g.T) ? g.Fz[z * tm + j] : 0.0f;
     GzT[z][j] = f32_to_bf16(BWD ? fz : gz);
     FzT[j][z] = f32_to_bf16(BWD ? gz : fz);
+  }
+  __shared__ float proj[2][MODE == LAYER_LAST ? 32 : 1];   // the projection's rows (bf16 values)
+  if constexpr (MODE == LAYER_LAST) {
+    if (threadIdx.x < 64) {
+      const int o = threadIdx.x >> 5, c = threadIdx.x & 31;
+      proj[o][c] = o < g.cout && c < C ? __uint_as_float(unsigned(f32_to_bf16(g.Q[o * C + c])) << 16) : 0.0f;
+    }
   }
   bf16x4 Wf[4];                                      // B = W^T: (k = c_in, n = c_out = lc)
 #pragma unroll
@@ -384,6 +405,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
   // power-of-two strides: with 4 KiB more between channels a layer takes 170 us.  Loading up or Z
   // a chunk or a line ahead was slower (backward 320 us, spilled registers).
   float (*tile)[36] = tiles[threadIdx.x >> 6];
+  const float qbias = MODE == LAYER_LAST && (kq >> 2) < g.cout ? g.qb[kq >> 2] : 0.0f;
   const int mc = lane >> 3, mz = 4 * (lane & 7);
   auto to_memory = [&](char* base, unsigned at) {
     __builtin_amdgcn_wave_barrier();
@@ -489,12 +511,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
       } else {
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[i] = acc[i] + bias_c;
-        if (ub) {
+        if (ub || MODE == LAYER_LAST) {
 #pragma unroll
           for (int q = 0; q < 4; ++q)
             *reinterpret_cast<float4*>(&tile[lc][8 * q + kq]) =
                 make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
-          to_memory(ub, at);
+          if (ub) to_memory(ub, at);
+        }
+        if constexpr (MODE == LAYER_LAST) {
+          // lane: z = lc, channels 16 (l / 32) ..; then the other half's sums, and half o stores row o
+          __builtin_amdgcn_wave_barrier();
+          float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const float y = tile[4 * kq + i][lc];
+            s0 = __builtin_fmaf(proj[0][4 * kq + i], y, s0);
+            s1 = __builtin_fmaf(proj[1][4 * kq + i], y, s1);
+          }
+          __builtin_amdgcn_wave_barrier();
+          const float mine = kq ? s1 : s0, other = __shfl_xor(kq ? s0 : s1, 32, 64);
+          const int o = kq >> 2;
+          if (o < g.cout) {
+            const unsigned e = unsigned(o) * P + at + unsigned(lc);
+            const float y = g.rscale * (mine + other + qbias);
+            g.out[e] = g.base ? g.base[e] + y : y;
+          }
+          return;
         }
 #pragma unroll
         for (int i = 0; i < 16; ++i) gv[i] = g.act ? gelu_f(acc[i]) : acc[i];
@@ -915,13 +957,13 @@ extern "C" int wfs_fno_modes(const float* Rr, const float* Ri, const float* X, f
 }
 
 // one wavefront per line, four per block
-template <bool BWD>
+template <int MODE>
 static void launch_layer(const LayerArgs& g, int n, hipStream_t s) {
   const long want = (g.rows + 3) / 4;
   const unsigned blocks = unsigned(want < 2048 ? want : 2048);
 #define WFS_LAYER(NZC)                                                                                    \
-  if (g.cin % 4 == 0) hipLaunchKernelGGL((fno_layer_kernel<NZC, BWD, true>), dim3(blocks), dim3(256), 0, s, g); \
-  else hipLaunchKernelGGL((fno_layer_kernel<NZC, BWD, false>), dim3(blocks), dim3(256), 0, s, g);
+  if (g.cin % 4 == 0) hipLaunchKernelGGL((fno_layer_kernel<NZC, MODE, true>), dim3(blocks), dim3(256), 0, s, g); \
+  else hipLaunchKernelGGL((fno_layer_kernel<NZC, MODE, false>), dim3(blocks), dim3(256), 0, s, g);
   switch (n / 32) {
     case 1: WFS_LAYER(1) break;
     case 2: WFS_LAYER(2) break;
@@ -950,8 +992,34 @@ extern "C" int wfs_fno_layer(const float* W, const float* v, const float* Z, con
     set_last_error("wfs_fno_layer: u, vn and Z must be 16-byte aligned");
     return WFS_ERR_INVALID;
   }
-  const LayerArgs g{W, v, Z, bias, Gz, Fz, u, vn, T, cin, C, tm, act, long(n) * n, nullptr};
-  launch_layer<false>(g, n, static_cast<hipStream_t>(stream));
+  const LayerArgs g{W, v, Z, bias, Gz, Fz, u, vn, T, cin, C, tm, act, long(n) * n};
+  launch_layer<LAYER_FORWARD>(g, n, static_cast<hipStream_t>(stream));
+  WFS_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
+extern "C" int wfs_fno_last_layer(const float* W, const float* v, const float* Z, const float* bias, const float* Gz,
+                                  const float* Q, const float* qb, const float* base, float rscale, float* u,
+                                  float* out, int cin, int C, int cout, int n, int tm, void* stream) {
+  if (!W || !v || !bias || !Q || !qb || !out || (Z && !Gz)) { set_last_error("wfs_fno_last_layer: null argument"); return WFS_ERR_INVALID; }
+  if (n % 32 != 0 || n < 32 || n > 128 || C < 1 || C > 32 || cin < 1 || cin > 32 || cout < 1 || cout > 2 || tm < 4 ||
+      tm > 32 || tm % 4) {
+    set_last_error("wfs_fno_last_layer: needs n in {32, 64, 96, 128}, C, cin <= 32, cout <= 2 and tm a multiple of 4 "
+                   "up to 32 (n=%d C=%d cin=%d cout=%d tm=%d)", n, C, cin, cout, tm);
+    return WFS_ERR_UNSUPPORTED;
+  }
+  if ((reinterpret_cast<unsigned long>(u) % 16) != 0 || (reinterpret_cast<unsigned long>(Z) % 16) != 0) {
+    set_last_error("wfs_fno_last_layer: u and Z must be 16-byte aligned");
+    return WFS_ERR_INVALID;
+  }
+  LayerArgs g{W, v, Z, bias, Gz, nullptr, u, nullptr, nullptr, cin, C, tm, 0, long(n) * n};
+  g.Q = Q;
+  g.qb = qb;
+  g.base = base;
+  g.out = out;
+  g.rscale = rscale;
+  g.cout = cout;
+  launch_layer<LAYER_LAST>(g, n, static_cast<hipStream_t>(stream));
   WFS_HIP_CHECK(hipGetLastError());
   return 0;
 }
@@ -971,7 +1039,7 @@ extern "C" int wfs_fno_layer_backward(const float* W, const float* g, const floa
     return WFS_ERR_INVALID;
   }
   const LayerArgs a{W, g, Tg, nullptr, Gz, Fz, nullptr, gn, Tn, cin, C, tm, 0, long(n) * n, u};
-  launch_layer<true>(a, n, static_cast<hipStream_t>(stream));
+  launch_layer<LAYER_BACKWARD>(a, n, static_cast<hipStream_t>(stream));
   WFS_HIP_CHECK(hipGetLastError());
   return 0;
 }

@@ -320,6 +320,17 @@ class FNO3d:
             for l in range(self.L):
                 self._spectral_mid(l, modes_buffer())
                 last = l == self.L - 1
+                if last and self._native and self.cout <= 2:
+                    # the projection and the residual ride on the last layer; u only for training
+                    u = torch.empty(C * P, dtype=self.dtype, device=self.device) if keep else None
+                    _abi.fno_last_layer(pr[f"W{l}"], v, ws["Z"], pr[f"b{l}"], self.tab["Gz"], pr["Q"], pr["qb"],
+                                        a if self.residual else None, self.rscale, u, ws["out"], C, C, self.cout,
+                                        self.n, 2 * self.m)
+                    if keep:
+                        saved_v.append(v)
+                        saved_u.append(u)
+                        self._saved = (a, saved_v, saved_u, u, saved_X)
+                    return ws["out"]
                 u = (torch.empty(C * P, dtype=self.dtype, device=self.device) if keep
                      else ws["d3"] if last else None)
                 vn = None if last else act_buffer(v)
