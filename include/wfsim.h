@@ -323,7 +323,8 @@ int wfs_potential_operator(long count, const void* V, double dt, int precision, 
 #define WFS_K_SLAB_EDGE 13
 #define WFS_K_SLAB_OBSERVE 14
 #define WFS_K_PV_PLANES 15
-#define WFS_K_COUNT 16
+#define WFS_K_YZ_SPLIT 16
+#define WFS_K_COUNT 17
 int wfs_plan_set_profiling(wfs_plan* plan, int enable);
 
 /*
@@ -358,6 +359,13 @@ int wfs_plan_set_profiling(wfs_plan* plan, int enable);
  * whose potential phase factors are bitwise equal (the planes away from walls
  * and absorbing x layers), so that those reads hit the caches instead of HBM;
  * variant 0 reads every plane's own copy.  The results are bit-identical.
+ * WFS_K_YZ_SPLIT (no launches of its own: they count as WFS_K_YZ_SLAB,
+ * WFS_K_X_SLAB and WFS_K_SLAB_EDGE): variant 1 (default where supported:
+ * complex128 grids with ny = nz in {64, 96, 128, 192} and nx <= 256, at 64 only
+ * below 192 x planes) runs the
+ * steps as the slab scheme's two launches, variant 0 as the plane pass or the
+ * axis passes; the results agree to rounding.  Setting WFS_K_YZ_PLANE or
+ * WFS_K_YZ_SLAB switches it off.
  */
 int wfs_plan_autotune(wfs_plan* plan, void* stream);
 int wfs_plan_set_variant(wfs_plan* plan, int kernel_class, int variant);

@@ -138,7 +138,9 @@ struct XSlabParams {
   long packets = 0;             // grids stacked along x
 };
 bool slab_supported(int precision, const int n[3]);
-// Per x plane (packets * nx planes of plane_elems complex64 factors, contiguous per plane): src[p]
+// the same two launches for complex128 planes (kernel class WFS_K_YZ_SPLIT)
+bool split_supported(int precision, const int n[3]);
+// Per x plane (packets * nx planes of plane_elems 64-bit words, contiguous per plane): src[p]
 // = the first plane of the run of bitwise-identical consecutive planes holding p, within its
 // packet.  flags: workspace of packets * nx ints.
 // flags[p] = plane p of the table equals plane p - 1 of its packet, for planes first .. first +
@@ -150,15 +152,15 @@ int launch_plane_dedup(const void* table, long plane_elems, int nx, int packets,
 struct SlabRows {
   int b, uy, uz, n1;
 };
-SlabRows slab_rows(int n);
+SlabRows slab_rows(int precision, int n);
 // the potential table order of the slab scheme's y-z launch (ny = nz = n)
-LinesOrder slab_lines_order(int n);
+LinesOrder slab_lines_order(int precision, int n);
 // YzPlaneParams.planes = packets * nx; variant 2 = persistent (one block per CU walking the
 // row groups, loading the next group during the current one's arithmetic), else one block
 // per group
-int launch_yz_slab(int n, int mode, int variant, void* data, const YzPlaneParams& p, hipStream_t s);
+int launch_yz_slab(int precision, int n, int mode, int variant, void* data, const YzPlaneParams& p, hipStream_t s);
 // variant 2: 8 z points per block, else 16
-int launch_x_slab(int nx, int n, int variant, void* data, const XSlabParams& p, hipStream_t s);
+int launch_x_slab(int precision, int nx, int n, int variant, void* data, const XSlabParams& p, hipStream_t s);
 
 // pv = cexp_i(-dt V) elementwise in the state precision
 int launch_potential_phase(int precision, long count, const float2* V, double dt, void* pv, hipStream_t s);

@@ -133,9 +133,19 @@ int upload_dithered(void** dst, const std::vector<double>& re, const std::vector
 // The twiddles W_L^{u k1} = W_N^{(M u k1) mod N} (u < U, k1 < K) of the length-L lines
 // of the slab scheme's y-z launch, each copy laid out [u][k1] so that a thread's K twiddles
 // are contiguous (wide scalar loads); entry for entry the values of the dithered N-table.
-int upload_rows_table(void** dst, const std::vector<double>& re, const std::vector<double>& im, int M, int U,
-                      int K) {
+int upload_rows_table(void** dst, const std::vector<double>& re, const std::vector<double>& im, int M, int U, int K,
+                      int precision) {
   const long n = long(re.size());
+  if (precision == WFS_C128) {
+    std::vector<double> rr(size_t(U) * K), ri(size_t(U) * K);
+    for (int u = 0; u < U; ++u)
+      for (int k1 = 0; k1 < K; ++k1) {
+        const long j = (long(M) * u * k1) % n;
+        rr[size_t(u) * K + k1] = re[j];
+        ri[size_t(u) * K + k1] = im[j];
+      }
+    return upload_table(dst, rr, ri, precision);
+  }
   std::vector<float2> h(size_t(kDither) * U * K);
   for (int c = 0; c < kDither; ++c)
     for (int u = 0; u < U; ++u)
@@ -323,7 +333,8 @@ int run_pass(wfs_plan* p, int axis, int mode, void* data, const void* pv, const 
 
 size_t grid_points(const wfs_plan* p) { return size_t(p->batch) * p->n[0] * p->n[1] * p->n[2]; }
 
-bool slab_on(const wfs_plan* p) { return p->variant[WFS_K_YZ_SLAB] != 0; }
+// steps run as two launches: the complex64 slab scheme or its complex128 counterpart
+bool slab_on(const wfs_plan* p) { return p->variant[WFS_K_YZ_SLAB] != 0 || p->variant[WFS_K_YZ_SPLIT] != 0; }
 
 int alloc_table(wfs_plan* p, void** t, hipStream_t s) {
   if (*t) return 0;
@@ -352,7 +363,7 @@ int share_planes(wfs_plan* p, hipStream_t s) {
       return WFS_ERR_ALLOC;
     }
   }
-  WFS_TRY(launch_plane_dedup(p->pv_lines, long(p->n[1]) * p->n[2], p->n[0], p->batch, 0, planes,
+  WFS_TRY(launch_plane_dedup(p->pv_lines, long(p->n[1]) * p->n[2] * long(p->elem / 8), p->n[0], p->batch, 0, planes,
                              p->pv_planes + planes, p->pv_planes, s));
   p->pv_planes_ok = true;
   return 0;
@@ -365,7 +376,7 @@ int set_potential(wfs_plan* p, const void* V, hipStream_t s) {
   if (slab_on(p)) {
     WFS_TRY(alloc_table(p, &p->pv_lines, s));
     WFS_TRY(launch_potential_phase_lines(p->precision, count, static_cast<const float2*>(V), p->dt, p->pv_lines,
-                                         slab_lines_order(p->n[1]), s));
+                                         slab_lines_order(p->precision, p->n[1]), s));
     p->pv_lines_ok = true;
     p->pv_nat_ok = false;
     if (capturing(s)) p->pv_in_graph = true;
@@ -395,13 +406,13 @@ int set_potential_planes(wfs_plan* p, const void* V, int x_begin, int x_end, hip
   const float2* v = static_cast<const float2*>(V) + off;
   if (slab_on(p)) {
     WFS_TRY(launch_potential_phase_lines(p->precision, count, v, p->dt, static_cast<char*>(p->pv_lines) + off * p->elem,
-                                         slab_lines_order(p->n[1]), s));
+                                         slab_lines_order(p->precision, p->n[1]), s));
     p->pv_nat_ok = false;
     if (capturing(s)) p->pv_in_graph = true;
     if (p->pv_planes_ok && !capturing(s)) {
       const long planes = p->n[0];
       const long last = x_end < p->n[0] ? x_end : p->n[0] - 1;
-      WFS_TRY(launch_plane_dedup(p->pv_lines, plane, p->n[0], 1, x_begin, last - x_begin + 1, p->pv_planes + planes,
+      WFS_TRY(launch_plane_dedup(p->pv_lines, plane * long(p->elem / 8), p->n[0], 1, x_begin, last - x_begin + 1, p->pv_planes + planes,
                                  p->pv_planes, s));
     } else {
       WFS_TRY(share_planes(p, s));
@@ -423,7 +434,7 @@ int current_table(wfs_plan* p, hipStream_t s, const void** out) {
   if (slab_on(p)) {
     if (!p->pv_lines_ok) {
       WFS_TRY(alloc_table(p, &p->pv_lines, s));
-      WFS_TRY(launch_table_reorder(p->precision, count, p->pv, p->pv_lines, slab_lines_order(p->n[1]), true, s));
+      WFS_TRY(launch_table_reorder(p->precision, count, p->pv, p->pv_lines, slab_lines_order(p->precision, p->n[1]), true, s));
       p->pv_lines_ok = !capturing(s);
       p->pv_planes_ok = false;
       if (capturing(s)) p->pv_in_graph = true;
@@ -433,7 +444,7 @@ int current_table(wfs_plan* p, hipStream_t s, const void** out) {
   } else {
     if (!p->pv_nat_ok) {
       WFS_TRY(alloc_table(p, &p->pv, s));
-      WFS_TRY(launch_table_reorder(p->precision, count, p->pv_lines, p->pv, slab_lines_order(p->n[1]), false, s));
+      WFS_TRY(launch_table_reorder(p->precision, count, p->pv_lines, p->pv, slab_lines_order(p->precision, p->n[1]), false, s));
       p->pv_nat_ok = !capturing(s);
     }
     *out = p->pv;
@@ -497,7 +508,7 @@ int run_yz(wfs_plan* p, void* data, const void* pv, hipStream_t s, int sel) {
 // LINES_FULL), or the entry (z, y forward) / exit (y, z inverse) launch of a call
 int run_slab_lines(wfs_plan* p, int mode, void* data, const void* pv, hipStream_t s, int sel) {
   YzPlaneParams pp;
-  const SlabRows g = slab_rows(p->n[1]);
+  const SlabRows g = slab_rows(p->precision, p->n[1]);
   const int c = sel % p->ntab;
   pp.tw_yi = static_cast<const char*>(p->tw_rows[0]) + size_t(c) * g.uy * g.n1 * p->elem;
   pp.tw_yf = pp.tw_yi;
@@ -518,7 +529,7 @@ int run_slab_lines(wfs_plan* p, int mode, void* data, const void* pv, hipStream_
   pp.nx = p->n[0];
   pp.planes = long(p->batch) * p->n[0];
   ProfileScope scope(p, mode == LINES_FULL ? WFS_K_YZ_SLAB : WFS_K_SLAB_EDGE, s);
-  return launch_yz_slab(p->n[1], mode, p->variant[WFS_K_YZ_SLAB], data, pp, s);
+  return launch_yz_slab(p->precision, p->n[1], mode, p->variant[WFS_K_YZ_SLAB], data, pp, s);
 }
 
 // Slab scheme: length-4 y stages around x forward -> K -> x inverse
@@ -531,7 +542,7 @@ int run_x_slab(wfs_plan* p, void* data, const void* const* ktab, hipStream_t s, 
   xp.kz = table_copy(p, ktab[2], 2, sel);
   xp.packets = p->batch;
   ProfileScope scope(p, WFS_K_X_SLAB, s);
-  return launch_x_slab(p->n[0], p->n[1], p->variant[WFS_K_X_SLAB], data, xp, s);
+  return launch_x_slab(p->precision, p->n[0], p->n[1], p->variant[WFS_K_X_SLAB], data, xp, s);
 }
 
 // Slab scheme, observing launches: LINES_OBSERVE runs the exit launch of one stretch (table copy
@@ -541,7 +552,7 @@ int run_x_slab(wfs_plan* p, void* data, const void* const* ktab, hipStream_t s, 
 // The records (obs_lines) are allocated with the plan.
 int run_slab_observe(wfs_plan* p, int mode, void* data, int sel_exit, int sel_entry, const wfs_box* boxes, int nb,
                      double* out, hipStream_t s) {
-  const SlabRows g = slab_rows(p->n[1]);
+  const SlabRows g = slab_rows(p->precision, p->n[1]);
   const long groups = long(p->batch) * p->n[0] * g.b;
   if (p->obs_lines_len < groups * kBoxesPerPass * 7) {
     set_last_error("wfs_step_observe: observing records missing");
@@ -575,7 +586,7 @@ int run_slab_observe(wfs_plan* p, int mode, void* data, int sel_exit, int sel_en
   pp.mom.partials = p->obs_lines;
   {
     ProfileScope scope(p, WFS_K_SLAB_OBSERVE, s);
-    WFS_TRY(launch_yz_slab(p->n[1], mode, 1, data, pp, s));
+    WFS_TRY(launch_yz_slab(p->precision, p->n[1], mode, 1, data, pp, s));
   }
   ProfileScope scope(p, WFS_K_OBSERVABLES, s);
   return launch_sum_partials(p->obs_lines, long(p->n[0]) * g.b, nb, p->batch, p->dx[0] * p->dx[1] * p->dx[2] / 27.0,
@@ -596,7 +607,7 @@ int fourier_steps(wfs_plan* p, void* psi, const void* V, int nsteps, hipStream_t
   // one long call does
   const int b = p->step_index;
   p->step_index = int((long(b) + nsteps) % p->ntab);
-  if (p->variant[WFS_K_YZ_SLAB] != 0) {
+  if (slab_on(p)) {
     // two launches per step; between them y holds the half-transformed Y[b][ka]
     WFS_TRY(run_slab_lines(p, LINES_ENTRY, psi, nullptr, s, b));
     WFS_TRY(run_x_slab(p, psi, kh, s, b));
@@ -766,6 +777,8 @@ extern "C" int wfs_plan_create_batched(const int n[3], const double dx[3], doubl
   const bool slab = slab_supported(precision, n) && (n[1] != 128 || long(batch) * n[0] < 256);
   p->variant[WFS_K_YZ_SLAB] = slab ? (n[1] == 192 ? 1 : 2) : 0;
   if (slab) p->variant[WFS_K_X_SLAB] = n[1] == 192 ? 1 : 2;
+  const bool two_launch = slab_supported(precision, n) || split_supported(precision, n);
+  p->variant[WFS_K_YZ_SPLIT] = split_supported(precision, n) && (n[1] != 64 || n[0] < 192) ? 1 : 0;
   p->pending = new std::vector<std::pair<hipEvent_t, hipEvent_t>>[WFS_K_COUNT];
   p->event_pool = new std::vector<hipEvent_t>();
   int rc = 0;
@@ -778,10 +791,10 @@ extern "C" int wfs_plan_create_batched(const int n[3], const double dx[3], doubl
     }
     rc = upload_dithered(&p->tw[a], re, im, precision);
     if (rc) break;
-    if (a > 0 && slab_supported(precision, n)) {
-      const SlabRows g = slab_rows(n[1]);
-      rc = a == 1 ? upload_rows_table(&p->tw_rows[0], re, im, g.b, g.uy, g.n1)
-                  : upload_rows_table(&p->tw_rows[1], re, im, 1, g.uz, g.n1);
+    if (a > 0 && two_launch) {
+      const SlabRows g = slab_rows(precision, n[1]);
+      rc = a == 1 ? upload_rows_table(&p->tw_rows[0], re, im, g.b, g.uy, g.n1, precision)
+                  : upload_rows_table(&p->tw_rows[1], re, im, 1, g.uz, g.n1, precision);
       if (rc) break;
     }
     kinetic_table(n[a], dx[a], dt, mass, 2.0, re, im);
@@ -802,7 +815,7 @@ extern "C" int wfs_plan_create_batched(const int n[3], const double dx[3], doubl
   }
   if (rc == 0 && slab_supported(precision, n)) {
     // box-moment records of the slab scheme's observing launch: one per row group and box
-    const long need = long(batch) * n[0] * slab_rows(n[1]).b * kBoxesPerPass * 7;
+    const long need = long(batch) * n[0] * slab_rows(precision, n[1]).b * kBoxesPerPass * 7;
     hipError_t e = hipMalloc(reinterpret_cast<void**>(&p->obs_lines), size_t(need) * sizeof(double));
     if (e != hipSuccess) { set_last_error("hipMalloc for observing records failed"); rc = WFS_ERR_ALLOC; }
     else p->obs_lines_len = need;
@@ -1016,7 +1029,7 @@ extern "C" int wfs_plan_profile(wfs_plan* p, int kc, int reset, long* launches, 
 }
 
 extern "C" int wfs_plan_set_variant(wfs_plan* p, int kc, int variant) {
-  const int vmax = kc == WFS_K_HORNER ? 5 : kc == WFS_K_PV_PLANES ? 1 : 2;
+  const int vmax = kc == WFS_K_HORNER ? 5 : kc == WFS_K_PV_PLANES || kc == WFS_K_YZ_SPLIT ? 1 : 2;
   if (!p || kc < 0 || kc >= WFS_K_COUNT || variant < 0 || variant > vmax) { set_last_error("wfs_plan_set_variant: bad argument"); return WFS_ERR_INVALID; }
   if (kc == WFS_K_YZ_PLANE && variant > 0 && !yz_plane_supported(p->precision, p->n[1], p->n[2], variant)) {
     set_last_error("wfs_plan_set_variant: fused plane pass variant %d unsupported for %d x %d planes", variant, p->n[1], p->n[2]);
@@ -1026,7 +1039,13 @@ extern "C" int wfs_plan_set_variant(wfs_plan* p, int kc, int variant) {
     set_last_error("wfs_plan_set_variant: the slab scheme needs complex64, ny = nz in {128, 192, 256} and nx <= 256");
     return WFS_ERR_UNSUPPORTED;
   }
+  if (kc == WFS_K_YZ_SPLIT && variant > 0 && !split_supported(p->precision, p->n)) {
+    set_last_error("wfs_plan_set_variant: the split scheme needs complex128, ny = nz in {64, 96, 128, 192} and nx <= 256");
+    return WFS_ERR_UNSUPPORTED;
+  }
   p->variant[kc] = variant;
+  // asking for a form of the plane pass or of the slab scheme means running it
+  if (kc == WFS_K_YZ_PLANE || kc == WFS_K_YZ_SLAB) p->variant[WFS_K_YZ_SPLIT] = 0;
   return 0;
 }
 

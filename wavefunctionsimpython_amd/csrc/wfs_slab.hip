@@ -1,5 +1,6 @@
-// Two-launch split step for complex64 grids with ny = nz in {128, 192, 256} and nx <= 256
-// (gfx950).
+// Two-launch split step for complex64 grids with ny = nz in {128, 192, 256} and complex128 grids
+// with ny = nz in {64, 96, 128, 192}, nx <= 256 (gfx950).  Compiled twice: WFS_SLAB_PREC=0
+// (complex64) and 1 (complex128).
 //
 // A 256^2 y-z plane (512 KiB) or a 192^2 one (288 KiB) does not fit in one CU, so the y
 // transform is split in two stages, ny = LY * B (B = 4, LY = 64 or 48; at 128, B = 2 and
@@ -28,10 +29,17 @@ namespace wfs {
 
 namespace {
 
-// rows y = B a + b of a row group: the length-B stage rides on the x launch (B = 4 at 256 and
-// 192, LY = 64 and 48 rows per group; B = 2 at 128, LY = 64)
-template <int N> struct SlabShape {
-  static constexpr int B = N == 128 ? 2 : 4;
+// z points per x block of the complex128 launch: half lines where whole ones leave too few blocks
+// (128^3: 16.5 us with 8, 18.3 with 4)
+template <int N> constexpr int kZB128 = N <= 64 ? 4 : 8;
+
+// rows y = B a + b of a row group: the length-B stage rides on the x launch (complex64: B = 4 at
+// 256 and 192, LY = 64 and 48 rows per group; B = 2 at 128, LY = 64; complex128: B = 2 up to 128,
+// where the x launch then holds one row a lane: 33, 74 and 129 KiB of LDS per group at 64, 96 and
+// 128, B = 4 at 192, 148 KiB).  Measured at 64^3 and 128^3 complex128, y-z and x launch: B = 2 8.0 +
+// 5.7 and 25.9 + 16.5 us, B = 4 7.3 + 7.5 and 24.2 + 21.9.
+template <typename R, int N> struct SlabShape {
+  static constexpr int B = (sizeof(R) == 4 ? N == 128 : N <= 128) ? 2 : 4;
   static constexpr int LY = N / B;
 };
 
@@ -73,6 +81,8 @@ __device__ __forceinline__ cx<R> partner_c(cx<R> v) {
     const auto sx = __builtin_amdgcn_permlane16_swap(__float_as_uint(v.x), __float_as_uint(v.x), false, false);
     const auto sy = __builtin_amdgcn_permlane16_swap(__float_as_uint(v.y), __float_as_uint(v.y), false, false);
     return mk<R>(__uint_as_float(odd_row ? sx[0] : sx[1]), __uint_as_float(odd_row ? sy[0] : sy[1]));
+  } else if constexpr (sizeof(R) == 8) {
+    return mk<R>(xor_lane<ZB>(v.x), xor_lane<ZB>(v.y));
   } else {
     return shfl_xor_c<R>(v, ZB);
   }
@@ -82,13 +92,13 @@ __device__ __forceinline__ cx<R> partner_c(cx<R> v) {
 // VGPRs: the x transforms' table twiddles are read from LDS one at a time where they are applied,
 // so no twiddle array is held; at nx = 256 one spilled register, 52.4 against 55.8 us per launch
 // with three waves, bit-identical); the 24 points of nx = 96 or 192 do not fit in 128.
-// ZB = 8: a block reads and writes 64-byte halves of 128-byte lines; the two blocks of a line
+// 64-byte segments (ZB = 8, complex128 ZB = 4): a block reads and writes halves of 128-byte lines; the two blocks of a line
 // get the block indices 16 g + x and 16 g + 8 + x, which the dispatcher sends to the same XCD
 // (blocks go round-robin over the 8 XCDs) one after the other, so the second half comes from
 // that XCD's L2.
 template <typename R, int NX, int NY, int NZ, int B, int ZB>
 __global__ __launch_bounds__(2 * ZB * split_of<NX>::n2)
-__attribute__((amdgpu_waves_per_eu(ZB == 8 && NX / split_of<NX>::n2 <= 16 ? 4 : 1))) void x_slab_kernel(
+__attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && ZB == 8 && NX / split_of<NX>::n2 <= 16 ? 4 : 1))) void x_slab_kernel(
     cx<R>* __restrict__ data, const XSlabParams p) {
   constexpr int N2 = split_of<NX>::n2;
   constexpr int N1 = NX / N2;
@@ -108,7 +118,7 @@ __attribute__((amdgpu_waves_per_eu(ZB == 8 && NX / split_of<NX>::n2 <= 16 ? 4 : 
   const int t = tid / (2 * ZB);            // thread of the x line: x = t + N2 i
   const int line = q * ZB + zl;
   long bid = blockIdx.x;
-  if constexpr (ZB == 8) bid = 2 * (8 * (bid / 16) + bid % 8) + (bid / 8) % 2;
+  if constexpr (ZB * sizeof(C) == 64) bid = 2 * (8 * (bid / 16) + bid % 8) + (bid / 8) % 2;
   const int zt = int(bid % TZ);
   const int ka = int((bid / TZ) % A);
   const long pk = bid / (long(TZ) * A);
@@ -243,6 +253,7 @@ __attribute__((amdgpu_waves_per_eu(ZB == 8 && NX / split_of<NX>::n2 <= 16 ? 4 : 
   }
 }
 
+#if WFS_SLAB_PREC == 0
 // flags[p] = 1 when x plane p equals plane p - 1 of the same packet bit for bit, else 0
 __global__ __launch_bounds__(256) void plane_equal_kernel(const unsigned long long* __restrict__ table,
                                                           long plane_elems, int nx, long first,
@@ -309,6 +320,8 @@ __global__ __launch_bounds__(256) void plane_runs_kernel(const int* __restrict__
   }
 }
 
+#endif
+
 // compute units of the current device (cached per device)
 int cu_count() {
   static int cache[64] = {0};
@@ -322,48 +335,56 @@ int cu_count() {
 }
 
 // persistent: one block per CU walking the row groups, else one block per group
-template <int N, int MODE, bool PERSIST>
+template <typename R, int N, int MODE, bool PERSIST>
 int launch_lines_m(void* data, const YzPlaneParams& p, hipStream_t s) {
-  constexpr int LY = SlabShape<N>::LY, B = SlabShape<N>::B;
-  static_assert(yz_lines_lds_bytes<float, N, LY, 1>() <= 160 * 1024, "rows do not fit in LDS");
+  constexpr int LY = SlabShape<R, N>::LY, B = SlabShape<R, N>::B;
+  static_assert(yz_lines_lds_bytes<R, N, LY, 1>() <= 160 * 1024, "rows do not fit in LDS");
   const long groups = p.planes * B;
   const long grid = PERSIST ? std::min<long>(groups, cu_count()) : groups;
-  WFS_LAUNCH((yz_lines_kernel<float, N, LY, B, 1, MODE, PERSIST, true>), dim3(unsigned(grid)),
-                     dim3(yz_lines_threads<N, LY, 1>()), 0, s, reinterpret_cast<float2*>(data), p);
+  WFS_LAUNCH((yz_lines_kernel<R, N, LY, B, 1, MODE, PERSIST, true>), dim3(unsigned(grid)),
+                     dim3(yz_lines_threads<N, LY, 1>()), 0, s, reinterpret_cast<cx<R>*>(data), p);
   return int(hipGetLastError());
 }
 
-template <int N>
+// complex128 has the one-block-per-group forms only, and takes its box moments in their own launches
+// (the sums of the plane pass and the axis passes, bit for bit)
+template <typename R, int N>
 int launch_lines_n(int mode, int variant, void* data, const YzPlaneParams& p, hipStream_t s) {
-  const bool persist = variant == 2;
-  if (mode == LINES_FULL)
-    return persist ? launch_lines_m<N, LINES_FULL, true>(data, p, s) : launch_lines_m<N, LINES_FULL, false>(data, p, s);
-  if (mode == LINES_ENTRY)
-    return persist ? launch_lines_m<N, LINES_ENTRY, true>(data, p, s) : launch_lines_m<N, LINES_ENTRY, false>(data, p, s);
-  if (mode == LINES_EXIT)
-    return persist ? launch_lines_m<N, LINES_EXIT, true>(data, p, s) : launch_lines_m<N, LINES_EXIT, false>(data, p, s);
-  if (mode == LINES_OBSERVE) return launch_lines_m<N, LINES_OBSERVE, false>(data, p, s);
-  if (mode == LINES_ENTRY_OBSERVE) return launch_lines_m<N, LINES_ENTRY_OBSERVE, false>(data, p, s);
+  if constexpr (sizeof(R) == 4) {
+    if (variant == 2) {
+      if (mode == LINES_FULL) return launch_lines_m<R, N, LINES_FULL, true>(data, p, s);
+      if (mode == LINES_ENTRY) return launch_lines_m<R, N, LINES_ENTRY, true>(data, p, s);
+      if (mode == LINES_EXIT) return launch_lines_m<R, N, LINES_EXIT, true>(data, p, s);
+    }
+  }
+  if (mode == LINES_FULL) return launch_lines_m<R, N, LINES_FULL, false>(data, p, s);
+  if (mode == LINES_ENTRY) return launch_lines_m<R, N, LINES_ENTRY, false>(data, p, s);
+  if (mode == LINES_EXIT) return launch_lines_m<R, N, LINES_EXIT, false>(data, p, s);
+  if constexpr (sizeof(R) == 4) {
+    if (mode == LINES_OBSERVE) return launch_lines_m<R, N, LINES_OBSERVE, false>(data, p, s);
+    if (mode == LINES_ENTRY_OBSERVE) return launch_lines_m<R, N, LINES_ENTRY_OBSERVE, false>(data, p, s);
+  }
   set_last_error("slab y-z pass: bad mode %d", mode);
   return WFS_ERR_INVALID;
 }
 
-template <int NX, int N, int ZB>
+template <typename R, int NX, int N, int ZB>
 int launch_x_slab_z(void* data, const XSlabParams& p, hipStream_t s) {
-  constexpr int B = SlabShape<N>::B;
+  constexpr int B = SlabShape<R, N>::B;
   constexpr long per_packet = long(N / B) * (N / ZB);
   static_assert(per_packet % 16 == 0, "the XCD pairing needs a multiple of 16 blocks");
-  WFS_LAUNCH((x_slab_kernel<float, NX, N, N, B, ZB>), dim3(unsigned(p.packets * per_packet)),
-                     dim3(2 * ZB * split_of<NX>::n2), 0, s, reinterpret_cast<float2*>(data), p);
+  WFS_LAUNCH((x_slab_kernel<R, NX, N, N, B, ZB>), dim3(unsigned(p.packets * per_packet)),
+                     dim3(2 * ZB * split_of<NX>::n2), 0, s, reinterpret_cast<cx<R>*>(data), p);
   return int(hipGetLastError());
 }
 
-// variant 2: 8 z points per block (256 threads at nx = 256), else 16
-template <int N>
+// complex64: variant 2: 8 z points per block (256 threads at nx = 256), else 16; complex128: ZB128
+template <typename R, int N>
 int launch_x_slab_ny(int nx, int variant, void* data, const XSlabParams& p, hipStream_t s) {
-#define WFS_X_SLAB_CASE(NX)                                                                              \
-  case NX:                                                                                               \
-    return variant == 2 ? launch_x_slab_z<NX, N, 8>(data, p, s) : launch_x_slab_z<NX, N, 16>(data, p, s);
+#define WFS_X_SLAB_CASE(NX)                                                                                    \
+  case NX:                                                                                                     \
+    if constexpr (sizeof(R) == 8) return launch_x_slab_z<R, NX, N, kZB128<N>>(data, p, s);                         \
+    else return variant == 2 ? launch_x_slab_z<R, NX, N, 8>(data, p, s) : launch_x_slab_z<R, NX, N, 16>(data, p, s);
   switch (nx) {
     WFS_X_SLAB_CASE(8)
     WFS_X_SLAB_CASE(16)
@@ -380,8 +401,34 @@ int launch_x_slab_ny(int nx, int variant, void* data, const XSlabParams& p, hipS
 #undef WFS_X_SLAB_CASE
 }
 
+template <typename R, int N>
+SlabRows slab_rows_n() {
+  SlabRows g;
+  g.b = SlabShape<R, N>::B;
+  g.n1 = N / split_of<N>::n2;
+  g.uy = SlabShape<R, N>::LY / g.n1;
+  g.uz = split_of<N>::n2;
+  return g;
+}
+
+template <typename R, int N>
+LinesOrder slab_lines_order_n() {
+  constexpr int LY = SlabShape<R, N>::LY;
+  LinesOrder m;
+  m.ny = N;
+  m.nz = N;
+  m.ly = LY;
+  m.b = SlabShape<R, N>::B;
+  m.rh = LY;
+  m.n2z = split_of<N>::n2;
+  m.n1 = N / split_of<N>::n2;
+  m.threads = yz_lines_threads<N, LY, 1>();
+  return m;
+}
+
 }  // namespace
 
+#if WFS_SLAB_PREC == 0
 int launch_plane_dedup(const void* table, long plane_elems, int nx, int packets, long first, long count, int* flags,
                        int* src, hipStream_t s) {
   const long planes = long(nx) * packets;
@@ -404,62 +451,87 @@ bool slab_supported(int precision, const int n[3]) {
          fft_length_supported(n[0]);
 }
 
-template <int N>
-static SlabRows slab_rows_n() {
-  SlabRows g;
-  g.b = SlabShape<N>::B;
-  g.n1 = N / split_of<N>::n2;
-  g.uy = SlabShape<N>::LY / g.n1;
-  g.uz = split_of<N>::n2;
-  return g;
+// complex128, ny = nz in {64, 96, 128, 192}: a row group of 256^2 planes (LY = 64 rows, 257 KiB)
+// does not fit in a CU.  us per step with a potential table, passes or plane pass against the two
+// launches: 64^3 18.1 -> 14.8, 96^3 54.8 -> 37.7, 128^3 57.5 -> 44.4, 192^3 198.7 -> 166.1, 64 x
+// 192^2 76.4 -> 46.0, 48 x 64^3 192 -> 144; only long x lines beside 64^2 planes were slower
+// (192 x 64^2 27.6 -> 29.9, 256 x 64^2 28.7 -> 34.6: x blocks of 128 and more points a lane pair),
+// so the plan leaves those to the plane pass.
+bool split_supported(int precision, const int n[3]) {
+  return precision == WFS_C128 && n[1] == n[2] && (n[1] == 64 || n[1] == 96 || n[1] == 128 || n[1] == 192) &&
+         n[0] <= 256 && fft_length_supported(n[0]);
 }
 
-SlabRows slab_rows(int n) {
-  return n == 128 ? slab_rows_n<128>() : n == 192 ? slab_rows_n<192>() : slab_rows_n<256>();
+SlabRows slab_rows_c128(int n);
+LinesOrder slab_lines_order_c128(int n);
+int launch_yz_slab_c128(int n, int mode, void* data, const YzPlaneParams& p, hipStream_t s);
+int launch_x_slab_c128(int nx, int n, void* data, const XSlabParams& p, hipStream_t s);
+
+SlabRows slab_rows(int precision, int n) {
+  if (precision == WFS_C128) return slab_rows_c128(n);
+  return n == 128 ? slab_rows_n<float, 128>() : n == 192 ? slab_rows_n<float, 192>() : slab_rows_n<float, 256>();
 }
 
-template <int N>
-static LinesOrder slab_lines_order_n() {
-  constexpr int LY = SlabShape<N>::LY;
-  LinesOrder m;
-  m.ny = N;
-  m.nz = N;
-  m.ly = LY;
-  m.b = SlabShape<N>::B;
-  m.rh = LY;
-  m.n2z = split_of<N>::n2;
-  m.n1 = N / split_of<N>::n2;
-  m.threads = yz_lines_threads<N, LY, 1>();
-  return m;
+LinesOrder slab_lines_order(int precision, int n) {
+  if (precision == WFS_C128) return slab_lines_order_c128(n);
+  return n == 128 ? slab_lines_order_n<float, 128>()
+                  : n == 192 ? slab_lines_order_n<float, 192>() : slab_lines_order_n<float, 256>();
 }
 
-LinesOrder slab_lines_order(int n) {
-  return n == 128 ? slab_lines_order_n<128>() : n == 192 ? slab_lines_order_n<192>() : slab_lines_order_n<256>();
-}
-
-int launch_yz_slab(int n, int mode, int variant, void* data, const YzPlaneParams& p, hipStream_t s) {
+int launch_yz_slab(int precision, int n, int mode, int variant, void* data, const YzPlaneParams& p, hipStream_t s) {
   if (p.planes <= 0 || p.planes * 4 > 0x7fffffffL) {
     set_last_error("slab y-z pass: bad plane count %ld", p.planes);
     return WFS_ERR_INVALID;
   }
-  if (n == 256) return launch_lines_n<256>(mode, variant, data, p, s);
-  if (n == 192) return launch_lines_n<192>(mode, variant, data, p, s);
-  if (n == 128) return launch_lines_n<128>(mode, variant, data, p, s);
+  if (precision == WFS_C128) return launch_yz_slab_c128(n, mode, data, p, s);
+  if (n == 256) return launch_lines_n<float, 256>(mode, variant, data, p, s);
+  if (n == 192) return launch_lines_n<float, 192>(mode, variant, data, p, s);
+  if (n == 128) return launch_lines_n<float, 128>(mode, variant, data, p, s);
   set_last_error("slab y-z pass: unsupported plane %d", n);
   return WFS_ERR_UNSUPPORTED;
 }
 
-int launch_x_slab(int nx, int n, int variant, void* data, const XSlabParams& p, hipStream_t s) {
-  const long blocks = p.packets * long(n / 2) * (n / 8);
+int launch_x_slab(int precision, int nx, int n, int variant, void* data, const XSlabParams& p, hipStream_t s) {
+  const long blocks = p.packets * long(n / 2) * (n / 4);
   if (p.packets <= 0 || blocks > 0x7fffffffL) {
     set_last_error("slab x pass: bad packet count %ld", p.packets);
     return WFS_ERR_INVALID;
   }
-  if (n == 256) return launch_x_slab_ny<256>(nx, variant, data, p, s);
-  if (n == 192) return launch_x_slab_ny<192>(nx, variant, data, p, s);
-  if (n == 128) return launch_x_slab_ny<128>(nx, variant, data, p, s);
+  if (precision == WFS_C128) return launch_x_slab_c128(nx, n, data, p, s);
+  if (n == 256) return launch_x_slab_ny<float, 256>(nx, variant, data, p, s);
+  if (n == 192) return launch_x_slab_ny<float, 192>(nx, variant, data, p, s);
+  if (n == 128) return launch_x_slab_ny<float, 128>(nx, variant, data, p, s);
   set_last_error("slab x pass: unsupported plane %d", n);
   return WFS_ERR_UNSUPPORTED;
 }
+#else
+SlabRows slab_rows_c128(int n) {
+  return n == 64 ? slab_rows_n<double, 64>() : n == 96 ? slab_rows_n<double, 96>()
+         : n == 128 ? slab_rows_n<double, 128>() : slab_rows_n<double, 192>();
+}
+
+LinesOrder slab_lines_order_c128(int n) {
+  return n == 64 ? slab_lines_order_n<double, 64>() : n == 96 ? slab_lines_order_n<double, 96>()
+         : n == 128 ? slab_lines_order_n<double, 128>() : slab_lines_order_n<double, 192>();
+}
+
+int launch_yz_slab_c128(int n, int mode, void* data, const YzPlaneParams& p, hipStream_t s) {
+  if (n == 64) return launch_lines_n<double, 64>(mode, 1, data, p, s);
+  if (n == 96) return launch_lines_n<double, 96>(mode, 1, data, p, s);
+  if (n == 128) return launch_lines_n<double, 128>(mode, 1, data, p, s);
+  if (n == 192) return launch_lines_n<double, 192>(mode, 1, data, p, s);
+  set_last_error("slab y-z pass: unsupported complex128 plane %d", n);
+  return WFS_ERR_UNSUPPORTED;
+}
+
+int launch_x_slab_c128(int nx, int n, void* data, const XSlabParams& p, hipStream_t s) {
+  if (n == 64) return launch_x_slab_ny<double, 64>(nx, 1, data, p, s);
+  if (n == 96) return launch_x_slab_ny<double, 96>(nx, 1, data, p, s);
+  if (n == 128) return launch_x_slab_ny<double, 128>(nx, 1, data, p, s);
+  if (n == 192) return launch_x_slab_ny<double, 192>(nx, 1, data, p, s);
+  set_last_error("slab x pass: unsupported complex128 plane %d", n);
+  return WFS_ERR_UNSUPPORTED;
+}
+#endif
 
 }  // namespace wfs
