@@ -347,8 +347,7 @@ int wfs_plan_set_profiling(wfs_plan* plan, int enable);
  * work (kernel class WFS_K_YZ_SLAB; the entry and exit launches of a call
  * count as WFS_K_SLAB_EDGE, the launches of wfs_step_observe that also take
  * the box moments as WFS_K_SLAB_OBSERVE) and a length-B stage fused with the x pass
- * (WFS_K_X_SLAB); variant 2 runs the y-z launch as one persistent block per
- * CU that loads the next row group during the current one's arithmetic;
+ * (WFS_K_X_SLAB); variants 1 and 2 are the same launches;
  * variant 0 runs the four axis passes.  The results agree to float rounding
  * (the length-ny y transform is factored differently); the slab variants
  * among themselves are bit-identical.  WFS_K_X_SLAB: variant 1 (default at

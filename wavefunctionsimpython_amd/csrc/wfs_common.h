@@ -376,6 +376,39 @@ __device__ __forceinline__ void column_dft_second(C (&a)[N / N2], C* lds, int t,
   }
 }
 
+// The same step through LDS of one part at a time, in half the space: the caller's slots hold
+// the real parts, then the imaginary parts (three barriers instead of one; the values and their
+// order in the DFTs are those of column_dft_second).
+template <int N, int N2, int SIGN, typename C, typename R, typename LIDX>
+__device__ __forceinline__ void column_dft_second_parts(C (&a)[N / N2], R* lds, int t, LIDX lidx) {
+  constexpr int N1 = N / N2;
+  constexpr int M = N1 / N2;
+#pragma unroll
+  for (int k1 = 0; k1 < N1; ++k1) lds[lidx(k1, t)] = a[k1].x;
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < M; ++m)
+#pragma unroll
+    for (int n2 = 0; n2 < N2; ++n2) a[m + M * n2].x = lds[lidx(t + N2 * m, n2)];
+  __syncthreads();
+#pragma unroll
+  for (int k1 = 0; k1 < N1; ++k1) lds[lidx(k1, t)] = a[k1].y;
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < M; ++m)
+#pragma unroll
+    for (int n2 = 0; n2 < N2; ++n2) a[m + M * n2].y = lds[lidx(t + N2 * m, n2)];
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    C b[N2];
+#pragma unroll
+    for (int n2 = 0; n2 < N2; ++n2) b[n2] = a[m + M * n2];
+    DFT<N2, SIGN>::run(b);
+#pragma unroll
+    for (int k2 = 0; k2 < N2; ++k2) a[m + M * k2] = b[k2];
+  }
+}
+
 template <int N, int N2, int SIGN, typename C, typename LIDX>
 __device__ __forceinline__ void column_dft(C (&a)[N / N2], const C (&w)[N / N2], C* lds, int t, LIDX lidx) {
   column_dft_first<N, N2, SIGN>(a, w);

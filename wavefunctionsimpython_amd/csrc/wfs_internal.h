@@ -155,10 +155,8 @@ struct SlabRows {
 SlabRows slab_rows(int precision, int n);
 // the potential table order of the slab scheme's y-z launch (ny = nz = n)
 LinesOrder slab_lines_order(int precision, int n);
-// YzPlaneParams.planes = packets * nx; variant 2 = persistent (one block per CU walking the
-// row groups, loading the next group during the current one's arithmetic), else one block
-// per group
-int launch_yz_slab(int precision, int n, int mode, int variant, void* data, const YzPlaneParams& p, hipStream_t s);
+// YzPlaneParams.planes = packets * nx
+int launch_yz_slab(int precision, int n, int mode, void* data, const YzPlaneParams& p, hipStream_t s);
 // variant 2: 8 z points per block, else 16
 int launch_x_slab(int precision, int nx, int n, int variant, void* data, const XSlabParams& p, hipStream_t s);
 

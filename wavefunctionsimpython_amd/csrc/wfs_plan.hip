@@ -529,7 +529,7 @@ int run_slab_lines(wfs_plan* p, int mode, void* data, const void* pv, hipStream_
   pp.nx = p->n[0];
   pp.planes = long(p->batch) * p->n[0];
   ProfileScope scope(p, mode == LINES_FULL ? WFS_K_YZ_SLAB : WFS_K_SLAB_EDGE, s);
-  return launch_yz_slab(p->precision, p->n[1], mode, p->variant[WFS_K_YZ_SLAB], data, pp, s);
+  return launch_yz_slab(p->precision, p->n[1], mode, data, pp, s);
 }
 
 // Slab scheme: length-4 y stages around x forward -> K -> x inverse
@@ -586,7 +586,7 @@ int run_slab_observe(wfs_plan* p, int mode, void* data, int sel_exit, int sel_en
   pp.mom.partials = p->obs_lines;
   {
     ProfileScope scope(p, WFS_K_SLAB_OBSERVE, s);
-    WFS_TRY(launch_yz_slab(p->precision, p->n[1], mode, 1, data, pp, s));
+    WFS_TRY(launch_yz_slab(p->precision, p->n[1], mode, data, pp, s));
   }
   ProfileScope scope(p, WFS_K_OBSERVABLES, s);
   return launch_sum_partials(p->obs_lines, long(p->n[0]) * g.b, nb, p->batch, p->dx[0] * p->dx[1] * p->dx[2] / 27.0,
@@ -768,10 +768,9 @@ extern "C" int wfs_plan_create_batched(const int n[3], const double dx[3], doubl
   p->variant[WFS_K_YZ_PLANE] =
       (yz_plane_supported(precision, n[1], n[2], 2) && n[1] == 128 && long(batch) * n[0] >= 512) ? 2
       : yz_plane_supported(precision, n[1], n[2], 1) ? 1 : 0;
-  // slab scheme at ny = nz = 256, 192 or 128 (complex64).  At 256 the persistent y-z launch
-  // and 8-z x blocks (measured fastest at 256^3: 90 and 66 us against 115 and 79 for the other
-  // forms); at 192 one block per row group (two 72 KiB blocks per CU) and 16-z x blocks
-  // (192^3 x 15: 662 and 460 us; 8-z x blocks 514 us); at 128 only while the x planes are too
+  // slab scheme at ny = nz = 256, 192 or 128 (complex64; both nonzero variants are the same y-z
+  // launch).  At 256 8-z x blocks (256^3 66 us against 79 with 16 z points), at 192 16-z x blocks
+  // (192^3 x 15: 460 us; 8-z x blocks 514 us); at 128 only while the x planes are too
   // few to fill the CUs with plane-pass blocks, fewer than 256 (128^3: 29 against 34 us per
   // step; from 8 packets on the plane pass is as fast)
   const bool slab = slab_supported(precision, n) && (n[1] != 128 || long(batch) * n[0] < 256);
@@ -1118,7 +1117,7 @@ extern "C" int wfs_plan_autotune(wfs_plan* p, void* stream) {
     p->variant[WFS_K_YZ_PLANE] = rc == 0 ? best_v : keep;
   }
   // slab scheme (two launches per step) against the tuned four axis passes: first the x
-  // launch's block width, then one step of each y-z form and of the passes
+  // launch's block width, then one step of the two launches and of the passes
   if (rc == 0 && slab_supported(p->precision, p->n)) {
     {
       const int keep = p->variant[WFS_K_X_SLAB];
@@ -1140,7 +1139,7 @@ extern "C" int wfs_plan_autotune(wfs_plan* p, void* stream) {
     const int keep = p->variant[WFS_K_YZ_SLAB];
     float best = 1e30f;
     int best_v = keep;
-    for (int v = 0; v < 3 && rc == 0; ++v) {
+    for (int v = 0; v < 2 && rc == 0; ++v) {
       p->variant[WFS_K_YZ_SLAB] = v;
       auto one_step = [&]() -> int {
         if (v) {

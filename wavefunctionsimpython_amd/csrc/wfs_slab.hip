@@ -23,7 +23,6 @@
 // bit for bit.
 #include "wfs_yz_lines.h"
 
-#include <algorithm>
 
 namespace wfs {
 
@@ -334,35 +333,53 @@ int cu_count() {
   return n;
 }
 
-// persistent: one block per CU walking the row groups, else one block per group
-template <typename R, int N, int MODE, bool PERSIST>
+template <typename R, int N, int MODE, int PARTS = 0>
 int launch_lines_m(void* data, const YzPlaneParams& p, hipStream_t s) {
   constexpr int LY = SlabShape<R, N>::LY, B = SlabShape<R, N>::B;
   static_assert(yz_lines_lds_bytes<R, N, LY, 1>() <= 160 * 1024, "rows do not fit in LDS");
   const long groups = p.planes * B;
-  const long grid = PERSIST ? std::min<long>(groups, cu_count()) : groups;
-  WFS_LAUNCH((yz_lines_kernel<R, N, LY, B, 1, MODE, PERSIST, true>), dim3(unsigned(grid)),
+  WFS_LAUNCH((yz_lines_kernel<R, N, LY, B, 1, MODE, true, PARTS>), dim3(unsigned(groups)),
                      dim3(yz_lines_threads<N, LY, 1>()), 0, s, reinterpret_cast<cx<R>*>(data), p);
   return int(hipGetLastError());
+}
+
+// Waves per SIMD asked of the compiler for the form that exchanges one part at a time (PARTS in
+// wfs_yz_lines.h; the bits are those of the whole form), 0 where the whole form is the better one at any
+// size.  256^2: a 1024-thread block in 64 VGPRs and 66 KB of LDS leaves room for a second one, so that one
+// block's loads and stores run beside the other's transforms.  192^2: one 768-thread block either way, but
+// the transforms no longer wait for the factor loads hoisted over them.  Not for complex128 (128^3 27.3 ->
+// 28.6, 192^3 80.3 -> 85.6, 96^3 17.2 -> 18.3 us: its 3 and more exchanges cost what the second block
+// gains) nor for complex64 128^2 planes (19.0 -> 19.3).
+template <typename R, int N> constexpr int lines_parts() { return sizeof(R) == 8 ? 0 : N == 256 ? 8 : N == 192 ? 3 : 0; }
+
+// The parts form is taken where the groups are more than the CUs.  us of the full / entry or exit launch,
+// whole against parts: 256^2 256 planes 85 / 57 -> 76 / 49, 192 planes 64 / 44 -> 57 / 39, 128 planes
+// 46 / 30 -> 36 / 26, 96 planes 40 / 27 -> 33 / 24; 192^2 256 planes 64 / 43 -> 59 / 39, 192 planes
+// 50 / 34 -> 40 / 27, 128 planes 34 / 22 -> 26 / 18.  With one group per CU there is nothing to overlap
+// and the extra barriers show: 256^2 64 planes 24.1 / 15.3 -> 26.2 / 16.4, 192^2 17.9 -> 19.0.
+template <typename R, int N>
+bool lines_in_parts(long planes) {
+  return lines_parts<R, N>() != 0 && planes * SlabShape<R, N>::B > cu_count();
 }
 
 // complex128 has the one-block-per-group forms only, and takes its box moments in their own launches
 // (the sums of the plane pass and the axis passes, bit for bit)
 template <typename R, int N>
-int launch_lines_n(int mode, int variant, void* data, const YzPlaneParams& p, hipStream_t s) {
-  if constexpr (sizeof(R) == 4) {
-    if (variant == 2) {
-      if (mode == LINES_FULL) return launch_lines_m<R, N, LINES_FULL, true>(data, p, s);
-      if (mode == LINES_ENTRY) return launch_lines_m<R, N, LINES_ENTRY, true>(data, p, s);
-      if (mode == LINES_EXIT) return launch_lines_m<R, N, LINES_EXIT, true>(data, p, s);
+int launch_lines_n(int mode, void* data, const YzPlaneParams& p, hipStream_t s) {
+  if constexpr (lines_parts<R, N>() != 0) {
+    constexpr int W = lines_parts<R, N>();
+    if (lines_in_parts<R, N>(p.planes)) {
+      if (mode == LINES_FULL) return launch_lines_m<R, N, LINES_FULL, W>(data, p, s);
+      if (mode == LINES_ENTRY) return launch_lines_m<R, N, LINES_ENTRY, W>(data, p, s);
+      if (mode == LINES_EXIT) return launch_lines_m<R, N, LINES_EXIT, W>(data, p, s);
     }
   }
-  if (mode == LINES_FULL) return launch_lines_m<R, N, LINES_FULL, false>(data, p, s);
-  if (mode == LINES_ENTRY) return launch_lines_m<R, N, LINES_ENTRY, false>(data, p, s);
-  if (mode == LINES_EXIT) return launch_lines_m<R, N, LINES_EXIT, false>(data, p, s);
+  if (mode == LINES_FULL) return launch_lines_m<R, N, LINES_FULL>(data, p, s);
+  if (mode == LINES_ENTRY) return launch_lines_m<R, N, LINES_ENTRY>(data, p, s);
+  if (mode == LINES_EXIT) return launch_lines_m<R, N, LINES_EXIT>(data, p, s);
   if constexpr (sizeof(R) == 4) {
-    if (mode == LINES_OBSERVE) return launch_lines_m<R, N, LINES_OBSERVE, false>(data, p, s);
-    if (mode == LINES_ENTRY_OBSERVE) return launch_lines_m<R, N, LINES_ENTRY_OBSERVE, false>(data, p, s);
+    if (mode == LINES_OBSERVE) return launch_lines_m<R, N, LINES_OBSERVE>(data, p, s);
+    if (mode == LINES_ENTRY_OBSERVE) return launch_lines_m<R, N, LINES_ENTRY_OBSERVE>(data, p, s);
   }
   set_last_error("slab y-z pass: bad mode %d", mode);
   return WFS_ERR_INVALID;
@@ -478,15 +495,15 @@ LinesOrder slab_lines_order(int precision, int n) {
                   : n == 192 ? slab_lines_order_n<float, 192>() : slab_lines_order_n<float, 256>();
 }
 
-int launch_yz_slab(int precision, int n, int mode, int variant, void* data, const YzPlaneParams& p, hipStream_t s) {
+int launch_yz_slab(int precision, int n, int mode, void* data, const YzPlaneParams& p, hipStream_t s) {
   if (p.planes <= 0 || p.planes * 4 > 0x7fffffffL) {
     set_last_error("slab y-z pass: bad plane count %ld", p.planes);
     return WFS_ERR_INVALID;
   }
   if (precision == WFS_C128) return launch_yz_slab_c128(n, mode, data, p, s);
-  if (n == 256) return launch_lines_n<float, 256>(mode, variant, data, p, s);
-  if (n == 192) return launch_lines_n<float, 192>(mode, variant, data, p, s);
-  if (n == 128) return launch_lines_n<float, 128>(mode, variant, data, p, s);
+  if (n == 256) return launch_lines_n<float, 256>(mode, data, p, s);
+  if (n == 192) return launch_lines_n<float, 192>(mode, data, p, s);
+  if (n == 128) return launch_lines_n<float, 128>(mode, data, p, s);
   set_last_error("slab y-z pass: unsupported plane %d", n);
   return WFS_ERR_UNSUPPORTED;
 }
@@ -516,10 +533,10 @@ LinesOrder slab_lines_order_c128(int n) {
 }
 
 int launch_yz_slab_c128(int n, int mode, void* data, const YzPlaneParams& p, hipStream_t s) {
-  if (n == 64) return launch_lines_n<double, 64>(mode, 1, data, p, s);
-  if (n == 96) return launch_lines_n<double, 96>(mode, 1, data, p, s);
-  if (n == 128) return launch_lines_n<double, 128>(mode, 1, data, p, s);
-  if (n == 192) return launch_lines_n<double, 192>(mode, 1, data, p, s);
+  if (n == 64) return launch_lines_n<double, 64>(mode, data, p, s);
+  if (n == 96) return launch_lines_n<double, 96>(mode, data, p, s);
+  if (n == 128) return launch_lines_n<double, 128>(mode, data, p, s);
+  if (n == 192) return launch_lines_n<double, 192>(mode, data, p, s);
   set_last_error("slab y-z pass: unsupported complex128 plane %d", n);
   return WFS_ERR_UNSUPPORTED;
 }

@@ -53,6 +53,13 @@ __device__ __forceinline__ double lines_simpson(int i, int n) {
 }
 
 
+// Orders the accesses to memory after it behind the computation of v (and those before it ahead
+// of what uses v): a load meant for later is not hoisted over the transform that fills the registers.
+template <typename C>
+__device__ __forceinline__ void settle(C& v) {
+  asm volatile("" : "+v"(v.x), "+v"(v.y)::"memory");
+}
+
 // Box moments of the position-space row a thread holds in the z-line mapping of a
 // yz_lines_kernel round (row c0 = tid mod LY of the group, z = u + N2Z i): per box
 //   sum w |psi|^2 [1, x, y, z, x^2, y^2, z^2],  w = s(ix) s(iy) s(iz)  (Simpson 1-4-2-...-4-1)
@@ -119,16 +126,18 @@ constexpr long yz_lines_lds_bytes() {
   return long(LY / H) * (NZ + 1) * long(sizeof(cx<R>));
 }
 
-// PERSIST: a grid of at most one block per CU walks the groups blockIdx.x, + gridDim.x, ...
-// and loads the next group's points while it transforms the current one (H = 1 only), so
-// that one block per CU still overlaps its memory traffic with its arithmetic.
 // PV_LINES: the potential table is in lines order (LinesOrder, wfs_internal.h), read as one
 // contiguous run per wavefront, and the twiddle tables hold each thread's twiddles
 // contiguously ([u][k1], u the thread's index within a line); else the potential table is
 // in the state's C order and the twiddles come from the length-N axis tables.
-template <typename R, int NZ, int LY, int B, int H, int MODE, bool PERSIST = false, bool PV_LINES = false>
+// PARTS != 0: the exchanges pass the real parts, then the imaginary parts, through half the LDS, and PARTS
+// waves per SIMD bound the registers (four potential factors in flight instead of sixteen), so that two
+// 1024-thread blocks share a CU at 256^2: 256 planes 85 -> 76 us (4.2 -> 4.7 TB/s with the table), entry and
+// exit 57 -> 49 (5.5 TB/s).  What bounds it then is memory, and in the full launch the barriers (20 against 8).
+template <typename R, int NZ, int LY, int B, int H, int MODE, bool PV_LINES = false,
+          int PARTS = 0>
 __global__ __launch_bounds__((yz_lines_threads<NZ, LY, H>()))
-__attribute__((amdgpu_waves_per_eu(H == 1 ? 1 : 4))) void yz_lines_kernel(cx<R>* __restrict__ data,
+__attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lines_kernel(cx<R>* __restrict__ data,
                                                                            const YzPlaneParams p) {
   constexpr int N2Z = split_of<NZ>::n2;
   constexpr int N1 = NZ / N2Z;               // points per thread and line, both directions
@@ -145,14 +154,14 @@ __attribute__((amdgpu_waves_per_eu(H == 1 ? 1 : 4))) void yz_lines_kernel(cx<R>*
   constexpr bool UNIFORM_Z = (RH % 64) == 0;
   using C = cx<R>;
   using CC = const __attribute__((address_space(4))) C;
-  __shared__ C lds[RH * TS];
+  using L = std::conditional_t<PARTS != 0, R, C>;
+  __shared__ L lds[RH * TS];
 
-  static_assert(!PERSIST || H == 1, "the persistent form holds one round");
+  static_assert(!PARTS || H == 1, "parts: one round");
   const int tid = threadIdx.x;
-  const long groups = p.planes * B;
-  long group = blockIdx.x;
-  long plane = group / B;                    // x plane, counted over all packets
-  int bres = int(group % B);                 // residue b of the block's rows
+  const long group = blockIdx.x;
+  const long plane = group / B;                    // x plane, counted over all packets
+  const int bres = int(group % B);                 // residue b of the block's rows
   C* __restrict__ blk = data + plane * long(NY) * NZ + long(bres) * NZ;
 
   C a[H][N1];
@@ -197,13 +206,15 @@ __attribute__((amdgpu_waves_per_eu(H == 1 ? 1 : 4))) void yz_lines_kernel(cx<R>*
   // the exchanges of column_dft for the lines of one round
   auto exchange_y = [&](C (&line)[N1], int u, auto sign_c) {
     const int c0 = opaque_v(tid) % CH;
-    column_dft_second<LY, N2Y, decltype(sign_c)::value>(line, lds, u,
-                                                        [&](int k1, int n2) { return (k1 * N2Y + n2) * CH + c0; });
+    auto slot = [&](int k1, int n2) { return (k1 * N2Y + n2) * CH + c0; };
+    if constexpr (PARTS) column_dft_second_parts<LY, N2Y, decltype(sign_c)::value>(line, lds, u, slot);
+    else column_dft_second<LY, N2Y, decltype(sign_c)::value>(line, lds, u, slot);
   };
   auto exchange_z = [&](C (&line)[N1], int u, auto sign_c) {
     const int c0 = opaque_v(tid) % RH;
-    column_dft_second<NZ, N2Z, decltype(sign_c)::value>(line, lds, u,
-                                                        [&](int k1, int n2) { return (k1 * N2Z + n2) * RH + c0; });
+    auto slot = [&](int k1, int n2) { return (k1 * N2Z + n2) * RH + c0; };
+    if constexpr (PARTS) column_dft_second_parts<NZ, N2Z, decltype(sign_c)::value>(line, lds, u, slot);
+    else column_dft_second<NZ, N2Z, decltype(sign_c)::value>(line, lds, u, slot);
   };
   // one transform of every y line, round by round (one round's temporaries live at a time)
   auto transform_y = [&](const void* twp, auto sign_c) {
@@ -232,6 +243,20 @@ __attribute__((amdgpu_waves_per_eu(H == 1 ? 1 : 4))) void yz_lines_kernel(cx<R>*
     const int t = opaque_v(tid);
     const int c0 = t % CH, u = t / CH;
     const int r0 = t % RH, v = t / RH;
+    if constexpr (PARTS) {
+#pragma unroll
+      for (int i = 0; i < N1; ++i) lds[(u + N2Y * i) * TS + c0] = a[0][i].x;
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < N1; ++i) a[0][i].x = lds[r0 * TS + v + N2Z * i];
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < N1; ++i) lds[(u + N2Y * i) * TS + c0] = a[0][i].y;
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < N1; ++i) a[0][i].y = lds[r0 * TS + v + N2Z * i];
+      return;
+    } else {
     C bb[H][N1];
 #pragma unroll
     for (int r = 0; r < H; ++r) {
@@ -248,11 +273,26 @@ __attribute__((amdgpu_waves_per_eu(H == 1 ? 1 : 4))) void yz_lines_kernel(cx<R>*
     for (int r = 0; r < H; ++r)
 #pragma unroll
       for (int i = 0; i < N1; ++i) a[r][i] = bb[r][i];
+    }
   };
   auto rows_to_cols = [&]() {
     const int t = opaque_v(tid);
     const int c0 = t % CH, u = t / CH;
     const int r0 = t % RH, v = t / RH;
+    if constexpr (PARTS) {
+#pragma unroll
+      for (int i = 0; i < N1; ++i) lds[r0 * TS + v + N2Z * i] = a[0][i].x;
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < N1; ++i) a[0][i].x = lds[(u + N2Y * i) * TS + c0];
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < N1; ++i) lds[r0 * TS + v + N2Z * i] = a[0][i].y;
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < N1; ++i) a[0][i].y = lds[(u + N2Y * i) * TS + c0];
+      return;
+    } else {
     C bb[H][N1];
 #pragma unroll
     for (int r = 0; r < H; ++r) {
@@ -269,6 +309,7 @@ __attribute__((amdgpu_waves_per_eu(H == 1 ? 1 : 4))) void yz_lines_kernel(cx<R>*
     for (int h = 0; h < H; ++h)
 #pragma unroll
       for (int i = 0; i < N1; ++i) a[h][i] = bb[h][i];
+    }
   };
 
   {
@@ -279,150 +320,145 @@ __attribute__((amdgpu_waves_per_eu(H == 1 ? 1 : 4))) void yz_lines_kernel(cx<R>*
       for (int i = 0; i < N1; ++i) a[h][i] = blk[unsigned(c0 + h * CH) + unsigned(u + N2Y * i) * RS];
   }
 
-  for (;;) {
-    // persistent form: the next group's points, loaded now and used after this group's store
-    C nxt[PERSIST ? N1 : 1];
-    const long next = group + gridDim.x;
-    const bool more = PERSIST && next < groups;
-    if constexpr (PERSIST) {
-      if (more) {
-        const long np = next / B;
-        const C* __restrict__ nb = data + np * long(NY) * NZ + long(next % B) * NZ;
-        const int c0 = tid % CH, u = tid / CH;
-#pragma unroll
-        for (int i = 0; i < N1; ++i) nxt[i] = nb[unsigned(c0) + unsigned(u + N2Y * i) * RS];
-      }
-    }
+  if constexpr (MODE == LINES_FULL) {
+    // y inverse on columns
+    transform_y(p.tw_yi, std::integral_constant<int, +1>{});
+    __syncthreads();
+    cols_to_rows();
+    __syncthreads();
 
-    if constexpr (MODE == LINES_FULL) {
-      // y inverse on columns
-      transform_y(p.tw_yi, std::integral_constant<int, +1>{});
-      __syncthreads();
-      cols_to_rows();
-      __syncthreads();
-
-      // z inverse, potential phase and z forward on rows c0 + r LY/H (z = u + N2Z i).  Each
-      // row round is finished (exchange, potential, first forward step) before the next one's
-      // exchange, so that only one round's potential factors are held.
-      {
-        const int u = thread_u_z();
+    // z inverse, potential phase and z forward on rows c0 + r LY/H (z = u + N2Z i).  Each
+    // row round is finished (exchange, potential, first forward step) before the next one's
+    // exchange, so that only one round's potential factors are held.
+    {
+      const int u = thread_u_z();
 #pragma unroll
-        for (int r = 0; r < H; ++r) {
-          if (r) __syncthreads();
-          load_wz(p.tw_z, u);
-          column_dft_first<NZ, N2Z, +1>(a[r], w);
-          exchange_z(a[r], u, std::integral_constant<int, +1>{});
-          const int c0 = opaque_v(tid) % RH;
-          if (p.spx) {
-            const long pk = plane / p.nx;
-            const C* __restrict__ px = reinterpret_cast<const C*>(p.spx);
-            const C* __restrict__ py = reinterpret_cast<const C*>(p.spy) + pk * NY;
-            const C* __restrict__ pzb = reinterpret_cast<const C*>(p.spz) + pk * NZ;
-            const C pxy = cmul(px[plane], py[bres + B * (c0 + r * RH)]);
-            const int ur = opaque_v(u);     // separate loads per round (not held across rounds)
+      for (int r = 0; r < H; ++r) {
+        if (r) __syncthreads();
+        load_wz(p.tw_z, u);
+        column_dft_first<NZ, N2Z, +1>(a[r], w);
+        exchange_z(a[r], u, std::integral_constant<int, +1>{});
+        const int c0 = opaque_v(tid) % RH;
+        if constexpr (PARTS) {
 #pragma unroll
-            for (int i = 0; i < N1; ++i) {
-              a[r][i] = cmul(a[r][i], cmul(pzb[ur + N2Z * i], pxy));
-              if (H > 1 && i % 4 == 3) asm volatile("" ::: "memory");   // at most 4 factors in flight
+          for (int i = 0; i < N1; ++i) settle(a[r][i]);
+        }
+        if (p.spx) {
+          const long pk = plane / p.nx;
+          const C* __restrict__ px = reinterpret_cast<const C*>(p.spx);
+          const C* __restrict__ py = reinterpret_cast<const C*>(p.spy) + pk * NY;
+          const C* __restrict__ pzb = reinterpret_cast<const C*>(p.spz) + pk * NZ;
+          const C pxy = cmul(px[plane], py[bres + B * (c0 + r * RH)]);
+          const int ur = opaque_v(u);     // separate loads per round (not held across rounds)
+#pragma unroll
+          for (int i = 0; i < N1; ++i) {
+            a[r][i] = cmul(a[r][i], cmul(pzb[ur + N2Z * i], pxy));
+            if (H > 1 && i % 4 == 3) asm volatile("" ::: "memory");   // at most 4 factors in flight
+            if (PARTS && i % 4 == 3) settle(a[r][i]);
+          }
+        } else if constexpr (PV_LINES) {
+          constexpr unsigned T = unsigned(yz_lines_threads<NZ, LY, H>());
+          // x planes whose factors equal the previous plane's read that plane's copy (PARTS: the index
+          // through the scalar cache, which frees the registers of a 64-bit address per factor)
+          using I = std::conditional_t<PARTS != 0, const __attribute__((address_space(4))) int, const int>;
+          const long tg = p.pv_planes ? long(((I*)p.pv_planes)[plane]) * B + bres : group;
+          const C* __restrict__ pvb = reinterpret_cast<const C*>(p.pv) + tg * (long(LY) * NZ);
+          if constexpr (PARTS) {
+#pragma unroll
+            for (int i = 0; i < N1; i += 4) {
+              C f[4];
+#pragma unroll
+              for (int j = 0; j < 4; ++j) f[j] = byte_at(pvb, (unsigned(i + j) * T + unsigned(tid)) * unsigned(sizeof(C)));
+#pragma unroll
+              for (int j = 0; j < 4; ++j) a[r][i + j] = cmul(a[r][i + j], f[j]);
+#pragma unroll
+              for (int j = 0; j < 4; ++j) settle(a[r][i + j]);
             }
-          } else if constexpr (PV_LINES) {
-            constexpr unsigned T = unsigned(yz_lines_threads<NZ, LY, H>());
-            // x planes whose factors equal the previous plane's read that plane's copy
-            const long tg = p.pv_planes ? long(p.pv_planes[plane]) * B + bres : group;
-            const C* __restrict__ pvb = reinterpret_cast<const C*>(p.pv) + tg * (long(LY) * NZ);
+          } else {
 #pragma unroll
             for (int i = 0; i < N1; ++i) {
               a[r][i] = cmul(a[r][i], pvb[unsigned(r * N1 + i) * T + unsigned(tid)]);
               if (H > 1 && i % 4 == 3) asm volatile("" ::: "memory");
             }
-          } else {
-            const C* __restrict__ pvb = reinterpret_cast<const C*>(p.pv) + plane * long(NY) * NZ + long(bres) * NZ;
-#pragma unroll
-            for (int i = 0; i < N1; ++i) {
-              a[r][i] = cmul(a[r][i], pvb[unsigned(c0 + r * RH) * RS + unsigned(u + N2Z * i)]);
-              if (H > 1 && i % 4 == 3) asm volatile("" ::: "memory");
-            }
           }
-          load_wz(p.tw_z, u);
-          column_dft_first<NZ, N2Z, -1>(a[r], w);
-        }
+        } else {
+          const C* __restrict__ pvb = reinterpret_cast<const C*>(p.pv) + plane * long(NY) * NZ + long(bres) * NZ;
 #pragma unroll
-        for (int r = 0; r < H; ++r) {
-          __syncthreads();
-          exchange_z(a[r], u, std::integral_constant<int, -1>{});
+          for (int i = 0; i < N1; ++i) {
+            a[r][i] = cmul(a[r][i], pvb[unsigned(c0 + r * RH) * RS + unsigned(u + N2Z * i)]);
+            if (H > 1 && i % 4 == 3) asm volatile("" ::: "memory");
+            if (PARTS && i % 4 == 3) settle(a[r][i]);
+          }
         }
+        load_wz(p.tw_z, u);
+        column_dft_first<NZ, N2Z, -1>(a[r], w);
       }
-      __syncthreads();
-      rows_to_cols();
-      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < H; ++r) {
+        __syncthreads();
+        exchange_z(a[r], u, std::integral_constant<int, -1>{});
+      }
+    }
+    __syncthreads();
+    rows_to_cols();
+    __syncthreads();
 
-      // y forward on columns
-      transform_y(p.tw_yf, std::integral_constant<int, -1>{});
-    } else if constexpr (MODE == LINES_ENTRY) {
-      cols_to_rows();
-      __syncthreads();
-      transform_z(p.tw_z, std::integral_constant<int, -1>{});
-      __syncthreads();
-      rows_to_cols();
-      __syncthreads();
-      transform_y(p.tw_yf, std::integral_constant<int, -1>{});
-    } else if constexpr (MODE == LINES_ENTRY_OBSERVE) {
-      // the entry launch with the box moments of the position-space rows it reads
-      static_assert(H == 1 && !PERSIST, "the observing launch holds one round, one group per block");
-      cols_to_rows();
-      lines_moments<R, NZ, LY, B, N2Z, N1, yz_lines_threads<NZ, LY, H>()>(a[0], p.mom, plane, bres, group, tid,
-                                                                          thread_u_z());
-      __syncthreads();
-      transform_z(p.tw_z, std::integral_constant<int, -1>{});
-      __syncthreads();
-      rows_to_cols();
-      __syncthreads();
-      transform_y(p.tw_yf, std::integral_constant<int, -1>{});
-    } else if constexpr (MODE == LINES_EXIT) {
-      transform_y(p.tw_yi, std::integral_constant<int, +1>{});
-      __syncthreads();
-      cols_to_rows();
-      __syncthreads();
-      transform_z(p.tw_z, std::integral_constant<int, +1>{});
-      __syncthreads();
-      rows_to_cols();
-    } else {
-      // LINES_OBSERVE: the exit launch, the box moments of the position-space rows it would
-      // store, and the entry launch that would read them back, in one pass (same arithmetic)
-      static_assert(H == 1 && !PERSIST, "the observing launch holds one round, one group per block");
-      transform_y(p.tw_yi, std::integral_constant<int, +1>{});
-      __syncthreads();
-      cols_to_rows();
-      __syncthreads();
-      transform_z(p.tw_z, std::integral_constant<int, +1>{});
-      lines_moments<R, NZ, LY, B, N2Z, N1, yz_lines_threads<NZ, LY, H>()>(a[0], p.mom, plane, bres, group, tid,
-                                                                          thread_u_z());
-      __syncthreads();
-      transform_z(p.tw_zf, std::integral_constant<int, -1>{});
-      __syncthreads();
-      rows_to_cols();
-      __syncthreads();
-      transform_y(p.tw_yf, std::integral_constant<int, -1>{});
-    }
+    // y forward on columns
+    transform_y(p.tw_yf, std::integral_constant<int, -1>{});
+  } else if constexpr (MODE == LINES_ENTRY) {
+    cols_to_rows();
+    __syncthreads();
+    transform_z(p.tw_z, std::integral_constant<int, -1>{});
+    __syncthreads();
+    rows_to_cols();
+    __syncthreads();
+    transform_y(p.tw_yf, std::integral_constant<int, -1>{});
+  } else if constexpr (MODE == LINES_ENTRY_OBSERVE) {
+    // the entry launch with the box moments of the position-space rows it reads
+    static_assert(H == 1, "the observing launch holds one round");
+    cols_to_rows();
+    lines_moments<R, NZ, LY, B, N2Z, N1, yz_lines_threads<NZ, LY, H>()>(a[0], p.mom, plane, bres, group, tid,
+                                                                        thread_u_z());
+    __syncthreads();
+    transform_z(p.tw_z, std::integral_constant<int, -1>{});
+    __syncthreads();
+    rows_to_cols();
+    __syncthreads();
+    transform_y(p.tw_yf, std::integral_constant<int, -1>{});
+  } else if constexpr (MODE == LINES_EXIT) {
+    transform_y(p.tw_yi, std::integral_constant<int, +1>{});
+    __syncthreads();
+    cols_to_rows();
+    __syncthreads();
+    transform_z(p.tw_z, std::integral_constant<int, +1>{});
+    __syncthreads();
+    rows_to_cols();
+  } else {
+    // LINES_OBSERVE: the exit launch, the box moments of the position-space rows it would
+    // store, and the entry launch that would read them back, in one pass (same arithmetic)
+    static_assert(H == 1, "the observing launch holds one round");
+    transform_y(p.tw_yi, std::integral_constant<int, +1>{});
+    __syncthreads();
+    cols_to_rows();
+    __syncthreads();
+    transform_z(p.tw_z, std::integral_constant<int, +1>{});
+    lines_moments<R, NZ, LY, B, N2Z, N1, yz_lines_threads<NZ, LY, H>()>(a[0], p.mom, plane, bres, group, tid,
+                                                                        thread_u_z());
+    __syncthreads();
+    transform_z(p.tw_zf, std::integral_constant<int, -1>{});
+    __syncthreads();
+    rows_to_cols();
+    __syncthreads();
+    transform_y(p.tw_yf, std::integral_constant<int, -1>{});
+  }
 
-    {
-      const int t = opaque_v(tid);
-      const int c0 = t % CH, u = t / CH;
+  {
+    const int t = opaque_v(tid);
+    const int c0 = t % CH, u = t / CH;
 #pragma unroll
-      for (int h = 0; h < H; ++h)
+    for (int h = 0; h < H; ++h)
 #pragma unroll
-        for (int i = 0; i < N1; ++i) blk[unsigned(c0 + h * CH) + unsigned(u + N2Y * i) * RS] = a[h][i];
-    }
-    if (!more) break;
-    if constexpr (PERSIST) {
-#pragma unroll
-      for (int i = 0; i < N1; ++i) a[0][i] = nxt[i];
-      group = next;
-      plane = group / B;
-      bres = int(group % B);
-      blk = data + plane * long(NY) * NZ + long(bres) * NZ;
-      __syncthreads();   // the LDS of this group's last exchange is written again next
-    }
+      for (int i = 0; i < N1; ++i) blk[unsigned(c0 + h * CH) + unsigned(u + N2Y * i) * RS] = a[h][i];
   }
 }
 
