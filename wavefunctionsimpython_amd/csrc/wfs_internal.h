@@ -138,7 +138,7 @@ struct XSlabParams {
   long packets = 0;             // grids stacked along x
 };
 bool slab_supported(int precision, const int n[3]);
-// the same two launches for complex128 planes (kernel class WFS_K_YZ_SPLIT)
+// the same two launches under kernel class WFS_K_YZ_SPLIT: complex128 planes, complex64 96^2 and 128^2 planes
 bool split_supported(int precision, const int n[3]);
 // Per x plane (packets * nx planes of plane_elems 64-bit words, contiguous per plane): src[p]
 // = the first plane of the run of bitwise-identical consecutive planes holding p, within its

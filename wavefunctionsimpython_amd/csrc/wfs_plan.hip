@@ -777,7 +777,12 @@ extern "C" int wfs_plan_create_batched(const int n[3], const double dx[3], doubl
   p->variant[WFS_K_YZ_SLAB] = slab ? (n[1] == 192 ? 1 : 2) : 0;
   if (slab) p->variant[WFS_K_X_SLAB] = n[1] == 192 ? 1 : 2;
   const bool two_launch = slab_supported(precision, n) || split_supported(precision, n);
-  p->variant[WFS_K_YZ_SPLIT] = split_supported(precision, n) && (n[1] != 64 || n[0] < 192) ? 1 : 0;
+  // the same two launches elsewhere (figures at split_supported); complex64 128^2 planes have them under
+  // the slab class below 256 planes, with the same bits, and under this one from there on.  Their x
+  // launch: 8-z blocks while 16-z ones are few (96^2 288 planes 13.7 against 14.4 us, 512 14.5 and 15.2),
+  // whole lines from 640 planes on (768 28.7 and 26.7, 1152 38.0 and 36.2; 128^2 1536 77.7 and 68.6)
+  p->variant[WFS_K_YZ_SPLIT] = !slab && split_supported(precision, n) && (n[1] != 64 || n[0] < 192) ? 1 : 0;
+  if (p->variant[WFS_K_YZ_SPLIT]) p->variant[WFS_K_X_SLAB] = long(batch) * n[0] < 640 ? 2 : 1;
   p->pending = new std::vector<std::pair<hipEvent_t, hipEvent_t>>[WFS_K_COUNT];
   p->event_pool = new std::vector<hipEvent_t>();
   int rc = 0;
@@ -1039,7 +1044,7 @@ extern "C" int wfs_plan_set_variant(wfs_plan* p, int kc, int variant) {
     return WFS_ERR_UNSUPPORTED;
   }
   if (kc == WFS_K_YZ_SPLIT && variant > 0 && !split_supported(p->precision, p->n)) {
-    set_last_error("wfs_plan_set_variant: the split scheme needs complex128, ny = nz in {64, 96, 128, 192} and nx <= 256");
+    set_last_error("wfs_plan_set_variant: the split scheme needs ny = nz in {64, 96, 128, 192} (complex64: 96, 128) and nx <= 256");
     return WFS_ERR_UNSUPPORTED;
   }
   p->variant[kc] = variant;
@@ -1159,6 +1164,7 @@ extern "C" int wfs_plan_autotune(wfs_plan* p, void* stream) {
       if (rc == 0 && ms < best) { best = ms; best_v = v; }
     }
     p->variant[WFS_K_YZ_SLAB] = rc == 0 ? best_v : keep;
+    if (rc == 0) p->variant[WFS_K_YZ_SPLIT] = 0;     // the same launches: the choice stands in WFS_K_YZ_SLAB
   }
   p->profiling = prof;
   (void)hipEventDestroy(a);

@@ -1,10 +1,10 @@
-// Two-launch split step for complex64 grids with ny = nz in {128, 192, 256} and complex128 grids
+// Two-launch split step for complex64 grids with ny = nz in {96, 128, 192, 256} and complex128 grids
 // with ny = nz in {64, 96, 128, 192}, nx <= 256 (gfx950).  Compiled twice: WFS_SLAB_PREC=0
 // (complex64) and 1 (complex128).
 //
 // A 256^2 y-z plane (512 KiB) or a 192^2 one (288 KiB) does not fit in one CU, so the y
-// transform is split in two stages, ny = LY * B (B = 4, LY = 64 or 48; at 128, B = 2 and
-// LY = 64), y = B a + b, ky = ka + LY kb:
+// transform is split in two stages, ny = LY * B (B = 4, LY = 64 or 48; at 128 and 96, B = 2 and
+// LY = 64 and 48), y = B a + b, ky = ka + LY kb:
 //   X[ka + LY kb] = sum_b W_B^{b kb} W_NY^{b ka} sum_a x[B a + b] W_LY^{a ka}
 // and each stage rides on a pass that is needed anyway:
 //
@@ -33,12 +33,12 @@ namespace {
 template <int N> constexpr int kZB128 = N <= 64 ? 4 : 8;
 
 // rows y = B a + b of a row group: the length-B stage rides on the x launch (complex64: B = 4 at
-// 256 and 192, LY = 64 and 48 rows per group; B = 2 at 128, LY = 64; complex128: B = 2 up to 128,
+// 256 and 192, LY = 64 and 48 rows per group; B = 2 at 128 and 96, LY = 64 and 48; complex128: B = 2 up to 128,
 // where the x launch then holds one row a lane: 33, 74 and 129 KiB of LDS per group at 64, 96 and
 // 128, B = 4 at 192, 148 KiB).  Measured at 64^3 and 128^3 complex128, y-z and x launch: B = 2 8.0 +
 // 5.7 and 25.9 + 16.5 us, B = 4 7.3 + 7.5 and 24.2 + 21.9.
 template <typename R, int N> struct SlabShape {
-  static constexpr int B = (sizeof(R) == 4 ? N == 128 : N <= 128) ? 2 : 4;
+  static constexpr int B = N <= 128 ? 2 : 4;
   static constexpr int LY = N / B;
 };
 
@@ -474,8 +474,16 @@ bool slab_supported(int precision, const int n[3]) {
 // 192^2 76.4 -> 46.0, 48 x 64^3 192 -> 144; only long x lines beside 64^2 planes were slower
 // (192 x 64^2 27.6 -> 29.9, 256 x 64^2 28.7 -> 34.6: x blocks of 128 and more points a lane pair),
 // so the plan leaves those to the plane pass.
+//
+// complex64, ny = nz = 96 or 128: the plane pass holds a whole plane per block, a 96^2 plane in 74 KB with 12
+// points of two lines a thread and one block a CU, against row groups of half a plane.  us per step with a
+// potential table / with per-axis factors: 96^2 8 planes 24.4 / 21.6 -> 15.1 / 15.3, 64 planes 29.5 / 26.8 ->
+// 20.0 / 20.2, 96^3 35.2 / 32.6 -> 26.8 / 27.0, 3 packets of it 57.9 / 56.8 -> 34.8 / 39.0, 12 packets 147 / 132
+// -> 93 / 90; 128^2 256 planes 49.6 / 43.3 -> 40.6 / 39.4, 512 planes 78 / 71 -> 70 / 68, 1536 planes 240 / 182
+// -> 191 / 172.  Not at 64^2: 14.0 / 12.7 -> 11.3 / 11.5 for one packet, but 12 packets of 96 x 64^2 47 / 42 ->
+// 45 / 44, and the tuned 64^2 forms are bit for bit the axis passes.
 bool split_supported(int precision, const int n[3]) {
-  return precision == WFS_C128 && n[1] == n[2] && (n[1] == 64 || n[1] == 96 || n[1] == 128 || n[1] == 192) &&
+  return n[1] == n[2] && (n[1] == 96 || n[1] == 128 || (precision == WFS_C128 && (n[1] == 64 || n[1] == 192))) &&
          n[0] <= 256 && fft_length_supported(n[0]);
 }
 
@@ -486,11 +494,13 @@ int launch_x_slab_c128(int nx, int n, void* data, const XSlabParams& p, hipStrea
 
 SlabRows slab_rows(int precision, int n) {
   if (precision == WFS_C128) return slab_rows_c128(n);
+  if (n == 96) return slab_rows_n<float, 96>();
   return n == 128 ? slab_rows_n<float, 128>() : n == 192 ? slab_rows_n<float, 192>() : slab_rows_n<float, 256>();
 }
 
 LinesOrder slab_lines_order(int precision, int n) {
   if (precision == WFS_C128) return slab_lines_order_c128(n);
+  if (n == 96) return slab_lines_order_n<float, 96>();
   return n == 128 ? slab_lines_order_n<float, 128>()
                   : n == 192 ? slab_lines_order_n<float, 192>() : slab_lines_order_n<float, 256>();
 }
@@ -504,6 +514,7 @@ int launch_yz_slab(int precision, int n, int mode, void* data, const YzPlanePara
   if (n == 256) return launch_lines_n<float, 256>(mode, data, p, s);
   if (n == 192) return launch_lines_n<float, 192>(mode, data, p, s);
   if (n == 128) return launch_lines_n<float, 128>(mode, data, p, s);
+  if (n == 96) return launch_lines_n<float, 96>(mode, data, p, s);
   set_last_error("slab y-z pass: unsupported plane %d", n);
   return WFS_ERR_UNSUPPORTED;
 }
@@ -518,6 +529,7 @@ int launch_x_slab(int precision, int nx, int n, int variant, void* data, const X
   if (n == 256) return launch_x_slab_ny<float, 256>(nx, variant, data, p, s);
   if (n == 192) return launch_x_slab_ny<float, 192>(nx, variant, data, p, s);
   if (n == 128) return launch_x_slab_ny<float, 128>(nx, variant, data, p, s);
+  if (n == 96) return launch_x_slab_ny<float, 96>(nx, variant, data, p, s);
   set_last_error("slab x pass: unsupported plane %d", n);
   return WFS_ERR_UNSUPPORTED;
 }
