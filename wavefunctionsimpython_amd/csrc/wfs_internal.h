@@ -75,17 +75,6 @@ struct LinesOrder {
   long ny = 0, nz = 0;
   int ly = 0, b = 1, rh = 0, n2z = 0, n1 = 0, threads = 0;
 };
-// natural (C-order) index of element o of a lines-ordered table
-__host__ __device__ inline long lines_source(long o, const LinesOrder& m) {
-  const long per = long(m.ly) * m.nz;
-  const long g = o / per, rem = o % per;
-  const long ri = rem / m.threads;
-  const int t = int(rem % m.threads);
-  const int r = int(ri / m.n1), i = int(ri % m.n1);
-  const long row = long(m.b) * ((t % m.rh) + long(r) * m.rh) + g % m.b;
-  return (g / m.b) * m.ny * m.nz + row * m.nz + (t / m.rh) + long(m.n2z) * i;
-}
-
 // boxes measured in one launch_box_moments call (and one LINES_OBSERVE launch)
 constexpr int kBoxesPerPass = 4;
 // Simpson box moments taken inside a LINES_OBSERVE launch: one record of 7 sums per row group
@@ -138,7 +127,7 @@ struct XSlabParams {
   long packets = 0;             // grids stacked along x
 };
 bool slab_supported(int precision, const int n[3]);
-// the same two launches under kernel class WFS_K_YZ_SPLIT: complex128 planes, complex64 96^2 and 128^2 planes
+// the same two launches under kernel class WFS_K_YZ_SPLIT: complex128 planes, complex64 96^2, 128^2 and 512^2 planes
 bool split_supported(int precision, const int n[3]);
 // Per x plane (packets * nx planes of plane_elems 64-bit words, contiguous per plane): src[p]
 // = the first plane of the run of bitwise-identical consecutive planes holding p, within its
@@ -162,11 +151,10 @@ int launch_x_slab(int precision, int nx, int n, int variant, void* data, const X
 
 // pv = cexp_i(-dt V) elementwise in the state precision
 int launch_potential_phase(int precision, long count, const float2* V, double dt, void* pv, hipStream_t s);
-// the same table written in lines order: pv[o] = cexp_i(-dt V[lines_source(o)])
+// the same table written in lines order
 int launch_potential_phase_lines(int precision, long count, const float2* V, double dt, void* pv,
                                  const LinesOrder& m, hipStream_t s);
-// move a table between natural and lines order (to_lines: dst[o] = src[lines_source(o)],
-// else dst[lines_source(o)] = src[o])
+// move a table between natural and lines order
 int launch_table_reorder(int precision, long count, const void* src, void* dst, const LinesOrder& m, bool to_lines,
                          hipStream_t s);
 

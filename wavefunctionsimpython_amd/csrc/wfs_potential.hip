@@ -288,25 +288,50 @@ __global__ __launch_bounds__(kGenThreads) void potential_table_kernel(cx<R>* __r
   out[i] = potential_factor<R>(V[i], dt);
 }
 
-// the same factors in the order the slab scheme's y-z launch reads them
-template <typename R>
-__global__ __launch_bounds__(kGenThreads) void potential_table_lines_kernel(cx<R>* __restrict__ out,
-                                                                            const float2* __restrict__ V, long n,
-                                                                            double dt, LinesOrder m) {
-  const long o = long(blockIdx.x) * kGenThreads + threadIdx.x;
-  if (o >= n) return;
-  out[o] = potential_factor<R>(V[lines_source(o, m)], dt);
-}
+// Table between C order and the order the slab scheme's y-z launch reads (LinesOrder: z-major within a row
+// group): 16 z points of one group through LDS, so that both sides move in runs (128-byte row pieces, whole
+// rows of the transpose).  TABLE_FACTORS computes the factors of V on the way; the FP64 sine, cosine and
+// exponential and the memory bound it: 256^3 complex64 120 -> 68 us, 512^3 970 -> 675, 192^3 52 -> 32,
+// 128^3 complex128 20 -> 14, against one element a thread that reads V down the rows (the table in C order
+// takes 60, 634, 24 and 11).
+enum { TABLE_FACTORS, TABLE_TO_LINES, TABLE_FROM_LINES };
+constexpr int kLinesTileZ = 16, kLinesTileRows = 64;
 
-template <typename R>
-__global__ __launch_bounds__(kGenThreads) void table_reorder_kernel(cx<R>* __restrict__ dst,
-                                                                    const cx<R>* __restrict__ src, long n,
-                                                                    LinesOrder m, int to_lines) {
-  const long o = long(blockIdx.x) * kGenThreads + threadIdx.x;
-  if (o >= n) return;
-  const long j = lines_source(o, m);
-  if (to_lines) dst[o] = src[j];
-  else dst[j] = src[o];
+template <typename R, int MODE>
+__global__ __launch_bounds__(kGenThreads) void table_lines_kernel(cx<R>* __restrict__ dst, const void* __restrict__ src,
+                                                                  double dt, LinesOrder m) {
+  __shared__ cx<R> tile[kLinesTileZ][kLinesTileRows + 1];
+  const long tiles = m.nz / kLinesTileZ;
+  const long g = blockIdx.x / tiles;
+  const int z0 = int(blockIdx.x % tiles) * kLinesTileZ;
+  const long nat = (g / m.b) * m.ny * m.nz + (g % m.b) * m.nz + z0;     // row b y, z: nat + b y nz + z - z0
+  const long lin = g * (long(m.ly) * m.nz) + long(z0) * m.ly;            // row b y, z: lin + (z - z0) ly + y
+  // 16 lanes along z and 16 rows a round on the C-order side, a wavefront per z on the other
+  constexpr int kRows = kGenThreads / kLinesTileZ, kLines = kGenThreads / 64;
+  const int zl = threadIdx.x % kLinesTileZ, yl = threadIdx.x / kLinesTileZ;
+  const int row = threadIdx.x % 64, zw = threadIdx.x / 64;
+  if constexpr (MODE == TABLE_FROM_LINES) {
+    const cx<R>* in = static_cast<const cx<R>*>(src);
+#pragma unroll
+    for (int z = zw; z < kLinesTileZ; z += kLines)
+      if (row < m.ly) tile[z][row] = in[lin + long(z) * m.ly + row];
+    __syncthreads();
+#pragma unroll
+    for (int y = yl; y < kLinesTileRows; y += kRows)
+      if (y < m.ly) dst[nat + long(m.b) * m.nz * y + zl] = tile[zl][y];
+  } else {
+#pragma unroll
+    for (int y = yl; y < kLinesTileRows; y += kRows) {
+      if (y >= m.ly) break;
+      const long j = nat + long(m.b) * m.nz * y + zl;
+      tile[zl][y] = MODE == TABLE_FACTORS ? potential_factor<R>(static_cast<const float2*>(src)[j], dt)
+                                          : static_cast<const cx<R>*>(src)[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int z = zw; z < kLinesTileZ; z += kLines)
+      if (row < m.ly) dst[lin + long(z) * m.ly + row] = tile[z][row];
+  }
 }
 
 }  // namespace
@@ -507,34 +532,36 @@ int launch_potential_phase(int precision, long count, const float2* V, double dt
   return int(hipGetLastError());
 }
 
+// one round of row groups (every row of a group in one round: rh = ly), as the slab scheme has them
 static bool lines_order_ok(long count, const LinesOrder& m) {
-  return m.ly > 0 && m.nz > 0 && m.b > 0 && m.rh > 0 && m.n1 > 0 && m.threads > 0 &&
-         count % (long(m.ly) * m.nz) == 0 && long(m.ly) * m.b == m.ny;
+  return m.ly > 0 && m.ly <= kLinesTileRows && m.nz > 0 && m.nz % kLinesTileZ == 0 && m.b > 0 && m.rh == m.ly &&
+         m.threads == m.n2z * m.rh && m.n1 * m.n2z == m.nz && count % (long(m.ly) * m.nz) == 0 &&
+         long(m.ly) * m.b == m.ny && count / (long(m.ly) * kLinesTileZ) <= 0x7fffffffL;
+}
+
+template <int MODE>
+static int launch_table_lines(int precision, long count, const void* src, double dt, void* dst, const LinesOrder& m,
+                              hipStream_t s) {
+  if (count <= 0) return 0;
+  if (!lines_order_ok(count, m)) { set_last_error("potential table: bad lines order"); return WFS_ERR_INVALID; }
+  const unsigned blocks = unsigned(count / (long(m.ly) * kLinesTileZ));
+  if (precision == WFS_C128)
+    hipLaunchKernelGGL((table_lines_kernel<double, MODE>), dim3(blocks), dim3(kGenThreads), 0, s,
+                       static_cast<double2*>(dst), src, dt, m);
+  else
+    hipLaunchKernelGGL((table_lines_kernel<float, MODE>), dim3(blocks), dim3(kGenThreads), 0, s,
+                       static_cast<float2*>(dst), src, dt, m);
+  return int(hipGetLastError());
 }
 
 int launch_potential_phase_lines(int precision, long count, const float2* V, double dt, void* pv,
                                  const LinesOrder& m, hipStream_t s) {
-  if (count <= 0) return 0;
-  if (!lines_order_ok(count, m)) { set_last_error("potential table: bad lines order"); return WFS_ERR_INVALID; }
-  if (precision == WFS_C128)
-    hipLaunchKernelGGL(potential_table_lines_kernel<double>, dim3(blocks_for(count)), dim3(kGenThreads), 0, s,
-                       static_cast<double2*>(pv), V, count, dt, m);
-  else
-    hipLaunchKernelGGL(potential_table_lines_kernel<float>, dim3(blocks_for(count)), dim3(kGenThreads), 0, s,
-                       static_cast<float2*>(pv), V, count, dt, m);
-  return int(hipGetLastError());
+  return launch_table_lines<TABLE_FACTORS>(precision, count, V, dt, pv, m, s);
 }
 
 int launch_table_reorder(int precision, long count, const void* src, void* dst, const LinesOrder& m, bool to_lines,
                          hipStream_t s) {
-  if (count <= 0) return 0;
-  if (!lines_order_ok(count, m)) { set_last_error("potential table: bad lines order"); return WFS_ERR_INVALID; }
-  if (precision == WFS_C128)
-    hipLaunchKernelGGL(table_reorder_kernel<double>, dim3(blocks_for(count)), dim3(kGenThreads), 0, s,
-                       static_cast<double2*>(dst), static_cast<const double2*>(src), count, m, int(to_lines));
-  else
-    hipLaunchKernelGGL(table_reorder_kernel<float>, dim3(blocks_for(count)), dim3(kGenThreads), 0, s,
-                       static_cast<float2*>(dst), static_cast<const float2*>(src), count, m, int(to_lines));
-  return int(hipGetLastError());
+  return to_lines ? launch_table_lines<TABLE_TO_LINES>(precision, count, src, 0.0, dst, m, s)
+                  : launch_table_lines<TABLE_FROM_LINES>(precision, count, src, 0.0, dst, m, s);
 }
 }  // namespace wfs
