@@ -362,7 +362,7 @@ int wfs_plan_set_profiling(wfs_plan* plan, int enable);
  * WFS_K_X_SLAB and WFS_K_SLAB_EDGE): variant 1 (default where supported:
  * complex128 grids with ny = nz in {64, 96, 128, 192} and complex64 grids with
  * ny = nz = 96 or, from 256 x planes on, 128, nx <= 256, at 64 only below 192 x
- * planes) runs the steps as the slab scheme's two launches, variant 0 as the plane pass or the
+ * planes; complex64 grids with ny = nz = 512 and nx >= 32) runs the steps as the slab scheme's two launches, variant 0 as the plane pass or the
  * axis passes; the results agree to rounding.  Setting WFS_K_YZ_PLANE or
  * WFS_K_YZ_SLAB switches it off.
  */

@@ -1,4 +1,4 @@
-"""complex64 96^2 and 128^2 planes stepped as two launches (kernel class yz_split) against the passes, the
+"""complex64 96^2, 128^2 and 512^2 planes stepped as two launches (kernel class yz_split) against the passes, the
 slab class's launches and the oracle."""
 
 import numpy as np
@@ -17,7 +17,9 @@ C64 = _abi.WFS_C64
 def _plan(shape, split=None, batch=1):
     p = _abi.Plan(shape, DX, DT, 1.0, C64, _abi.WFS_METHOD_FOURIER, batch=batch)
     if split is not None:
-        p.set_variant("yz_slab", 0)
+        p.set_variant("yz_plane", 0)
+        if shape[1] == 128:
+            p.set_variant("yz_slab", 0)
         p.set_variant("yz_split", split)
     return p
 
@@ -31,9 +33,11 @@ def _state(shape, dev, seed=0):
 
 
 # a few roundings of 6e-8 per transform and axis, steps transforms there and back
-@pytest.mark.parametrize("n", [96, 128])
-@pytest.mark.parametrize("nx,steps", [(8, 1), (32, 3), (96, 2), (256, 2)])
-def test_split_matches_passes(dev, n, nx, steps):
+@pytest.mark.parametrize("nx,n,steps", [(nx, n, steps) for n in (96, 128)
+                                        for nx, steps in ((8, 1), (32, 3), (96, 2), (256, 2))]
+                         + [(32, 512, 3), (64, 512, 1), (96, 512, 2), (128, 512, 1), (192, 512, 1), (256, 512, 2),
+                            (512, 512, 1)])
+def test_split_matches_passes(dev, nx, n, steps):
     shape = (nx, n, n)
     psi, V = _state(shape, dev, n + nx)
     out = []
@@ -46,9 +50,9 @@ def test_split_matches_passes(dev, n, nx, steps):
     assert oracle.relative_l2(out[1].cpu().numpy(), out[0].cpu().numpy()) < 2e-6
 
 
-@pytest.mark.parametrize("n", [96, 128])
-def test_split_matches_oracle_and_follows_the_potential(dev, n):
-    shape = (16, n, n)
+@pytest.mark.parametrize("nx,n", [(16, 96), (16, 128), (32, 512)])
+def test_split_matches_oracle_and_follows_the_potential(dev, nx, n):
+    shape = (nx, n, n)
     psi, V = _state(shape, dev, 3)
     p = _plan(shape, 1)
     a = psi.clone()
@@ -68,12 +72,13 @@ def test_split_matches_oracle_and_follows_the_potential(dev, n):
 
 
 # 3 packets stay below 256 planes of 128^2 (slab class), 10 pass it and the 640 of the 16-z x launch
-@pytest.mark.parametrize("shape,batch", [((16, 96, 96), 3), ((64, 96, 96), 10), ((64, 128, 128), 3), ((64, 128, 128), 10)])
+@pytest.mark.parametrize("shape,batch", [((32, 512, 512), 2), ((16, 96, 96), 3), ((64, 96, 96), 10), ((64, 128, 128), 3), ((64, 128, 128), 10)])
 def test_default_packets_equal_single_runs(dev, shape, batch):
     rng = np.random.default_rng(batch)
     axes = [rng.uniform(-1, 1, (batch, m)) for m in shape]
     psi = _state((batch,) + shape, dev, batch)[0]
     p = _plan(shape, batch=batch)
+    assert p.variants()["yz_split"] or p.variants()["yz_slab"]
     p.set_potential_axes(*axes)
     a = psi.clone()
     p.step(a, None, 3)
@@ -93,5 +98,7 @@ def test_split_defaults(dev):
     assert on((128, 128, 128)) == (0, 2) and on((256, 128, 128)) == (1, 0) and on((64, 128, 128), 8) == (1, 0)
     assert on((64, 64, 64)) == (0, 0) and on((512, 96, 96)) == (0, 0) and on((32, 96, 128)) == (0, 0)
     assert on((192, 192, 192)) == (0, 1)
+    assert on((512, 512, 512)) == (1, 0) and on((32, 512, 512)) == (1, 0) and on((16, 512, 512)) == (0, 0)
+    assert on((512, 256, 256)) == (0, 0) and on((32, 512, 256)) == (0, 0)
     with pytest.raises(_abi.WfsError):
         _plan((64, 64, 64)).set_variant("yz_split", 1)

@@ -1044,7 +1044,7 @@ extern "C" int wfs_plan_set_variant(wfs_plan* p, int kc, int variant) {
     return WFS_ERR_UNSUPPORTED;
   }
   if (kc == WFS_K_YZ_SPLIT && variant > 0 && !split_supported(p->precision, p->n)) {
-    set_last_error("wfs_plan_set_variant: the split scheme needs ny = nz in {64, 96, 128, 192} (complex64: 96, 128) and nx <= 256");
+    set_last_error("wfs_plan_set_variant: the split scheme needs ny = nz in {64, 96, 128, 192} and nx <= 256 (complex64: 96, 128, or 512 with nx >= 32)");
     return WFS_ERR_UNSUPPORTED;
   }
   p->variant[kc] = variant;

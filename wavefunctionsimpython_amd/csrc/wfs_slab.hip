@@ -1,10 +1,10 @@
-// Two-launch split step for complex64 grids with ny = nz in {96, 128, 192, 256} and complex128 grids
-// with ny = nz in {64, 96, 128, 192}, nx <= 256 (gfx950).  Compiled twice: WFS_SLAB_PREC=0
+// Two-launch split step for complex64 grids with ny = nz in {96, 128, 192, 256, 512} and complex128 grids
+// with ny = nz in {64, 96, 128, 192}, nx <= 256 (512 beside 512^2 planes; gfx950).  Compiled twice: WFS_SLAB_PREC=0
 // (complex64) and 1 (complex128).
 //
 // A 256^2 y-z plane (512 KiB) or a 192^2 one (288 KiB) does not fit in one CU, so the y
 // transform is split in two stages, ny = LY * B (B = 4, LY = 64 or 48; at 128 and 96, B = 2 and
-// LY = 64 and 48), y = B a + b, ky = ka + LY kb:
+// LY = 64 and 48; at 512, B = 8 and LY = 64), y = B a + b, ky = ka + LY kb:
 //   X[ka + LY kb] = sum_b W_B^{b kb} W_NY^{b ka} sum_a x[B a + b] W_LY^{a ka}
 // and each stage rides on a pass that is needed anyway:
 //
@@ -33,12 +33,12 @@ namespace {
 template <int N> constexpr int kZB128 = N <= 64 ? 4 : 8;
 
 // rows y = B a + b of a row group: the length-B stage rides on the x launch (complex64: B = 4 at
-// 256 and 192, LY = 64 and 48 rows per group; B = 2 at 128 and 96, LY = 64 and 48; complex128: B = 2 up to 128,
+// 256 and 192, LY = 64 and 48 rows per group; B = 2 at 128 and 96, LY = 64 and 48; B = 8 at 512, LY = 64; complex128: B = 2 up to 128,
 // where the x launch then holds one row a lane: 33, 74 and 129 KiB of LDS per group at 64, 96 and
 // 128, B = 4 at 192, 148 KiB).  Measured at 64^3 and 128^3 complex128, y-z and x launch: B = 2 8.0 +
 // 5.7 and 25.9 + 16.5 us, B = 4 7.3 + 7.5 and 24.2 + 21.9.
 template <typename R, int N> struct SlabShape {
-  static constexpr int B = N <= 128 ? 2 : 4;
+  static constexpr int B = N <= 128 ? 2 : N <= 256 ? 4 : 8;
   static constexpr int LY = N / B;
 };
 
@@ -253,6 +253,140 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && ZB == 8 && NX / split_of<NX
 }
 
 #if WFS_SLAB_PREC == 0
+// Moves the 8 x 8 matrix (lane bits 3..5, register r) of a wavefront to its transpose: register r of the
+// lanes with bits q holds afterwards what register q of the lanes with bits r held.  One pass per bit
+// pair; the halves of two registers are exchanged by gfx950's row and half-wavefront swaps, and 8 lanes
+// along by a DPP rotation that writes the masked banks only.
+__device__ __forceinline__ void transpose8_words(float (&v)[8]) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[r]), __float_as_uint(v[r + 4]), false, false);
+    v[r] = __uint_as_float(s[0]);
+    v[r + 4] = __uint_as_float(s[1]);
+  }
+#pragma unroll
+  for (int h = 0; h < 8; h += 4)
+#pragma unroll
+    for (int r = h; r < h + 2; ++r) {
+      const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[r]), __float_as_uint(v[r + 2]), false, false);
+      v[r] = __uint_as_float(s[0]);
+      v[r + 2] = __uint_as_float(s[1]);
+    }
+  constexpr int kRowRor8 = 0x128;
+#pragma unroll
+  for (int r = 0; r < 8; r += 2) {
+    const int lo = __float_as_int(v[r]), hi = __float_as_int(v[r + 1]);
+    v[r] = __int_as_float(__builtin_amdgcn_update_dpp(lo, hi, kRowRor8, 0xF, 0xC, false));
+    v[r + 1] = __int_as_float(__builtin_amdgcn_update_dpp(hi, lo, kRowRor8, 0xF, 0x3, false));
+  }
+}
+
+__device__ __forceinline__ void transpose8(cx<float>* a) {
+  float x[8], y[8];
+#pragma unroll
+  for (int r = 0; r < 8; ++r) { x[r] = a[r].x; y[r] = a[r].y; }
+  transpose8_words(x);
+  transpose8_words(y);
+#pragma unroll
+  for (int r = 0; r < 8; ++r) a[r] = mk<float>(x[r], y[r]);
+}
+
+// x launch of planes whose y transform is split off a length-8 stage (512^2: rows y = 8 a + b).  A block
+// owns the 8 rows of one ka over 8 z points and all x; lane 8 q + z of every wavefront holds row b = q at
+// x = t + N2 i, t the wavefront's index, so that the x transforms' twiddles and kinetic factors are the
+// same in all lanes and come through the scalar cache.  For the y stage 8 rows are brought into one lane
+// (transpose8, 8 x points at a time), transformed there and sent back; the x transforms exchange one part
+// at a time through 4 NX 64 bytes of LDS, 128 KiB at nx = 512 (one block of 1024 threads, 128 registers).
+// Memory is touched in 64-byte segments; all z tiles of a ka go to one XCD (blocks go round-robin over the 8
+// of them), so that the halves of a line and the rows of a page stay with one L2: 512^3 597 us against 646
+// with the tiles of a ka spread over the XCDs in pairs (the axis pass alone takes 688, 256 x 512^2 317 -> 233,
+// 64 x 512^2 46 -> 50), bound by the 400 us of its arithmetic beside one block's waits.  Lanes along x instead
+// of the rows at the loads save a transposition and lose more to eight pages a load: 692 us.
+template <int NX, int N>
+__global__ __launch_bounds__(64 * split_of<NX>::n2) void x_rows8_kernel(cx<float>* __restrict__ data,
+                                                                        const XSlabParams p) {
+  constexpr int B = 8, ZB = 8, A = N / B, TZ = N / ZB;
+  constexpr int N2 = split_of<NX>::n2, N1 = NX / N2;
+  static_assert(N1 % 8 == 0 && (long(A) * TZ) % 16 == 0, "bad split of the x line");
+  using C = cx<float>;
+  using CC = const __attribute__((address_space(4))) C;
+  __shared__ float lds[64 * NX];
+
+  const int lane = threadIdx.x & 63;
+  const int t = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long bid = blockIdx.x;
+  const int zt = int((bid / 8) % TZ);
+  const int ka = int((bid / (8 * TZ)) % (A / 8)) * 8 + int(bid % 8);
+  const long pk = bid / (long(TZ) * A);
+  C* __restrict__ blk = data + pk * (long(NX) * N * N) + long(B * ka) * N + long(zt) * ZB;
+  constexpr unsigned XS = unsigned(N) * N, EB = unsigned(sizeof(C));
+  static_assert(long(NX) * N * N * sizeof(C) <= (1L << 32), "32-bit byte offsets");
+
+  auto off = [&](int l, int i) {
+    return (unsigned(l & 7) + unsigned(l >> 3) * N + (unsigned(t) + unsigned(N2) * unsigned(i)) * XS) * EB;
+  };
+  C a[N1];
+#pragma unroll
+  for (int i = 0; i < N1; ++i) a[i] = byte_at(blk, off(lane, i));
+
+  CC* twy = (CC*)(p.tw_y);
+  // forward y stage X[kb] = sum_b W_8^{b kb} W_N^{b ka} Y[b] on 8 x points at a time
+#pragma unroll
+  for (int g = 0; g < N1; g += 8) {
+    transpose8(a + g);
+    C r[B];
+    r[0] = a[g];
+#pragma unroll
+    for (int b = 1; b < B; ++b) r[b] = cmul(a[g + b], mk<float>(twy[(b * ka) % N].x, twy[(b * ka) % N].y));
+    DFT<B, -1>::run(r);
+#pragma unroll
+    for (int b = 0; b < B; ++b) a[g + b] = r[b];
+    transpose8(a + g);
+  }
+  CC* twx = (CC*)(p.tw_x);
+  auto lidx = [&](int k1, int n2) { return (k1 * N2 + n2) * 64 + lane; };
+  auto transform_x = [&](auto sign_c) {
+    constexpr int SG = decltype(sign_c)::value;
+    DFT<N1, SG>::run(a);
+#pragma unroll
+    for (int k1 = 1; k1 < N1; ++k1) {
+      const C w = mk<float>(twx[(t * k1) % NX].x, twx[(t * k1) % NX].y);
+      a[k1] = SG < 0 ? cmul(a[k1], w) : cmulc(a[k1], w);
+    }
+    column_dft_second_parts<NX, N2, SG>(a, lds, t, lidx);
+  };
+
+  transform_x(std::integral_constant<int, -1>{});
+  {
+    const C ky = reinterpret_cast<const C*>(p.ky)[ka + A * (lane >> 3)];
+    const C kyz = cmul(ky, reinterpret_cast<const C*>(p.kz)[zt * ZB + (lane & 7)]);
+    CC* kx = (CC*)(p.kx) + t;
+#pragma unroll
+    for (int i = 0; i < N1; ++i) a[i] = cmul(a[i], cmul(mk<float>(kx[N2 * i].x, kx[N2 * i].y), kyz));
+  }
+  __syncthreads();
+  transform_x(std::integral_constant<int, +1>{});
+
+  // inverse y stage Y'[b] = W_N^{-b ka} sum_kb W_8^{-b kb} X[kb], stored 8 x points at a time
+  const int l = opaque_v(lane);
+#pragma unroll
+  for (int g = 0; g < N1; g += 8) {
+    transpose8(a + g);
+    C r[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) r[b] = a[g + b];
+    DFT<B, +1>::run(r);
+    a[g] = r[0];
+#pragma unroll
+    for (int b = 1; b < B; ++b) a[g + b] = cmulc(r[b], mk<float>(twy[(b * ka) % N].x, twy[(b * ka) % N].y));
+    transpose8(a + g);
+#pragma unroll
+    for (int i = g; i < g + 8; ++i) byte_at(blk, off(l, i)) = a[i];
+  }
+}
+#endif
+
+#if WFS_SLAB_PREC == 0
 // flags[p] = 1 when x plane p equals plane p - 1 of the same packet bit for bit, else 0
 __global__ __launch_bounds__(256) void plane_equal_kernel(const unsigned long long* __restrict__ table,
                                                           long plane_elems, int nx, long first,
@@ -336,7 +470,7 @@ int cu_count() {
 template <typename R, int N, int MODE, int PARTS = 0>
 int launch_lines_m(void* data, const YzPlaneParams& p, hipStream_t s) {
   constexpr int LY = SlabShape<R, N>::LY, B = SlabShape<R, N>::B;
-  static_assert(yz_lines_lds_bytes<R, N, LY, 1>() <= 160 * 1024, "rows do not fit in LDS");
+  static_assert(yz_lines_lds_bytes<R, N, LY, 1>() / (PARTS ? 2 : 1) <= 160 * 1024, "rows do not fit in LDS");
   const long groups = p.planes * B;
   WFS_LAUNCH((yz_lines_kernel<R, N, LY, B, 1, MODE, true, PARTS>), dim3(unsigned(groups)),
                      dim3(yz_lines_threads<N, LY, 1>()), 0, s, reinterpret_cast<cx<R>*>(data), p);
@@ -349,8 +483,9 @@ int launch_lines_m(void* data, const YzPlaneParams& p, hipStream_t s) {
 // block's loads and stores run beside the other's transforms.  192^2: one 768-thread block either way, but
 // the transforms no longer wait for the factor loads hoisted over them.  Not for complex128 (128^3 27.3 ->
 // 28.6, 192^3 80.3 -> 85.6, 96^3 17.2 -> 18.3 us: its 3 and more exchanges cost what the second block
-// gains) nor for complex64 128^2 planes (19.0 -> 19.3).
-template <typename R, int N> constexpr int lines_parts() { return sizeof(R) == 8 ? 0 : N == 256 ? 8 : N == 192 ? 3 : 0; }
+// gains) nor for complex64 128^2 planes (19.0 -> 19.3).  512^2: the only form that fits, 131 KB of LDS and 128
+// registers a block of 1024 threads; 512^3 830 us a full launch (3.3 GB: 4.0 TB/s), 510 an entry or exit.
+template <typename R, int N> constexpr int lines_parts() { return sizeof(R) == 8 ? 0 : N == 512 ? 4 : N == 256 ? 8 : N == 192 ? 3 : 0; }
 
 // The parts form is taken where the groups are more than the CUs.  us of the full / entry or exit launch,
 // whole against parts: 256^2 256 planes 85 / 57 -> 76 / 49, 192 planes 64 / 44 -> 57 / 39, 128 planes
@@ -359,7 +494,7 @@ template <typename R, int N> constexpr int lines_parts() { return sizeof(R) == 8
 // and the extra barriers show: 256^2 64 planes 24.1 / 15.3 -> 26.2 / 16.4, 192^2 17.9 -> 19.0.
 template <typename R, int N>
 bool lines_in_parts(long planes) {
-  return lines_parts<R, N>() != 0 && planes * SlabShape<R, N>::B > cu_count();
+  return N == 512 || (lines_parts<R, N>() != 0 && planes * SlabShape<R, N>::B > cu_count());
 }
 
 // complex128 has the one-block-per-group forms only, and takes its box moments in their own launches
@@ -374,10 +509,12 @@ int launch_lines_n(int mode, void* data, const YzPlaneParams& p, hipStream_t s) 
       if (mode == LINES_EXIT) return launch_lines_m<R, N, LINES_EXIT, W>(data, p, s);
     }
   }
-  if (mode == LINES_FULL) return launch_lines_m<R, N, LINES_FULL>(data, p, s);
-  if (mode == LINES_ENTRY) return launch_lines_m<R, N, LINES_ENTRY>(data, p, s);
-  if (mode == LINES_EXIT) return launch_lines_m<R, N, LINES_EXIT>(data, p, s);
-  if constexpr (sizeof(R) == 4) {
+  if constexpr (N < 512) {
+    if (mode == LINES_FULL) return launch_lines_m<R, N, LINES_FULL>(data, p, s);
+    if (mode == LINES_ENTRY) return launch_lines_m<R, N, LINES_ENTRY>(data, p, s);
+    if (mode == LINES_EXIT) return launch_lines_m<R, N, LINES_EXIT>(data, p, s);
+  }
+  if constexpr (sizeof(R) == 4 && N >= 128 && N < 512) {
     if (mode == LINES_OBSERVE) return launch_lines_m<R, N, LINES_OBSERVE>(data, p, s);
     if (mode == LINES_ENTRY_OBSERVE) return launch_lines_m<R, N, LINES_ENTRY_OBSERVE>(data, p, s);
   }
@@ -417,6 +554,30 @@ int launch_x_slab_ny(int nx, int variant, void* data, const XSlabParams& p, hipS
   }
 #undef WFS_X_SLAB_CASE
 }
+
+#if WFS_SLAB_PREC == 0
+int launch_x_rows8(int nx, void* data, const XSlabParams& p, hipStream_t s) {
+  constexpr int N = 512;
+#define WFS_X_ROWS8_CASE(NX)                                                                                 \
+  case NX:                                                                                                   \
+    WFS_LAUNCH((x_rows8_kernel<NX, N>), dim3(unsigned(p.packets * (N / 8) * (N / 8))),                          \
+               dim3(64 * split_of<NX>::n2), 0, s, reinterpret_cast<cx<float>*>(data), p);                         \
+    return int(hipGetLastError());
+  switch (nx) {
+    WFS_X_ROWS8_CASE(32)
+    WFS_X_ROWS8_CASE(64)
+    WFS_X_ROWS8_CASE(96)
+    WFS_X_ROWS8_CASE(128)
+    WFS_X_ROWS8_CASE(192)
+    WFS_X_ROWS8_CASE(256)
+    WFS_X_ROWS8_CASE(512)
+    default:
+      set_last_error("slab x pass: unsupported length %d", nx);
+      return WFS_ERR_UNSUPPORTED;
+  }
+#undef WFS_X_ROWS8_CASE
+}
+#endif
 
 template <typename R, int N>
 SlabRows slab_rows_n() {
@@ -482,7 +643,12 @@ bool slab_supported(int precision, const int n[3]) {
 // -> 93 / 90; 128^2 256 planes 49.6 / 43.3 -> 40.6 / 39.4, 512 planes 78 / 71 -> 70 / 68, 1536 planes 240 / 182
 // -> 191 / 172.  Not at 64^2: 14.0 / 12.7 -> 11.3 / 11.5 for one packet, but 12 packets of 96 x 64^2 47 / 42 ->
 // 45 / 44, and the tuned 64^2 forms are bit for bit the axis passes.
+//
+// complex64 512^2 planes (B = 8, x_rows8_kernel), us per step with a potential table against the four axis
+// passes: 512^3 2407 -> 1654, 256 x 512^2 1158 -> 798, 64 x 512^2 230 -> 182.  Its x launch takes 8 x points
+// of a lane at a time, so nx = 8 and 16 (4 points a lane) stay with the passes.
 bool split_supported(int precision, const int n[3]) {
+  if (precision == WFS_C64 && n[1] == 512 && n[2] == 512) return n[0] >= 32 && fft_length_supported(n[0]);
   return n[1] == n[2] && (n[1] == 96 || n[1] == 128 || (precision == WFS_C128 && (n[1] == 64 || n[1] == 192))) &&
          n[0] <= 256 && fft_length_supported(n[0]);
 }
@@ -495,18 +661,20 @@ int launch_x_slab_c128(int nx, int n, void* data, const XSlabParams& p, hipStrea
 SlabRows slab_rows(int precision, int n) {
   if (precision == WFS_C128) return slab_rows_c128(n);
   if (n == 96) return slab_rows_n<float, 96>();
+  if (n == 512) return slab_rows_n<float, 512>();
   return n == 128 ? slab_rows_n<float, 128>() : n == 192 ? slab_rows_n<float, 192>() : slab_rows_n<float, 256>();
 }
 
 LinesOrder slab_lines_order(int precision, int n) {
   if (precision == WFS_C128) return slab_lines_order_c128(n);
   if (n == 96) return slab_lines_order_n<float, 96>();
+  if (n == 512) return slab_lines_order_n<float, 512>();
   return n == 128 ? slab_lines_order_n<float, 128>()
                   : n == 192 ? slab_lines_order_n<float, 192>() : slab_lines_order_n<float, 256>();
 }
 
 int launch_yz_slab(int precision, int n, int mode, void* data, const YzPlaneParams& p, hipStream_t s) {
-  if (p.planes <= 0 || p.planes * 4 > 0x7fffffffL) {
+  if (p.planes <= 0 || p.planes * 8 > 0x7fffffffL) {
     set_last_error("slab y-z pass: bad plane count %ld", p.planes);
     return WFS_ERR_INVALID;
   }
@@ -515,6 +683,7 @@ int launch_yz_slab(int precision, int n, int mode, void* data, const YzPlanePara
   if (n == 192) return launch_lines_n<float, 192>(mode, data, p, s);
   if (n == 128) return launch_lines_n<float, 128>(mode, data, p, s);
   if (n == 96) return launch_lines_n<float, 96>(mode, data, p, s);
+  if (n == 512) return launch_lines_n<float, 512>(mode, data, p, s);
   set_last_error("slab y-z pass: unsupported plane %d", n);
   return WFS_ERR_UNSUPPORTED;
 }
@@ -530,6 +699,7 @@ int launch_x_slab(int precision, int nx, int n, int variant, void* data, const X
   if (n == 192) return launch_x_slab_ny<float, 192>(nx, variant, data, p, s);
   if (n == 128) return launch_x_slab_ny<float, 128>(nx, variant, data, p, s);
   if (n == 96) return launch_x_slab_ny<float, 96>(nx, variant, data, p, s);
+  if (n == 512) return launch_x_rows8(nx, data, p, s);
   set_last_error("slab x pass: unsupported plane %d", n);
   return WFS_ERR_UNSUPPORTED;
 }
