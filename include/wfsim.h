@@ -350,10 +350,8 @@ int wfs_plan_set_profiling(wfs_plan* plan, int enable);
  * (WFS_K_X_SLAB); variants 1 and 2 are the same launches;
  * variant 0 runs the four axis passes.  The results agree to float rounding
  * (the length-ny y transform is factored differently); the slab variants
- * among themselves are bit-identical.  WFS_K_X_SLAB: variant 1 (default at
- * 192) puts 16 z points in an x block, variant 2 (default at 256) 8, pairing
- * the two blocks of a 128-byte line on one XCD.  The autotuner keeps the
- * fastest.  WFS_K_PV_PLANES (no launches of its own): variant 1 (default)
+ * among themselves are bit-identical.  WFS_K_X_SLAB: variants 1 and 2 are the
+ * same launch.  The autotuner keeps the faster.  WFS_K_PV_PLANES (no launches of its own): variant 1 (default)
  * lets the slab scheme's y-z launch read one copy of each run of x planes
  * whose potential phase factors are bitwise equal (the planes away from walls
  * and absorbing x layers), so that those reads hit the caches instead of HBM;

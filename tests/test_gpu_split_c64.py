@@ -71,8 +71,12 @@ def test_split_matches_oracle_and_follows_the_potential(dev, nx, n):
     assert oracle.relative_l2(a.cpu().numpy(), ref) < 3e-6
 
 
+# (x launches of few blocks run as lane pairs, a batch's as rows: the same bits at every length of x)
 # 3 packets stay below 256 planes of 128^2 (slab class), 10 pass it and the 640 of the 16-z x launch
-@pytest.mark.parametrize("shape,batch", [((32, 512, 512), 2), ((16, 96, 96), 3), ((64, 96, 96), 10), ((64, 128, 128), 3), ((64, 128, 128), 10)])
+@pytest.mark.parametrize("shape,batch", [((32, 512, 512), 2), ((16, 96, 96), 3), ((8, 96, 96), 3),
+                                         ((32, 96, 96), 3), ((128, 96, 96), 3), ((192, 96, 96), 3), ((256, 96, 96), 3),
+                                         ((8, 128, 128), 2), ((96, 128, 128), 2), ((256, 128, 128), 2),
+                                         ((64, 96, 96), 10), ((64, 128, 128), 3), ((64, 128, 128), 10)])
 def test_default_packets_equal_single_runs(dev, shape, batch):
     rng = np.random.default_rng(batch)
     axes = [rng.uniform(-1, 1, (batch, m)) for m in shape]

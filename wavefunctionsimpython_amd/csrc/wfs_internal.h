@@ -146,8 +146,7 @@ SlabRows slab_rows(int precision, int n);
 LinesOrder slab_lines_order(int precision, int n);
 // YzPlaneParams.planes = packets * nx
 int launch_yz_slab(int precision, int n, int mode, void* data, const YzPlaneParams& p, hipStream_t s);
-// variant 2: 8 z points per block, else 16
-int launch_x_slab(int precision, int nx, int n, int variant, void* data, const XSlabParams& p, hipStream_t s);
+int launch_x_slab(int precision, int nx, int n, void* data, const XSlabParams& p, hipStream_t s);
 
 // pv = cexp_i(-dt V) elementwise in the state precision
 int launch_potential_phase(int precision, long count, const float2* V, double dt, void* pv, hipStream_t s);

@@ -542,7 +542,7 @@ int run_x_slab(wfs_plan* p, void* data, const void* const* ktab, hipStream_t s, 
   xp.kz = table_copy(p, ktab[2], 2, sel);
   xp.packets = p->batch;
   ProfileScope scope(p, WFS_K_X_SLAB, s);
-  return launch_x_slab(p->precision, p->n[0], p->n[1], p->variant[WFS_K_X_SLAB], data, xp, s);
+  return launch_x_slab(p->precision, p->n[0], p->n[1], data, xp, s);
 }
 
 // Slab scheme, observing launches: LINES_OBSERVE runs the exit launch of one stretch (table copy
@@ -768,21 +768,14 @@ extern "C" int wfs_plan_create_batched(const int n[3], const double dx[3], doubl
   p->variant[WFS_K_YZ_PLANE] =
       (yz_plane_supported(precision, n[1], n[2], 2) && n[1] == 128 && long(batch) * n[0] >= 512) ? 2
       : yz_plane_supported(precision, n[1], n[2], 1) ? 1 : 0;
-  // slab scheme at ny = nz = 256, 192 or 128 (complex64; both nonzero variants are the same y-z
-  // launch).  At 256 8-z x blocks (256^3 66 us against 79 with 16 z points), at 192 16-z x blocks
-  // (192^3 x 15: 460 us; 8-z x blocks 514 us); at 128 only while the x planes are too
-  // few to fill the CUs with plane-pass blocks, fewer than 256 (128^3: 29 against 34 us per
-  // step; from 8 packets on the plane pass is as fast)
+  // slab scheme at ny = nz = 256, 192 or 128 (complex64; both nonzero variants of either launch are the
+  // same one); at 128 below 256 x planes, from there on under WFS_K_YZ_SPLIT
   const bool slab = slab_supported(precision, n) && (n[1] != 128 || long(batch) * n[0] < 256);
   p->variant[WFS_K_YZ_SLAB] = slab ? (n[1] == 192 ? 1 : 2) : 0;
   if (slab) p->variant[WFS_K_X_SLAB] = n[1] == 192 ? 1 : 2;
   const bool two_launch = slab_supported(precision, n) || split_supported(precision, n);
-  // the same two launches elsewhere (figures at split_supported); complex64 128^2 planes have them under
-  // the slab class below 256 planes, with the same bits, and under this one from there on.  Their x
-  // launch: 8-z blocks while 16-z ones are few (96^2 288 planes 13.7 against 14.4 us, 512 14.5 and 15.2),
-  // whole lines from 640 planes on (768 28.7 and 26.7, 1152 38.0 and 36.2; 128^2 1536 77.7 and 68.6)
+  // the same two launches elsewhere, figures at split_supported
   p->variant[WFS_K_YZ_SPLIT] = !slab && split_supported(precision, n) && (n[1] != 64 || n[0] < 192) ? 1 : 0;
-  if (p->variant[WFS_K_YZ_SPLIT]) p->variant[WFS_K_X_SLAB] = long(batch) * n[0] < 640 ? 2 : 1;
   p->pending = new std::vector<std::pair<hipEvent_t, hipEvent_t>>[WFS_K_COUNT];
   p->event_pool = new std::vector<hipEvent_t>();
   int rc = 0;
@@ -1121,26 +1114,8 @@ extern "C" int wfs_plan_autotune(wfs_plan* p, void* stream) {
     }
     p->variant[WFS_K_YZ_PLANE] = rc == 0 ? best_v : keep;
   }
-  // slab scheme (two launches per step) against the tuned four axis passes: first the x
-  // launch's block width, then one step of the two launches and of the passes
+  // slab scheme (two launches per step) against the tuned four axis passes
   if (rc == 0 && slab_supported(p->precision, p->n)) {
-    {
-      const int keep = p->variant[WFS_K_X_SLAB];
-      float best = 1e30f;
-      int best_v = keep;
-      for (int v = 1; v < 3 && rc == 0; ++v) {
-        p->variant[WFS_K_X_SLAB] = v;
-        rc = run_x_slab(p, buf, p->kfull, s, 1);
-        (void)hipEventRecord(a, s);
-        for (int r = 0; r < 3 && rc == 0; ++r) rc = run_x_slab(p, buf, p->kfull, s, 1);
-        (void)hipEventRecord(b, s);
-        (void)hipEventSynchronize(b);
-        float ms = 0.0f;
-        (void)hipEventElapsedTime(&ms, a, b);
-        if (rc == 0 && ms < best) { best = ms; best_v = v; }
-      }
-      p->variant[WFS_K_X_SLAB] = rc == 0 ? best_v : keep;
-    }
     const int keep = p->variant[WFS_K_YZ_SLAB];
     float best = 1e30f;
     int best_v = keep;

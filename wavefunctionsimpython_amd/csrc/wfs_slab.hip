@@ -11,7 +11,7 @@
 //   yz_lines_kernel<NZ, LY, B>  (one block per x plane and residue b: the LY rows
 //     y = B a + b with all z, 128 KiB at 256, 72 KiB at 192, 66 KiB at 128):  length-LY
 //     inverse y stage over a, z inverse, potential phase, z forward, length-LY forward y stage
-//   x_slab_kernel  (one block per packet, ka and 8 or 16 consecutive z: the B rows
+//   x_rows_kernel or x_slab_kernel  (one block per packet, ka and 8 to 32 consecutive z: the B rows
 //     y = B ka + b with all x):  twiddles W_NY^{b ka} and length-B forward y stage over b,
 //     x forward, kinetic phase K(kx, ky, kz), x inverse, length-B inverse y stage and twiddles
 //
@@ -57,37 +57,17 @@ template <typename R, int N> struct SlabShape {
 // holds s times its second column through the x transforms (all linear) and uses s W_NY^{b ka}
 // as that row's twiddle.  Negation commutes exactly with every rounded operation, so the
 // results are bit for bit those of the selecting form, with one select per value left.
-template <typename R>
-__device__ __forceinline__ cx<R> shfl_xor_c(cx<R> v, int m) {
-  return mk<R>(__shfl_xor(v.x, m, 64), __shfl_xor(v.y, m, 64));
-}
-
-// the partner's value, partner = tid ^ ZB: for ZB = 8 the partner sits in the same row of 16
-// lanes, 8 along, so a DPP row rotation by 8 (row_ror:8, one VALU move per part) replaces the
-// LDS-unit permute; for ZB = 16 it sits in the neighbouring row, and gfx950's row swap
-// (v_permlane16_swap: odd rows of the first operand with even rows of the second, both the
-// value itself) leaves it in one of the two results, picked by the lane's row; other widths use
-// the permute
+// the partner's value, partner = tid ^ ZB, by DPP moves and row swaps (xor_lane)
 template <int ZB, typename R>
 __device__ __forceinline__ cx<R> partner_c(cx<R> v) {
-  if constexpr (ZB == 8 && sizeof(R) == 4) {
-    constexpr int kRowRor8 = 0x128;
-    const int x = __builtin_amdgcn_update_dpp(0, __float_as_int(v.x), kRowRor8, 0xF, 0xF, false);
-    const int y = __builtin_amdgcn_update_dpp(0, __float_as_int(v.y), kRowRor8, 0xF, 0xF, false);
-    return mk<R>(__int_as_float(x), __int_as_float(y));
-  } else if constexpr (ZB == 16 && sizeof(R) == 4) {
-    const bool odd_row = threadIdx.x & 16;
-    const auto sx = __builtin_amdgcn_permlane16_swap(__float_as_uint(v.x), __float_as_uint(v.x), false, false);
-    const auto sy = __builtin_amdgcn_permlane16_swap(__float_as_uint(v.y), __float_as_uint(v.y), false, false);
-    return mk<R>(__uint_as_float(odd_row ? sx[0] : sx[1]), __uint_as_float(odd_row ? sy[0] : sy[1]));
-  } else if constexpr (sizeof(R) == 8) {
-    return mk<R>(xor_lane<ZB>(v.x), xor_lane<ZB>(v.y));
+  if constexpr (sizeof(R) == 4) {
+    return mk<R>(__int_as_float(xor_lane_b32<ZB>(__float_as_int(v.x))), __int_as_float(xor_lane_b32<ZB>(__float_as_int(v.y))));
   } else {
-    return shfl_xor_c<R>(v, ZB);
+    return mk<R>(xor_lane<ZB>(v.x), xor_lane<ZB>(v.y));
   }
 }
 
-// ZB = 8 runs four waves per SIMD where a lane holds at most 16 points of an x line (at most 128
+// complex64 grids of few blocks and complex128.  ZB = 8 runs four waves per SIMD where a lane holds at most 16 points of an x line (at most 128
 // VGPRs: the x transforms' table twiddles are read from LDS one at a time where they are applied,
 // so no twiddle array is held; at nx = 256 one spilled register, 52.4 against 55.8 us per launch
 // with three waves, bit-identical); the 24 points of nx = 96 or 192 do not fit in 128.
@@ -253,61 +233,71 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && ZB == 8 && NX / split_of<NX
 }
 
 #if WFS_SLAB_PREC == 0
-// Moves the 8 x 8 matrix (lane bits 3..5, register r) of a wavefront to its transpose: register r of the
-// lanes with bits q holds afterwards what register q of the lanes with bits r held.  One pass per bit
-// pair; the halves of two registers are exchanged by gfx950's row and half-wavefront swaps, and 8 lanes
-// along by a DPP rotation that writes the masked banks only.
-__device__ __forceinline__ void transpose8_words(float (&v)[8]) {
+// Moves the B x B matrix (upper log2 B lane bits, register r) of a wavefront to its transpose: register r
+// of the lanes with upper bits q holds afterwards what register q of the lanes with upper bits r held.  One
+// pass per bit pair; the halves of two registers are exchanged by gfx950's half-wavefront and row swaps, and
+// 8 lanes along by a DPP rotation that writes the masked banks only.
+template <int B>
+__device__ __forceinline__ void transpose_words(float (&v)[B]) {
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[r]), __float_as_uint(v[r + 4]), false, false);
+  for (int r = 0; r < B / 2; ++r) {
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[r]), __float_as_uint(v[r + B / 2]), false, false);
     v[r] = __uint_as_float(s[0]);
-    v[r + 4] = __uint_as_float(s[1]);
+    v[r + B / 2] = __uint_as_float(s[1]);
   }
+  if constexpr (B >= 4) {
 #pragma unroll
-  for (int h = 0; h < 8; h += 4)
+    for (int h = 0; h < B; h += B / 2)
 #pragma unroll
-    for (int r = h; r < h + 2; ++r) {
-      const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[r]), __float_as_uint(v[r + 2]), false, false);
-      v[r] = __uint_as_float(s[0]);
-      v[r + 2] = __uint_as_float(s[1]);
+      for (int r = h; r < h + B / 4; ++r) {
+        const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[r]), __float_as_uint(v[r + B / 4]), false, false);
+        v[r] = __uint_as_float(s[0]);
+        v[r + B / 4] = __uint_as_float(s[1]);
+      }
+  }
+  if constexpr (B == 8) {
+    constexpr int kRowRor8 = 0x128;
+#pragma unroll
+    for (int r = 0; r < 8; r += 2) {
+      const int lo = __float_as_int(v[r]), hi = __float_as_int(v[r + 1]);
+      v[r] = __int_as_float(__builtin_amdgcn_update_dpp(lo, hi, kRowRor8, 0xF, 0xC, false));
+      v[r + 1] = __int_as_float(__builtin_amdgcn_update_dpp(hi, lo, kRowRor8, 0xF, 0x3, false));
     }
-  constexpr int kRowRor8 = 0x128;
-#pragma unroll
-  for (int r = 0; r < 8; r += 2) {
-    const int lo = __float_as_int(v[r]), hi = __float_as_int(v[r + 1]);
-    v[r] = __int_as_float(__builtin_amdgcn_update_dpp(lo, hi, kRowRor8, 0xF, 0xC, false));
-    v[r + 1] = __int_as_float(__builtin_amdgcn_update_dpp(hi, lo, kRowRor8, 0xF, 0x3, false));
   }
 }
 
-__device__ __forceinline__ void transpose8(cx<float>* a) {
-  float x[8], y[8];
+template <int B>
+__device__ __forceinline__ void transpose_rows(cx<float>* a) {
+  float x[B], y[B];
 #pragma unroll
-  for (int r = 0; r < 8; ++r) { x[r] = a[r].x; y[r] = a[r].y; }
-  transpose8_words(x);
-  transpose8_words(y);
+  for (int r = 0; r < B; ++r) { x[r] = a[r].x; y[r] = a[r].y; }
+  transpose_words<B>(x);
+  transpose_words<B>(y);
 #pragma unroll
-  for (int r = 0; r < 8; ++r) a[r] = mk<float>(x[r], y[r]);
+  for (int r = 0; r < B; ++r) a[r] = mk<float>(x[r], y[r]);
 }
 
-// x launch of planes whose y transform is split off a length-8 stage (512^2: rows y = 8 a + b).  A block
-// owns the 8 rows of one ka over 8 z points and all x; lane 8 q + z of every wavefront holds row b = q at
-// x = t + N2 i, t the wavefront's index, so that the x transforms' twiddles and kinetic factors are the
-// same in all lanes and come through the scalar cache.  For the y stage 8 rows are brought into one lane
-// (transpose8, 8 x points at a time), transformed there and sent back; the x transforms exchange one part
-// at a time through 4 NX 64 bytes of LDS, 128 KiB at nx = 512 (one block of 1024 threads, 128 registers).
-// Memory is touched in 64-byte segments; all z tiles of a ka go to one XCD (blocks go round-robin over the 8
-// of them), so that the halves of a line and the rows of a page stay with one L2: 512^3 597 us against 646
-// with the tiles of a ka spread over the XCDs in pairs (the axis pass alone takes 688, 256 x 512^2 317 -> 233,
-// 64 x 512^2 46 -> 50), bound by the 400 us of its arithmetic beside one block's waits.  Lanes along x instead
-// of the rows at the loads save a transposition and lose more to eight pages a load: 692 us.
-template <int NX, int N>
-__global__ __launch_bounds__(64 * split_of<NX>::n2) void x_rows8_kernel(cx<float>* __restrict__ data,
+// The complex64 x launch.  A block owns the B rows of one ka over 64 / B z points (64, 128 or 256 bytes of a
+// row) and all x; lane q 64 / B + z of every wavefront holds row b = q at x = t + N2 i, t the wavefront's
+// index, so that the x transforms' twiddles and the kinetic factors are the same in all lanes and come
+// through the scalar cache.  For the y stage the B rows are brought into one lane (transpose_rows, B x
+// points at a time), transformed there and sent back; the x transforms exchange one part at a time through
+// 256 NX bytes of LDS.  At nx = 256 that leaves 44 registers and 64 KiB, two blocks of 1024 threads a CU, at
+// nx = 512 (128 registers, 128 KiB) one.  Whole lines (B < 8) go down the rows, ka fastest (256^3 49.8 us against
+// 51.6 with z fastest); the half lines of B = 8 go with all z tiles of a ka to one XCD (blocks go round-robin
+// over the 8 of them), whose L2 then joins them.
+//   us per launch, lane pairs (x_slab_kernel, the better of 8 and 16 z points) against this form: 2 x 256^3
+//   134 -> 105 (536 MB: 5.1 TB/s), 192 x 256^2 53 -> 38, 192^3 37 -> 28, 3 of them 85 -> 69, 12 x 96^3 37 -> 28,
+//   8 x 128^3 45 -> 42, 256^3 alike at 50 (5.4 TB/s); the bits are the same.
+//   512^2 planes (B = 8): 512^3 597 us, 646 with the tiles of a ka in pairs over the XCDs (the axis pass alone
+//   688), 256 x 512^2 317 -> 233, 64 x 512^2 46 -> 50; 400 us of arithmetic beside one block's waits.  Lanes along
+//   x instead of the rows at the loads save a transposition and lose more to eight pages a load: 692 us.
+template <int NX, int N, int B>
+__global__ __launch_bounds__(64 * split_of<NX>::n2) void x_rows_kernel(cx<float>* __restrict__ data,
                                                                         const XSlabParams p) {
-  constexpr int B = 8, ZB = 8, A = N / B, TZ = N / ZB;
+  constexpr int ZB = 64 / B, A = N / B, TZ = N / ZB;
   constexpr int N2 = split_of<NX>::n2, N1 = NX / N2;
-  static_assert(N1 % 8 == 0 && (long(A) * TZ) % 16 == 0, "bad split of the x line");
+  static_assert(N1 % B == 0 && A % 8 == 0 && N % ZB == 0, "bad split of the x line");
   using C = cx<float>;
   using CC = const __attribute__((address_space(4))) C;
   __shared__ float lds[64 * NX];
@@ -315,25 +305,25 @@ __global__ __launch_bounds__(64 * split_of<NX>::n2) void x_rows8_kernel(cx<float
   const int lane = threadIdx.x & 63;
   const int t = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long bid = blockIdx.x;
-  const int zt = int((bid / 8) % TZ);
-  const int ka = int((bid / (8 * TZ)) % (A / 8)) * 8 + int(bid % 8);
+  const int zt = B == 8 ? int((bid / 8) % TZ) : int((bid / A) % TZ);
+  const int ka = B == 8 ? int((bid / (8 * TZ)) % (A / 8)) * 8 + int(bid % 8) : int(bid % A);
   const long pk = bid / (long(TZ) * A);
   C* __restrict__ blk = data + pk * (long(NX) * N * N) + long(B * ka) * N + long(zt) * ZB;
   constexpr unsigned XS = unsigned(N) * N, EB = unsigned(sizeof(C));
   static_assert(long(NX) * N * N * sizeof(C) <= (1L << 32), "32-bit byte offsets");
 
   auto off = [&](int l, int i) {
-    return (unsigned(l & 7) + unsigned(l >> 3) * N + (unsigned(t) + unsigned(N2) * unsigned(i)) * XS) * EB;
+    return (unsigned(l % ZB) + unsigned(l / ZB) * N + (unsigned(t) + unsigned(N2) * unsigned(i)) * XS) * EB;
   };
   C a[N1];
 #pragma unroll
   for (int i = 0; i < N1; ++i) a[i] = byte_at(blk, off(lane, i));
 
   CC* twy = (CC*)(p.tw_y);
-  // forward y stage X[kb] = sum_b W_8^{b kb} W_N^{b ka} Y[b] on 8 x points at a time
+  // forward y stage X[kb] = sum_b W_B^{b kb} W_N^{b ka} Y[b] on B x points at a time
 #pragma unroll
-  for (int g = 0; g < N1; g += 8) {
-    transpose8(a + g);
+  for (int g = 0; g < N1; g += B) {
+    transpose_rows<B>(a + g);
     C r[B];
     r[0] = a[g];
 #pragma unroll
@@ -341,7 +331,7 @@ __global__ __launch_bounds__(64 * split_of<NX>::n2) void x_rows8_kernel(cx<float
     DFT<B, -1>::run(r);
 #pragma unroll
     for (int b = 0; b < B; ++b) a[g + b] = r[b];
-    transpose8(a + g);
+    transpose_rows<B>(a + g);
   }
   CC* twx = (CC*)(p.tw_x);
   auto lidx = [&](int k1, int n2) { return (k1 * N2 + n2) * 64 + lane; };
@@ -358,8 +348,8 @@ __global__ __launch_bounds__(64 * split_of<NX>::n2) void x_rows8_kernel(cx<float
 
   transform_x(std::integral_constant<int, -1>{});
   {
-    const C ky = reinterpret_cast<const C*>(p.ky)[ka + A * (lane >> 3)];
-    const C kyz = cmul(ky, reinterpret_cast<const C*>(p.kz)[zt * ZB + (lane & 7)]);
+    const C ky = reinterpret_cast<const C*>(p.ky)[ka + A * (lane / ZB)];
+    const C kyz = cmul(ky, reinterpret_cast<const C*>(p.kz)[zt * ZB + (lane % ZB)]);
     CC* kx = (CC*)(p.kx) + t;
 #pragma unroll
     for (int i = 0; i < N1; ++i) a[i] = cmul(a[i], cmul(mk<float>(kx[N2 * i].x, kx[N2 * i].y), kyz));
@@ -367,11 +357,11 @@ __global__ __launch_bounds__(64 * split_of<NX>::n2) void x_rows8_kernel(cx<float
   __syncthreads();
   transform_x(std::integral_constant<int, +1>{});
 
-  // inverse y stage Y'[b] = W_N^{-b ka} sum_kb W_8^{-b kb} X[kb], stored 8 x points at a time
+  // inverse y stage Y'[b] = W_N^{-b ka} sum_kb W_B^{-b kb} X[kb], stored B x points at a time
   const int l = opaque_v(lane);
 #pragma unroll
-  for (int g = 0; g < N1; g += 8) {
-    transpose8(a + g);
+  for (int g = 0; g < N1; g += B) {
+    transpose_rows<B>(a + g);
     C r[B];
 #pragma unroll
     for (int b = 0; b < B; ++b) r[b] = a[g + b];
@@ -379,9 +369,9 @@ __global__ __launch_bounds__(64 * split_of<NX>::n2) void x_rows8_kernel(cx<float
     a[g] = r[0];
 #pragma unroll
     for (int b = 1; b < B; ++b) a[g + b] = cmulc(r[b], mk<float>(twy[(b * ka) % N].x, twy[(b * ka) % N].y));
-    transpose8(a + g);
+    transpose_rows<B>(a + g);
 #pragma unroll
-    for (int i = g; i < g + 8; ++i) byte_at(blk, off(l, i)) = a[i];
+    for (int i = g; i < g + B; ++i) byte_at(blk, off(l, i)) = a[i];
   }
 }
 #endif
@@ -532,13 +522,12 @@ int launch_x_slab_z(void* data, const XSlabParams& p, hipStream_t s) {
   return int(hipGetLastError());
 }
 
-// complex64: variant 2: 8 z points per block (256 threads at nx = 256), else 16; complex128: ZB128
+// z points per block: complex64 8 (256 threads at nx = 256), complex128 kZB128
 template <typename R, int N>
-int launch_x_slab_ny(int nx, int variant, void* data, const XSlabParams& p, hipStream_t s) {
+int launch_x_slab_ny(int nx, void* data, const XSlabParams& p, hipStream_t s) {
 #define WFS_X_SLAB_CASE(NX)                                                                                    \
   case NX:                                                                                                     \
-    if constexpr (sizeof(R) == 8) return launch_x_slab_z<R, NX, N, kZB128<N>>(data, p, s);                         \
-    else return variant == 2 ? launch_x_slab_z<R, NX, N, 8>(data, p, s) : launch_x_slab_z<R, NX, N, 16>(data, p, s);
+    return launch_x_slab_z<R, NX, N, sizeof(R) == 8 ? kZB128<N> : 8>(data, p, s);
   switch (nx) {
     WFS_X_SLAB_CASE(8)
     WFS_X_SLAB_CASE(16)
@@ -556,26 +545,39 @@ int launch_x_slab_ny(int nx, int variant, void* data, const XSlabParams& p, hipS
 }
 
 #if WFS_SLAB_PREC == 0
-int launch_x_rows8(int nx, void* data, const XSlabParams& p, hipStream_t s) {
-  constexpr int N = 512;
-#define WFS_X_ROWS8_CASE(NX)                                                                                 \
+// x_rows_kernel's N^2 / 64 blocks a packet fill the card from 1.5 of them a CU on; below that the smaller blocks
+// of x_slab_kernel are the faster ones or level.  us per launch, lane pairs against rows: 256 x 128^2 (256
+// blocks a packet) 17.0 / 16.7, 2 packets 27.9 / 26.2; 128^3 11.4 / 11.8, 2 packets 14.6 / 14.1, 4 packets 25.5 /
+// 21.1; 256 x 96^2 (144 blocks a packet) 14.6 / 16.3, 2 packets 18.1 / 20.9, 3 packets 24.2 / 22.2; 128 x 96^2
+// 9.7 / 10.4, 14.0 / 15.3.  192^2 and 256^2 planes have 576 and 1024 blocks a packet.
+bool x_rows_fill(int n, long packets) { return packets * (long(n) * n / 64) * 2 >= 3L * cu_count(); }
+
+template <int N>
+int launch_x_rows(int nx, void* data, const XSlabParams& p, hipStream_t s) {
+  constexpr int B = SlabShape<float, N>::B;
+#define WFS_X_ROWS_CASE(NX)                                                                                  \
   case NX:                                                                                                   \
-    WFS_LAUNCH((x_rows8_kernel<NX, N>), dim3(unsigned(p.packets * (N / 8) * (N / 8))),                          \
-               dim3(64 * split_of<NX>::n2), 0, s, reinterpret_cast<cx<float>*>(data), p);                         \
-    return int(hipGetLastError());
+    if constexpr ((NX / split_of<NX>::n2) % B == 0 && (NX <= 256 || N == 512)) {                              \
+      WFS_LAUNCH((x_rows_kernel<NX, N, B>), dim3(unsigned(p.packets * (N / 8) * (N / 8))),                    \
+                 dim3(64 * split_of<NX>::n2), 0, s, reinterpret_cast<cx<float>*>(data), p);                  \
+      return int(hipGetLastError());                                                                         \
+    }                                                                                                        \
+    break;
   switch (nx) {
-    WFS_X_ROWS8_CASE(32)
-    WFS_X_ROWS8_CASE(64)
-    WFS_X_ROWS8_CASE(96)
-    WFS_X_ROWS8_CASE(128)
-    WFS_X_ROWS8_CASE(192)
-    WFS_X_ROWS8_CASE(256)
-    WFS_X_ROWS8_CASE(512)
-    default:
-      set_last_error("slab x pass: unsupported length %d", nx);
-      return WFS_ERR_UNSUPPORTED;
+    WFS_X_ROWS_CASE(8)
+    WFS_X_ROWS_CASE(16)
+    WFS_X_ROWS_CASE(32)
+    WFS_X_ROWS_CASE(64)
+    WFS_X_ROWS_CASE(96)
+    WFS_X_ROWS_CASE(128)
+    WFS_X_ROWS_CASE(192)
+    WFS_X_ROWS_CASE(256)
+    WFS_X_ROWS_CASE(512)
+    default: break;
   }
-#undef WFS_X_ROWS8_CASE
+#undef WFS_X_ROWS_CASE
+  set_last_error("slab x pass: unsupported length %d", nx);
+  return WFS_ERR_UNSUPPORTED;
 }
 #endif
 
@@ -644,7 +646,7 @@ bool slab_supported(int precision, const int n[3]) {
 // -> 191 / 172.  Not at 64^2: 14.0 / 12.7 -> 11.3 / 11.5 for one packet, but 12 packets of 96 x 64^2 47 / 42 ->
 // 45 / 44, and the tuned 64^2 forms are bit for bit the axis passes.
 //
-// complex64 512^2 planes (B = 8, x_rows8_kernel), us per step with a potential table against the four axis
+// complex64 512^2 planes (B = 8, x_rows_kernel), us per step with a potential table against the four axis
 // passes: 512^3 2407 -> 1654, 256 x 512^2 1158 -> 798, 64 x 512^2 230 -> 182.  Its x launch takes 8 x points
 // of a lane at a time, so nx = 8 and 16 (4 points a lane) stay with the passes.
 bool split_supported(int precision, const int n[3]) {
@@ -688,18 +690,19 @@ int launch_yz_slab(int precision, int n, int mode, void* data, const YzPlanePara
   return WFS_ERR_UNSUPPORTED;
 }
 
-int launch_x_slab(int precision, int nx, int n, int variant, void* data, const XSlabParams& p, hipStream_t s) {
+int launch_x_slab(int precision, int nx, int n, void* data, const XSlabParams& p, hipStream_t s) {
   const long blocks = p.packets * long(n / 2) * (n / 4);
   if (p.packets <= 0 || blocks > 0x7fffffffL) {
     set_last_error("slab x pass: bad packet count %ld", p.packets);
     return WFS_ERR_INVALID;
   }
   if (precision == WFS_C128) return launch_x_slab_c128(nx, n, data, p, s);
-  if (n == 256) return launch_x_slab_ny<float, 256>(nx, variant, data, p, s);
-  if (n == 192) return launch_x_slab_ny<float, 192>(nx, variant, data, p, s);
-  if (n == 128) return launch_x_slab_ny<float, 128>(nx, variant, data, p, s);
-  if (n == 96) return launch_x_slab_ny<float, 96>(nx, variant, data, p, s);
-  if (n == 512) return launch_x_rows8(nx, data, p, s);
+  if (n == 512) return launch_x_rows<512>(nx, data, p, s);
+  if (n == 256) return launch_x_rows<256>(nx, data, p, s);
+  if (n == 192) return launch_x_rows<192>(nx, data, p, s);
+  const bool rows = x_rows_fill(n, p.packets);
+  if (n == 128) return rows ? launch_x_rows<128>(nx, data, p, s) : launch_x_slab_ny<float, 128>(nx, data, p, s);
+  if (n == 96) return rows ? launch_x_rows<96>(nx, data, p, s) : launch_x_slab_ny<float, 96>(nx, data, p, s);
   set_last_error("slab x pass: unsupported plane %d", n);
   return WFS_ERR_UNSUPPORTED;
 }
@@ -724,10 +727,10 @@ int launch_yz_slab_c128(int n, int mode, void* data, const YzPlaneParams& p, hip
 }
 
 int launch_x_slab_c128(int nx, int n, void* data, const XSlabParams& p, hipStream_t s) {
-  if (n == 64) return launch_x_slab_ny<double, 64>(nx, 1, data, p, s);
-  if (n == 96) return launch_x_slab_ny<double, 96>(nx, 1, data, p, s);
-  if (n == 128) return launch_x_slab_ny<double, 128>(nx, 1, data, p, s);
-  if (n == 192) return launch_x_slab_ny<double, 192>(nx, 1, data, p, s);
+  if (n == 64) return launch_x_slab_ny<double, 64>(nx, data, p, s);
+  if (n == 96) return launch_x_slab_ny<double, 96>(nx, data, p, s);
+  if (n == 128) return launch_x_slab_ny<double, 128>(nx, data, p, s);
+  if (n == 192) return launch_x_slab_ny<double, 192>(nx, data, p, s);
   set_last_error("slab x pass: unsupported complex128 plane %d", n);
   return WFS_ERR_UNSUPPORTED;
 }
