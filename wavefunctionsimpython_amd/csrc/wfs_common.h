@@ -409,6 +409,50 @@ __device__ __forceinline__ void column_dft_second_parts(C (&a)[N / N2], R* lds, 
   }
 }
 
+// Moves the B x B matrix (upper log2 B lane bits, register r) of a wavefront to its transpose: register r
+// of the lanes with upper bits q holds afterwards what register q of the lanes with upper bits r held.  One
+// pass per bit pair; the halves of two registers are exchanged by gfx950's half-wavefront and row swaps, and
+// 8 lanes along by a DPP rotation that writes the masked banks only.
+template <int B>
+__device__ __forceinline__ void transpose_words(float (&v)[B]) {
+#pragma unroll
+  for (int r = 0; r < B / 2; ++r) {
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[r]), __float_as_uint(v[r + B / 2]), false, false);
+    v[r] = __uint_as_float(s[0]);
+    v[r + B / 2] = __uint_as_float(s[1]);
+  }
+  if constexpr (B >= 4) {
+#pragma unroll
+    for (int h = 0; h < B; h += B / 2)
+#pragma unroll
+      for (int r = h; r < h + B / 4; ++r) {
+        const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[r]), __float_as_uint(v[r + B / 4]), false, false);
+        v[r] = __uint_as_float(s[0]);
+        v[r + B / 4] = __uint_as_float(s[1]);
+      }
+  }
+  if constexpr (B == 8) {
+    constexpr int kRowRor8 = 0x128;
+#pragma unroll
+    for (int r = 0; r < 8; r += 2) {
+      const int lo = __float_as_int(v[r]), hi = __float_as_int(v[r + 1]);
+      v[r] = __int_as_float(__builtin_amdgcn_update_dpp(lo, hi, kRowRor8, 0xF, 0xC, false));
+      v[r + 1] = __int_as_float(__builtin_amdgcn_update_dpp(hi, lo, kRowRor8, 0xF, 0x3, false));
+    }
+  }
+}
+
+template <int B>
+__device__ __forceinline__ void transpose_rows(cx<float>* a) {
+  float x[B], y[B];
+#pragma unroll
+  for (int r = 0; r < B; ++r) { x[r] = a[r].x; y[r] = a[r].y; }
+  transpose_words<B>(x);
+  transpose_words<B>(y);
+#pragma unroll
+  for (int r = 0; r < B; ++r) a[r] = mk<float>(x[r], y[r]);
+}
+
 template <int N, int N2, int SIGN, typename C, typename LIDX>
 __device__ __forceinline__ void column_dft(C (&a)[N / N2], const C (&w)[N / N2], C* lds, int t, LIDX lidx) {
   column_dft_first<N, N2, SIGN>(a, w);

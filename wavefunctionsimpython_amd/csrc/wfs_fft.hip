@@ -153,7 +153,7 @@ __global__ __launch_bounds__(N2 * G) void fft_pass_kernel(cx<R>* __restrict__ da
 // loads and stores overlap the other's arithmetic.
 template <typename R, int N, int H>
 static int launch_yz_plane_n(void* data, const YzPlaneParams& p, hipStream_t s) {
-  static_assert(yz_lines_lds_bytes<R, N, N, H>() <= 160 * 1024, "plane does not fit in LDS");
+  static_assert(yz_lines_lds_bytes<R, N, N, 1, H>() <= 160 * 1024, "plane does not fit in LDS");
   if (p.planes <= 0 || p.planes > 0x7fffffffL) {
     set_last_error("yz plane pass: bad plane count %ld", p.planes);
     return WFS_ERR_INVALID;

@@ -233,50 +233,6 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && ZB == 8 && NX / split_of<NX
 }
 
 #if WFS_SLAB_PREC == 0
-// Moves the B x B matrix (upper log2 B lane bits, register r) of a wavefront to its transpose: register r
-// of the lanes with upper bits q holds afterwards what register q of the lanes with upper bits r held.  One
-// pass per bit pair; the halves of two registers are exchanged by gfx950's half-wavefront and row swaps, and
-// 8 lanes along by a DPP rotation that writes the masked banks only.
-template <int B>
-__device__ __forceinline__ void transpose_words(float (&v)[B]) {
-#pragma unroll
-  for (int r = 0; r < B / 2; ++r) {
-    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[r]), __float_as_uint(v[r + B / 2]), false, false);
-    v[r] = __uint_as_float(s[0]);
-    v[r + B / 2] = __uint_as_float(s[1]);
-  }
-  if constexpr (B >= 4) {
-#pragma unroll
-    for (int h = 0; h < B; h += B / 2)
-#pragma unroll
-      for (int r = h; r < h + B / 4; ++r) {
-        const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[r]), __float_as_uint(v[r + B / 4]), false, false);
-        v[r] = __uint_as_float(s[0]);
-        v[r + B / 4] = __uint_as_float(s[1]);
-      }
-  }
-  if constexpr (B == 8) {
-    constexpr int kRowRor8 = 0x128;
-#pragma unroll
-    for (int r = 0; r < 8; r += 2) {
-      const int lo = __float_as_int(v[r]), hi = __float_as_int(v[r + 1]);
-      v[r] = __int_as_float(__builtin_amdgcn_update_dpp(lo, hi, kRowRor8, 0xF, 0xC, false));
-      v[r + 1] = __int_as_float(__builtin_amdgcn_update_dpp(hi, lo, kRowRor8, 0xF, 0x3, false));
-    }
-  }
-}
-
-template <int B>
-__device__ __forceinline__ void transpose_rows(cx<float>* a) {
-  float x[B], y[B];
-#pragma unroll
-  for (int r = 0; r < B; ++r) { x[r] = a[r].x; y[r] = a[r].y; }
-  transpose_words<B>(x);
-  transpose_words<B>(y);
-#pragma unroll
-  for (int r = 0; r < B; ++r) a[r] = mk<float>(x[r], y[r]);
-}
-
 // The complex64 x launch.  A block owns the B rows of one ka over 64 / B z points (64, 128 or 256 bytes of a
 // row) and all x; lane q 64 / B + z of every wavefront holds row b = q at x = t + N2 i, t the wavefront's
 // index, so that the x transforms' twiddles and the kinetic factors are the same in all lanes and come
@@ -460,7 +416,7 @@ int cu_count() {
 template <typename R, int N, int MODE, int PARTS = 0>
 int launch_lines_m(void* data, const YzPlaneParams& p, hipStream_t s) {
   constexpr int LY = SlabShape<R, N>::LY, B = SlabShape<R, N>::B;
-  static_assert(yz_lines_lds_bytes<R, N, LY, 1>() / (PARTS ? 2 : 1) <= 160 * 1024, "rows do not fit in LDS");
+  static_assert(yz_lines_lds_bytes<R, N, LY, B, 1, PARTS>() <= 160 * 1024, "rows do not fit in LDS");
   const long groups = p.planes * B;
   WFS_LAUNCH((yz_lines_kernel<R, N, LY, B, 1, MODE, true, PARTS>), dim3(unsigned(groups)),
                      dim3(yz_lines_threads<N, LY, 1>()), 0, s, reinterpret_cast<cx<R>*>(data), p);
@@ -474,7 +430,7 @@ int launch_lines_m(void* data, const YzPlaneParams& p, hipStream_t s) {
 // the transforms no longer wait for the factor loads hoisted over them.  Not for complex128 (128^3 27.3 ->
 // 28.6, 192^3 80.3 -> 85.6, 96^3 17.2 -> 18.3 us: its 3 and more exchanges cost what the second block
 // gains) nor for complex64 128^2 planes (19.0 -> 19.3).  512^2: the only form that fits, 131 KB of LDS and 128
-// registers a block of 1024 threads; 512^3 830 us a full launch (3.3 GB: 4.0 TB/s), 510 an entry or exit.
+// registers a block of 1024 threads; 512^3 748 us a full launch (3.3 GB: 4.4 TB/s), 465 an entry or exit.
 template <typename R, int N> constexpr int lines_parts() { return sizeof(R) == 8 ? 0 : N == 512 ? 4 : N == 256 ? 8 : N == 192 ? 3 : 0; }
 
 // The parts form is taken where the groups are more than the CUs.  us of the full / entry or exit launch,
@@ -647,7 +603,7 @@ bool slab_supported(int precision, const int n[3]) {
 // 45 / 44, and the tuned 64^2 forms are bit for bit the axis passes.
 //
 // complex64 512^2 planes (B = 8, x_rows_kernel), us per step with a potential table against the four axis
-// passes: 512^3 2407 -> 1654, 256 x 512^2 1158 -> 798, 64 x 512^2 230 -> 182.  Its x launch takes 8 x points
+// passes: 512^3 2407 -> 1412, 256 x 512^2 1158 -> 798, 64 x 512^2 230 -> 182.  Its x launch takes 8 x points
 // of a lane at a time, so nx = 8 and 16 (4 points a lane) stay with the passes.
 bool split_supported(int precision, const int n[3]) {
   if (precision == WFS_C64 && n[1] == 512 && n[2] == 512) return n[0] >= 32 && fft_length_supported(n[0]);

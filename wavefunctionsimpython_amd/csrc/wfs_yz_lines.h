@@ -121,9 +121,28 @@ constexpr int yz_lines_threads() {
   return NZ * (LY / (NZ / split_of<NZ>::n2)) / H;
 }
 
-template <typename R, int NZ, int LY, int H>
+// The y lines' second stage inside a wavefront (SWAP_Y below): complex64 row groups whose y lines are split
+// over 2 threads (512^2, 192^2 and 96^2 planes).  It takes two of the six exchanges, and their barriers, off
+// the LDS: us of the full / entry or exit launch 512^3 825 / 510 -> 748 / 465, 3 x 192^3 126 / 72 -> 120 / 63,
+// 192^3 39.5 / 27 -> 37.5 / 25, 12 x 96^3 46 / 32 -> 44 / 30, 96^3 13.8 / 8.7 -> 13.0 / 8.3.  Over 4 threads a line
+// (256^2, 128^2) the lanes of a wavefront need four sets of y twiddles, read from LDS, and that is no gain:
+// 256^3 77.5 / 51 -> 80 / 51 with a table, 73.5 -> 71 without, 128^3 14.3 / 9.6 -> 16.3 / 10.8.
+template <typename R, int NZ, int LY, int B, int H>
+constexpr bool yz_lines_swap() {
+  constexpr int n2y = LY / (NZ / split_of<NZ>::n2);
+  return sizeof(R) == 4 && B > 1 && H == 1 && n2y == 2;
+}
+// Row stride of the transposition tile: odd, so that the rows a wavefront reads at one z lie in different
+// banks; 4-byte elements (PARTS) with SWAP_Y: 1 more than the 32 columns of a row that a wavefront writes at
+// once (modulo the 64 banks), so that the two rows it writes lie beside each other.
+template <typename R, int NZ, int LY, int B, int H, int PARTS>
+constexpr int yz_lines_stride() {
+  return PARTS && yz_lines_swap<R, NZ, LY, B, H>() ? NZ + (97 - NZ % 64) % 64 : NZ + 1;
+}
+
+template <typename R, int NZ, int LY, int B, int H, int PARTS = 0>
 constexpr long yz_lines_lds_bytes() {
-  return long(LY / H) * (NZ + 1) * long(sizeof(cx<R>));
+  return long(LY / H) * yz_lines_stride<R, NZ, LY, B, H, PARTS>() * long(PARTS ? sizeof(R) : sizeof(cx<R>));
 }
 
 // PV_LINES: the potential table is in lines order (LinesOrder, wfs_internal.h), read as one
@@ -147,10 +166,13 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lin
   constexpr int CH = NZ / H;                 // y lines (columns z) per round
   constexpr int RH = LY / H;                 // z lines (rows) per round
   constexpr int N1H = N1 / H;                // points of a y line per round of the transposition
-  constexpr int TS = NZ + 1;                 // padded row stride of the transposition
+  constexpr int TS = yz_lines_stride<R, NZ, LY, B, H, PARTS>();   // padded row stride of the transposition
+  // A wavefront holds 32 columns, the two threads u of their y lines in its halves, and the y lines' exchange
+  // is a transposition by half-wavefront swaps: no LDS, no barrier
+  constexpr bool SWAP_Y = yz_lines_swap<R, NZ, LY, B, H>();
   constexpr unsigned RS = unsigned(B) * NZ;  // element stride between the block's rows
   static_assert(N1 % H == 0 && N2Y >= H && N2Z >= H, "bad round split");
-  constexpr bool UNIFORM_Y = (CH % 64) == 0;
+  constexpr bool UNIFORM_Y = !SWAP_Y && (CH % 64) == 0;
   constexpr bool UNIFORM_Z = (RH % 64) == 0;
   using C = cx<R>;
   using CC = const __attribute__((address_space(4))) C;
@@ -166,9 +188,14 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lin
 
   C a[H][N1];
   C w[N1];
+  // column and index within the y line of thread t
+  auto col_c = [&](int t) { return SWAP_Y ? t % 32 + 32 * (t / 64) : t % CH; };
+  auto col_u = [&](int t) { return SWAP_Y ? (t / 32) % 2 : t / CH; };
+  // barrier that only the LDS form of the y exchange needs
+  auto sync_y = [&]() { if constexpr (!SWAP_Y) __syncthreads(); };
   auto thread_u_y = [&]() -> int {
     if constexpr (UNIFORM_Y) return __builtin_amdgcn_readfirstlane(tid / CH);
-    else return opaque_v(tid) / CH;
+    else return col_u(opaque_v(tid));
   };
   auto thread_u_z = [&]() -> int {
     if constexpr (UNIFORM_Z) return __builtin_amdgcn_readfirstlane(tid / RH);
@@ -219,12 +246,40 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lin
   // one transform of every y line, round by round (one round's temporaries live at a time)
   auto transform_y = [&](const void* twp, auto sign_c) {
     const int u = thread_u_y();
+    if constexpr (SWAP_Y) {
+      constexpr int SG = decltype(sign_c)::value;
+      constexpr int M = N1 / N2Y;
+      DFT<N1, SG>::run(a[0]);
+      if (u) {                                 // u = 0 has unit twiddles, u = 1 one set for all lanes
+        CC* tw = (CC*)(twp) + N1;
+#pragma unroll
+        for (int k1 = 1; k1 < N1; ++k1) {
+          const C v = mk<R>(tw[k1].x, tw[k1].y);
+          a[0][k1] = SG < 0 ? cmul(a[0][k1], v) : cmulc(a[0][k1], v);
+        }
+      }
+      C o[N1];
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        C b[N2Y];
+#pragma unroll
+        for (int r = 0; r < N2Y; ++r) b[r] = a[0][N2Y * m + r];
+        transpose_rows<N2Y>(b);
+        DFT<N2Y, SG>::run(b);
+#pragma unroll
+        for (int k2 = 0; k2 < N2Y; ++k2) o[m + M * k2] = b[k2];
+      }
+#pragma unroll
+      for (int i = 0; i < N1; ++i) a[0][i] = o[i];
+      return;
+    } else {
 #pragma unroll
     for (int h = 0; h < H; ++h) {
       if (h) __syncthreads();
       load_wy(twp, u);
       column_dft_first<LY, N2Y, decltype(sign_c)::value>(a[h], w);
       exchange_y(a[h], u, sign_c);
+    }
     }
   };
   // one transform of every z line (no potential), round by round
@@ -241,7 +296,7 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lin
   // transpositions between the y lines and the z lines, LY/H rows a round
   auto cols_to_rows = [&]() {
     const int t = opaque_v(tid);
-    const int c0 = t % CH, u = t / CH;
+    const int c0 = col_c(t), u = col_u(t);
     const int r0 = t % RH, v = t / RH;
     if constexpr (PARTS) {
 #pragma unroll
@@ -277,7 +332,7 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lin
   };
   auto rows_to_cols = [&]() {
     const int t = opaque_v(tid);
-    const int c0 = t % CH, u = t / CH;
+    const int c0 = col_c(t), u = col_u(t);
     const int r0 = t % RH, v = t / RH;
     if constexpr (PARTS) {
 #pragma unroll
@@ -313,7 +368,7 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lin
   };
 
   {
-    const int c0 = tid % CH, u = tid / CH;
+    const int c0 = col_c(tid), u = col_u(tid);
 #pragma unroll
     for (int h = 0; h < H; ++h)
 #pragma unroll
@@ -323,7 +378,7 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lin
   if constexpr (MODE == LINES_FULL) {
     // y inverse on columns
     transform_y(p.tw_yi, std::integral_constant<int, +1>{});
-    __syncthreads();
+    sync_y();
     cols_to_rows();
     __syncthreads();
 
@@ -401,7 +456,7 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lin
     }
     __syncthreads();
     rows_to_cols();
-    __syncthreads();
+    sync_y();
 
     // y forward on columns
     transform_y(p.tw_yf, std::integral_constant<int, -1>{});
@@ -411,7 +466,7 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lin
     transform_z(p.tw_z, std::integral_constant<int, -1>{});
     __syncthreads();
     rows_to_cols();
-    __syncthreads();
+    sync_y();
     transform_y(p.tw_yf, std::integral_constant<int, -1>{});
   } else if constexpr (MODE == LINES_ENTRY_OBSERVE) {
     // the entry launch with the box moments of the position-space rows it reads
@@ -423,11 +478,11 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lin
     transform_z(p.tw_z, std::integral_constant<int, -1>{});
     __syncthreads();
     rows_to_cols();
-    __syncthreads();
+    sync_y();
     transform_y(p.tw_yf, std::integral_constant<int, -1>{});
   } else if constexpr (MODE == LINES_EXIT) {
     transform_y(p.tw_yi, std::integral_constant<int, +1>{});
-    __syncthreads();
+    sync_y();
     cols_to_rows();
     __syncthreads();
     transform_z(p.tw_z, std::integral_constant<int, +1>{});
@@ -438,7 +493,7 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lin
     // store, and the entry launch that would read them back, in one pass (same arithmetic)
     static_assert(H == 1, "the observing launch holds one round");
     transform_y(p.tw_yi, std::integral_constant<int, +1>{});
-    __syncthreads();
+    sync_y();
     cols_to_rows();
     __syncthreads();
     transform_z(p.tw_z, std::integral_constant<int, +1>{});
@@ -448,13 +503,13 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lin
     transform_z(p.tw_zf, std::integral_constant<int, -1>{});
     __syncthreads();
     rows_to_cols();
-    __syncthreads();
+    sync_y();
     transform_y(p.tw_yf, std::integral_constant<int, -1>{});
   }
 
   {
     const int t = opaque_v(tid);
-    const int c0 = t % CH, u = t / CH;
+    const int c0 = col_c(t), u = col_u(t);
 #pragma unroll
     for (int h = 0; h < H; ++h)
 #pragma unroll
