@@ -338,7 +338,8 @@ int wfs_plan_set_profiling(wfs_plan* plan, int enable);
  * WFS_K_YZ_PLANE: variant 1 (default where supported: complex64 planes of
  * ny = nz <= 128, complex128 planes of ny = nz <= 64) runs the y inverse, z
  * inverse / potential / z forward and y forward passes of each step as one
- * kernel on whole x planes held in LDS; variant 0 runs the three passes.  The
+ * kernel on whole x planes held in LDS, and at up to 64 x 64 planes the first
+ * and last two passes of a call likewise (kernel class WFS_K_SLAB_EDGE); variant 0 runs the three passes.  The
  * results are identical; the autotuner keeps the faster.
  * WFS_K_YZ_SLAB: variants 1 and 2 (the default where supported: complex64
  * grids with ny = nz = 256 or 192 and nx <= 256, 2 at 256 and 1 at 192; at

@@ -151,14 +151,14 @@ __global__ __launch_bounds__(N2 * G) void fft_pass_kernel(cx<R>* __restrict__ da
 // (16 B per point for complex64) instead of three times (48 B per point).  For N = 128
 // complex64 and H = 2: 66 KiB of LDS and 512 threads, two blocks per CU, so one block's
 // loads and stores overlap the other's arithmetic.
-template <typename R, int N, int H>
+template <typename R, int N, int H, int MODE = LINES_FULL>
 static int launch_yz_plane_n(void* data, const YzPlaneParams& p, hipStream_t s) {
   static_assert(yz_lines_lds_bytes<R, N, N, 1, H>() <= 160 * 1024, "plane does not fit in LDS");
   if (p.planes <= 0 || p.planes > 0x7fffffffL) {
     set_last_error("yz plane pass: bad plane count %ld", p.planes);
     return WFS_ERR_INVALID;
   }
-  WFS_LAUNCH((yz_lines_kernel<R, N, N, 1, H, LINES_FULL>), dim3(unsigned(p.planes)),
+  WFS_LAUNCH((yz_lines_kernel<R, N, N, 1, H, MODE>), dim3(unsigned(p.planes)),
                      dim3(yz_lines_threads<N, N, H>()), 0, s, reinterpret_cast<cx<R>*>(data), p);
   return int(hipGetLastError());
 }
@@ -244,6 +244,40 @@ int launch_fft_pass_t(int n, int layout, int mode, void* data, const PassParams&
 }
 
 // This file is compiled twice: WFS_FFT_PREC=0 (complex64) and 1 (complex128).
+// The entry (z, y forward) or exit (y, z inverse) transforms of whole planes in one launch, bit for bit the two
+// passes: a short call is bound by its launches (one step 7 -> 5 of them) and a long batch by the passes over
+// memory.  us of a one-step call, passes against this: 32^3 24.5 -> 19.5, 64^3 30.5 -> 27.5, 256 x 64^2 52.5 ->
+// 44.7, 48 x 64^3 240 -> 186, 8 x 64 x 16^2 24 -> 19.7; complex128 32^3 25.8 -> 20.6, 256 x 64^2 74 -> 55.  Planes above
+// 64^2 step in two launches, or beside 512 x planes keep the passes.
+template <typename R>
+static int launch_yz_edge_t(int n, bool entry, void* data, const YzPlaneParams& p, hipStream_t s) {
+#define WFS_YZ_EDGE(N)                                                                                       \
+  case N: return entry ? launch_yz_plane_n<R, N, 1, LINES_ENTRY>(data, p, s)                                   \
+                       : launch_yz_plane_n<R, N, 1, LINES_EXIT>(data, p, s);
+  switch (n) {
+    WFS_YZ_EDGE(16)
+    WFS_YZ_EDGE(32)
+    WFS_YZ_EDGE(64)
+    default:
+      set_last_error("yz plane edge: unsupported plane %d", n);
+      return WFS_ERR_UNSUPPORTED;
+  }
+#undef WFS_YZ_EDGE
+}
+
+#if WFS_FFT_PREC == 0
+bool yz_edge_supported(int precision, int ny, int nz) { return ny <= 64 && yz_plane_supported(precision, ny, nz, 1); }
+
+int launch_yz_edge_c128(int n, bool entry, void* data, const YzPlaneParams& p, hipStream_t s);
+int launch_yz_edge(int precision, int n, bool entry, void* data, const YzPlaneParams& p, hipStream_t s) {
+  return precision == WFS_C128 ? launch_yz_edge_c128(n, entry, data, p, s) : launch_yz_edge_t<float>(n, entry, data, p, s);
+}
+#else
+int launch_yz_edge_c128(int n, bool entry, void* data, const YzPlaneParams& p, hipStream_t s) {
+  return launch_yz_edge_t<double>(n, entry, data, p, s);
+}
+#endif
+
 #if WFS_FFT_PREC == 0
 template int launch_fft_pass_t<float>(int, int, int, void*, const PassParams&, long, int, hipStream_t);
 

@@ -107,6 +107,9 @@ struct YzPlaneParams {
 // halves: lines per thread (1 or 2), the plane passing through LDS in that many rounds
 bool yz_plane_supported(int precision, int ny, int nz, int halves);
 int launch_yz_plane(int precision, int n, int halves, void* data, const YzPlaneParams& p, hipStream_t s);
+// a call's first two transforms (z, y forward) or last two (y, z inverse) on whole planes of up to 64^2
+bool yz_edge_supported(int precision, int ny, int nz);
+int launch_yz_edge(int precision, int n, bool entry, void* data, const YzPlaneParams& p, hipStream_t s);
 
 // Two-launch split step for complex64 grids with ny = nz = 256 or 192 (wfs_slab.hip): the y
 // transform split in a length-ny/4 stage (on rows y = 4 a + b, with the z work) and a

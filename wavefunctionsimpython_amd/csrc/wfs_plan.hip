@@ -497,6 +497,27 @@ int run_yz_plane(wfs_plan* p, void* data, const void* pv, hipStream_t s, int sel
 }
 
 // the passes between two x passes: fused plane kernel or three axis passes
+// entry (z, y forward) or exit (y, z inverse) transforms of a call, table copy sel: with the plane pass of
+// small planes one launch, else two passes; the same bits
+int run_edge(wfs_plan* p, bool entry, void* data, hipStream_t s, int sel) {
+  if (p->variant[WFS_K_YZ_PLANE] != 0 && yz_edge_supported(p->precision, p->n[1], p->n[2])) {
+    YzPlaneParams pp;
+    pp.tw_yi = table_copy(p, p->tw[1], 1, sel);
+    pp.tw_yf = pp.tw_yi;
+    pp.tw_z = table_copy(p, p->tw[2], 2, sel);
+    pp.nx = p->n[0];
+    pp.planes = long(p->batch) * p->n[0];
+    ProfileScope scope(p, WFS_K_SLAB_EDGE, s);
+    return launch_yz_edge(p->precision, p->n[1], entry, data, pp, s);
+  }
+  if (entry) {
+    WFS_TRY(run_pass(p, 2, MODE_FWD, data, nullptr, nullptr, 1.0, s, sel));
+    return run_pass(p, 1, MODE_FWD, data, nullptr, nullptr, 1.0, s, sel);
+  }
+  WFS_TRY(run_pass(p, 1, MODE_INV, data, nullptr, nullptr, 1.0, s, sel));
+  return run_pass(p, 2, MODE_INV, data, nullptr, nullptr, 1.0, s, sel);
+}
+
 int run_yz(wfs_plan* p, void* data, const void* pv, hipStream_t s, int sel) {
   if (p->variant[WFS_K_YZ_PLANE] != 0) return run_yz_plane(p, data, pv, s, sel);
   WFS_TRY(run_pass(p, 1, MODE_INV, data, nullptr, nullptr, 1.0, s, sel - 1));
@@ -617,16 +638,13 @@ int fourier_steps(wfs_plan* p, void* psi, const void* V, int nsteps, hipStream_t
     }
     return run_slab_lines(p, LINES_EXIT, psi, nullptr, s, b + nsteps);
   }
-  WFS_TRY(run_pass(p, 2, MODE_FWD, psi, nullptr, nullptr, 1.0, s, b));
-  WFS_TRY(run_pass(p, 1, MODE_FWD, psi, nullptr, nullptr, 1.0, s, b));
+  WFS_TRY(run_edge(p, true, psi, s, b));
   WFS_TRY(run_pass(p, 0, MODE_FKI, psi, nullptr, kh, 1.0, s, b));
   for (int step = 1; step <= nsteps; ++step) {
     WFS_TRY(run_yz(p, psi, pv, s, b + step));
     WFS_TRY(run_pass(p, 0, MODE_FKI, psi, nullptr, step == nsteps ? kh : kf, 1.0, s, b + step));
   }
-  WFS_TRY(run_pass(p, 1, MODE_INV, psi, nullptr, nullptr, 1.0, s, b + nsteps));
-  WFS_TRY(run_pass(p, 2, MODE_INV, psi, nullptr, nullptr, 1.0, s, b + nsteps));
-  return 0;
+  return run_edge(p, false, psi, s, b + nsteps);
 }
 
 // nsteps steps with the box observables of the state before steps 0, every, 2 every, ...
