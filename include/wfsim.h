@@ -339,8 +339,9 @@ int wfs_plan_set_profiling(wfs_plan* plan, int enable);
  * ny = nz <= 128, complex128 planes of ny = nz <= 64) runs the y inverse, z
  * inverse / potential / z forward and y forward passes of each step as one
  * kernel on whole x planes held in LDS, and at up to 64 x 64 planes the first
- * and last two passes of a call likewise (kernel class WFS_K_SLAB_EDGE); variant 0 runs the three passes.  The
- * results are identical; the autotuner keeps the faster.
+ * and last two passes of a call likewise (kernel class WFS_K_SLAB_EDGE);
+ * variant 0 runs the single passes.  The results are identical; the autotuner
+ * keeps the faster.
  * WFS_K_YZ_SLAB: variants 1 and 2 (the default where supported: complex64
  * grids with ny = nz = 256 or 192 and nx <= 256, 2 at 256 and 1 at 192; at
  * ny = nz = 128 variant 2 below 256 x planes) run a step as two launches, the
@@ -358,12 +359,17 @@ int wfs_plan_set_profiling(wfs_plan* plan, int enable);
  * and absorbing x layers), so that those reads hit the caches instead of HBM;
  * variant 0 reads every plane's own copy.  The results are bit-identical.
  * WFS_K_YZ_SPLIT (no launches of its own: they count as WFS_K_YZ_SLAB,
- * WFS_K_X_SLAB and WFS_K_SLAB_EDGE): variant 1 (default where supported:
- * complex128 grids with ny = nz in {64, 96, 128, 192} and complex64 grids with
- * ny = nz = 96 or, from 256 x planes on, 128, nx <= 256, at 64 only below 192 x
- * planes; complex64 grids with ny = nz = 512 and nx >= 32) runs the steps as the slab scheme's two launches, variant 0 as the plane pass or the
- * axis passes; the results agree to rounding.  Setting WFS_K_YZ_PLANE or
- * WFS_K_YZ_SLAB switches it off.
+ * WFS_K_X_SLAB and WFS_K_SLAB_EDGE): variant 1 (the default where supported,
+ * but for complex128 64 x 64 planes beside 192 and more x planes) runs the
+ * steps as the slab scheme's two launches, variant 0 as the plane pass or the
+ * axis passes; the results agree to rounding.  Supported: complex128 grids with
+ * ny = nz in {64, 96, 128, 192}, nx <= 256; complex64 grids with ny = nz = 96 or
+ * 128, with ny = nz = 512 and nx >= 32, with ny = nz = 192 or 256 and nx = 512,
+ * and with ny != nz in {32, 64, 96, 128, 192, 256, 512}, but for nx < 32 beside
+ * planes of 8 residue classes (from 96 x 512 and 256 x 192 points on) and
+ * nx = 512 beside 32 x 64.  At complex64 128 x 128 planes WFS_K_YZ_SLAB runs
+ * them below 256 x planes.  Setting WFS_K_YZ_PLANE or WFS_K_YZ_SLAB switches
+ * it off.
  */
 int wfs_plan_autotune(wfs_plan* plan, void* stream);
 int wfs_plan_set_variant(wfs_plan* plan, int kernel_class, int variant);

@@ -100,9 +100,9 @@ def test_split_defaults(dev):
         return v["yz_split"], v["yz_slab"]
     assert on((96, 96, 96)) == (1, 0) and on((8, 96, 96), 40) == (1, 0)
     assert on((128, 128, 128)) == (0, 2) and on((256, 128, 128)) == (1, 0) and on((64, 128, 128), 8) == (1, 0)
-    assert on((64, 64, 64)) == (0, 0) and on((512, 96, 96)) == (0, 0) and on((32, 96, 128)) == (0, 0)
+    assert on((64, 64, 64)) == (0, 0) and on((512, 64, 64)) == (0, 0) and on((32, 96, 16)) == (0, 0)
     assert on((192, 192, 192)) == (0, 1)
     assert on((512, 512, 512)) == (1, 0) and on((32, 512, 512)) == (1, 0) and on((16, 512, 512)) == (0, 0)
-    assert on((512, 256, 256)) == (0, 0) and on((32, 512, 256)) == (0, 0)
+    assert on((512, 256, 256)) == (1, 0) and on((32, 512, 256)) == (1, 0) and on((16, 512, 256)) == (0, 0)
     with pytest.raises(_abi.WfsError):
         _plan((64, 64, 64)).set_variant("yz_split", 1)

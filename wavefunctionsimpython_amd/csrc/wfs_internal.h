@@ -128,10 +128,13 @@ struct XSlabParams {
   const void* ky = nullptr;
   const void* kz = nullptr;
   long packets = 0;             // grids stacked along x
+  int ny = 0, nz = 0;
 };
 bool slab_supported(int precision, const int n[3]);
 // the same two launches under kernel class WFS_K_YZ_SPLIT: complex128 planes, complex64 96^2, 128^2 and 512^2 planes
 bool split_supported(int precision, const int n[3]);
+// and for complex64 planes of unequal sides (wfs_rect.hip; the same class)
+bool rect_supported(int precision, const int n[3]);
 // Per x plane (packets * nx planes of plane_elems 64-bit words, contiguous per plane): src[p]
 // = the first plane of the run of bitwise-identical consecutive planes holding p, within its
 // packet.  flags: workspace of packets * nx ints.
@@ -140,16 +143,18 @@ bool split_supported(int precision, const int n[3]);
 int launch_plane_dedup(const void* table, long plane_elems, int nx, int packets, long first, long count, int* flags,
                        int* src, hipStream_t s);
 // thread geometry of the slab scheme's y-z launch: y lines split over uy threads, z lines
-// over uz threads, n1 points per thread; y-line twiddle stride b in the ny table
+// over uz threads, n1y and n1z points per thread; y-line twiddle stride b in the ny table
 struct SlabRows {
-  int b, uy, uz, n1;
+  int b = 0, uy = 0, uz = 0, n1y = 0, n1z = 0;
 };
-SlabRows slab_rows(int precision, int n);
-// the potential table order of the slab scheme's y-z launch (ny = nz = n)
-LinesOrder slab_lines_order(int precision, int n);
+SlabRows slab_rows(int precision, const int n[3]);
+SlabRows rect_rows(int ny, int nz);
+int launch_yz_rect(int ny, int nz, int mode, void* data, const YzPlaneParams& p, hipStream_t s);
+// the potential table order of the slab scheme's y-z launch
+LinesOrder slab_lines_order(int precision, const int n[3]);
 // YzPlaneParams.planes = packets * nx
-int launch_yz_slab(int precision, int n, int mode, void* data, const YzPlaneParams& p, hipStream_t s);
-int launch_x_slab(int precision, int nx, int n, void* data, const XSlabParams& p, hipStream_t s);
+int launch_yz_slab(int precision, const int n[3], int mode, void* data, const YzPlaneParams& p, hipStream_t s);
+int launch_x_slab(int precision, const int n[3], void* data, const XSlabParams& p, hipStream_t s);
 
 // pv = cexp_i(-dt V) elementwise in the state precision
 int launch_potential_phase(int precision, long count, const float2* V, double dt, void* pv, hipStream_t s);

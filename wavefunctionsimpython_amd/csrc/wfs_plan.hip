@@ -376,7 +376,7 @@ int set_potential(wfs_plan* p, const void* V, hipStream_t s) {
   if (slab_on(p)) {
     WFS_TRY(alloc_table(p, &p->pv_lines, s));
     WFS_TRY(launch_potential_phase_lines(p->precision, count, static_cast<const float2*>(V), p->dt, p->pv_lines,
-                                         slab_lines_order(p->precision, p->n[1]), s));
+                                         slab_lines_order(p->precision, p->n), s));
     p->pv_lines_ok = true;
     p->pv_nat_ok = false;
     if (capturing(s)) p->pv_in_graph = true;
@@ -406,7 +406,7 @@ int set_potential_planes(wfs_plan* p, const void* V, int x_begin, int x_end, hip
   const float2* v = static_cast<const float2*>(V) + off;
   if (slab_on(p)) {
     WFS_TRY(launch_potential_phase_lines(p->precision, count, v, p->dt, static_cast<char*>(p->pv_lines) + off * p->elem,
-                                         slab_lines_order(p->precision, p->n[1]), s));
+                                         slab_lines_order(p->precision, p->n), s));
     p->pv_nat_ok = false;
     if (capturing(s)) p->pv_in_graph = true;
     if (p->pv_planes_ok && !capturing(s)) {
@@ -434,7 +434,7 @@ int current_table(wfs_plan* p, hipStream_t s, const void** out) {
   if (slab_on(p)) {
     if (!p->pv_lines_ok) {
       WFS_TRY(alloc_table(p, &p->pv_lines, s));
-      WFS_TRY(launch_table_reorder(p->precision, count, p->pv, p->pv_lines, slab_lines_order(p->precision, p->n[1]), true, s));
+      WFS_TRY(launch_table_reorder(p->precision, count, p->pv, p->pv_lines, slab_lines_order(p->precision, p->n), true, s));
       p->pv_lines_ok = !capturing(s);
       p->pv_planes_ok = false;
       if (capturing(s)) p->pv_in_graph = true;
@@ -444,7 +444,7 @@ int current_table(wfs_plan* p, hipStream_t s, const void** out) {
   } else {
     if (!p->pv_nat_ok) {
       WFS_TRY(alloc_table(p, &p->pv, s));
-      WFS_TRY(launch_table_reorder(p->precision, count, p->pv_lines, p->pv, slab_lines_order(p->precision, p->n[1]), false, s));
+      WFS_TRY(launch_table_reorder(p->precision, count, p->pv_lines, p->pv, slab_lines_order(p->precision, p->n), false, s));
       p->pv_nat_ok = !capturing(s);
     }
     *out = p->pv;
@@ -529,11 +529,11 @@ int run_yz(wfs_plan* p, void* data, const void* pv, hipStream_t s, int sel) {
 // LINES_FULL), or the entry (z, y forward) / exit (y, z inverse) launch of a call
 int run_slab_lines(wfs_plan* p, int mode, void* data, const void* pv, hipStream_t s, int sel) {
   YzPlaneParams pp;
-  const SlabRows g = slab_rows(p->precision, p->n[1]);
+  const SlabRows g = slab_rows(p->precision, p->n);
   const int c = sel % p->ntab;
-  pp.tw_yi = static_cast<const char*>(p->tw_rows[0]) + size_t(c) * g.uy * g.n1 * p->elem;
+  pp.tw_yi = static_cast<const char*>(p->tw_rows[0]) + size_t(c) * g.uy * g.n1y * p->elem;
   pp.tw_yf = pp.tw_yi;
-  pp.tw_z = static_cast<const char*>(p->tw_rows[1]) + size_t(c) * g.uz * g.n1 * p->elem;
+  pp.tw_z = static_cast<const char*>(p->tw_rows[1]) + size_t(c) * g.uz * g.n1z * p->elem;
   if (mode == LINES_FULL) {
     if (p->sep_set) {
       const size_t per = size_t(p->batch) * p->elem;
@@ -550,7 +550,7 @@ int run_slab_lines(wfs_plan* p, int mode, void* data, const void* pv, hipStream_
   pp.nx = p->n[0];
   pp.planes = long(p->batch) * p->n[0];
   ProfileScope scope(p, mode == LINES_FULL ? WFS_K_YZ_SLAB : WFS_K_SLAB_EDGE, s);
-  return launch_yz_slab(p->precision, p->n[1], mode, data, pp, s);
+  return launch_yz_slab(p->precision, p->n, mode, data, pp, s);
 }
 
 // Slab scheme: length-4 y stages around x forward -> K -> x inverse
@@ -562,8 +562,10 @@ int run_x_slab(wfs_plan* p, void* data, const void* const* ktab, hipStream_t s, 
   xp.ky = table_copy(p, ktab[1], 1, sel);
   xp.kz = table_copy(p, ktab[2], 2, sel);
   xp.packets = p->batch;
+  xp.ny = p->n[1];
+  xp.nz = p->n[2];
   ProfileScope scope(p, WFS_K_X_SLAB, s);
-  return launch_x_slab(p->precision, p->n[0], p->n[1], data, xp, s);
+  return launch_x_slab(p->precision, p->n, data, xp, s);
 }
 
 // Slab scheme, observing launches: LINES_OBSERVE runs the exit launch of one stretch (table copy
@@ -573,14 +575,14 @@ int run_x_slab(wfs_plan* p, void* data, const void* const* ktab, hipStream_t s, 
 // The records (obs_lines) are allocated with the plan.
 int run_slab_observe(wfs_plan* p, int mode, void* data, int sel_exit, int sel_entry, const wfs_box* boxes, int nb,
                      double* out, hipStream_t s) {
-  const SlabRows g = slab_rows(p->precision, p->n[1]);
+  const SlabRows g = slab_rows(p->precision, p->n);
   const long groups = long(p->batch) * p->n[0] * g.b;
   if (p->obs_lines_len < groups * kBoxesPerPass * 7) {
     set_last_error("wfs_step_observe: observing records missing");
     return WFS_ERR_INVALID;
   }
   YzPlaneParams pp;
-  const size_t ysz = size_t(g.uy) * g.n1 * p->elem, zsz = size_t(g.uz) * g.n1 * p->elem;
+  const size_t ysz = size_t(g.uy) * g.n1y * p->elem, zsz = size_t(g.uz) * g.n1z * p->elem;
   const char* ty = static_cast<const char*>(p->tw_rows[0]);
   const char* tz = static_cast<const char*>(p->tw_rows[1]);
   if (mode == LINES_OBSERVE) {
@@ -607,7 +609,7 @@ int run_slab_observe(wfs_plan* p, int mode, void* data, int sel_exit, int sel_en
   pp.mom.partials = p->obs_lines;
   {
     ProfileScope scope(p, WFS_K_SLAB_OBSERVE, s);
-    WFS_TRY(launch_yz_slab(p->precision, p->n[1], mode, data, pp, s));
+    WFS_TRY(launch_yz_slab(p->precision, p->n, mode, data, pp, s));
   }
   ProfileScope scope(p, WFS_K_OBSERVABLES, s);
   return launch_sum_partials(p->obs_lines, long(p->n[0]) * g.b, nb, p->batch, p->dx[0] * p->dx[1] * p->dx[2] / 27.0,
@@ -793,7 +795,7 @@ extern "C" int wfs_plan_create_batched(const int n[3], const double dx[3], doubl
   if (slab) p->variant[WFS_K_X_SLAB] = n[1] == 192 ? 1 : 2;
   const bool two_launch = slab_supported(precision, n) || split_supported(precision, n);
   // the same two launches elsewhere, figures at split_supported
-  p->variant[WFS_K_YZ_SPLIT] = !slab && split_supported(precision, n) && (n[1] != 64 || n[0] < 192) ? 1 : 0;
+  p->variant[WFS_K_YZ_SPLIT] = !slab && split_supported(precision, n) && (n[1] != n[2] || n[1] != 64 || n[0] < 192) ? 1 : 0;
   p->pending = new std::vector<std::pair<hipEvent_t, hipEvent_t>>[WFS_K_COUNT];
   p->event_pool = new std::vector<hipEvent_t>();
   int rc = 0;
@@ -807,9 +809,9 @@ extern "C" int wfs_plan_create_batched(const int n[3], const double dx[3], doubl
     rc = upload_dithered(&p->tw[a], re, im, precision);
     if (rc) break;
     if (a > 0 && two_launch) {
-      const SlabRows g = slab_rows(precision, n[1]);
-      rc = a == 1 ? upload_rows_table(&p->tw_rows[0], re, im, g.b, g.uy, g.n1, precision)
-                  : upload_rows_table(&p->tw_rows[1], re, im, 1, g.uz, g.n1, precision);
+      const SlabRows g = slab_rows(precision, n);
+      rc = a == 1 ? upload_rows_table(&p->tw_rows[0], re, im, g.b, g.uy, g.n1y, precision)
+                  : upload_rows_table(&p->tw_rows[1], re, im, 1, g.uz, g.n1z, precision);
       if (rc) break;
     }
     kinetic_table(n[a], dx[a], dt, mass, 2.0, re, im);
@@ -830,7 +832,7 @@ extern "C" int wfs_plan_create_batched(const int n[3], const double dx[3], doubl
   }
   if (rc == 0 && slab_supported(precision, n)) {
     // box-moment records of the slab scheme's observing launch: one per row group and box
-    const long need = long(batch) * n[0] * slab_rows(precision, n[1]).b * kBoxesPerPass * 7;
+    const long need = long(batch) * n[0] * slab_rows(precision, n).b * kBoxesPerPass * 7;
     hipError_t e = hipMalloc(reinterpret_cast<void**>(&p->obs_lines), size_t(need) * sizeof(double));
     if (e != hipSuccess) { set_last_error("hipMalloc for observing records failed"); rc = WFS_ERR_ALLOC; }
     else p->obs_lines_len = need;
@@ -1055,7 +1057,8 @@ extern "C" int wfs_plan_set_variant(wfs_plan* p, int kc, int variant) {
     return WFS_ERR_UNSUPPORTED;
   }
   if (kc == WFS_K_YZ_SPLIT && variant > 0 && !split_supported(p->precision, p->n)) {
-    set_last_error("wfs_plan_set_variant: the split scheme needs ny = nz in {64, 96, 128, 192} and nx <= 256 (complex64: 96, 128, or 512 with nx >= 32)");
+    set_last_error("wfs_plan_set_variant: the split scheme does not take %d x %d x %d grids of this precision", p->n[0],
+                   p->n[1], p->n[2]);
     return WFS_ERR_UNSUPPORTED;
   }
   p->variant[kc] = variant;

@@ -295,7 +295,7 @@ __global__ __launch_bounds__(kGenThreads) void potential_table_kernel(cx<R>* __r
 // 128^3 complex128 20 -> 14, against one element a thread that reads V down the rows (the table in C order
 // takes 60, 634, 24 and 11).
 enum { TABLE_FACTORS, TABLE_TO_LINES, TABLE_FROM_LINES };
-constexpr int kLinesTileZ = 16, kLinesTileRows = 64;
+constexpr int kLinesTileZ = 16, kLinesTileRows = 128;
 
 template <typename R, int MODE>
 __global__ __launch_bounds__(kGenThreads) void table_lines_kernel(cx<R>* __restrict__ dst, const void* __restrict__ src,
@@ -309,12 +309,12 @@ __global__ __launch_bounds__(kGenThreads) void table_lines_kernel(cx<R>* __restr
   // 16 lanes along z and 16 rows a round on the C-order side, a wavefront per z on the other
   constexpr int kRows = kGenThreads / kLinesTileZ, kLines = kGenThreads / 64;
   const int zl = threadIdx.x % kLinesTileZ, yl = threadIdx.x / kLinesTileZ;
-  const int row = threadIdx.x % 64, zw = threadIdx.x / 64;
+  const int zw = threadIdx.x / 64;
   if constexpr (MODE == TABLE_FROM_LINES) {
     const cx<R>* in = static_cast<const cx<R>*>(src);
 #pragma unroll
     for (int z = zw; z < kLinesTileZ; z += kLines)
-      if (row < m.ly) tile[z][row] = in[lin + long(z) * m.ly + row];
+      for (int row = threadIdx.x % 64; row < m.ly; row += 64) tile[z][row] = in[lin + long(z) * m.ly + row];
     __syncthreads();
 #pragma unroll
     for (int y = yl; y < kLinesTileRows; y += kRows)
@@ -330,7 +330,7 @@ __global__ __launch_bounds__(kGenThreads) void table_lines_kernel(cx<R>* __restr
     __syncthreads();
 #pragma unroll
     for (int z = zw; z < kLinesTileZ; z += kLines)
-      if (row < m.ly) dst[lin + long(z) * m.ly + row] = tile[z][row];
+      for (int row = threadIdx.x % 64; row < m.ly; row += 64) dst[lin + long(z) * m.ly + row] = tile[z][row];
   }
 }
 

@@ -248,28 +248,34 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && ZB == 8 && NX / split_of<NX
 //   512^2 planes (B = 8): 512^3 597 us, 646 with the tiles of a ka in pairs over the XCDs (the axis pass alone
 //   688), 256 x 512^2 317 -> 233, 64 x 512^2 46 -> 50; 400 us of arithmetic beside one block's waits.  Lanes along
 //   x instead of the rows at the loads save a transposition and lose more to eight pages a load: 692 us.
-template <int NX, int N, int B>
-__global__ __launch_bounds__(64 * split_of<NX>::n2) void x_rows_kernel(cx<float>* __restrict__ data,
+// N: the sides of square planes at compile time, or 0 (256^3 49.3 us, with sides at run time 52).
+template <int NX, int B, int N>
+__global__ __launch_bounds__(64 * split_of<NX>::n2)
+__attribute__((amdgpu_waves_per_eu(NX == 256 && B >= 4 ? 8 : 1))) void x_rows_kernel(cx<float>* __restrict__ data,
                                                                         const XSlabParams p) {
-  constexpr int ZB = 64 / B, A = N / B, TZ = N / ZB;
+  constexpr int ZB = 64 / B;
+  // B = 1: 64 consecutive points of the plane, taken as one row
+  const unsigned NY = N ? unsigned(N) : B == 1 ? 1u : unsigned(p.ny);
+  const unsigned NZ = N ? unsigned(N) : B == 1 ? unsigned(p.ny) * unsigned(p.nz) : unsigned(p.nz);
+  const unsigned A = NY / B, TZ = NZ / ZB;
   constexpr int N2 = split_of<NX>::n2, N1 = NX / N2;
-  static_assert(N1 % B == 0 && A % 8 == 0 && N % ZB == 0, "bad split of the x line");
+  static_assert(N1 % B == 0, "bad split of the x line");
   using C = cx<float>;
   using CC = const __attribute__((address_space(4))) C;
   __shared__ float lds[64 * NX];
 
   const int lane = threadIdx.x & 63;
   const int t = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const long bid = blockIdx.x;
-  const int zt = B == 8 ? int((bid / 8) % TZ) : int((bid / A) % TZ);
-  const int ka = B == 8 ? int((bid / (8 * TZ)) % (A / 8)) * 8 + int(bid % 8) : int(bid % A);
-  const long pk = bid / (long(TZ) * A);
-  C* __restrict__ blk = data + pk * (long(NX) * N * N) + long(B * ka) * N + long(zt) * ZB;
-  constexpr unsigned XS = unsigned(N) * N, EB = unsigned(sizeof(C));
-  static_assert(long(NX) * N * N * sizeof(C) <= (1L << 32), "32-bit byte offsets");
+  const unsigned pk = blockIdx.x / (TZ * A), bid = blockIdx.x % (TZ * A);
+  const bool by_xcd = B == 8 && A % 8 == 0;
+  const int zt = int(by_xcd ? (bid / 8) % TZ : bid / A);
+  const int ka = int(by_xcd ? (bid / (8 * TZ)) * 8 + bid % 8 : bid % A);
+  const unsigned XS = NY * NZ;
+  constexpr unsigned EB = unsigned(sizeof(C));           // byte offsets within a packet: nx ny nz 8 <= 2^32
+  C* __restrict__ blk = data + long(pk) * NX * XS + long(B * ka) * NZ + long(zt) * ZB;
 
   auto off = [&](int l, int i) {
-    return (unsigned(l % ZB) + unsigned(l / ZB) * N + (unsigned(t) + unsigned(N2) * unsigned(i)) * XS) * EB;
+    return (unsigned(l % ZB) + unsigned(l / ZB) * NZ + (unsigned(t) + unsigned(N2) * unsigned(i)) * XS) * EB;
   };
   C a[N1];
 #pragma unroll
@@ -278,12 +284,12 @@ __global__ __launch_bounds__(64 * split_of<NX>::n2) void x_rows_kernel(cx<float>
   CC* twy = (CC*)(p.tw_y);
   // forward y stage X[kb] = sum_b W_B^{b kb} W_N^{b ka} Y[b] on B x points at a time
 #pragma unroll
-  for (int g = 0; g < N1; g += B) {
+  for (int g = 0; g < (B > 1 ? N1 : 0); g += B) {
     transpose_rows<B>(a + g);
     C r[B];
     r[0] = a[g];
 #pragma unroll
-    for (int b = 1; b < B; ++b) r[b] = cmul(a[g + b], mk<float>(twy[(b * ka) % N].x, twy[(b * ka) % N].y));
+    for (int b = 1; b < B; ++b) r[b] = cmul(a[g + b], mk<float>(twy[b * ka].x, twy[b * ka].y));
     DFT<B, -1>::run(r);
 #pragma unroll
     for (int b = 0; b < B; ++b) a[g + b] = r[b];
@@ -304,8 +310,9 @@ __global__ __launch_bounds__(64 * split_of<NX>::n2) void x_rows_kernel(cx<float>
 
   transform_x(std::integral_constant<int, -1>{});
   {
-    const C ky = reinterpret_cast<const C*>(p.ky)[ka + A * (lane / ZB)];
-    const C kyz = cmul(ky, reinterpret_cast<const C*>(p.kz)[zt * ZB + (lane % ZB)]);
+    const int y = B == 1 ? (zt * ZB + lane) / p.nz : ka + int(A) * (lane / ZB);
+    const int z = B == 1 ? (zt * ZB + lane) % p.nz : zt * ZB + lane % ZB;
+    const C kyz = cmul(reinterpret_cast<const C*>(p.ky)[y], reinterpret_cast<const C*>(p.kz)[z]);
     CC* kx = (CC*)(p.kx) + t;
 #pragma unroll
     for (int i = 0; i < N1; ++i) a[i] = cmul(a[i], cmul(mk<float>(kx[N2 * i].x, kx[N2 * i].y), kyz));
@@ -317,15 +324,17 @@ __global__ __launch_bounds__(64 * split_of<NX>::n2) void x_rows_kernel(cx<float>
   const int l = opaque_v(lane);
 #pragma unroll
   for (int g = 0; g < N1; g += B) {
-    transpose_rows<B>(a + g);
-    C r[B];
+    if constexpr (B > 1) {
+      transpose_rows<B>(a + g);
+      C r[B];
 #pragma unroll
-    for (int b = 0; b < B; ++b) r[b] = a[g + b];
-    DFT<B, +1>::run(r);
-    a[g] = r[0];
+      for (int b = 0; b < B; ++b) r[b] = a[g + b];
+      DFT<B, +1>::run(r);
+      a[g] = r[0];
 #pragma unroll
-    for (int b = 1; b < B; ++b) a[g + b] = cmulc(r[b], mk<float>(twy[(b * ka) % N].x, twy[(b * ka) % N].y));
-    transpose_rows<B>(a + g);
+      for (int b = 1; b < B; ++b) a[g + b] = cmulc(r[b], mk<float>(twy[b * ka].x, twy[b * ka].y));
+      transpose_rows<B>(a + g);
+    }
 #pragma unroll
     for (int i = g; i < g + B; ++i) byte_at(blk, off(l, i)) = a[i];
   }
@@ -508,14 +517,14 @@ int launch_x_slab_ny(int nx, void* data, const XSlabParams& p, hipStream_t s) {
 // 9.7 / 10.4, 14.0 / 15.3.  192^2 and 256^2 planes have 576 and 1024 blocks a packet.
 bool x_rows_fill(int n, long packets) { return packets * (long(n) * n / 64) * 2 >= 3L * cu_count(); }
 
-template <int N>
+template <int B, int N = 0>
 int launch_x_rows(int nx, void* data, const XSlabParams& p, hipStream_t s) {
-  constexpr int B = SlabShape<float, N>::B;
+  const unsigned blocks = unsigned(p.packets * (long(p.ny) * p.nz / 64));
 #define WFS_X_ROWS_CASE(NX)                                                                                  \
   case NX:                                                                                                   \
-    if constexpr ((NX / split_of<NX>::n2) % B == 0 && (NX <= 256 || N == 512)) {                              \
-      WFS_LAUNCH((x_rows_kernel<NX, N, B>), dim3(unsigned(p.packets * (N / 8) * (N / 8))),                    \
-                 dim3(64 * split_of<NX>::n2), 0, s, reinterpret_cast<cx<float>*>(data), p);                  \
+    if constexpr ((NX / split_of<NX>::n2) % B == 0 && (N == 0 || NX <= 256)) {                                                    \
+      WFS_LAUNCH((x_rows_kernel<NX, B, N>), dim3(blocks), dim3(64 * split_of<NX>::n2), 0, s,                     \
+                 reinterpret_cast<cx<float>*>(data), p);                                                     \
       return int(hipGetLastError());                                                                         \
     }                                                                                                        \
     break;
@@ -541,25 +550,10 @@ template <typename R, int N>
 SlabRows slab_rows_n() {
   SlabRows g;
   g.b = SlabShape<R, N>::B;
-  g.n1 = N / split_of<N>::n2;
-  g.uy = SlabShape<R, N>::LY / g.n1;
+  g.n1y = g.n1z = N / split_of<N>::n2;
+  g.uy = SlabShape<R, N>::LY / g.n1y;
   g.uz = split_of<N>::n2;
   return g;
-}
-
-template <typename R, int N>
-LinesOrder slab_lines_order_n() {
-  constexpr int LY = SlabShape<R, N>::LY;
-  LinesOrder m;
-  m.ny = N;
-  m.nz = N;
-  m.ly = LY;
-  m.b = SlabShape<R, N>::B;
-  m.rh = LY;
-  m.n2z = split_of<N>::n2;
-  m.n1 = N / split_of<N>::n2;
-  m.threads = yz_lines_threads<N, LY, 1>();
-  return m;
 }
 
 }  // namespace
@@ -605,33 +599,46 @@ bool slab_supported(int precision, const int n[3]) {
 // complex64 512^2 planes (B = 8, x_rows_kernel), us per step with a potential table against the four axis
 // passes: 512^3 2407 -> 1412, 256 x 512^2 1158 -> 798, 64 x 512^2 230 -> 182.  Its x launch takes 8 x points
 // of a lane at a time, so nx = 8 and 16 (4 points a lane) stay with the passes.
+//
+// complex64 with 512 x planes (x_rows_kernel alone takes them): 512 x 96^2 75 / 69 -> 56 / 55, x 128^2 87 / 81 -> 81 /
+// 78, x 192^2 256 / 243 -> 218 / 200, x 256^2 450 / 374 -> 339 / 310.
 bool split_supported(int precision, const int n[3]) {
-  if (precision == WFS_C64 && n[1] == 512 && n[2] == 512) return n[0] >= 32 && fft_length_supported(n[0]);
-  return n[1] == n[2] && (n[1] == 96 || n[1] == 128 || (precision == WFS_C128 && (n[1] == 64 || n[1] == 192))) &&
-         n[0] <= 256 && fft_length_supported(n[0]);
+  if (n[1] != n[2]) return rect_supported(precision, n);
+  if (!fft_length_supported(n[0])) return false;
+  if (precision == WFS_C128) return (n[1] == 64 || n[1] == 96 || n[1] == 128 || n[1] == 192) && n[0] <= 256;
+  if (n[1] == 512) return n[0] >= 32;
+  return n[1] == 96 || n[1] == 128 || (n[0] == 512 && (n[1] == 192 || n[1] == 256));
 }
 
 SlabRows slab_rows_c128(int n);
-LinesOrder slab_lines_order_c128(int n);
 int launch_yz_slab_c128(int n, int mode, void* data, const YzPlaneParams& p, hipStream_t s);
 int launch_x_slab_c128(int nx, int n, void* data, const XSlabParams& p, hipStream_t s);
 
-SlabRows slab_rows(int precision, int n) {
+SlabRows slab_rows(int precision, const int nn[3]) {
+  if (nn[1] != nn[2]) return rect_rows(nn[1], nn[2]);
+  const int n = nn[1];
   if (precision == WFS_C128) return slab_rows_c128(n);
   if (n == 96) return slab_rows_n<float, 96>();
   if (n == 512) return slab_rows_n<float, 512>();
   return n == 128 ? slab_rows_n<float, 128>() : n == 192 ? slab_rows_n<float, 192>() : slab_rows_n<float, 256>();
 }
 
-LinesOrder slab_lines_order(int precision, int n) {
-  if (precision == WFS_C128) return slab_lines_order_c128(n);
-  if (n == 96) return slab_lines_order_n<float, 96>();
-  if (n == 512) return slab_lines_order_n<float, 512>();
-  return n == 128 ? slab_lines_order_n<float, 128>()
-                  : n == 192 ? slab_lines_order_n<float, 192>() : slab_lines_order_n<float, 256>();
+LinesOrder slab_lines_order(int precision, const int n[3]) {
+  const SlabRows g = slab_rows(precision, n);
+  LinesOrder m;
+  m.ny = n[1];
+  m.nz = n[2];
+  m.b = g.b;
+  m.ly = m.rh = n[1] / g.b;
+  m.n2z = g.uz;
+  m.n1 = g.n1z;
+  m.threads = g.uz * m.rh;
+  return m;
 }
 
-int launch_yz_slab(int precision, int n, int mode, void* data, const YzPlaneParams& p, hipStream_t s) {
+int launch_yz_slab(int precision, const int nn[3], int mode, void* data, const YzPlaneParams& p, hipStream_t s) {
+  if (nn[1] != nn[2]) return launch_yz_rect(nn[1], nn[2], mode, data, p, s);
+  const int n = nn[1];
   if (p.planes <= 0 || p.planes * 8 > 0x7fffffffL) {
     set_last_error("slab y-z pass: bad plane count %ld", p.planes);
     return WFS_ERR_INVALID;
@@ -646,19 +653,26 @@ int launch_yz_slab(int precision, int n, int mode, void* data, const YzPlanePara
   return WFS_ERR_UNSUPPORTED;
 }
 
-int launch_x_slab(int precision, int nx, int n, void* data, const XSlabParams& p, hipStream_t s) {
-  const long blocks = p.packets * long(n / 2) * (n / 4);
-  if (p.packets <= 0 || blocks > 0x7fffffffL) {
+int launch_x_slab(int precision, const int nn[3], void* data, const XSlabParams& p, hipStream_t s) {
+  const int nx = nn[0], n = nn[1];
+  const long blocks = p.packets * (nn[1] == nn[2] ? long(n / 2) * (n / 4) : long(nn[1]) * nn[2] / 64);
+  if (p.packets <= 0 || blocks > 0x7fffffffL || p.ny != nn[1] || p.nz != nn[2]) {
     set_last_error("slab x pass: bad packet count %ld", p.packets);
     return WFS_ERR_INVALID;
   }
+  if (nn[1] != nn[2]) {
+    const int b = rect_rows(nn[1], nn[2]).b;
+    return b == 1   ? launch_x_rows<1>(nx, data, p, s)
+           : b == 2 ? launch_x_rows<2>(nx, data, p, s)
+           : b == 4 ? launch_x_rows<4>(nx, data, p, s) : launch_x_rows<8>(nx, data, p, s);
+  }
   if (precision == WFS_C128) return launch_x_slab_c128(nx, n, data, p, s);
-  if (n == 512) return launch_x_rows<512>(nx, data, p, s);
-  if (n == 256) return launch_x_rows<256>(nx, data, p, s);
-  if (n == 192) return launch_x_rows<192>(nx, data, p, s);
-  const bool rows = x_rows_fill(n, p.packets);
-  if (n == 128) return rows ? launch_x_rows<128>(nx, data, p, s) : launch_x_slab_ny<float, 128>(nx, data, p, s);
-  if (n == 96) return rows ? launch_x_rows<96>(nx, data, p, s) : launch_x_slab_ny<float, 96>(nx, data, p, s);
+  if (n == 512) return launch_x_rows<8>(nx, data, p, s);
+  if (n == 256) return nx <= 256 ? launch_x_rows<4, 256>(nx, data, p, s) : launch_x_rows<4>(nx, data, p, s);
+  if (n == 192) return nx <= 256 ? launch_x_rows<4, 192>(nx, data, p, s) : launch_x_rows<4>(nx, data, p, s);
+  const bool rows = nx == 512 || x_rows_fill(n, p.packets);
+  if (n == 128) return rows ? launch_x_rows<2>(nx, data, p, s) : launch_x_slab_ny<float, 128>(nx, data, p, s);
+  if (n == 96) return rows ? launch_x_rows<2>(nx, data, p, s) : launch_x_slab_ny<float, 96>(nx, data, p, s);
   set_last_error("slab x pass: unsupported plane %d", n);
   return WFS_ERR_UNSUPPORTED;
 }
@@ -666,11 +680,6 @@ int launch_x_slab(int precision, int nx, int n, void* data, const XSlabParams& p
 SlabRows slab_rows_c128(int n) {
   return n == 64 ? slab_rows_n<double, 64>() : n == 96 ? slab_rows_n<double, 96>()
          : n == 128 ? slab_rows_n<double, 128>() : slab_rows_n<double, 192>();
-}
-
-LinesOrder slab_lines_order_c128(int n) {
-  return n == 64 ? slab_lines_order_n<double, 64>() : n == 96 ? slab_lines_order_n<double, 96>()
-         : n == 128 ? slab_lines_order_n<double, 128>() : slab_lines_order_n<double, 192>();
 }
 
 int launch_yz_slab_c128(int n, int mode, void* data, const YzPlaneParams& p, hipStream_t s) {
