@@ -345,7 +345,8 @@ int alloc_table(wfs_plan* p, void** t, hipStream_t s) {
 }
 
 // the map of x planes of pv_lines that repeat the previous plane (kernel class WFS_K_PV_PLANES,
-// variant 1): built with the lines table, so that graph capture finds it ready.  Under capture
+// variant 1): built with the lines table (fourier_steps: or at the first longer use of it), so that
+// graph capture finds it ready.  Under capture
 // it is not built (its kernels would run only at replay, and an uncaptured call before that
 // would read an unwritten map): the captured steps read every plane's own copy, and the next
 // uncaptured call builds it.  Once the table itself has been written inside a captured graph
@@ -371,7 +372,7 @@ int share_planes(wfs_plan* p, hipStream_t s) {
 
 // the phase table in the order the current scheme reads (the other order is rebuilt from it
 // on demand)
-int set_potential(wfs_plan* p, const void* V, hipStream_t s) {
+int set_potential(wfs_plan* p, const void* V, hipStream_t s, bool share = true) {
   const long count = long(grid_points(p));
   if (slab_on(p)) {
     WFS_TRY(alloc_table(p, &p->pv_lines, s));
@@ -380,7 +381,8 @@ int set_potential(wfs_plan* p, const void* V, hipStream_t s) {
     p->pv_lines_ok = true;
     p->pv_nat_ok = false;
     if (capturing(s)) p->pv_in_graph = true;
-    WFS_TRY(share_planes(p, s));
+    p->pv_planes_ok = false;
+    if (share) WFS_TRY(share_planes(p, s));
   } else {
     WFS_TRY(alloc_table(p, &p->pv, s));
     WFS_TRY(launch_potential_phase(p->precision, count, static_cast<const float2*>(V), p->dt, p->pv, s));
@@ -427,7 +429,7 @@ int set_potential_planes(wfs_plan* p, const void* V, int x_begin, int x_end, hip
 // the table the next steps read: C order for the axis passes and the plane pass, lines order
 // for the slab scheme.  A reorder issued under graph capture runs only at replay, so it does
 // not mark the other order current: the next uncaptured call reorders again.
-int current_table(wfs_plan* p, hipStream_t s, const void** out) {
+int current_table(wfs_plan* p, hipStream_t s, const void** out, bool share = true) {
   *out = nullptr;
   if (p->sep_set) return 0;
   const long count = long(grid_points(p));
@@ -439,7 +441,7 @@ int current_table(wfs_plan* p, hipStream_t s, const void** out) {
       p->pv_planes_ok = false;
       if (capturing(s)) p->pv_in_graph = true;
     }
-    if (!p->pv_planes_ok && p->variant[WFS_K_PV_PLANES] != 0) WFS_TRY(share_planes(p, s));
+    if (share && !p->pv_planes_ok && p->variant[WFS_K_PV_PLANES] != 0) WFS_TRY(share_planes(p, s));
     *out = p->pv_lines;
   } else {
     if (!p->pv_nat_ok) {
@@ -619,10 +621,15 @@ int run_slab_observe(wfs_plan* p, int mode, void* data, int sel_exit, int sel_en
 int observe(wfs_plan* p, const void* psi, const wfs_box* boxes, int nboxes, double* out, hipStream_t s);
 
 int fourier_steps(wfs_plan* p, void* psi, const void* V, int nsteps, hipStream_t s) {
-  if (V) WFS_TRY(set_potential(p, V, s));
+  // The map of repeated planes costs two launches that read the table twice (256^3 37 us, 96 x 192 x 128 13)
+  // and saves a step up to the table's read (256^3 6 us, 96 x 192 x 128 2): a call that brings its potential
+  // for a few steps leaves it to the next call that steps on the same table.  The bits are the same.
+  constexpr int kShareSteps = 8;
+  const bool share = !V || nsteps >= kShareSteps;
+  if (V) WFS_TRY(set_potential(p, V, s, share));
   if (!p->pv_set) { set_last_error("wfs_step: no potential (pass V or call wfs_set_potential first)"); return WFS_ERR_INVALID; }
   const void* pv = nullptr;
-  WFS_TRY(current_table(p, s, &pv));
+  WFS_TRY(current_table(p, s, &pv, share));
   const void* const* kh = p->khalf;
   const void* const* kf = p->kfull;
   // every pass of the call's step k uses table copy b + k (mod ntab), the entry passes copy b:
