@@ -53,18 +53,24 @@ struct BoxSet {
   int bot[kBoxesPerPass][3], num[kBoxesPerPass][3];
 };
 
-template <typename R>
+// NB boxes.  A lane's z positions and each box's weights at them are the same for every row, so they are
+// held over the rows, 256 points of z at a time, and a point costs three multiply-adds a box on rho, rho z and
+// rho z^2, with weight 0 outside the box.  0 times a non-finite density would reach boxes that do not hold
+// the point, so rows with one in any lane (or one near overflow) take the selecting form.  Bound by the reads
+// (256^3, one box 23 us: 5.8 TB/s, partly cached) and at more boxes by the registers, 137 at three (128 with
+// spills: 47 instead of 44).  us a call with the summing launch, against weights formed at every point: 256^3 one
+// box 72 -> 28, three 76 -> 44, four 76 -> 50; 48 x 64^3 three 188 -> 105; 128^3 complex128 three 26 -> 16.
+template <typename R, int NB>
 __global__ __launch_bounds__(kObsThreads) void box_moments_kernel(const cx<R>* __restrict__ psi, int nx, int ny,
                                                                   int nz, double dx, double dy, double dz,
                                                                   BoxSet set, double* __restrict__ partials) {
-  constexpr int kWaves = kObsThreads / 64;
-  constexpr int NB = kBoxesPerPass;
+  constexpr int kWaves = kObsThreads / 64, U = 4;
   const long nrows = long(set.cnt[0]) * set.cnt[1];
   // packet blockIdx.y of a stack of independent grids
   psi += long(blockIdx.y) * nx * ny * nz;
-  partials += long(blockIdx.y) * gridDim.x * set.n * kObsQ;
+  partials += long(blockIdx.y) * gridDim.x * NB * kObsQ;
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long row0 = long(blockIdx.x) * kRowsPerBlock;
   // lane partial sums; every term is linear in the lane's z sums, so the row weights
   // (uniform over the wavefront) multiply them before the one reduction at the end
@@ -74,60 +80,80 @@ __global__ __launch_bounds__(kObsThreads) void box_moments_kernel(const cx<R>* _
 #pragma unroll
     for (int q = 0; q < kObsQ; ++q) acc[b][q] = 0.0;
 
-  for (int rr = wave; rr < kRowsPerBlock; rr += kWaves) {
-    const long row = row0 + rr;
-    if (row >= nrows) break;
-    const int gx = set.lo[0] + int(row / set.cnt[1]);
-    const int gy = set.lo[1] + int(row % set.cnt[1]);
-    double wxy[NB];
-    bool any = false;
+  const int zend = set.lo[2] + set.cnt[2];
+  for (int z0 = set.lo[2]; z0 < zend; z0 += 64 * U) {
+    double rz[U], wz[NB][U];
+    int zi[U];                                 // lanes beyond the bounding box read its last point, weight 0
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const int ix = gx - set.bot[b][0], iy = gy - set.bot[b][1];
-      const bool in = b < set.n && ix >= 0 && ix < set.num[b][0] && iy >= 0 && iy < set.num[b][1];
-      wxy[b] = in ? simpson_s(ix, set.num[b][0]) * simpson_s(iy, set.num[b][1]) : 0.0;
-      any = any || in;
-    }
-    if (!any) continue;
-    const double rx = dx * double(gx - nx / 2);
-    const double ry = dy * double(gy - ny / 2);
-    const cx<R>* rowp = psi + (long(gx) * ny + gy) * long(nz);
-    double s0[NB], sz1[NB], sz2[NB];
+    for (int u = 0; u < U; ++u) {
+      const int gz = z0 + lane + 64 * u;
+      zi[u] = min(gz, zend - 1);
+      rz[u] = dz * double(gz - nz / 2);
 #pragma unroll
-    for (int b = 0; b < NB; ++b) s0[b] = sz1[b] = sz2[b] = 0.0;
-    // 256 points of the row at a time: four loads issued together (indices clamped into the
-    // row, the excess lanes masked afterwards), so that each wavefront has four in flight
-    const int zend = set.lo[2] + set.cnt[2];
-    for (int z0 = set.lo[2]; z0 < zend; z0 += 256) {
-      cx<R> v[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] = rowp[min(z0 + lane + 64 * u, zend - 1)];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int gz = z0 + lane + 64 * u;
-        const double rho = gz < zend ? double(v[u].x) * double(v[u].x) + double(v[u].y) * double(v[u].y) : 0.0;
-        const double rz = dz * double(gz - nz / 2);
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-          const int iz = gz - set.bot[b][2];
-          const bool in = wxy[b] != 0.0 && iz >= 0 && iz < set.num[b][2];
-          const double wr = in ? simpson_s(iz, set.num[b][2]) * rho : 0.0;
-          s0[b] += wr;
-          sz1[b] += wr * rz;
-          sz2[b] += wr * rz * rz;
-        }
+      for (int b = 0; b < NB; ++b) {
+        const int iz = gz - set.bot[b][2];
+        wz[b][u] = iz >= 0 && iz < set.num[b][2] ? simpson_s(iz, set.num[b][2]) : 0.0;
       }
     }
+    for (int rr = wave; rr < kRowsPerBlock; rr += kWaves) {
+      const long row = row0 + rr;
+      if (row >= nrows) break;
+      const int gx = set.lo[0] + int(row / set.cnt[1]);
+      const int gy = set.lo[1] + int(row % set.cnt[1]);
+      double wxy[NB];
+      bool any = false;
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const double w = wxy[b];
-      acc[b][0] += w * s0[b];
-      acc[b][1] += w * rx * s0[b];
-      acc[b][2] += w * ry * s0[b];
-      acc[b][3] += w * sz1[b];
-      acc[b][4] += w * rx * rx * s0[b];
-      acc[b][5] += w * ry * ry * s0[b];
-      acc[b][6] += w * sz2[b];
+      for (int b = 0; b < NB; ++b) {
+        const int ix = gx - set.bot[b][0], iy = gy - set.bot[b][1];
+        const bool in = ix >= 0 && ix < set.num[b][0] && iy >= 0 && iy < set.num[b][1];
+        wxy[b] = in ? simpson_s(ix, set.num[b][0]) * simpson_s(iy, set.num[b][1]) : 0.0;
+        any = any || in;
+      }
+      if (!any) continue;
+      const double rx = dx * double(gx - nx / 2);
+      const double ry = dy * double(gy - ny / 2);
+      const cx<R>* rowp = psi + (long(gx) * ny + gy) * long(nz);
+      cx<R> v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = rowp[zi[u]];
+      double m0[U], m1[U], m2[U], total = 0.0;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        m0[u] = double(v[u].x) * double(v[u].x) + double(v[u].y) * double(v[u].y);
+        m1[u] = m0[u] * rz[u];
+        m2[u] = m1[u] * rz[u];
+        total += m0[u];
+      }
+      const bool select = __any(!(total < 1e280));
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const double w = wxy[b];
+        if (w == 0.0) continue;
+        double s0 = 0.0, sz1 = 0.0, sz2 = 0.0;
+        if (select) {
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const bool in = wz[b][u] != 0.0;
+            s0 += in ? wz[b][u] * m0[u] : 0.0;
+            sz1 += in ? wz[b][u] * m1[u] : 0.0;
+            sz2 += in ? wz[b][u] * m2[u] : 0.0;
+          }
+        } else {
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            s0 += wz[b][u] * m0[u];
+            sz1 += wz[b][u] * m1[u];
+            sz2 += wz[b][u] * m2[u];
+          }
+        }
+        acc[b][0] += w * s0;
+        acc[b][1] += w * rx * s0;
+        acc[b][2] += w * ry * s0;
+        acc[b][3] += w * sz1;
+        acc[b][4] += w * rx * rx * s0;
+        acc[b][5] += w * ry * ry * s0;
+        acc[b][6] += w * sz2;
+      }
     }
   }
 
@@ -135,17 +161,16 @@ __global__ __launch_bounds__(kObsThreads) void box_moments_kernel(const cx<R>* _
   static_assert(kObsQ == 7, "the wavefront sums take seven values");
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
-    if (b >= set.n) break;
     const double v = wave_sum7(acc[b], lane);
     const int q = (lane >> 3) & 7;
     if ((lane & 7) == 0 && q < kObsQ) red[wave][b * kObsQ + q] = v;
   }
   __syncthreads();
-  if (int(threadIdx.x) < set.n * kObsQ) {
+  if (int(threadIdx.x) < NB * kObsQ) {
     double v = 0.0;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) v += red[w][threadIdx.x];
-    partials[long(blockIdx.x) * set.n * kObsQ + threadIdx.x] = v;
+    partials[long(blockIdx.x) * NB * kObsQ + threadIdx.x] = v;
   }
 }
 
@@ -223,13 +248,24 @@ int launch_box_moments(int precision, int batch, int nx, int ny, int nz, const d
   }
   // the Simpson weight products carry 1/27 and the volume element dx dy dz
   const double sc = dx[0] * dx[1] * dx[2] / 27.0;
-  if (precision == WFS_C128) {
-    WFS_LAUNCH(box_moments_kernel<double>, dim3(unsigned(nblocks), unsigned(batch)), dim3(kObsThreads), 0, s,
-                       static_cast<const double2*>(psi), nx, ny, nz, dx[0], dx[1], dx[2], set, partials);
-  } else {
-    WFS_LAUNCH(box_moments_kernel<float>, dim3(unsigned(nblocks), unsigned(batch)), dim3(kObsThreads), 0, s,
-                       static_cast<const float2*>(psi), nx, ny, nz, dx[0], dx[1], dx[2], set, partials);
+  const dim3 grid{unsigned(nblocks), unsigned(batch)}, block{unsigned(kObsThreads)};
+#define WFS_BOX_MOMENTS(NB)                                                                                  \
+  case NB:                                                                                                   \
+    if (precision == WFS_C128)                                                                               \
+      WFS_LAUNCH((box_moments_kernel<double, NB>), grid, block, 0, s, static_cast<const double2*>(psi), nx, ny, \
+                 nz, dx[0], dx[1], dx[2], set, partials);                                                    \
+    else                                                                                                     \
+      WFS_LAUNCH((box_moments_kernel<float, NB>), grid, block, 0, s, static_cast<const float2*>(psi), nx, ny,  \
+                 nz, dx[0], dx[1], dx[2], set, partials);                                                    \
+    break;
+  static_assert(kBoxesPerPass == 4, "one case per number of boxes");
+  switch (nb) {
+    WFS_BOX_MOMENTS(1)
+    WFS_BOX_MOMENTS(2)
+    WFS_BOX_MOMENTS(3)
+    WFS_BOX_MOMENTS(4)
   }
+#undef WFS_BOX_MOMENTS
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return int(e);
   WFS_LAUNCH(sum_partials_kernel, dim3(unsigned(nb), unsigned(batch)), dim3(kObsThreads), 0, s, partials,
