@@ -443,14 +443,30 @@ __device__ __forceinline__ void transpose_words(float (&v)[B]) {
 }
 
 template <int B>
-__device__ __forceinline__ void transpose_rows(cx<float>* a) {
-  float x[B], y[B];
+__device__ __forceinline__ void transpose_words(double (&v)[B]) {
+  float lo[B], hi[B];
+#pragma unroll
+  for (int r = 0; r < B; ++r) {
+    const long long b = __double_as_longlong(v[r]);
+    lo[r] = __int_as_float(int(b));
+    hi[r] = __int_as_float(int(b >> 32));
+  }
+  transpose_words<B>(lo);
+  transpose_words<B>(hi);
+#pragma unroll
+  for (int r = 0; r < B; ++r)
+    v[r] = __longlong_as_double((static_cast<long long>(__float_as_int(hi[r])) << 32) | static_cast<unsigned>(__float_as_int(lo[r])));
+}
+
+template <int B, typename R>
+__device__ __forceinline__ void transpose_rows(cx<R>* a) {
+  R x[B], y[B];
 #pragma unroll
   for (int r = 0; r < B; ++r) { x[r] = a[r].x; y[r] = a[r].y; }
   transpose_words<B>(x);
   transpose_words<B>(y);
 #pragma unroll
-  for (int r = 0; r < B; ++r) a[r] = mk<float>(x[r], y[r]);
+  for (int r = 0; r < B; ++r) a[r] = mk<R>(x[r], y[r]);
 }
 
 template <int N, int N2, int SIGN, typename C, typename LIDX>

@@ -232,8 +232,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && ZB == 8 && NX / split_of<NX
   }
 }
 
-#if WFS_SLAB_PREC == 0
-// The complex64 x launch.  A block owns the B rows of one ka over 64 / B z points (64, 128 or 256 bytes of a
+// The complex64 x launch (and complex128 at 192^2).  A block owns the B rows of one ka over 64 / B z points (64, 128 or 256 bytes of a
 // row) and all x; lane q 64 / B + z of every wavefront holds row b = q at x = t + N2 i, t the wavefront's
 // index, so that the x transforms' twiddles and the kinetic factors are the same in all lanes and come
 // through the scalar cache.  For the y stage the B rows are brought into one lane (transpose_rows, B x
@@ -249,9 +248,9 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && ZB == 8 && NX / split_of<NX
 //   688), 256 x 512^2 317 -> 233, 64 x 512^2 46 -> 50; 400 us of arithmetic beside one block's waits.  Lanes along
 //   x instead of the rows at the loads save a transposition and lose more to eight pages a load: 692 us.
 // N: the sides of square planes at compile time, or 0 (256^3 49.3 us, with sides at run time 52).
-template <int NX, int B, int N>
+template <typename R, int NX, int B, int N>
 __global__ __launch_bounds__(64 * split_of<NX>::n2)
-__attribute__((amdgpu_waves_per_eu(NX == 256 && B >= 4 ? 8 : 1))) void x_rows_kernel(cx<float>* __restrict__ data,
+__attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && NX == 256 && B >= 4 ? 8 : 1))) void x_rows_kernel(cx<R>* __restrict__ data,
                                                                         const XSlabParams p) {
   constexpr int ZB = 64 / B;
   // B = 1: 64 consecutive points of the plane, taken as one row
@@ -260,9 +259,9 @@ __attribute__((amdgpu_waves_per_eu(NX == 256 && B >= 4 ? 8 : 1))) void x_rows_ke
   const unsigned A = NY / B, TZ = NZ / ZB;
   constexpr int N2 = split_of<NX>::n2, N1 = NX / N2;
   static_assert(N1 % B == 0, "bad split of the x line");
-  using C = cx<float>;
+  using C = cx<R>;
   using CC = const __attribute__((address_space(4))) C;
-  __shared__ float lds[64 * NX];
+  __shared__ R lds[64 * NX];
 
   const int lane = threadIdx.x & 63;
   const int t = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -285,15 +284,15 @@ __attribute__((amdgpu_waves_per_eu(NX == 256 && B >= 4 ? 8 : 1))) void x_rows_ke
   // forward y stage X[kb] = sum_b W_B^{b kb} W_N^{b ka} Y[b] on B x points at a time
 #pragma unroll
   for (int g = 0; g < (B > 1 ? N1 : 0); g += B) {
-    transpose_rows<B>(a + g);
+    transpose_rows<B, R>(a + g);
     C r[B];
     r[0] = a[g];
 #pragma unroll
-    for (int b = 1; b < B; ++b) r[b] = cmul(a[g + b], mk<float>(twy[b * ka].x, twy[b * ka].y));
+    for (int b = 1; b < B; ++b) r[b] = cmul(a[g + b], mk<R>(twy[b * ka].x, twy[b * ka].y));
     DFT<B, -1>::run(r);
 #pragma unroll
     for (int b = 0; b < B; ++b) a[g + b] = r[b];
-    transpose_rows<B>(a + g);
+    transpose_rows<B, R>(a + g);
   }
   CC* twx = (CC*)(p.tw_x);
   auto lidx = [&](int k1, int n2) { return (k1 * N2 + n2) * 64 + lane; };
@@ -302,7 +301,7 @@ __attribute__((amdgpu_waves_per_eu(NX == 256 && B >= 4 ? 8 : 1))) void x_rows_ke
     DFT<N1, SG>::run(a);
 #pragma unroll
     for (int k1 = 1; k1 < N1; ++k1) {
-      const C w = mk<float>(twx[(t * k1) % NX].x, twx[(t * k1) % NX].y);
+      const C w = mk<R>(twx[(t * k1) % NX].x, twx[(t * k1) % NX].y);
       a[k1] = SG < 0 ? cmul(a[k1], w) : cmulc(a[k1], w);
     }
     column_dft_second_parts<NX, N2, SG>(a, lds, t, lidx);
@@ -315,7 +314,7 @@ __attribute__((amdgpu_waves_per_eu(NX == 256 && B >= 4 ? 8 : 1))) void x_rows_ke
     const C kyz = cmul(reinterpret_cast<const C*>(p.ky)[y], reinterpret_cast<const C*>(p.kz)[z]);
     CC* kx = (CC*)(p.kx) + t;
 #pragma unroll
-    for (int i = 0; i < N1; ++i) a[i] = cmul(a[i], cmul(mk<float>(kx[N2 * i].x, kx[N2 * i].y), kyz));
+    for (int i = 0; i < N1; ++i) a[i] = cmul(a[i], cmul(mk<R>(kx[N2 * i].x, kx[N2 * i].y), kyz));
   }
   __syncthreads();
   transform_x(std::integral_constant<int, +1>{});
@@ -325,21 +324,20 @@ __attribute__((amdgpu_waves_per_eu(NX == 256 && B >= 4 ? 8 : 1))) void x_rows_ke
 #pragma unroll
   for (int g = 0; g < N1; g += B) {
     if constexpr (B > 1) {
-      transpose_rows<B>(a + g);
+      transpose_rows<B, R>(a + g);
       C r[B];
 #pragma unroll
       for (int b = 0; b < B; ++b) r[b] = a[g + b];
       DFT<B, +1>::run(r);
       a[g] = r[0];
 #pragma unroll
-      for (int b = 1; b < B; ++b) a[g + b] = cmulc(r[b], mk<float>(twy[b * ka].x, twy[b * ka].y));
-      transpose_rows<B>(a + g);
+      for (int b = 1; b < B; ++b) a[g + b] = cmulc(r[b], mk<R>(twy[b * ka].x, twy[b * ka].y));
+      transpose_rows<B, R>(a + g);
     }
 #pragma unroll
     for (int i = g; i < g + B; ++i) byte_at(blk, off(l, i)) = a[i];
   }
 }
-#endif
 
 #if WFS_SLAB_PREC == 0
 // flags[p] = 1 when x plane p equals plane p - 1 of the same packet bit for bit, else 0
@@ -509,7 +507,6 @@ int launch_x_slab_ny(int nx, void* data, const XSlabParams& p, hipStream_t s) {
 #undef WFS_X_SLAB_CASE
 }
 
-#if WFS_SLAB_PREC == 0
 // x_rows_kernel's N^2 / 64 blocks a packet fill the card from 1.5 of them a CU on; below that the smaller blocks
 // of x_slab_kernel are the faster ones or level.  us per launch, lane pairs against rows: 256 x 128^2 (256
 // blocks a packet) 17.0 / 16.7, 2 packets 27.9 / 26.2; 128^3 11.4 / 11.8, 2 packets 14.6 / 14.1, 4 packets 25.5 /
@@ -517,14 +514,14 @@ int launch_x_slab_ny(int nx, void* data, const XSlabParams& p, hipStream_t s) {
 // 9.7 / 10.4, 14.0 / 15.3.  192^2 and 256^2 planes have 576 and 1024 blocks a packet.
 bool x_rows_fill(int n, long packets) { return packets * (long(n) * n / 64) * 2 >= 3L * cu_count(); }
 
-template <int B, int N = 0>
+template <typename R, int B, int N = 0>
 int launch_x_rows(int nx, void* data, const XSlabParams& p, hipStream_t s) {
   const unsigned blocks = unsigned(p.packets * (long(p.ny) * p.nz / 64));
 #define WFS_X_ROWS_CASE(NX)                                                                                  \
   case NX:                                                                                                   \
-    if constexpr ((NX / split_of<NX>::n2) % B == 0 && (N == 0 || NX <= 256)) {                                                    \
-      WFS_LAUNCH((x_rows_kernel<NX, B, N>), dim3(blocks), dim3(64 * split_of<NX>::n2), 0, s,                     \
-                 reinterpret_cast<cx<float>*>(data), p);                                                     \
+    if constexpr ((NX / split_of<NX>::n2) % B == 0 && (NX <= 256 || (N == 0 && sizeof(R) == 4))) {                                                    \
+      WFS_LAUNCH((x_rows_kernel<R, NX, B, N>), dim3(blocks), dim3(64 * split_of<NX>::n2), 0, s,                     \
+                 reinterpret_cast<cx<R>*>(data), p);                                                         \
       return int(hipGetLastError());                                                                         \
     }                                                                                                        \
     break;
@@ -544,7 +541,6 @@ int launch_x_rows(int nx, void* data, const XSlabParams& p, hipStream_t s) {
   set_last_error("slab x pass: unsupported length %d", nx);
   return WFS_ERR_UNSUPPORTED;
 }
-#endif
 
 template <typename R, int N>
 SlabRows slab_rows_n() {
@@ -662,17 +658,17 @@ int launch_x_slab(int precision, const int nn[3], void* data, const XSlabParams&
   }
   if (nn[1] != nn[2]) {
     const int b = rect_rows(nn[1], nn[2]).b;
-    return b == 1   ? launch_x_rows<1>(nx, data, p, s)
-           : b == 2 ? launch_x_rows<2>(nx, data, p, s)
-           : b == 4 ? launch_x_rows<4>(nx, data, p, s) : launch_x_rows<8>(nx, data, p, s);
+    return b == 1   ? launch_x_rows<float, 1>(nx, data, p, s)
+           : b == 2 ? launch_x_rows<float, 2>(nx, data, p, s)
+           : b == 4 ? launch_x_rows<float, 4>(nx, data, p, s) : launch_x_rows<float, 8>(nx, data, p, s);
   }
   if (precision == WFS_C128) return launch_x_slab_c128(nx, n, data, p, s);
-  if (n == 512) return launch_x_rows<8>(nx, data, p, s);
-  if (n == 256) return nx <= 256 ? launch_x_rows<4, 256>(nx, data, p, s) : launch_x_rows<4>(nx, data, p, s);
-  if (n == 192) return nx <= 256 ? launch_x_rows<4, 192>(nx, data, p, s) : launch_x_rows<4>(nx, data, p, s);
+  if (n == 512) return launch_x_rows<float, 8>(nx, data, p, s);
+  if (n == 256) return nx <= 256 ? launch_x_rows<float, 4, 256>(nx, data, p, s) : launch_x_rows<float, 4>(nx, data, p, s);
+  if (n == 192) return nx <= 256 ? launch_x_rows<float, 4, 192>(nx, data, p, s) : launch_x_rows<float, 4>(nx, data, p, s);
   const bool rows = nx == 512 || x_rows_fill(n, p.packets);
-  if (n == 128) return rows ? launch_x_rows<2>(nx, data, p, s) : launch_x_slab_ny<float, 128>(nx, data, p, s);
-  if (n == 96) return rows ? launch_x_rows<2>(nx, data, p, s) : launch_x_slab_ny<float, 96>(nx, data, p, s);
+  if (n == 128) return rows ? launch_x_rows<float, 2>(nx, data, p, s) : launch_x_slab_ny<float, 128>(nx, data, p, s);
+  if (n == 96) return rows ? launch_x_rows<float, 2>(nx, data, p, s) : launch_x_slab_ny<float, 96>(nx, data, p, s);
   set_last_error("slab x pass: unsupported plane %d", n);
   return WFS_ERR_UNSUPPORTED;
 }
@@ -695,7 +691,12 @@ int launch_x_slab_c128(int nx, int n, void* data, const XSlabParams& p, hipStrea
   if (n == 64) return launch_x_slab_ny<double, 64>(nx, data, p, s);
   if (n == 96) return launch_x_slab_ny<double, 96>(nx, data, p, s);
   if (n == 128) return launch_x_slab_ny<double, 128>(nx, data, p, s);
-  if (n == 192) return launch_x_slab_ny<double, 192>(nx, data, p, s);
+  // 192^2 (B = 4: a lane pair holds two rows a lane): rows in one lane, but for 128 and 256 x planes (16 points
+  // a lane), us per launch lane pairs / rows: nx = 192 79 / 67, 96 47 / 26, 64 16.8 / 15.9, 32 15.0 / 12.5, 8 6.5 / 4.9, 3
+  // packets of 96 107 / 65; 128 32.4 / 34.2, 256 63 / 76.  B = 2 planes stay with lane pairs: 64^3 5.5 / 6.8, 128^3
+  // 15.4 / 16.2, 96^3 15.1 / 17.1 (6 packets 44 / 37).
+  if (n == 192)
+    return nx % 128 ? launch_x_rows<double, 4, 192>(nx, data, p, s) : launch_x_slab_ny<double, 192>(nx, data, p, s);
   set_last_error("slab x pass: unsupported complex128 plane %d", n);
   return WFS_ERR_UNSUPPORTED;
 }

@@ -264,7 +264,7 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lin
         C b[N2Y];
 #pragma unroll
         for (int r = 0; r < N2Y; ++r) b[r] = a[0][N2Y * m + r];
-        transpose_rows<N2Y>(b);
+        transpose_rows<N2Y, R>(b);
         DFT<N2Y, SG>::run(b);
 #pragma unroll
         for (int k2 = 0; k2 < N2Y; ++k2) o[m + M * k2] = b[k2];
