@@ -420,12 +420,12 @@ int cu_count() {
   return n;
 }
 
-template <typename R, int N, int MODE, int PARTS = 0>
+template <typename R, int N, int MODE, int PARTS = 0, int PV = PV_ANY>
 int launch_lines_m(void* data, const YzPlaneParams& p, hipStream_t s) {
   constexpr int LY = SlabShape<R, N>::LY, B = SlabShape<R, N>::B;
   static_assert(yz_lines_lds_bytes<R, N, LY, B, 1, PARTS>() <= 160 * 1024, "rows do not fit in LDS");
   const long groups = p.planes * B;
-  WFS_LAUNCH((yz_lines_kernel<R, N, LY, B, 1, MODE, true, PARTS>), dim3(unsigned(groups)),
+  WFS_LAUNCH((yz_lines_kernel<R, N, LY, B, 1, MODE, true, PARTS, PV>), dim3(unsigned(groups)),
                      dim3(yz_lines_threads<N, LY, 1>()), 0, s, reinterpret_cast<cx<R>*>(data), p);
   return int(hipGetLastError());
 }
@@ -437,7 +437,7 @@ int launch_lines_m(void* data, const YzPlaneParams& p, hipStream_t s) {
 // the transforms no longer wait for the factor loads hoisted over them.  Not for complex128 (128^3 27.3 ->
 // 28.6, 192^3 80.3 -> 85.6, 96^3 17.2 -> 18.3 us: its 3 and more exchanges cost what the second block
 // gains) nor for complex64 128^2 planes (19.0 -> 19.3).  512^2: the only form that fits, 131 KB of LDS and 128
-// registers a block of 1024 threads; 512^3 748 us a full launch (3.3 GB: 4.4 TB/s), 465 an entry or exit.
+// registers a block of 1024 threads; 512^3 701 us a full launch (3.3 GB: 4.7 TB/s), 465 an entry or exit.
 template <typename R, int N> constexpr int lines_parts() { return sizeof(R) == 8 ? 0 : N == 512 ? 4 : N == 256 ? 8 : N == 192 ? 3 : 0; }
 
 // The parts form is taken where the groups are more than the CUs.  us of the full / entry or exit launch,
@@ -457,7 +457,9 @@ int launch_lines_n(int mode, void* data, const YzPlaneParams& p, hipStream_t s) 
   if constexpr (lines_parts<R, N>() != 0) {
     constexpr int W = lines_parts<R, N>();
     if (lines_in_parts<R, N>(p.planes)) {
-      if (mode == LINES_FULL) return launch_lines_m<R, N, LINES_FULL, W>(data, p, s);
+      if (mode == LINES_FULL)
+        return p.spx ? launch_lines_m<R, N, LINES_FULL, W, PV_AXES>(data, p, s)
+                     : launch_lines_m<R, N, LINES_FULL, W, PV_TABLE>(data, p, s);
       if (mode == LINES_ENTRY) return launch_lines_m<R, N, LINES_ENTRY, W>(data, p, s);
       if (mode == LINES_EXIT) return launch_lines_m<R, N, LINES_EXIT, W>(data, p, s);
     }
@@ -593,7 +595,7 @@ bool slab_supported(int precision, const int n[3]) {
 // 45 / 44, and the tuned 64^2 forms are bit for bit the axis passes.
 //
 // complex64 512^2 planes (B = 8, x_rows_kernel), us per step with a potential table against the four axis
-// passes: 512^3 2407 -> 1412, 256 x 512^2 1158 -> 798, 64 x 512^2 230 -> 182.  Its x launch takes 8 x points
+// passes: 512^3 2407 -> 1367, 256 x 512^2 1158 -> 798, 64 x 512^2 230 -> 182.  Its x launch takes 8 x points
 // of a lane at a time, so nx = 8 and 16 (4 points a lane) stay with the passes.
 //
 // complex64 with 512 x planes (x_rows_kernel alone takes them): 512 x 96^2 75 / 69 -> 56 / 55, x 128^2 87 / 81 -> 81 /

@@ -145,16 +145,23 @@ constexpr long yz_lines_lds_bytes() {
   return long(LY / H) * yz_lines_stride<R, NZ, LY, B, H, PARTS>() * long(PARTS ? sizeof(R) : sizeof(cx<R>));
 }
 
+// How LINES_FULL gets the potential factors: by the parameters (spx set or not), or fixed at compile time, which
+// frees the registers that the other form would hold.  The PARTS launches fix it (256^2: 56 and 63 registers
+// instead of 64 and 5 spilled, 20 of a launch's 320 MB written; 192^2 94 and 106 instead of 127): us per launch with a
+// table / with per-axis factors 512^3 744 / 730 -> 701 / 615, 3 x 192^3 121 / 103 -> 111 / 102, 256^3 77 / 73 -> 76 / 67
+// (66 with repeated planes).  Whole launches gain nothing by it (128^3 complex128 25 -> 28).
+enum { PV_ANY, PV_TABLE, PV_AXES };
+
 // PV_LINES: the potential table is in lines order (LinesOrder, wfs_internal.h), read as one
 // contiguous run per wavefront, and the twiddle tables hold each thread's twiddles
 // contiguously ([u][k1], u the thread's index within a line); else the potential table is
 // in the state's C order and the twiddles come from the length-N axis tables.
 // PARTS != 0: the exchanges pass the real parts, then the imaginary parts, through half the LDS, and PARTS
 // waves per SIMD bound the registers (four potential factors in flight instead of sixteen), so that two
-// 1024-thread blocks share a CU at 256^2: 256 planes 85 -> 76 us (4.2 -> 4.7 TB/s with the table), entry and
+// 1024-thread blocks share a CU at 256^2: 256 planes 85 -> 76 us (5.3 TB/s with the table), entry and
 // exit 57 -> 49 (5.5 TB/s).  What bounds it then is memory, and in the full launch the barriers (20 against 8).
 template <typename R, int NZ, int LY, int B, int H, int MODE, bool PV_LINES = false,
-          int PARTS = 0>
+          int PARTS = 0, int PV = PV_ANY>
 __global__ __launch_bounds__((yz_lines_threads<NZ, LY, H>()))
 __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lines_kernel(cx<R>* __restrict__ data,
                                                                            const YzPlaneParams p) {
@@ -398,7 +405,7 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lin
 #pragma unroll
           for (int i = 0; i < N1; ++i) settle(a[r][i]);
         }
-        if (p.spx) {
+        if (PV == PV_ANY ? p.spx != nullptr : PV == PV_AXES) {
           const long pk = plane / p.nx;
           const C* __restrict__ px = reinterpret_cast<const C*>(p.spx);
           const C* __restrict__ py = reinterpret_cast<const C*>(p.spy) + pk * NY;
