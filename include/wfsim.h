@@ -469,6 +469,18 @@ int wfs_fno_weight_grad(const float* g, const float* v, float* gW, float* gb, in
                         long work_elems, void* stream);
 int wfs_fno_modes_backward(const float* Rr, const float* Ri, const float* X, const float* dO, float* dX, float* gRr,
                            float* gRi, int m3, int C, void* stream);
+/*
+ * wfs_fno_spectral (no reference counterpart): a layer's spectral path between its z stages, in five
+ * launches: wfs_fno_stage along y and x with the table F2 [2m][2n], wfs_fno_modes, wfs_fno_stage along x
+ * and y with G2 [2n][2m].  T and Z [C][n^2][2m], U [C][n][2m][m], X and O [C][2][m^3], Y [C][2n][m^2],
+ * 2m <= 32.  U, X, O and Y are written too.  wfs_fno_spectral_backward is its transposition (tables G2t
+ * [2m][2n], F2t [2n][2m], X the layer's modes; Zg may be Tg); gRr, gRi are accumulated, C <= 256.
+ */
+int wfs_fno_spectral(const void* F2, const void* G2, const float* Rr, const float* Ri, const float* T, float* U,
+                     float* X, float* O, float* Y, float* Z, int n, int m, int C, void* stream);
+int wfs_fno_spectral_backward(const void* G2t, const void* F2t, const float* Rr, const float* Ri, const float* X,
+                              const float* Tg, float* Y, float* O, float* dX, float* U, float* Zg, float* gRr,
+                              float* gRi, int n, int m, int C, void* stream);
 int wfs_fno_gelu_backward(const float* u, const float* dv, float* du, long n, void* stream);
 /*
  * wfs_spectral_resample (no reference counterpart): the spectrum of an ndst grid from that of

@@ -59,6 +59,8 @@ SIGNATURES = {
     "wfs_fno_stage": (ctypes.c_int, [_vp] * 3 + [ctypes.c_int] * 3 + [ctypes.c_long, _vp]),
     "wfs_fno_weight_grad": (ctypes.c_int, [_vp] * 4 + [ctypes.c_int] * 2 + [ctypes.c_long, _vp, ctypes.c_long, _vp]),
     "wfs_fno_modes_backward": (ctypes.c_int, [_vp] * 7 + [ctypes.c_int] * 2 + [_vp]),
+    "wfs_fno_spectral": (ctypes.c_int, [_vp] * 10 + [ctypes.c_int] * 3 + [_vp]),
+    "wfs_fno_spectral_backward": (ctypes.c_int, [_vp] * 13 + [ctypes.c_int] * 3 + [_vp]),
     "wfs_fno_pack": (ctypes.c_int, [_vp, ctypes.c_int, _vp, ctypes.c_float, ctypes.c_float, _vp, ctypes.c_long,
                                     _vp]),
     "wfs_fno_unpack": (ctypes.c_int, [_vp, ctypes.c_float, _vp, ctypes.c_long, _vp]),
@@ -533,8 +535,9 @@ def _check_f32(tensors) -> None:
     for t, size, name in tensors:
         if t is None:
             continue
-        _require_device_any(t, name)
-        if t.dtype != torch.float32 or not t.is_contiguous() or t.numel() < size:
+        if not isinstance(t, torch.Tensor) or not t.is_cuda:
+            raise ValueError(f"{name} must be a device tensor")
+        if t.dtype is not torch.float32 or not t.is_contiguous() or t.numel() < size:
             raise ValueError(f"{name} must be a contiguous float32 tensor of at least {size} elements")
 
 
@@ -583,6 +586,40 @@ def fno_layer_backward(W: torch.Tensor, g: torch.Tensor, Tg: torch.Tensor | None
                                        ptr(u) if u is not None else None, ptr(Gz), ptr(Fz), ptr(gn),
                                        ptr(Tn) if Tn is not None else None, int(cin), int(C), int(n), int(tm),
                                        stream_handle(stream)), "wfs_fno_layer_backward")
+
+
+def _stage_tables(tables) -> None:
+    """(name, table, rows, columns) of the padded bf16 tables of fno_stage_table."""
+    for name, A, M, K in tables:
+        if (not isinstance(A, torch.Tensor) or not A.is_cuda or A.dtype is not torch.bfloat16
+                or not A.is_contiguous() or tuple(A.shape) != (-(-M // 32) * 32, -(-K // 16) * 16)):
+            raise ValueError(f"{name} must be the padded bf16 table of a {M} x {K} stage")
+
+
+def fno_spectral(F2: torch.Tensor, G2: torch.Tensor, Rr: torch.Tensor, Ri: torch.Tensor, T: torch.Tensor,
+                 U: torch.Tensor, X: torch.Tensor, O: torch.Tensor, Y: torch.Tensor, Z: torch.Tensor, n: int, m: int,
+                 C: int, stream=None) -> None:
+    """A layer's spectral path between its z stages, T -> Z (``wfs_fno_spectral``)."""
+    _stage_tables((("F2", F2, 2 * m, 2 * n), ("G2", G2, 2 * n, 2 * m)))
+    zs, xs, ms, w = C * n * n * 2 * m, 2 * C * n * m * m, 2 * C * m ** 3, m ** 3 * C * C
+    _check_f32([(Rr, w, "Rr"), (Ri, w, "Ri"), (T, zs, "T"), (U, xs, "U"), (X, ms, "X"), (O, ms, "O"), (Y, xs, "Y"),
+                (Z, zs, "Z")])
+    check(lib().wfs_fno_spectral(ptr(F2), ptr(G2), ptr(Rr), ptr(Ri), ptr(T), ptr(U), ptr(X), ptr(O), ptr(Y), ptr(Z),
+                                 int(n), int(m), int(C), stream_handle(stream)), "wfs_fno_spectral")
+
+
+def fno_spectral_backward(G2t: torch.Tensor, F2t: torch.Tensor, Rr: torch.Tensor, Ri: torch.Tensor, X: torch.Tensor,
+                          Tg: torch.Tensor, Y: torch.Tensor, O: torch.Tensor, dX: torch.Tensor, U: torch.Tensor,
+                          Zg: torch.Tensor, gRr: torch.Tensor, gRi: torch.Tensor, n: int, m: int, C: int,
+                          stream=None) -> None:
+    """The transposition of fno_spectral, Tg -> Zg; gRr, gRi accumulated (``wfs_fno_spectral_backward``)."""
+    _stage_tables((("G2t", G2t, 2 * m, 2 * n), ("F2t", F2t, 2 * n, 2 * m)))
+    zs, xs, ms, w = C * n * n * 2 * m, 2 * C * n * m * m, 2 * C * m ** 3, m ** 3 * C * C
+    _check_f32([(Rr, w, "Rr"), (Ri, w, "Ri"), (X, ms, "X"), (Tg, zs, "Tg"), (Y, xs, "Y"), (O, ms, "O"), (dX, ms, "dX"),
+                (U, xs, "U"), (Zg, zs, "Zg"), (gRr, w, "gRr"), (gRi, w, "gRi")])
+    check(lib().wfs_fno_spectral_backward(ptr(G2t), ptr(F2t), ptr(Rr), ptr(Ri), ptr(X), ptr(Tg), ptr(Y), ptr(O),
+                                          ptr(dX), ptr(U), ptr(Zg), ptr(gRr), ptr(gRi), int(n), int(m), int(C),
+                                          stream_handle(stream)), "wfs_fno_spectral_backward")
 
 
 # floats wfs_fno_weight_grad may need in its workspace (512 records of a 32 x 32 tile and 32 sums)

@@ -1111,6 +1111,31 @@ extern "C" int wfs_fno_modes_backward(const float* Rr, const float* Ri, const fl
   return 0;
 }
 
+// The spectral path between the z stages, T -> Z, in one call: its five launches are 4 to 10 us each, and
+// called one by one from Python they cost more host time than that (32^3, width 32, 12 modes, 4 layers:
+// 246 -> 153 us a forward, 750 -> 470 a training sample with the gradients cleared in one launch).
+extern "C" int wfs_fno_spectral(const void* F2, const void* G2, const float* Rr, const float* Ri, const float* T,
+                                float* U, float* X, float* O, float* Y, float* Z, int n, int m, int C, void* stream) {
+  const int m2 = m * m;
+  if (int rc = wfs_fno_stage(F2, T, U, 2 * m, 2 * n, m, long(C) * n, stream)) return rc;
+  if (int rc = wfs_fno_stage(F2, U, X, 2 * m, 2 * n, m2, C, stream)) return rc;
+  if (int rc = wfs_fno_modes(Rr, Ri, X, O, m2 * m, C, stream)) return rc;
+  if (int rc = wfs_fno_stage(G2, O, Y, 2 * n, 2 * m, m2, C, stream)) return rc;
+  return wfs_fno_stage(G2, Y, Z, 2 * n, 2 * m, m, long(C) * n, stream);
+}
+
+// its transposition, Tg -> Zg (Zg may be Tg): G2t and F2t are the transposed tables
+extern "C" int wfs_fno_spectral_backward(const void* G2t, const void* F2t, const float* Rr, const float* Ri,
+                                         const float* X, const float* Tg, float* Y, float* O, float* dX, float* U,
+                                         float* Zg, float* gRr, float* gRi, int n, int m, int C, void* stream) {
+  const int m2 = m * m;
+  if (int rc = wfs_fno_stage(G2t, Tg, Y, 2 * m, 2 * n, m, long(C) * n, stream)) return rc;
+  if (int rc = wfs_fno_stage(G2t, Y, O, 2 * m, 2 * n, m2, C, stream)) return rc;
+  if (int rc = wfs_fno_modes_backward(Rr, Ri, X, O, dX, gRr, gRi, m2 * m, C, stream)) return rc;
+  if (int rc = wfs_fno_stage(F2t, dX, U, 2 * n, 2 * m, m2, C, stream)) return rc;
+  return wfs_fno_stage(F2t, U, Zg, 2 * n, 2 * m, m, long(C) * n, stream);
+}
+
 template <int WM, int WN>
 static void launch_tile(dim3 grid, hipStream_t s, const GemmArgs& g) {
   switch (g.flags & 3) {
