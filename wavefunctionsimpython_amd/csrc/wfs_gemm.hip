@@ -278,6 +278,16 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(GemmArgs g) {
 // At 64^3, C = 32: 47 us, against 150 us for the four launches it replaces (27 + 27 us for the two
 // GEMMs that write W^T g and add the spectral term, 23 for GELU', 73 for the z stage).
 //
+// Wavefronts in flight: the kernel waits for memory, so it is held to 128 registers, four wavefronts per
+// SIMD, where that goes without spills that cost more.  The next chunk's loads then go into the registers
+// of the chunk that the matrix cores have just taken (ONE_BUF), the chunk loop is unrolled (rolled, its
+// addresses spill 12 to 21 registers), and n <= 64, whose 1024 (64^3) blocks of a line per wavefront were
+// 1.33 rounds at three per SIMD, loses the loop over lines (ONE_LINE).  us, three per SIMD with two buffers
+// against this: 64^3 forward 253 -> 226 and a training sample 805 -> 727 (C = 32, 4 layers), 128^3 forward
+// 981 -> 973, with C = 16 and 16 modes 628 -> 595, 96^3 with C = 24 285 -> 274.  Three per SIMD and two
+// buffers stay at n >= 96 for channel counts that are no multiple of four (every row has its own address) and
+// for the backward form (a training sample at 128^3 3520 us, 3587 at four; 96^3 815 and 847).
+//
 // LAYER_LAST: the last layer with the projection, out = base + rscale (Q u + qb) for one or two
 // rows (Q bf16 as in the GEMM, u FP32): the lanes sum their half of the channels of one z from the
 // chunk's LDS tile.  Without it the layer wrote u and a GEMM with 2 useful rows of 32 and an
@@ -315,9 +325,15 @@ __device__ __forceinline__ void split4(const float (&x)[4], bf16x4& hi, bf16x4& 
   }
 }
 
+// whether a layer kernel runs four wavefronts per SIMD (above)
 template <int NZC, int MODE, bool QUADS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void fno_layer_kernel(LayerArgs g) {
+constexpr bool layer_four() { return NZC <= 2 || (QUADS && MODE != LAYER_BACKWARD); }
+
+template <int NZC, int MODE, bool QUADS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(layer_four<NZC, MODE, QUADS>() ? 4 : 3))) void fno_layer_kernel(LayerArgs g) {
   constexpr bool BWD = MODE == LAYER_BACKWARD;
+  constexpr bool ONE_LINE = NZC <= 2;                // the grid then has a wavefront per line
+  constexpr bool ONE_BUF = layer_four<NZC, MODE, QUADS>();   // the next chunk's loads reuse this chunk's registers
   constexpr int n = 32 * NZC;
   constexpr int GP = kBK + 4;                        // padded rows of the transform tables
   __shared__ unsigned short GzT[n][GP];              // A = Gz^T: [z][j]
@@ -449,6 +465,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
     for (int i = 0; i < 16; ++i) accT[i] = 0.0f;
     const unsigned line = ru * n;
     const long rnext = r + stride;
+    // the chunk after ch: this line's ch + 1, or the next line's first
+    auto prefetch = [&](int ch, float (&x)[16]) {
+      if (ch + 1 < NZC) load_v(ru, ch + 1, x);
+      else if (!ONE_LINE && rnext < rows) load_v(unsigned(rnext), 0, x);
+    };
     // chunk ch of this line from x (its loads were issued one chunk earlier)
     auto process = [&](int ch, float (&x)[16]) {
       float4 up[4];
@@ -473,6 +494,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
           acc = mfma16(cat8(ah0, ah1), w, acc);
         }
       }
+      if constexpr (ONE_BUF) prefetch(ch, x);
 #pragma unroll
       for (int S = 0; S < 2; ++S) {
         if (2 * S < ktm) {
@@ -566,23 +588,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
         }
       }
     };
-    // the chunk after ch: this line's ch + 1, or the next line's first
-    auto prefetch = [&](int ch, float (&x)[16]) {
-      if (ch + 1 < NZC) load_v(ru, ch + 1, x);
-      else if (rnext < rows) load_v(unsigned(rnext), 0, x);
-    };
-    // chunks in pairs through two buffers, so that no register copy waits for a load in flight
-    float xw[16];
-#pragma unroll 1
-    for (int ch = 0; ch < NZC; ch += 2) {
-      prefetch(ch, xw);
-      process(ch, xv);
-      if (ch + 1 < NZC) {
-        prefetch(ch + 1, xv);
-        process(ch + 1, xw);
-      } else {
+    if constexpr (ONE_BUF) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) xv[i] = xw[i];   // odd chunk count: next line's first chunk
+      for (int ch = 0; ch < NZC; ++ch) process(ch, xv);
+    } else {
+      // chunks in pairs through two buffers, so that no register copy waits for a load in flight
+      float xw[16];
+#pragma unroll 1
+      for (int ch = 0; ch < NZC; ch += 2) {
+        prefetch(ch, xw);
+        process(ch, xv);
+        if (ch + 1 < NZC) {
+          prefetch(ch + 1, xv);
+          process(ch + 1, xw);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) xv[i] = xw[i];   // odd chunk count: next line's first chunk
+        }
       }
     }
     if (tb && lc < tm) {
@@ -594,6 +616,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
           *reinterpret_cast<float*>(tb + ((unsigned(c) * unsigned(rows) + ru) * unsigned(tm) + lc) * 4u) = accT[i];
       }
     }
+    if constexpr (ONE_LINE) break;
   }
 }
 
@@ -960,7 +983,7 @@ extern "C" int wfs_fno_modes(const float* Rr, const float* Ri, const float* X, f
 template <int MODE>
 static void launch_layer(const LayerArgs& g, int n, hipStream_t s) {
   const long want = (g.rows + 3) / 4;
-  const unsigned blocks = unsigned(want < 2048 ? want : 2048);
+  const unsigned blocks = unsigned(want < 2048 ? want : 2048);   // all lines at n <= 64 (ONE_LINE): 1024 blocks at most
 #define WFS_LAYER(NZC)                                                                                    \
   if (g.cin % 4 == 0) hipLaunchKernelGGL((fno_layer_kernel<NZC, MODE, true>), dim3(blocks), dim3(256), 0, s, g); \
   else hipLaunchKernelGGL((fno_layer_kernel<NZC, MODE, false>), dim3(blocks), dim3(256), 0, s, g);
