@@ -278,15 +278,15 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(GemmArgs g) {
 // At 64^3, C = 32: 47 us, against 150 us for the four launches it replaces (27 + 27 us for the two
 // GEMMs that write W^T g and add the spectral term, 23 for GELU', 73 for the z stage).
 //
-// Wavefronts in flight: the kernel waits for memory, so it is held to 128 registers, four wavefronts per
-// SIMD, where that goes without spills that cost more.  The next chunk's loads then go into the registers
-// of the chunk that the matrix cores have just taken (ONE_BUF), the chunk loop is unrolled (rolled, its
-// addresses spill 12 to 21 registers), and n <= 64, whose 1024 (64^3) blocks of a line per wavefront were
-// 1.33 rounds at three per SIMD, loses the loop over lines (ONE_LINE).  us, three per SIMD with two buffers
-// against this: 64^3 forward 253 -> 226 and a training sample 805 -> 727 (C = 32, 4 layers), 128^3 forward
-// 981 -> 973, with C = 16 and 16 modes 628 -> 595, 96^3 with C = 24 285 -> 274.  Three per SIMD and two
-// buffers stay at n >= 96 for channel counts that are no multiple of four (every row has its own address) and
-// for the backward form (a training sample at 128^3 3520 us, 3587 at four; 96^3 815 and 847).
+// Wavefronts in flight: the kernel waits for memory.  n <= 64 has at most 4096 lines, one a wavefront (ONE_LINE):
+// its next chunk's loads go into the registers of the chunk that the matrix cores have just taken, and the
+// unrolled chunk loop (rolled, its addresses spill 12 to 21 registers) holds 128 registers at most, four
+// wavefronts per SIMD; at three, 64^3 was 1.33 rounds of the card: 64^3 forward 253 -> 226 us, a training sample
+// 805 -> 727 (C = 32, 4 layers).  Larger n keeps three (four spill: a training sample at 128^3 3415 -> 3512 us) and
+// two chunk buffers, and its blocks, as many as fit the card at once (kLayerBlocks), walk the lines: the
+// tables are staged once a block and no load waits for a block's start.  us, 2048 blocks against 768: 128^3 forward
+// 981 -> 890 (942 with four wavefronts), C = 16 with 16 modes 628 -> 530, C = 18 506 -> 441, 96^3 with C = 24 285 ->
+// 241, training samples at 128^3 3525 -> 3415, at 96^3 with C = 20 826 -> 770.
 //
 // LAYER_LAST: the last layer with the projection, out = base + rscale (Q u + qb) for one or two
 // rows (Q bf16 as in the GEMM, u FP32): the lanes sum their half of the channels of one z from the
@@ -325,15 +325,10 @@ __device__ __forceinline__ void split4(const float (&x)[4], bf16x4& hi, bf16x4& 
   }
 }
 
-// whether a layer kernel runs four wavefronts per SIMD (above)
 template <int NZC, int MODE, bool QUADS>
-constexpr bool layer_four() { return NZC <= 2 || (QUADS && MODE != LAYER_BACKWARD); }
-
-template <int NZC, int MODE, bool QUADS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(layer_four<NZC, MODE, QUADS>() ? 4 : 3))) void fno_layer_kernel(LayerArgs g) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NZC <= 2 ? 4 : 3))) void fno_layer_kernel(LayerArgs g) {
   constexpr bool BWD = MODE == LAYER_BACKWARD;
-  constexpr bool ONE_LINE = NZC <= 2;                // the grid then has a wavefront per line
-  constexpr bool ONE_BUF = layer_four<NZC, MODE, QUADS>();   // the next chunk's loads reuse this chunk's registers
+  constexpr bool ONE_LINE = NZC <= 2;                // a wavefront per line
   constexpr int n = 32 * NZC;
   constexpr int GP = kBK + 4;                        // padded rows of the transform tables
   __shared__ unsigned short GzT[n][GP];              // A = Gz^T: [z][j]
@@ -494,7 +489,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(layer_four<
           acc = mfma16(cat8(ah0, ah1), w, acc);
         }
       }
-      if constexpr (ONE_BUF) prefetch(ch, x);
+      if constexpr (ONE_LINE) prefetch(ch, x);
 #pragma unroll
       for (int S = 0; S < 2; ++S) {
         if (2 * S < ktm) {
@@ -588,7 +583,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(layer_four<
         }
       }
     };
-    if constexpr (ONE_BUF) {
+    if constexpr (ONE_LINE) {
 #pragma unroll
       for (int ch = 0; ch < NZC; ++ch) process(ch, xv);
     } else {
@@ -979,14 +974,21 @@ extern "C" int wfs_fno_modes(const float* Rr, const float* Ri, const float* X, f
   return 0;
 }
 
-// one wavefront per line, four per block
+constexpr long kLayerBlocks = 3 * 256;   // three blocks of four wavefronts on each of the 256 CUs
+
+// a block takes four lines at a time
+template <int NZC, int MODE, bool QUADS>
+static void launch_layer_form(const LayerArgs& g, hipStream_t s) {
+  const long want = (g.rows + 3) / 4;
+  const unsigned blocks = unsigned(NZC <= 2 || want < kLayerBlocks ? want : kLayerBlocks);   // ONE_LINE: all lines
+  hipLaunchKernelGGL((fno_layer_kernel<NZC, MODE, QUADS>), dim3(blocks), dim3(256), 0, s, g);
+}
+
 template <int MODE>
 static void launch_layer(const LayerArgs& g, int n, hipStream_t s) {
-  const long want = (g.rows + 3) / 4;
-  const unsigned blocks = unsigned(want < 2048 ? want : 2048);   // all lines at n <= 64 (ONE_LINE): 1024 blocks at most
-#define WFS_LAYER(NZC)                                                                                    \
-  if (g.cin % 4 == 0) hipLaunchKernelGGL((fno_layer_kernel<NZC, MODE, true>), dim3(blocks), dim3(256), 0, s, g); \
-  else hipLaunchKernelGGL((fno_layer_kernel<NZC, MODE, false>), dim3(blocks), dim3(256), 0, s, g);
+#define WFS_LAYER(NZC)                                                   \
+  if (g.cin % 4 == 0) launch_layer_form<NZC, MODE, true>(g, s);          \
+  else launch_layer_form<NZC, MODE, false>(g, s);
   switch (n / 32) {
     case 1: WFS_LAYER(1) break;
     case 2: WFS_LAYER(2) break;
