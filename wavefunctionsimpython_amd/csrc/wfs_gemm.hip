@@ -275,7 +275,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(GemmArgs g) {
 // with g in v, T' (the gradient of the layer's z stage) in Z, W stored [cin][C], the two tables
 // exchanged, u in up (null: no factor) and no bias: what the composition writes and reads in
 // between (W^T g, its sum with the spectral term, the product with GELU') stays in registers.
-// At 64^3, C = 32: 47 us, against 150 us for the four launches it replaces (27 + 27 us for the two
+// At 64^3, C = 32: 41 us, against 150 us for the four launches it replaces (27 + 27 us for the two
 // GEMMs that write W^T g and add the spectral term, 23 for GELU', 73 for the z stage).
 //
 // Wavefronts in flight: the kernel waits for memory.  n <= 64 has at most 4096 lines, one a wavefront (ONE_LINE):

@@ -9,14 +9,16 @@ Architecture (channel-major FP32 activations v[c][p], p over the n^3 grid):
 
 DFT_m is the 3-D DFT restricted to the m lowest frequencies per axis,
 f in {0..m/2-1, -m/2..-1}; it is evaluated as three successive contractions
-with small cos/sin tables (z, then y, then x), each one call of the strided
-bf16 GEMM ``wfs_gemm_bf16``; IDFT_m (1/n per axis) likewise in reverse.  The
+with small cos/sin tables (z, then y, then x); IDFT_m (1/n per axis) likewise
+in reverse.  The
 complex spectral weights R_l[q][i][o] mix channels per mode q.  Every weight
-and activation enters the matrix cores as bf16; accumulation is FP32.  The
-backward pass is the same contractions with transposed strides; weight
-gradients use deterministic split-K reductions.  Adam updates FP32 master
-weights.  Only elementwise work (bias, GELU, loss, Adam) runs outside the
-GEMM, in the library's own kernels.
+and activation enters the matrix cores as bf16 (activations as hi + lo parts);
+accumulation is FP32.  Where the sizes allow (``fused``) a layer is one kernel
+over the grid's lines with the z stages in it, ``wfs_fno_layer``, and the
+spectral path between the z stages one call, ``wfs_fno_spectral``; other sizes
+compose strided bf16 GEMMs (``wfs_gemm_bf16``).  The backward pass is the
+transposed layer kernel or the same GEMMs with transposed strides; weight
+gradients sum in a fixed order.  Adam updates FP32 master weights.
 """
 
 from __future__ import annotations
