@@ -38,6 +38,8 @@ struct wfs_plan {
   bool pv_planes_ok;      // pv_planes describes the current pv_lines
   bool pv_in_graph;       // pv_lines was written inside a captured graph: its content changes at
                           // replays the plan does not see, so the plane map is not used again
+  bool pv_planes_held;    // a captured launch took pv_planes: from then on the map is rebuilt with
+                          // every writing of pv_lines, so that its replays find the two in step
   bool pv_set;
   void* tw_rows[2];       // slab scheme: the y and z twiddles of each thread's lines, [ntab][u][k1]
   void* sep[3];           // separable potential: per-axis exp(-i dt f_d), [ntab][batch][n_d]
@@ -351,11 +353,18 @@ int alloc_table(wfs_plan* p, void** t, hipStream_t s) {
 // would read an unwritten map): the captured steps read every plane's own copy, and the next
 // uncaptured call builds it.  Once the table itself has been written inside a captured graph
 // (a potential set or a reorder under capture), every replay may change it behind the map, so
-// from then on the plan reads every plane's own copy.
+// from then on the plan reads every plane's own copy.  A graph that has the map among its launches'
+// arguments goes on reading it whatever the plan decides later: once there is one (pv_planes_held)
+// the map is rebuilt each time the table is written, under capture by launches recorded behind the
+// table's own.
+bool planes_wanted(const wfs_plan* p, hipStream_t s) {
+  return p->variant[WFS_K_PV_PLANES] != 0 && !p->pv_in_graph && !capturing(s);
+}
+
 int share_planes(wfs_plan* p, hipStream_t s) {
   p->pv_planes_ok = false;
-  if (p->variant[WFS_K_PV_PLANES] == 0 || p->pv_in_graph) return 0;
-  if (capturing(s)) return 0;
+  const bool wanted = planes_wanted(p, s);
+  if (!wanted && !p->pv_planes_held) return 0;
   const long planes = long(p->batch) * p->n[0];
   if (!p->pv_planes) {
     if (hipMalloc(&p->pv_planes, size_t(2 * planes) * sizeof(int)) != hipSuccess) {
@@ -366,7 +375,7 @@ int share_planes(wfs_plan* p, hipStream_t s) {
   }
   WFS_TRY(launch_plane_dedup(p->pv_lines, long(p->n[1]) * p->n[2] * long(p->elem / 8), p->n[0], p->batch, 0, planes,
                              p->pv_planes + planes, p->pv_planes, s));
-  p->pv_planes_ok = true;
+  p->pv_planes_ok = wanted;
   return 0;
 }
 
@@ -382,7 +391,7 @@ int set_potential(wfs_plan* p, const void* V, hipStream_t s, bool share = true) 
     p->pv_nat_ok = false;
     if (capturing(s)) p->pv_in_graph = true;
     p->pv_planes_ok = false;
-    if (share) WFS_TRY(share_planes(p, s));
+    if (share || p->pv_planes_held) WFS_TRY(share_planes(p, s));
   } else {
     WFS_TRY(alloc_table(p, &p->pv, s));
     WFS_TRY(launch_potential_phase(p->precision, count, static_cast<const float2*>(V), p->dt, p->pv, s));
@@ -440,8 +449,11 @@ int current_table(wfs_plan* p, hipStream_t s, const void** out, bool share = tru
       p->pv_lines_ok = !capturing(s);
       p->pv_planes_ok = false;
       if (capturing(s)) p->pv_in_graph = true;
+      if (p->pv_planes_held) WFS_TRY(share_planes(p, s));
     }
-    if (share && !p->pv_planes_ok && p->variant[WFS_K_PV_PLANES] != 0) WFS_TRY(share_planes(p, s));
+    if (share && !p->pv_planes_ok && planes_wanted(p, s)) WFS_TRY(share_planes(p, s));
+    if (!p->pv_planes_held && p->pv_planes_ok && p->variant[WFS_K_PV_PLANES] != 0)
+      p->pv_planes_held = capturing(s);
     *out = p->pv_lines;
   } else {
     if (!p->pv_nat_ok) {
@@ -623,7 +635,8 @@ int observe(wfs_plan* p, const void* psi, const wfs_box* boxes, int nboxes, doub
 int fourier_steps(wfs_plan* p, void* psi, const void* V, int nsteps, hipStream_t s) {
   // The map of repeated planes costs two launches that read the table twice (256^3 37 us, 96 x 192 x 128 13)
   // and saves a step up to the table's read (256^3 6 us, 96 x 192 x 128 2): a call that brings its potential
-  // for a few steps leaves it to the next call that steps on the same table.  The bits are the same.
+  // for a few steps leaves it to the next call that steps on the same table (set_potential: unless a graph
+  // reads the map).  The bits are the same.
   constexpr int kShareSteps = 8;
   const bool share = !V || nsteps >= kShareSteps;
   if (V) WFS_TRY(set_potential(p, V, s, share));
