@@ -453,9 +453,13 @@ class FNO3d:
         return {"flops": flops, "hbm_bytes": bytes_}
 
     def zero_grad(self) -> None:
-        self._grad_all.zero_()
+        # one launch while every gradient is still its part of the buffer; a part that the caller took out
+        # (and put another tensor in its place) is the caller's
+        own = all(self.grads.get(k) is g for k, g in self._grad_views.items())
+        if own:
+            self._grad_all.zero_()
         for k, g in self.grads.items():
-            if g is not self._grad_views.get(k):      # a tensor the caller put there
+            if not own or k not in self._grad_views:
                 g.zero_()
 
     def adam(self, lr: float = 1e-3, beta1: float = 0.9, beta2: float = 0.999, eps: float = 1e-8) -> None:
