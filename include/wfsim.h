@@ -331,7 +331,9 @@ int wfs_plan_set_profiling(wfs_plan* plan, int enable);
  * FFT tile autotuner (no reference counterpart).  Times each tile variant
  * (0, 1, 2 = half, default, double the columns per block) of every
  * split-step pass on plan-owned scratch buffers and keeps the fastest per
- * kernel class.  Variants give bit-identical results.  Synchronises stream.
+ * kernel class, then times the step in two launches (WFS_K_YZ_SLAB,
+ * WFS_K_YZ_SPLIT) against the tuned passes.  The variants of a pass give
+ * bit-identical results.  Synchronises stream.
  * WFS_K_HORNER: variant 0 runs one launch per power-series stage, 1 (default)
  * fuses up to three stages a launch (two in complex128), 2 up to two; 3 to 5
  * are as 1.  The results are bit-identical.
@@ -362,7 +364,8 @@ int wfs_plan_set_profiling(wfs_plan* plan, int enable);
  * WFS_K_X_SLAB and WFS_K_SLAB_EDGE): variant 1 (the default where supported,
  * but for complex128 64 x 64 planes beside 192 and more x planes) runs the
  * steps as the slab scheme's two launches, variant 0 as the plane pass or the
- * axis passes; the results agree to rounding.  Supported: complex128 grids with
+ * axis passes; the results agree to rounding and the autotuner keeps the
+ * faster.  Supported: complex128 grids with
  * ny = nz in {64, 96, 128, 192}, nx <= 256; complex64 grids with ny = nz = 96 or
  * 128, with ny = nz = 512 and nx >= 32, with ny = nz = 192 or 256 and nx = 512,
  * and with ny != nz in {32, 64, 96, 128, 192, 256, 512}, but for nx < 32 beside

@@ -1093,8 +1093,10 @@ extern "C" int wfs_plan_get_variant(wfs_plan* p, int kc) {
 }
 
 // Time every tile variant of each split-step pass on scratch data and keep
-// the fastest.  Variants only change how many columns a block owns, so the
-// arithmetic per point, and hence the result, is identical for all of them.
+// the fastest.  The variants of a pass only change how many columns a block
+// owns, so the arithmetic per point, and hence the result, is identical for
+// all of them.  The two launches of the slab and split schemes are timed
+// against the tuned passes (or plane pass) last; those agree to rounding.
 extern "C" int wfs_plan_autotune(wfs_plan* p, void* stream) {
   if (!p) { set_last_error("wfs_plan_autotune: null plan"); return WFS_ERR_INVALID; }
   if (p->method != WFS_METHOD_FOURIER) return 0;
@@ -1155,13 +1157,15 @@ extern "C" int wfs_plan_autotune(wfs_plan* p, void* stream) {
     }
     p->variant[WFS_K_YZ_PLANE] = rc == 0 ? best_v : keep;
   }
-  // slab scheme (two launches per step) against the tuned four axis passes
-  if (rc == 0 && slab_supported(p->precision, p->n)) {
-    const int keep = p->variant[WFS_K_YZ_SLAB];
+  // two launches per step against the tuned plane pass or axis passes
+  const bool slab = slab_supported(p->precision, p->n);
+  if (rc == 0 && (slab || split_supported(p->precision, p->n))) {
+    int& two_launches = p->variant[slab ? WFS_K_YZ_SLAB : WFS_K_YZ_SPLIT];
+    const int keep = two_launches;
     float best = 1e30f;
     int best_v = keep;
     for (int v = 0; v < 2 && rc == 0; ++v) {
-      p->variant[WFS_K_YZ_SLAB] = v;
+      two_launches = v;
       auto one_step = [&]() -> int {
         if (v) {
           WFS_TRY(run_slab_lines(p, LINES_FULL, buf, tab, s, 1));
@@ -1179,8 +1183,8 @@ extern "C" int wfs_plan_autotune(wfs_plan* p, void* stream) {
       (void)hipEventElapsedTime(&ms, a, b);
       if (rc == 0 && ms < best) { best = ms; best_v = v; }
     }
-    p->variant[WFS_K_YZ_SLAB] = rc == 0 ? best_v : keep;
-    if (rc == 0) p->variant[WFS_K_YZ_SPLIT] = 0;     // the same launches: the choice stands in WFS_K_YZ_SLAB
+    two_launches = rc == 0 ? best_v : keep;
+    if (rc == 0 && slab) p->variant[WFS_K_YZ_SPLIT] = 0;     // the same launches: the choice stands in WFS_K_YZ_SLAB
   }
   p->profiling = prof;
   (void)hipEventDestroy(a);
