@@ -190,24 +190,28 @@ int launch_rect(int mode, int b, void* data, const YzPlaneParams& p, hipStream_t
   return int(hipGetLastError());
 }
 
-bool rect_length(int n) {
-  return n == 32 || n == 64 || n == 96 || n == 128 || n == 192 || n == 256 || n == 512;
+constexpr int kSides[] = {32, 64, 96, 128, 192, 256, 512};
+
+constexpr bool rect_length(int n) {
+  for (int m : kSides)
+    if (n == m) return true;
+  return false;
 }
 
 // Residue classes of the y axis: the whole plane while it has at most 4608 points (36 KiB), else the fewest
 // that leave row groups of at most 8192 points (two or more blocks a CU), at most 8, and of at most 128 rows.
-int rect_b(int ny, int nz) {
+constexpr int rect_b(int ny, int nz) {
   if (ny <= 128 && ny * nz <= 4608) return 1;
   int b = 2;
   while (b < 8 && (ny * nz / b > 8192 || ny / b > 128)) b *= 2;
   return b;
 }
 
-// calls f with the row group's (NZ, LY) as types
+// calls f with the row group's (NZ, LY) as types; false where there is no such row group
 template <typename F>
-auto rect_dispatch(int nz, int ly, F f) -> decltype(f(std::integral_constant<int, 32>{}, std::integral_constant<int, 64>{})) {
+constexpr bool rect_dispatch(int nz, int ly, F f) {
 #define WFS_RECT(NZ, LY) \
-  if (nz == NZ && ly == LY) return f(std::integral_constant<int, NZ>{}, std::integral_constant<int, LY>{});
+  if (nz == NZ && ly == LY) { f(std::integral_constant<int, NZ>{}, std::integral_constant<int, LY>{}); return true; }
   WFS_RECT(32, 64) WFS_RECT(32, 96) WFS_RECT(32, 128)
   WFS_RECT(64, 32) WFS_RECT(64, 48) WFS_RECT(64, 64) WFS_RECT(64, 96) WFS_RECT(64, 128)
   WFS_RECT(96, 32) WFS_RECT(96, 48) WFS_RECT(96, 64)
@@ -216,8 +220,17 @@ auto rect_dispatch(int nz, int ly, F f) -> decltype(f(std::integral_constant<int
   WFS_RECT(256, 16) WFS_RECT(256, 24) WFS_RECT(256, 32) WFS_RECT(256, 64)
   WFS_RECT(512, 12) WFS_RECT(512, 16) WFS_RECT(512, 24) WFS_RECT(512, 32)
 #undef WFS_RECT
-  return {};
+  return false;
 }
+
+// every pair of sides that rect_supported takes has its row group above
+constexpr bool rect_complete() {
+  for (int ny : kSides)
+    for (int nz : kSides)
+      if (ny != nz && !rect_dispatch(nz, ny / rect_b(ny, nz), [](auto, auto) {})) return false;
+  return true;
+}
+static_assert(rect_complete(), "a pair of sides without its row group");
 
 }  // namespace
 
@@ -229,27 +242,29 @@ bool rect_supported(int precision, const int n[3]) {
 
 SlabRows rect_rows(int ny, int nz) {
   const int b = rect_b(ny, nz);
-  return rect_dispatch(nz, ny / b, [&](auto z, auto y) {
+  SlabRows g;
+  rect_dispatch(nz, ny / b, [&](auto z, auto y) {
     using S = RectShape<decltype(z)::value, decltype(y)::value>;
-    SlabRows g;
     g.b = b;
     g.uy = S::N2Y;
     g.n1y = S::N1Y;
     g.uz = S::N2Z;
     g.n1z = S::N1Z;
-    return g;
   });
+  return g;
 }
 
 int launch_yz_rect(int ny, int nz, int mode, void* data, const YzPlaneParams& p, hipStream_t s) {
   const int b = rect_b(ny, nz);
-  if (p.planes <= 0 || p.planes * b > 0x7fffffffL || !rect_length(ny) || !rect_length(nz) || ny == nz) {
+  int rc = 0;
+  if (p.planes <= 0 || p.planes * b > 0x7fffffffL || !rect_length(ny) || !rect_length(nz) || ny == nz ||
+      !rect_dispatch(nz, ny / b, [&](auto z, auto y) {
+        rc = launch_rect<decltype(z)::value, decltype(y)::value>(mode, b, data, p, s);
+      })) {
     set_last_error("two-launch y-z pass: unsupported %d x %d planes", ny, nz);
     return WFS_ERR_UNSUPPORTED;
   }
-  return rect_dispatch(nz, ny / b, [&](auto z, auto y) {
-    return launch_rect<decltype(z)::value, decltype(y)::value>(mode, b, data, p, s);
-  });
+  return rc;
 }
 
 }  // namespace wfs
