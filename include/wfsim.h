@@ -356,7 +356,7 @@ int wfs_plan_set_profiling(wfs_plan* plan, int enable);
  * (the length-ny y transform is factored differently); the slab variants
  * among themselves are bit-identical.  WFS_K_X_SLAB: variants 1 and 2 are the
  * same launch.  The autotuner keeps the faster.  WFS_K_PV_PLANES (no launches of its own): variant 1 (default)
- * lets the slab scheme's y-z launch read one copy of each run of x planes
+ * lets the two-launch steps' y-z launch read one copy of each run of x planes
  * whose potential phase factors are bitwise equal (the planes away from walls
  * and absorbing x layers), so that those reads hit the caches instead of HBM;
  * variant 0 reads every plane's own copy.  The results are bit-identical.
@@ -517,11 +517,16 @@ int wfs_narrow_c128(const void* U, void* out, long n, void* stream);
  * wfs_* call ordered on it (and on streams joined to it by events) is
  * recorded instead of executed; wfs_graph_end instantiates the graph;
  * wfs_graph_launch replays it.  Plans used inside must not allocate during
- * capture: power-series scratch is allocated by a first uncaptured wfs_step,
+ * capture: power-series scratch is allocated by a first uncaptured wfs_step
+ * (two states, and a third by a first call of two or more steps, which spares a
+ * copy a step; without it, or without the memory for it, the copy is made),
  * the potential table by a first uncaptured wfs_set_potential, a plane-current
  * workspace by a first uncaptured wfs_plane_current; a call that would allocate
- * on a capturing stream returns WFS_ERR_INVALID instead.  A graph replays the
- * table copies of its capture (wfs_plan_set_step_index).
+ * on a capturing stream returns WFS_ERR_INVALID instead.  The map of repeated
+ * planes (WFS_K_PV_PLANES) is not built under capture: wfs_set_potential, a call
+ * of 8 or more steps with V or any call without V makes it ready.  Between the
+ * replays the plan's potential may be set anew; the replays read it.  A graph
+ * replays the table copies of its capture (wfs_plan_set_step_index).
  */
 typedef struct wfs_graph wfs_graph;
 int wfs_graph_begin(void* stream, wfs_graph** out);

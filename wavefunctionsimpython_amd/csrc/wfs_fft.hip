@@ -243,7 +243,6 @@ int launch_fft_pass_t(int n, int layout, int mode, void* data, const PassParams&
   return WFS_ERR_INVALID;
 }
 
-// This file is compiled twice: WFS_FFT_PREC=0 (complex64) and 1 (complex128).
 // The entry (z, y forward) or exit (y, z inverse) transforms of whole planes in one launch, bit for bit the two
 // passes: a short call is bound by its launches (one step 7 -> 5 of them) and a long batch by the passes over
 // memory.  us of a one-step call, passes against this: 32^3 24.5 -> 19.5, 64^3 30.5 -> 27.5, 256 x 64^2 52.5 ->
@@ -278,6 +277,7 @@ int launch_yz_edge_c128(int n, bool entry, void* data, const YzPlaneParams& p, h
 }
 #endif
 
+// This file is compiled twice: WFS_FFT_PREC=0 (complex64) and 1 (complex128).
 #if WFS_FFT_PREC == 0
 template int launch_fft_pass_t<float>(int, int, int, void*, const PassParams&, long, int, hipStream_t);
 

@@ -111,9 +111,8 @@ int launch_yz_plane(int precision, int n, int halves, void* data, const YzPlaneP
 bool yz_edge_supported(int precision, int ny, int nz);
 int launch_yz_edge(int precision, int n, bool entry, void* data, const YzPlaneParams& p, hipStream_t s);
 
-// Two-launch split step for complex64 grids with ny = nz = 256 or 192 (wfs_slab.hip): the y
-// transform split in a length-ny/4 stage (on rows y = 4 a + b, with the z work) and a
-// length-4 stage (with the x pass); see there.
+// Two-launch split step (wfs_slab.hip, wfs_rect.hip): the y transform split in a length-ny/B
+// stage (on rows y = B a + b, with the z work) and a length-B stage (with the x pass); see there.
 enum {
   LINES_FULL = 0,    // y inverse, z inverse, potential phase, z forward, y forward
   LINES_ENTRY = 1,   // z forward, y forward (position space in)
@@ -131,9 +130,10 @@ struct XSlabParams {
   int ny = 0, nz = 0;
 };
 bool slab_supported(int precision, const int n[3]);
-// the same two launches under kernel class WFS_K_YZ_SPLIT: complex128 planes, complex64 96^2, 128^2 and 512^2 planes
+// the same two launches under kernel class WFS_K_YZ_SPLIT: complex128 planes of 64^2 to 192^2, complex64 planes of
+// 96^2, 128^2 and 512^2, of 192^2 and 256^2 beside 512 x planes, and what rect_supported takes
 bool split_supported(int precision, const int n[3]);
-// and for complex64 planes of unequal sides (wfs_rect.hip; the same class)
+// complex64 planes of unequal sides (wfs_rect.hip; the same class)
 bool rect_supported(int precision, const int n[3]);
 // Per x plane (packets * nx planes of plane_elems 64-bit words, contiguous per plane): src[p]
 // = the first plane of the run of bitwise-identical consecutive planes holding p, within its

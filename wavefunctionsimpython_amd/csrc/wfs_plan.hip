@@ -28,12 +28,12 @@ struct wfs_plan {
   long plane_work_len;
   double* plane_out;      // 7 doubles
   void* pv;               // potential phase table cexp_i(-dt V), state precision, C order
-  void* pv_lines;         // the same table in the slab scheme's lines order (LinesOrder)
+  void* pv_lines;         // the same table in the two-launch steps' lines order (LinesOrder)
   double* obs_lines;      // slab scheme: box moment records of an observing launch (lazy)
   long obs_lines_len;
   bool pv_nat_ok;         // pv holds the current potential
   bool pv_lines_ok;       // pv_lines holds the current potential
-  int* pv_planes;         // slab scheme: per x plane the first plane of its run of identical
+  int* pv_planes;         // two-launch steps: per x plane the first plane of its run of identical
                           // planes of pv_lines, then as many ints of workspace (lazy)
   bool pv_planes_ok;      // pv_planes describes the current pv_lines
   bool pv_in_graph;       // pv_lines was written inside a captured graph: its content changes at
@@ -335,7 +335,7 @@ int run_pass(wfs_plan* p, int axis, int mode, void* data, const void* pv, const 
 
 size_t grid_points(const wfs_plan* p) { return size_t(p->batch) * p->n[0] * p->n[1] * p->n[2]; }
 
-// steps run as two launches: the complex64 slab scheme or its complex128 counterpart
+// steps run as two launches: the slab scheme, or the same launches under WFS_K_YZ_SPLIT
 bool slab_on(const wfs_plan* p) { return p->variant[WFS_K_YZ_SLAB] != 0 || p->variant[WFS_K_YZ_SPLIT] != 0; }
 
 int alloc_table(wfs_plan* p, void** t, hipStream_t s) {
@@ -510,7 +510,6 @@ int run_yz_plane(wfs_plan* p, void* data, const void* pv, hipStream_t s, int sel
   return launch_yz_plane(p->precision, p->n[1], p->variant[WFS_K_YZ_PLANE], data, pp, s);
 }
 
-// the passes between two x passes: fused plane kernel or three axis passes
 // entry (z, y forward) or exit (y, z inverse) transforms of a call, table copy sel: with the plane pass of
 // small planes one launch, else two passes; the same bits
 int run_edge(wfs_plan* p, bool entry, void* data, hipStream_t s, int sel) {
@@ -532,6 +531,7 @@ int run_edge(wfs_plan* p, bool entry, void* data, hipStream_t s, int sel) {
   return run_pass(p, 2, MODE_INV, data, nullptr, nullptr, 1.0, s, sel);
 }
 
+// the passes between two x passes: fused plane kernel or three axis passes
 int run_yz(wfs_plan* p, void* data, const void* pv, hipStream_t s, int sel) {
   if (p->variant[WFS_K_YZ_PLANE] != 0) return run_yz_plane(p, data, pv, s, sel);
   WFS_TRY(run_pass(p, 1, MODE_INV, data, nullptr, nullptr, 1.0, s, sel - 1));
@@ -539,7 +539,7 @@ int run_yz(wfs_plan* p, void* data, const void* pv, hipStream_t s, int sel) {
   return run_pass(p, 1, MODE_FWD, data, nullptr, nullptr, 1.0, s, sel);
 }
 
-// Slab scheme (ny = nz = 256): the y-z launch of one step on rows y = 4 a + b (mode
+// Two-launch steps: the y-z launch of one step on rows y = B a + b (mode
 // LINES_FULL), or the entry (z, y forward) / exit (y, z inverse) launch of a call
 int run_slab_lines(wfs_plan* p, int mode, void* data, const void* pv, hipStream_t s, int sel) {
   YzPlaneParams pp;
@@ -567,7 +567,7 @@ int run_slab_lines(wfs_plan* p, int mode, void* data, const void* pv, hipStream_
   return launch_yz_slab(p->precision, p->n, mode, data, pp, s);
 }
 
-// Slab scheme: length-4 y stages around x forward -> K -> x inverse
+// Two-launch steps: length-B y stages around x forward -> K -> x inverse
 int run_x_slab(wfs_plan* p, void* data, const void* const* ktab, hipStream_t s, int sel) {
   XSlabParams xp;
   xp.tw_x = table_copy(p, p->tw[0], 0, sel);

@@ -1,6 +1,6 @@
 // Two-launch split step for complex64 grids with ny = nz in {96, 128, 192, 256, 512} and complex128 grids
-// with ny = nz in {64, 96, 128, 192}, nx <= 256 (512 beside 512^2 planes; gfx950).  Compiled twice: WFS_SLAB_PREC=0
-// (complex64) and 1 (complex128).
+// with ny = nz in {64, 96, 128, 192} (gfx950), nx <= 512 in complex64 and <= 256 in complex128; planes of unequal
+// sides (wfs_rect.hip) share the x launch.  Compiled twice: WFS_SLAB_PREC=0 (complex64) and 1 (complex128).
 //
 // A 256^2 y-z plane (512 KiB) or a 192^2 one (288 KiB) does not fit in one CU, so the y
 // transform is split in two stages, ny = LY * B (B = 4, LY = 64 or 48; at 128 and 96, B = 2 and
@@ -9,7 +9,8 @@
 // and each stage rides on a pass that is needed anyway:
 //
 //   yz_lines_kernel<NZ, LY, B>  (one block per x plane and residue b: the LY rows
-//     y = B a + b with all z, 128 KiB at 256, 72 KiB at 192, 66 KiB at 128):  length-LY
+//     y = B a + b with all z, 128 KiB at 256, 72 KiB at 192, 66 KiB at 128; half of it where the
+//     exchanges go in parts, 64 KiB at 256 and 136 KiB at 512):  length-LY
 //     inverse y stage over a, z inverse, potential phase, z forward, length-LY forward y stage
 //   x_rows_kernel or x_slab_kernel  (one block per packet, ka and 8 to 32 consecutive z: the B rows
 //     y = B ka + b with all x):  twiddles W_NY^{b ka} and length-B forward y stage over b,
@@ -22,7 +23,6 @@
 // in how the y transform is factored, so the results agree with theirs to float rounding, not
 // bit for bit.
 #include "wfs_yz_lines.h"
-
 
 namespace wfs {
 
@@ -436,7 +436,7 @@ int launch_lines_m(void* data, const YzPlaneParams& p, hipStream_t s) {
 // block's loads and stores run beside the other's transforms.  192^2: one 768-thread block either way, but
 // the transforms no longer wait for the factor loads hoisted over them.  Not for complex128 (128^3 27.3 ->
 // 28.6, 192^3 80.3 -> 85.6, 96^3 17.2 -> 18.3 us: its 3 and more exchanges cost what the second block
-// gains) nor for complex64 128^2 planes (19.0 -> 19.3).  512^2: the only form that fits, 131 KB of LDS and 128
+// gains) nor for complex64 128^2 planes (19.0 -> 19.3).  512^2: the only form that fits, 136 KiB of LDS and 128
 // registers a block of 1024 threads; 512^3 701 us a full launch (3.3 GB: 4.7 TB/s), 465 an entry or exit.
 template <typename R, int N> constexpr int lines_parts() { return sizeof(R) == 8 ? 0 : N == 512 ? 4 : N == 256 ? 8 : N == 192 ? 3 : 0; }
 
@@ -595,8 +595,9 @@ bool slab_supported(int precision, const int n[3]) {
 // 45 / 44, and the tuned 64^2 forms are bit for bit the axis passes.
 //
 // complex64 512^2 planes (B = 8, x_rows_kernel), us per step with a potential table against the four axis
-// passes: 512^3 2407 -> 1367, 256 x 512^2 1158 -> 798, 64 x 512^2 230 -> 182.  Its x launch takes 8 x points
-// of a lane at a time, so nx = 8 and 16 (4 points a lane) stay with the passes.
+// passes: 512^3 2407 -> 1367 (20 steps a call, entry and exit counted in; the two launches alone 1311), 256 x 512^2
+// 1158 -> 798, 64 x 512^2 230 -> 182.  Its x launch takes 8 x points of a lane at a time, so nx = 8 and 16 (4 points
+// a lane) stay with the passes.
 //
 // complex64 with 512 x planes (x_rows_kernel alone takes them): 512 x 96^2 75 / 69 -> 56 / 55, x 128^2 87 / 81 -> 81 /
 // 78, x 192^2 256 / 243 -> 218 / 200, x 256^2 450 / 374 -> 339 / 310.

@@ -103,11 +103,11 @@ __global__ __launch_bounds__(TZ* TY) void horner_stage_kernel(const cx<R>* __res
 //
 // Every fused launch moves 32 B per point (complex64), 16 at S = 2 and 10.7 at S = 3 per stage:
 // at 256^3 two stages take 112 us (4.9 TB/s, the rate of a large copy) and three 136 us, where the
-// arithmetic and the LDS reads of the halo cells bound the launch.  Keeping the centre and the
+// arithmetic and the LDS reads of the halo cells bound the launch (530 MB, 3.6 to 3.9 TB/s).  Keeping the centre and the
 // previous plane of every level in registers spilled 30 of them (290 us at S = 3).  The pair
 // kernel before this one held three planes of every level in LDS, took 111 us at 256^3 and, with
 // too few blocks on smaller grids, 49 us at 128^3 (now 20), 46 at 64^3 (7.8), and in complex128
-// 63 us at 64 x 96 x 128 (14.6) and 322 at 256^3 (185).
+// 63 us at 64 x 96 x 128 (16 to 19) and 322 at 256^3 (185 to 225).
 struct ChainArgs {
   int nx, ny, nz;
   int w;                    // window columns
@@ -352,7 +352,9 @@ static int launch_chain_form(ChainArgs g, const void* u_in, void* u_out, const v
 
 int horner_chain_stages(int precision) { return precision == WFS_C128 ? 2 : 3; }
 
-// The window by grid, measured per launch in us (the other forms beside it):
+// The window by grid, measured per launch in us, the forms of a pair of figures side by side on one box (on another
+// box, by the launches' own times: S = 3 256^3 140, 192^3 55, 128^3 26, 64^3 13, 32^3 9.7; S = 2 256^3 108, 192^3 41,
+// 128^3 19, 64^3 9.4, 64 x 64 x 512 19; complex128 256^3 225, 64 x 96 x 128 16, 32^3 6.4):
 // complex64, S = 3: columns past 64 in tiles of 64 (a wide tile has few rows, most of them halo):
 //   256^3 136 (whole rows 157, tiles of 128 143), 192^3 54 (59), 128^3 28 (26); nz <= 64 whole
 //   rows, 512 threads (64^3 11.5 against 15 with 1024) or 256 on small grids (32^3 9.0 against 10.2)

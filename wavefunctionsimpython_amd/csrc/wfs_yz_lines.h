@@ -186,7 +186,7 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lin
   using L = std::conditional_t<PARTS != 0, R, C>;
   __shared__ L lds[RH * TS];
 
-  static_assert(!PARTS || H == 1, "parts: one round");
+  static_assert(!PARTS || (H == 1 && PV_LINES), "parts: one round, the table in lines order");
   const int tid = threadIdx.x;
   const long group = blockIdx.x;
   const long plane = group / B;                    // x plane, counted over all packets
@@ -449,7 +449,6 @@ __attribute__((amdgpu_waves_per_eu(PARTS ? PARTS : H == 1 ? 1 : 4))) void yz_lin
           for (int i = 0; i < N1; ++i) {
             a[r][i] = cmul(a[r][i], pvb[unsigned(c0 + r * RH) * RS + unsigned(u + N2Z * i)]);
             if (H > 1 && i % 4 == 3) asm volatile("" ::: "memory");
-            if (PARTS && i % 4 == 3) settle(a[r][i]);
           }
         }
         load_wz(p.tw_z, u);
