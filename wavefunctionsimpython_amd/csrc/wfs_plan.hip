@@ -470,11 +470,14 @@ int current_table(wfs_plan* p, hipStream_t s, const void** out, bool share = tru
 // reduced mod 2 pi; dithered copies for complex64 plans)
 int set_potential_axes(wfs_plan* p, const double* const f[3]) {
   const long double two_pi = 2.0L * 3.14159265358979323846264338327950288L;
+  // a refused potential leaves the one in force
+  for (int a = 0; a < 3; ++a)
+    for (long j = 0; j < long(p->batch) * p->n[a]; ++j)
+      if (!std::isfinite(f[a][j])) { set_last_error("wfs_set_potential_axes: non-finite potential"); return WFS_ERR_INVALID; }
   for (int a = 0; a < 3; ++a) {
     const long len = long(p->batch) * p->n[a];
     std::vector<double> re(len), im(len);
     for (long j = 0; j < len; ++j) {
-      if (!std::isfinite(f[a][j])) { set_last_error("wfs_set_potential_axes: non-finite potential"); return WFS_ERR_INVALID; }
       long double th = -(long double)p->dt * (long double)f[a][j];
       th = fmodl(th, two_pi);
       re[j] = double(cosl(th));
