@@ -46,3 +46,28 @@ def test_refused_axes_leave_the_potential(dev, shape, precision, axis):
         p.step(out[-1], None, 2)
     torch.cuda.synchronize()
     assert torch.equal(*out)
+
+
+@pytest.mark.parametrize("shape,precision", GRIDS)
+def test_replay_reads_axes_set_after_its_capture(dev, shape, precision):
+    start = _state(shape, precision, dev)
+    p = _plan(shape, precision)
+    p.set_potential_axes(*_axes(shape, 1))
+    psi = start.clone()
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with _abi.Graph(s) as graph:
+        p.step(psi, None, 2, stream=s)
+    for seed in (1, 2, 3, 1):
+        axes = _axes(shape, seed)
+        p.set_potential_axes(*axes)
+        psi.copy_(start)
+        torch.cuda.synchronize()
+        graph.launch()
+        s.synchronize()
+        q = _plan(shape, precision)                    # the table copies of a first call, as in the capture
+        q.set_potential_axes(*axes)
+        want = start.clone()
+        q.step(want, None, 2)
+        torch.cuda.synchronize()
+        assert torch.equal(psi, want), seed

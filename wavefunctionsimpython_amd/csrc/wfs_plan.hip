@@ -80,9 +80,10 @@ namespace {
 // numpy.fft.fftfreq index -> signed frequency index
 long freq_index(long j, long n) { return (j <= (n - 1) / 2) ? j : j - n; }
 
+// host -> *dst, allocated where it is null; a table uploaded again (the same size) keeps its address
 int upload(void** dst, const void* host, size_t bytes) {
-  hipError_t e = hipMalloc(dst, bytes);
-  if (e != hipSuccess) { set_last_error("hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e)); return WFS_ERR_ALLOC; }
+  hipError_t e = *dst ? hipSuccess : hipMalloc(dst, bytes);
+  if (e != hipSuccess) { *dst = nullptr; set_last_error("hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e)); return WFS_ERR_ALLOC; }
   e = hipMemcpy(*dst, host, bytes, hipMemcpyHostToDevice);
   if (e != hipSuccess) { set_last_error("hipMemcpy failed: %s", hipGetErrorString(e)); return int(e); }
   return 0;
@@ -474,6 +475,9 @@ int set_potential_axes(wfs_plan* p, const double* const f[3]) {
   for (int a = 0; a < 3; ++a)
     for (long j = 0; j < long(p->batch) * p->n[a]; ++j)
       if (!std::isfinite(f[a][j])) { set_last_error("wfs_set_potential_axes: non-finite potential"); return WFS_ERR_INVALID; }
+  // The tables stay where they are, since a captured graph has their addresses among its launches' arguments;
+  // steps that still read them end first.
+  if (p->sep[0]) WFS_HIP_CHECK(hipDeviceSynchronize());
   for (int a = 0; a < 3; ++a) {
     const long len = long(p->batch) * p->n[a];
     std::vector<double> re(len), im(len);
@@ -483,7 +487,6 @@ int set_potential_axes(wfs_plan* p, const double* const f[3]) {
       re[j] = double(cosl(th));
       im[j] = double(sinl(th));
     }
-    if (p->sep[a]) { (void)hipFree(p->sep[a]); p->sep[a] = nullptr; }
     WFS_TRY(upload_dithered(&p->sep[a], re, im, p->precision));
   }
   p->sep_set = true;
