@@ -26,6 +26,8 @@ struct wfs_plan {
   long obs_work_len;
   double* plane_work;     // plane-current partial records (grown on demand)
   long plane_work_len;
+  bool plane_work_held;   // a captured launch took plane_work: it outlives a larger one
+  std::vector<double*>* plane_work_kept;
   double* plane_out;      // 7 doubles
   void* pv;               // potential phase table cexp_i(-dt V), state precision, C order
   void* pv_lines;         // the same table in the two-launch steps' lines order (LinesOrder)
@@ -758,6 +760,9 @@ extern "C" int wfs_plan_destroy(wfs_plan* p) {
   if (p->state2) (void)hipFree(p->state2);
   if (p->obs_work) (void)hipFree(p->obs_work);
   if (p->plane_work) (void)hipFree(p->plane_work);
+  if (p->plane_work_kept)
+    for (double* w : *p->plane_work_kept) (void)hipFree(w);
+  delete p->plane_work_kept;
   if (p->plane_out) (void)hipFree(p->plane_out);
   if (p->pv) (void)hipFree(p->pv);
   if (p->pv_lines) (void)hipFree(p->pv_lines);
@@ -824,6 +829,7 @@ extern "C" int wfs_plan_create_batched(const int n[3], const double dx[3], doubl
   p->variant[WFS_K_YZ_SPLIT] = !slab && split_supported(precision, n) && (n[1] != n[2] || n[1] != 64 || n[0] < 192) ? 1 : 0;
   p->pending = new std::vector<std::pair<hipEvent_t, hipEvent_t>>[WFS_K_COUNT];
   p->event_pool = new std::vector<hipEvent_t>();
+  p->plane_work_kept = new std::vector<double*>();
   int rc = 0;
   for (int a = 0; a < 3 && rc == 0; ++a) {
     std::vector<double> re(n[a]), im(n[a]);
@@ -1258,10 +1264,19 @@ extern "C" int wfs_plane_current(wfs_plan* p, const void* psi, const double cent
   if (need > p->plane_work_len) {
     // grown on demand: the pixel count is known only here
     WFS_TRY(refuse_if_capturing(s, "wfs_plane_current"));
-    if (p->plane_work) { WFS_HIP_CHECK(hipStreamSynchronize(s)); (void)hipFree(p->plane_work); p->plane_work = nullptr; }
-    WFS_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&p->plane_work), size_t(need) * sizeof(double)));
+    double* work = nullptr;
+    WFS_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&work), size_t(need) * sizeof(double)));
+    if (p->plane_work_held) {
+      p->plane_work_kept->push_back(p->plane_work);
+      p->plane_work_held = false;
+    } else if (p->plane_work) {
+      (void)hipStreamSynchronize(s);
+      (void)hipFree(p->plane_work);
+    }
+    p->plane_work = work;
     p->plane_work_len = need;
   }
+  if (!p->plane_work_held) p->plane_work_held = capturing(s);
   ProfileScope scope(p, WFS_K_OBSERVABLES, s);
   WFS_TRY(launch_plane_current(p->precision, p->n[0], p->n[1], p->n[2], p->dx, psi, center, normal, size, count,
                                p->mass, density, p->plane_work, p->plane_work_len, p->plane_out, s));
