@@ -525,8 +525,10 @@ int wfs_narrow_c128(const void* U, void* out, long n, void* stream);
  * on a capturing stream returns WFS_ERR_INVALID instead.  The map of repeated
  * planes (WFS_K_PV_PLANES) is not built under capture: wfs_set_potential, a call
  * of 8 or more steps with V or any call without V makes it ready.  Between the
- * replays the plan's potential may be set anew; the replays read it.  A graph
- * replays the table copies of its capture (wfs_plan_set_step_index).
+ * replays the plan's potential may be set anew, and the replays read it: a table
+ * where the graph was captured with a table, per-axis factors where with those,
+ * in the variants of the capture.  A graph replays the table copies of its
+ * capture (wfs_plan_set_step_index).
  */
 typedef struct wfs_graph wfs_graph;
 int wfs_graph_begin(void* stream, wfs_graph** out);
